@@ -90,7 +90,7 @@ struct bh_ctx_s {
     // flagged list and groups, per-block sums of M^2
     double rc_kappa = 1.5;
     int rc_deferred = 0;
-    int rc_ready = 0;        // the last force pass prepared a32 / s2n
+    int rc_ready = 0;        // 1: the last force pass prepared a32 / s2n; 2: it left nothing to recompute
     double* rc_a32 = nullptr;      // the FP32 pass: x plane, y plane, near-field sums
     int32_t* rc_list = nullptr;    // flagged particles, system s at [p_off_s, p_off_s + cnt_s)
     int32_t* rc_cnt = nullptr;     // per system
@@ -100,6 +100,11 @@ struct bh_ctx_s {
     double* rc_blk = nullptr;      // per block: sum of M^2
     double* rc_bfar = nullptr;     // per block: its far-block part of the bound
     int64_t nblocks = 0;
+    // grouped far field (bh_fmm.hip): which passes take it is a rule on the
+    // systems' sizes (fmm_wanted)
+    bool fmm_on = false;
+    FmmPlan fmm;
+    FmmArgs fa = {};         // device buffers and sizes; the per-pass fields are set by each pass
     hipStream_t cap_stream = nullptr;   // graph capture only; replays run on the caller's stream
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     GraphKey gkey[2];
@@ -197,6 +202,158 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
     c->max_items = C + cols + 2 * cdiv(N, 64) + 64;
 }
 
+// Far terms of a pass (at most N x cells) from which the grouped far field
+// (bh_fmm.hip) is used, by passes of the fp64 and fp32 precisions.  At the
+// line a term-by-term pass takes ~5 ms in FP32 and ~9 ms in FP64 and the
+// grouped one 1.1 and 2.4 ms (600,001 uniform particles, 193^2 cells: 2.2e10
+// terms); the two meet near 3e9 terms.  The line is above that because short
+// passes over many uneven systems are where a learned queue order shortens
+// the term-by-term pass, and because the allocation-free step (at most 1.7e10
+// terms) has no scratch for the squares and gives the bits of bh_step.
+static constexpr double FMM_MIN_TERMS = 2e10;
+static constexpr size_t FMM_MAX_BYTES = (size_t)48 << 30;
+
+static bool fmm_wanted(const std::vector<SysDev>& sh)
+{
+    double terms = 0.0, tiles = 0.0;
+    int64_t side = 0;
+    for (const SysDev& d : sh) {
+        if (d.G < FMM_MIN_GRID) continue;
+        terms += (double)d.n * std::min((double)d.n, (double)d.G * d.G);
+        const double n0 = (double)cdiv(d.G, FMM_TILE);
+        tiles += n0 * n0 * (4.0 / 3.0);
+        side = std::max(side, cdiv(d.G, FMM_TILE));
+    }
+    // a nearly empty huge grid has more squares to serve than terms to save
+    return terms >= FMM_MIN_TERMS && terms >= 1e6 * tiles &&
+           tiles * 3.0 * FMM_P64 * FMM_P64 * sizeof(double) <= (double)FMM_MAX_BYTES &&
+           side <= 1024;   // a level's node masses are addressed with 32 bits
+}
+
+// Chebyshev nodes, transform and parent-child interpolation for P nodes.
+static std::vector<double> fmm_table(int P)
+{
+    std::vector<double> v(P + 3 * P * P);
+    double *nodes = v.data(), *cheb = nodes + P, *shift = cheb + P * P;
+    const long double pi = 3.14159265358979323846264338327950288L;
+    auto T = [&](int k, long double u) { return cosl(k * acosl(u)); };
+    std::vector<long double> x(P);
+    for (int i = 0; i < P; ++i) {
+        x[i] = cosl((2 * i + 1) * pi / (2 * P));
+        nodes[i] = (double)x[i];
+    }
+    for (int k = 0; k < P; ++k)
+        for (int i = 0; i < P; ++i) cheb[k * P + i] = (double)((k ? 2.0L : 1.0L) / P * T(k, x[i]));
+    for (int a = 0; a < 2; ++a)
+        for (int i = 0; i < P; ++i)
+            for (int I = 0; I < P; ++I) {
+                const long double u = 0.5L * x[I] + (a ? 0.5L : -0.5L);
+                long double c = 0.0L;
+                for (int k = 0; k < P; ++k) c += (k ? 2.0L : 1.0L) / P * T(k, x[i]) * T(k, u);
+                shift[(a * P + i) * P + I] = (double)c;
+            }
+    return v;
+}
+
+// Lays out the squares of every system and allocates the grouped far field's
+// buffers (c->sys_h and the sizes are set).
+static int fmm_configure(Ctx* c)
+{
+    c->fmm_on = false;
+    if (!fmm_wanted(c->sys_h)) return BH_OK;
+    const int S = c->S;
+    std::vector<FmmSys> fs(S);
+    int nlev = 0;
+    for (int s = 0; s < S; ++s) {
+        const int G = c->sys_h[s].G;
+        FmmSys& f = fs[s];
+        std::memset(&f, 0, sizeof(f));
+        f.T = G < FMM_MIN_GRID ? G : FMM_TILE;
+        f.n[0] = (int32_t)cdiv(G, f.T);
+        f.nlev = f.n[0] > 1 ? 1 : 0;
+        while (f.nlev && f.n[f.nlev - 1] > 4) {
+            f.n[f.nlev] = (f.n[f.nlev - 1] + 1) / 2;
+            ++f.nlev;
+        }
+        nlev = std::max(nlev, std::max(f.nlev, 1));
+    }
+    FmmArgs& a = c->fa;
+    a = FmmArgs{};
+    std::vector<FmmTile> tiles;
+    std::vector<FmmGroup> groups;
+    int64_t slots = 0;
+    for (int l = 0; l < nlev; ++l) {
+        a.lev_off[l] = (int64_t)tiles.size();
+        for (int s = 0; s < S; ++s) {
+            FmmSys& f = fs[s];
+            if (l >= std::max(f.nlev, 1)) continue;
+            f.off[l] = (int32_t)tiles.size();
+            const int n = f.n[l];
+            for (int x = 0; x < n; ++x)
+                for (int y = 0; y < n; ++y) tiles.push_back({s, (int16_t)x, (int16_t)y});
+            if (f.nlev == 0) continue;
+            f.moff[l] = slots;
+            slots += fmm_plane(n);
+            for (int p = 0; p < 4; ++p) {
+                const int ga = p >> 1, gb = p & 1;
+                const int cnt = ((n - ga + 1) / 2) * ((n - gb + 1) / 2);
+                for (int t0 = 0; t0 < cnt; t0 += 64)
+                    groups.push_back({s, t0, (int16_t)l, (int8_t)ga, (int8_t)gb});
+            }
+        }
+    }
+    for (int l = nlev; l <= FMM_LEVELS; ++l) a.lev_off[l] = (int64_t)tiles.size();
+    a.S = S;
+    a.N = c->N;
+    a.nleaf = a.lev_off[1];
+    a.ntiles = (int64_t)tiles.size();
+    a.max_chunks = cdiv(c->N, 64) + a.nleaf;
+    c->fmm.nlev = nlev;
+    c->fmm.ngroups = (int64_t)groups.size();
+    const std::vector<double> tab[2] = {fmm_table(FMM_P32), fmm_table(FMM_P64)};
+    const int P[2] = {FMM_P32, FMM_P64};
+    FmmSys* dfs = nullptr;
+    FmmTile* dt = nullptr;
+    FmmGroup* dg = nullptr;
+    int r;
+    for (int i = 0; i < 2; ++i) {
+        double* d = nullptr;
+        if ((r = dalloc(c, &d, (int64_t)tab[i].size()))) return r;
+        HIP_TRY(hipMemcpy(d, tab[i].data(), tab[i].size() * sizeof(double), hipMemcpyHostToDevice));
+        c->fmm.tab[i].nodes = d;
+        c->fmm.tab[i].cheb = d + P[i];
+        c->fmm.tab[i].shift = d + P[i] + P[i] * P[i];
+    }
+    const int64_t Q = FMM_P64 * FMM_P64;
+    if ((r = dalloc(c, &dfs, S)) || (r = dalloc(c, &dt, a.ntiles)) ||
+        (r = dalloc(c, &dg, (int64_t)groups.size())) || (r = dalloc(c, &a.tcnt, a.ntiles)) ||
+        (r = dalloc(c, &a.tstart, a.nleaf)) || (r = dalloc(c, &a.tne, a.nleaf)) ||
+        (r = dalloc(c, &a.cnt, 2 + S)) || (r = dalloc(c, &a.chunks, a.max_chunks)) ||
+        (r = dalloc(c, &a.list, c->C + 4 * a.nleaf)) || (r = dalloc(c, &a.pack, c->N)) ||
+        (r = dalloc(c, &a.loc, a.ntiles * 2 * Q)))
+        return r;
+    for (int i = 0; i < 2; ++i) {   // the borders stay zero
+        const int64_t cnt = slots * P[i] * P[i];
+        if ((r = dalloc(c, &c->fmm.mult[i], cnt))) return r;
+        HIP_TRY(hipMemset(c->fmm.mult[i], 0, sizeof(double) * cnt));
+    }
+    HIP_TRY(hipMemcpy(dfs, fs.data(), sizeof(FmmSys) * S, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dt, tiles.data(), sizeof(FmmTile) * tiles.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dg, groups.data(), sizeof(FmmGroup) * groups.size(), hipMemcpyHostToDevice));
+    a.sbad = a.cnt + 2;
+    a.fsys = dfs;
+    a.tiles = dt;
+    a.groups = dg;
+    a.sys = c->sys;
+    a.sys_of = c->sys_of;
+    a.offsets = c->offsets;
+    a.neprefix = c->neprefix;
+    a.key_sorted = c->key_sorted;
+    a.l64 = c->l64;
+    c->fmm_on = true;
+    return BH_OK;
+}
+
 // Every device buffer of a configured context with its element count, for the
 // sizes set by set_sizes.  bh_set_systems gives each buffer its own
 // allocation; the allocation-free step carves them out of one static array.
@@ -262,6 +419,7 @@ static void unconfigure(Ctx* c)
     c->sys_h.clear();
     c->energy_buf = nullptr;
     c->rc_ready = 0;
+    c->fmm_on = false;
 }
 
 // Allocates and initialises the buffers for sizes already validated by
@@ -280,6 +438,7 @@ static int configure(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, i
     HIP_TRY(hipMemset(c->stats, 0, sizeof(int32_t) * ST_COUNT));
     HIP_TRY(hipMemset(c->offsets, 0, sizeof(int32_t) * (C + 1)));
     HIP_TRY(hipMemset(c->neprefix, 0, sizeof(int32_t) * (C + 1)));
+    if ((r = fmm_configure(c)) != BH_OK) return r;
     HIP_TRY(hipDeviceSynchronize());
     return BH_OK;
 }
@@ -645,6 +804,28 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     const void* fn = bh_force_kernel(precision, pidx, lawi);
     if (!fn) return fail(BH_EINVAL, "no force kernel for this configuration");
     ForceArgs fa;
+    if (c->fmm_on && (precision == 0 || precision == 1) && !c->cost_log_on) {
+        // Grouped far field: its chunks replace the work items, so the queue
+        // order does not enter.  Near and mid terms are FP64 in both
+        // precisions: nothing is left for the recompute to mend.
+        FmmArgs A = c->fa;
+        A.x = p->px;
+        A.y = p->py;
+        A.m = p->mass;
+        A.ax = p->ax;
+        A.ay = p->ay;
+        const bool rc = precision == 1 && c->rc_kappa > 0.0;
+        if (part == 0) c->rc_ready = 0;
+        bh_fmm_pass(A, c->fmm, precision == 0, law->G, law->eps2, law->r2_cut, part, nparts,
+                    c->num_cu, st);
+        if (part == nparts - 1) {
+            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
+                               (int64_t)2, 0);
+            c->rc_ready = rc ? 2 : 0;
+        }
+        LAUNCH_CHECK("evaluate");
+        return BH_OK;
+    }
     fa.items = c->items;
     fa.order = order;
     fa.stats = c->stats;
@@ -726,6 +907,7 @@ int bh_recompute(void* ctx, const bh_particles* p, const bh_law* law, void* stre
     if (!(law->eps2 >= 0.0) || !(law->r2_cut >= 0.0) || !std::isfinite(law->G))
         return fail(BH_EINVAL, "law needs finite G, eps2 >= 0, r2_cut >= 0");
     if (!c->rc_ready) return fail(BH_ESTATE, "no FP32 force pass prepared a recompute");
+    if (c->rc_ready == 2) return BH_OK;   // the pass formed its sums in FP64: nothing flagged
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP, (int64_t)2, 0);
     if (law->G == 0.0) return BH_OK;   // every term, and so the FP32 result, is zero

@@ -1,0 +1,810 @@
+// Grouped far field: the same sums as the term-by-term force kernels, with
+// the COMs of distant cells taken in groups.
+//
+// A system's grid is covered by square tiles of FMM_TILE cells per side.  A
+// particle's terms split into
+//   near     the particles of its 3x3 cells, one by one;
+//   mid      the COMs of the other non-empty cells of its 3x3 tiles, one by one;
+//   distant  the COMs of all other cells, at least FMM_TILE cells away.
+// The law's weight 1 / (r^2 + eps2) is smooth over the distant part (softening
+// only makes it smoother), so that part is interpolated: on each tile, and on
+// each square of 2^l tiles per side, a P x P Chebyshev grid carries the
+// sources up (anterpolated masses at the nodes) and the field down (ax, ay at
+// the nodes).  Two squares interact directly (the law between their nodes) at
+// the coarsest level where they are not neighbours while their parents are.
+// Interpolating across a gap of one square converges as 5.8^-P: P = 12 leaves
+// 1.3e-10 of the far field (the FP32 precision's own rounding was 4e-8), and
+// P = 20 leaves 1e-15, below the rounding of a term-by-term FP64 sum over
+// 10^4 cells and more.  Everything here is FP64.
+//
+// Work per pass: 27 node-to-node products of (2 P^2) x P^2 per square instead
+// of one term per (particle, cell): 4.2M particles on 1024^2 cells go from
+// 2.0e12 far terms to ~4e9 terms and ~4.4e5 products.
+#include "bh_common.h"
+#include "bh_kernels.h"
+
+#define FMM_IN 1.0001   // |coordinate| on a square up to which it counts as inside
+
+typedef double fd4 __attribute__((ext_vector_type(4)));
+typedef double fd2 __attribute__((ext_vector_type(2)));
+
+// Wave-uniform reads through the constant address space: scalar loads, so
+// every lane gets the value from a scalar register.
+template <typename T>
+using cptr = const T __attribute__((address_space(4)))*;
+
+template <typename T>
+__device__ __forceinline__ cptr<T> as_const(const T* p)
+{
+    return (cptr<T>)(uintptr_t)p;
+}
+
+// The power of two that brings the cell side into [1, 2): positions scaled by
+// it are exact, and a distance to another cell's COM is at least 1.
+__device__ __forceinline__ double step_scale(double step)
+{
+    if (!(step > 0.0) || !(step < __builtin_huge_val())) return 1.0;
+    int e2;
+    (void)frexp(step, &e2);
+    return ldexp(1.0, 1 - e2);
+}
+
+__device__ __forceinline__ double rcp64(double q)
+{
+    const double r0 = __builtin_amdgcn_rcp(q);
+    const double e = fma(-q, r0, 1.0);
+    return fma(r0, fma(e, e, e), r0);
+}
+
+// ---------------------------------------------------------------- tiles
+// Eight lanes per tile add up its columns' particles and non-empty cells; the
+// block reserves a run of the chunk list (64 particles of one tile each) and
+// of the tile-ordered COM list with one atomic.  The order of the runs varies
+// from launch to launch; no result depends on it.
+__global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
+{
+    __shared__ int wc[4], we[4], base_c, base_e;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int64_t t = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
+    const int sub = threadIdx.x & 7;
+    int np = 0, ne = 0;
+    FmmTile tl = {0, 0, 0};
+    if (t < A.nleaf) {
+        tl = A.tiles[t];
+        const SysDev& d = A.sys[tl.sys];
+        const int T = A.fsys[tl.sys].T;
+        const int x0 = tl.tx * T, y0 = tl.ty * T;
+        const int x1 = min(x0 + T, d.G), y1 = min(y0 + T, d.G);
+        for (int x = x0 + sub; x < x1; x += 8) {
+            const int64_t cl = d.c_off + (int64_t)x * d.G;
+            np += A.offsets[cl + y1] - A.offsets[cl + y0];
+            ne += A.neprefix[cl + y1] - A.neprefix[cl + y0];
+        }
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        np += __shfl_xor(np, o, BH_WAVE);
+        ne += __shfl_xor(ne, o, BH_WAVE);
+    }
+    const int nc = (np + 63) >> 6;
+    const int ner = (ne + 3) & ~3;   // a tile's run of the list is padded to whole quads
+    // exclusive prefix over the wave's eight tiles
+    int pc = nc, pe = ner;
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) {
+        const int a = __shfl_up(pc, o, BH_WAVE), b = __shfl_up(pe, o, BH_WAVE);
+        if (lane >= o) {
+            pc += a;
+            pe += b;
+        }
+    }
+    if (lane == 63) {
+        wc[wid] = pc;
+        we[wid] = pe;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int c = 0, e = 0;
+        for (int w = 0; w < 4; ++w) {
+            const int a = wc[w], b = we[w];
+            wc[w] = c;
+            we[w] = e;
+            c += a;
+            e += b;
+        }
+        base_c = c ? atomicAdd(&A.cnt[0], c) : 0;
+        base_e = e ? atomicAdd(&A.cnt[1], e) : 0;
+    }
+    __syncthreads();
+    if (t >= A.nleaf) return;
+    const int c0 = base_c + wc[wid] + pc - nc, e0 = base_e + we[wid] + pe - ner;
+    if (sub == 0) {
+        A.tcnt[t] = np;
+        A.tstart[t] = e0;
+        A.tne[t] = ne;
+    }
+    for (int k = sub; k < nc; k += 8) {
+        FmmChunk c;
+        c.tile = (int32_t)t;
+        c.k = k;
+        A.chunks[c0 + k] = c;
+    }
+}
+
+// ---------------------------------------------------------------- sources up
+// One block per tile: the tile's COMs into the tile-ordered list, and their
+// masses anterpolated to the tile's nodes: Chebyshev moments
+// W_kl = sum M T_k(x) T_l(y) over the entries, then nodes = C^T W C.
+template <int P>
+__global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __restrict__ ctab)
+{
+    constexpr int Q = P * P;
+    constexpr int PER = (Q + 255) / 256;
+    __shared__ double tx[32][P], ty[32][P], mm[32], W[Q], V[Q], ct[Q];
+    const int tid = threadIdx.x;
+    const int64_t t = blockIdx.x;
+    const FmmTile tl = A.tiles[t];
+    const SysDev& d = A.sys[tl.sys];
+    const FmmSys& fs = A.fsys[tl.sys];
+    const int T = fs.T, ne = A.tne[t], e0 = A.tstart[t];
+    const int x0 = tl.tx * T, y0 = tl.ty * T;
+    const int x1 = min(x0 + T, d.G), y1 = min(y0 + T, d.G);
+    const double sig = step_scale(d.step);
+    double* M = nullptr;   // node q's mass goes to M[q * plane]
+    int64_t plane = 0;
+    if (fs.nlev > 0) {
+        plane = fmm_plane(fs.n[0]);
+        M = A.mult + fs.moff[0] * Q + fmm_slot(fs.n[0], tl.tx, tl.ty);
+    }
+    const bool up = fs.nlev > 0;
+    for (int i = tid; i < Q; i += 256) ct[i] = ctab[i];
+    double acc[PER] = {};
+    const double h = (double)T * d.step;
+    int cx = x0, cb = A.neprefix[d.c_off + (int64_t)x0 * d.G + y0];
+    int cn = A.neprefix[d.c_off + (int64_t)x0 * d.G + y1] - cb, cpre = 0;
+    for (int b = 0; b < ne; b += 32) {
+        const int nb = min(32, ne - b);
+        if (tid < nb) {
+            const int r = b + tid;   // entry rank in the tile, columns in order
+            while (r - cpre >= cn && cx + 1 < x1) {
+                cpre += cn;
+                ++cx;
+                const int64_t cl = d.c_off + (int64_t)cx * d.G;
+                cb = A.neprefix[cl + y0];
+                cn = A.neprefix[cl + y1] - cb;
+            }
+            const Com64 c = A.l64[cb + (r - cpre)];
+            FmmCom f;
+            f.X = c.X * sig;
+            f.Y = c.Y * sig;
+            f.M = c.M;
+            f.kx = c.kx;
+            f.ky = c.ky;
+            if (c.M == 0.0) {   // no COM: any point of the cell, at weight 0
+                f.X = fma((double)c.kx + 0.5, d.step, d.min_x) * sig;
+                f.Y = fma((double)c.ky + 0.5, d.step, d.min_y) * sig;
+            }
+            A.list[e0 + r] = f;
+            if (up) {
+                const double ux = 2.0 * ((c.X - d.min_x) / h - tl.tx) - 1.0;
+                const double uy = 2.0 * ((c.Y - d.min_y) / h - tl.ty) - 1.0;
+                // masses of both signs can put a COM outside its cell, where
+                // the interpolation does not hold: that system goes term by term
+                if (c.M != 0.0 && !(fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN)) A.sbad[tl.sys] = 1;
+                mm[tid] = c.M;
+                double a0 = 1.0, a1 = ux, b0 = 1.0, b1 = uy;
+                if (c.M == 0.0) a0 = a1 = b0 = b1 = 0.0;
+#pragma unroll
+                for (int k = 0; k < P; ++k) {
+                    tx[tid][k] = a0;
+                    ty[tid][k] = b0;
+                    const double an = fma(2.0 * ux, a1, -a0), bn = fma(2.0 * uy, b1, -b0);
+                    a0 = a1;
+                    a1 = c.M == 0.0 ? 0.0 : an;
+                    b0 = b1;
+                    b1 = c.M == 0.0 ? 0.0 : bn;
+                }
+            }
+        }
+        __syncthreads();
+        if (up) {
+#pragma unroll
+            for (int p = 0; p < PER; ++p) {
+                const int q = tid + 256 * p;
+                if (q < Q) {
+                    const int k = q / P, l = q - (q / P) * P;
+                    for (int e = 0; e < nb; ++e) acc[p] = fma(mm[e] * tx[e][k], ty[e][l], acc[p]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (tid < (-ne & 3)) {   // padding: no mass, far from everything
+        FmmCom f;
+        f.X = 1e60;
+        f.Y = 1e60;
+        f.M = 0.0;
+        f.kx = -100000;
+        f.ky = -100000;
+        A.list[e0 + ne + tid] = f;
+    }
+    if (!up) return;
+    if (ne == 0) {   // uniform over the block
+        for (int q = tid; q < Q; q += 256) M[q * plane] = 0.0;
+        return;
+    }
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+        if (tid + 256 * p < Q) W[tid + 256 * p] = acc[p];
+    __syncthreads();
+    for (int q = tid; q < Q; q += 256) {   // V[i][l] = sum_k ct[k][i] W[k][l]
+        const int i = q / P, l = q - i * P;
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < P; ++k) s = fma(ct[k * P + i], W[k * P + l], s);
+        V[q] = s;
+    }
+    __syncthreads();
+    for (int q = tid; q < Q; q += 256) {
+        const int i = q / P, j = q - i * P;
+        double s = 0.0;
+#pragma unroll
+        for (int l = 0; l < P; ++l) s = fma(V[i * P + l], ct[l * P + j], s);
+        M[q * plane] = s;
+    }
+}
+
+// One block per square of level lev: its children's node masses anterpolated
+// to its own nodes (shift[a][i][I]: the parent's cardinal i at child node I).
+template <int P>
+__global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __restrict__ shift,
+                                                 int lev)
+{
+    constexpr int Q = P * P;
+    constexpr int PER = (Q + 255) / 256;
+    __shared__ double S[2 * Q], C[Q], V[Q];
+    const int tid = threadIdx.x;
+    const int64_t t = A.lev_off[lev] + blockIdx.x;
+    const FmmTile tl = A.tiles[t];
+    const FmmSys& fs = A.fsys[tl.sys];
+    const int nc = fs.n[lev - 1];
+    const int64_t cplane = fmm_plane(nc), plane = fmm_plane(fs.n[lev]);
+    for (int i = tid; i < 2 * Q; i += 256) S[i] = shift[i];
+    double acc[PER] = {};
+    int np = 0;
+    for (int ch = 0; ch < 4; ++ch) {
+        const int a = ch >> 1, b = ch & 1;
+        const int cx = 2 * tl.tx + a, cy = 2 * tl.ty + b;
+        if (cx >= nc || cy >= nc) continue;
+        const int64_t c = fs.off[lev - 1] + (int64_t)cx * nc + cy;
+        const int n = A.tcnt[c];
+        if (n == 0) continue;
+        np += n;
+        __syncthreads();
+        const double* src = A.mult + fs.moff[lev - 1] * Q + fmm_slot(nc, cx, cy);
+        for (int q = tid; q < Q; q += 256) C[q] = src[q * cplane];
+        __syncthreads();
+        for (int q = tid; q < Q; q += 256) {
+            const int i = q / P, J = q - i * P;
+            double s = 0.0;
+#pragma unroll
+            for (int I = 0; I < P; ++I) s = fma(S[a * Q + i * P + I], C[I * P + J], s);
+            V[q] = s;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            const int q = tid + 256 * p;
+            if (q < Q) {
+                const int i = q / P, j = q - (q / P) * P;
+                double s = acc[p];
+#pragma unroll
+                for (int J = 0; J < P; ++J) s = fma(V[i * P + J], S[b * Q + j * P + J], s);
+                acc[p] = s;
+            }
+        }
+    }
+    if (tid == 0) A.tcnt[t] = np;
+    double* M = A.mult + fs.moff[lev] * Q + fmm_slot(fs.n[lev], tl.tx, tl.ty);
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+        if (tid + 256 * p < Q) M[(tid + 256 * p) * plane] = acc[p];
+}
+
+// ---------------------------------------------------------------- node to node
+// One wave per (64 targets of one level and child position, 16 target nodes);
+// the block's waves take neighbouring node rows of the same targets, so their
+// reads of the sources meet in the CU's cache.  For each of the 27 offsets a
+// wave forms its 16 x Q slice of the law between target and source nodes in
+// registers, one entry per lane and step (two components), and multiplies it
+// with the 64 sources' node masses on the FP64 matrix unit: A = 16 target
+// nodes x 4 source nodes, B = 4 source nodes x 16 squares, four B blocks per A.
+// Forming an entry costs ~11 issue slots per lane, the eight products it feeds
+// 8 x 16, so the matrix unit is the bound.  Softening enters relative to the
+// square's size, which differs by level and system; forming the slice on the
+// fly needs no table of them.
+template <int P>
+struct M2LWaves {
+    static constexpr int value = (P * P / 16) % 5 == 0 ? 5 : 3;
+};
+
+// NB: blocks of 16 targets (no branch inside: a branch around a product would
+// copy its accumulators).
+template <int P, int NB>
+__device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, int rb, double eps2,
+                                         const double* hn)
+{
+    constexpr int Q = P * P, QP = P / 4;
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const FmmSys& fs = A.fsys[gr.sys];
+    const int lev = gr.lev, n = fs.n[lev], off = fs.off[lev];
+    const int nx = (n - gr.a + 1) >> 1, ny = (n - gr.b + 1) >> 1;   // targets of this child position
+    const int w = fmm_pitch(n);
+    const int64_t plane = fmm_plane(n);
+    const double* M = A.mult + fs.moff[lev] * Q;
+    const double h = (double)fs.T * A.sys[gr.sys].step * (double)(1 << lev);
+    const double e2 = eps2 / (h * h);
+    int tx[NB], ty[NB], tg[NB];
+    unsigned pos[NB];   // byte offset of the target's place in a class, plus the lane's first node
+    bool any = false;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int t = gr.t0 + 16 * b + c;
+        const bool ok = t < nx * ny;
+        const int i = ok ? t / ny : 0, j = ok ? t - i * ny : 0;
+        tx[b] = 2 * i + gr.a;
+        ty[b] = 2 * j + gr.b;
+        tg[b] = ok ? off + tx[b] * n + ty[b] : -1;
+        if (ok && A.tcnt[tg[b]] == 0) tg[b] = -1;
+        pos[b] = (unsigned)(((i + 1) * w + j + 1 + g * (Q / 4) * plane) * sizeof(double));
+        any = any || tg[b] >= 0;
+    }
+    if (!__any(any)) return;
+    const int row = 16 * rb + c;
+    const double xt = hn[row / P], yt = hn[row % P];
+    fd4 ax[NB] = {}, ay[NB] = {};
+    for (int o = 0; o < 36; ++o) {
+        const int pi = o / 12 - 1, ca = (o / 6) & 1, pj = (o % 6) / 2 - 1, cb = o & 1;
+        const int ox = 2 * pi + ca - gr.a, oy = 2 * pj + cb - gr.b;
+        if (abs(ox) <= 1 && abs(oy) <= 1) continue;
+        bool act = false;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int sx = tx[b] + ox, sy = ty[b] + oy;
+            const bool in = tg[b] >= 0 && sx >= 0 && sx < n && sy >= 0 && sy < n;
+            act = act || (in && A.tcnt[in ? off + sx * n + sy : 0] > 0);
+        }
+        if (!__any(act)) continue;
+        // the sources' class, shifted by (pi, pj)
+        const char* mp = (const char*)(M + ((2 * ca + cb) * w + pi) * w + pj);
+        const double dy0 = (double)oy - yt;
+        double m[2][NB];   // the next step's node masses, on their way
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) m[u][b] = *(const double*)(mp + pos[b]);
+            mp += plane * sizeof(double);
+        }
+#pragma unroll 1
+        for (int k = 0; k < QP; ++k) {
+            const double dx = ((double)ox - xt) + hn[g * QP + k];
+            const double dx2 = fma(dx, dx, e2);
+#pragma unroll 1
+            for (int j = 0; j < P; j += 2) {
+                double mc[2][NB], kx[2], ky[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) mc[u][b] = m[u][b];
+                    const double dy = hn[j + u] + dy0;
+                    const double r = rcp64(fma(dy, dy, dx2));
+                    kx[u] = dx * r;
+                    ky[u] = dy * r;
+                }
+                if (k < QP - 1 || j + 2 < P) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) m[u][b] = *(const double*)(mp + pos[b]);
+                        mp += plane * sizeof(double);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        ax[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(kx[u], mc[u][b], ax[b], 0, 0, 0);
+                        ay[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ky[u], mc[u][b], ay[b], 0, 0, 0);
+                    }
+            }
+        }
+    }
+    const double inv_h = 1.0 / h;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (tg[b] < 0) continue;
+        double* L = A.loc + (int64_t)tg[b] * (2 * Q) + 16 * rb;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {   // register v of lane (c, g): row 4 v + g, column c
+            L[4 * v + g] = ax[b][v] * inv_h;
+            L[Q + 4 * v + g] = ay[b][v] * inv_h;
+        }
+    }
+}
+
+template <int P>
+__global__ __launch_bounds__(64 * M2LWaves<P>::value, 3) void k_fmm_m2l(
+    FmmArgs A, const double* __restrict__ nodes, double eps2)
+{
+    constexpr int W = M2LWaves<P>::value, RB = P * P / 16 / W;
+    __shared__ double hn[P];   // nodes on [-1/2, 1/2]
+    if (threadIdx.x < P) hn[threadIdx.x] = 0.5 * nodes[threadIdx.x];
+    __syncthreads();
+    const int gi = blockIdx.x / RB;
+    const int rb = uniform_int((blockIdx.x - gi * RB) * W + (threadIdx.x >> 6));
+    const FmmGroup gr = A.groups[gi];
+    const int n = A.fsys[gr.sys].n[gr.lev];
+    const int cnt = ((n - gr.a + 1) >> 1) * ((n - gr.b + 1) >> 1) - gr.t0;
+    if (cnt > 32) m2l_wave<P, 4>(A, gr, rb, eps2, hn);
+    else if (cnt > 16) m2l_wave<P, 2>(A, gr, rb, eps2, hn);
+    else m2l_wave<P, 1>(A, gr, rb, eps2, hn);
+}
+
+// ---------------------------------------------------------------- field down
+// One block per square of level lev: adds the parent's field, interpolated at
+// the square's nodes; on tiles (lev 0) the sum becomes Chebyshev coefficients.
+template <int P>
+__global__ __launch_bounds__(256) void k_fmm_l2l(FmmArgs A, const double* __restrict__ shift,
+                                                 const double* __restrict__ ctab, int lev)
+{
+    constexpr int Q = P * P;
+    constexpr int PER = (2 * Q + 255) / 256;
+    __shared__ double S[2 * Q], C[2 * Q], V[2 * Q];
+    const int tid = threadIdx.x;
+    const int64_t t = A.lev_off[lev] + blockIdx.x;
+    if (A.tcnt[t] == 0) return;
+    const FmmTile tl = A.tiles[t];
+    const FmmSys& fs = A.fsys[tl.sys];
+    if (fs.nlev <= lev) return;
+    const bool par = lev + 1 < fs.nlev;
+    if (!par && lev > 0) return;
+    double* L = A.loc + t * (int64_t)(2 * Q);
+    double acc[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) acc[p] = tid + 256 * p < 2 * Q ? L[tid + 256 * p] : 0.0;
+    if (par) {
+        const int64_t pt = fs.off[lev + 1] + (int64_t)(tl.tx >> 1) * fs.n[lev + 1] + (tl.ty >> 1);
+        const int a = tl.tx & 1, b = tl.ty & 1;
+        for (int q = tid; q < 2 * Q; q += 256) {
+            S[q] = shift[q];
+            C[q] = A.loc[pt * (2 * Q) + q];
+        }
+        __syncthreads();
+        for (int q = tid; q < 2 * Q; q += 256) {   // V[I][j] = sum_i shift_a[i][I] C[i][j]
+            const int z = q >= Q ? Q : 0, I = (q - z) / P, j = (q - z) - I * P;
+            double s = 0.0;
+#pragma unroll
+            for (int i = 0; i < P; ++i) s = fma(S[a * Q + i * P + I], C[z + i * P + j], s);
+            V[q] = s;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            const int q = tid + 256 * p;
+            if (q < 2 * Q) {
+                const int z = q >= Q ? Q : 0, I = (q - z) / P, J = (q - z) - I * P;
+                double s = acc[p];
+#pragma unroll
+                for (int j = 0; j < P; ++j) s = fma(V[z + I * P + j], S[b * Q + j * P + J], s);
+                acc[p] = s;
+            }
+        }
+    }
+    if (lev > 0) {
+#pragma unroll
+        for (int p = 0; p < PER; ++p)
+            if (tid + 256 * p < 2 * Q) L[tid + 256 * p] = acc[p];
+        return;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+        if (tid + 256 * p < 2 * Q) C[tid + 256 * p] = acc[p];
+    for (int q = tid; q < Q; q += 256) S[q] = ctab[q];
+    __syncthreads();
+    for (int q = tid; q < 2 * Q; q += 256) {   // V[k][J] = sum_I ct[k][I] C[I][J]
+        const int z = q >= Q ? Q : 0, k = (q - z) / P, J = (q - z) - k * P;
+        double s = 0.0;
+#pragma unroll
+        for (int I = 0; I < P; ++I) s = fma(S[k * P + I], C[z + I * P + J], s);
+        V[q] = s;
+    }
+    __syncthreads();
+    for (int q = tid; q < 2 * Q; q += 256) {
+        const int z = q >= Q ? Q : 0, k = (q - z) / P, l = (q - z) - k * P;
+        double s = 0.0;
+#pragma unroll
+        for (int J = 0; J < P; ++J) s = fma(V[z + k * P + J], S[l * P + J], s);
+        L[q] = s;
+    }
+}
+
+// ---------------------------------------------------------------- particles
+__global__ __launch_bounds__(256) void k_fmm_pack(FmmArgs A)
+{
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.N; i += stride) {
+        const double sig = step_scale(A.sys[A.sys_of[i]].step);
+        FmmPart p;
+        p.x = A.x[i] * sig;
+        p.y = A.y[i] * sig;
+        p.m = A.m[i];
+        p.pad = 0.0;
+        A.pack[i] = p;
+    }
+}
+
+// Two terms of the law from one reciprocal: Q = q0 q1, R = 1 / Q, so the
+// weights are (m0 R) q1 and (m1 R) q0.  An entry that the particle does not
+// keep enters as q = 1 with weight 0.
+template <int LAW, bool MASK>
+__device__ __forceinline__ void pair_terms(double X0, double Y0, double m0, double X1, double Y1,
+                                           double m1, double x, double y, bool k0, bool k1,
+                                           double eps2, double r2cut, double& sx, double& sy)
+{
+    const double wx0 = X0 - x, wy0 = Y0 - y, wx1 = X1 - x, wy1 = Y1 - y;
+    double q0 = fma(wx0, wx0, fma(wy0, wy0, eps2)), q1 = fma(wx1, wx1, fma(wy1, wy1, eps2));
+    if (LAW == 1) {
+        const bool c0 = fma(wx0, wx0, wy0 * wy0) > r2cut, c1 = fma(wx1, wx1, wy1 * wy1) > r2cut;
+        k0 = MASK ? k0 && c0 : c0;
+        k1 = MASK ? k1 && c1 : c1;
+    }
+    if (MASK || LAW == 1) {
+        q0 = k0 ? q0 : 1.0;
+        q1 = k1 ? q1 : 1.0;
+    }
+    const double R = rcp64(q0 * q1);
+    double w0 = (m0 * R) * q1, w1 = (m1 * R) * q0;
+    if (MASK || LAW == 1) {
+        w0 = k0 ? w0 : 0.0;
+        w1 = k1 ? w1 : 0.0;
+    }
+    sx = fma(wx0, w0, sx);
+    sy = fma(wy0, w0, sy);
+    sx = fma(wx1, w1, sx);
+    sy = fma(wy1, w1, sy);
+}
+
+// One wave per chunk of 64 particles of one tile.  The tile's coefficients
+// and the mid entries are the same for every lane: scalar loads.  Near
+// candidates: if the wave lies in one column and spans at most
+// FMM_UNIFORM_ROWS rows, the union of its lanes' ranges is walked with scalar
+// loads and a row test; otherwise each lane walks its own three ranges with
+// vector loads (a union would spend most of its pairs on the test).  Either
+// way a particle's terms come in the same order.
+template <int P, int LAW>
+__global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2p,
+                                                  double r2cutp, int qpart, int nqparts)
+{
+    constexpr int Q = P * P;
+    const int lane = threadIdx.x;
+    const int total = A.cnt[0];
+    const int qb = (int)(((int64_t)total * qpart) / nqparts);
+    const int qe = (int)(((int64_t)total * (qpart + 1)) / nqparts);
+    for (int ci = qb + blockIdx.x; ci < qe; ci += gridDim.x) {
+        const FmmChunk ch = A.chunks[ci];
+        const int t = uniform_int(ch.tile);
+        const FmmTile tl = A.tiles[t];
+        const int s = uniform_int(tl.sys);
+        const int ttx = uniform_int(tl.tx), tty = uniform_int(tl.ty);
+        const SysDev& d = A.sys[s];
+        const FmmSys& fs = A.fsys[s];
+        const int G = d.G, T = fs.T;
+        const int64_t coff = d.c_off;
+        const double step = d.step, sig = step_scale(step);
+        const double eps2 = eps2p * sig * sig, r2cut = r2cutp * sig * sig;
+        const double h = (double)T * step;
+        const int x0 = ttx * T, y0 = tty * T, x1 = min(x0 + T, G), y1 = min(y0 + T, G);
+
+        // lane -> particle: rank 64 k + lane in the tile, columns in order
+        int r = 64 * uniform_int(ch.k) + lane, gi = -1;
+        for (int x = x0; x < x1; ++x) {
+            const int64_t cl = coff + (int64_t)x * G;
+            const int a = A.offsets[cl + y0], b = A.offsets[cl + y1];
+            if (gi < 0 && r < b - a) gi = a + r;
+            r -= b - a;
+        }
+        const bool act = gi >= 0;
+        double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, fx = 0.0, fy = 0.0;
+        int cx = -100000, cy = -100000;
+        if (act) {
+            const FmmPart p = A.pack[gi];
+            x = p.x;
+            y = p.y;
+            const int key = A.key_sorted[gi] - (int)coff;
+            cx = key / G;
+            cy = key - cx * G;
+        }
+        const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
+        const int cxh = uniform_int(wave_max(act ? cx : -1));
+        const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
+        const int cyh = uniform_int(wave_max(act ? cy : -1));
+
+        // the particle on its tile, [-1, 1]^2
+        const double ux = 2.0 * ((x / sig - d.min_x) / h - ttx) - 1.0;
+        const double uy = 2.0 * ((y / sig - d.min_y) / h - tty) - 1.0;
+
+        // near pairs, two at a time; the second of an odd count is the particle
+        // itself, not kept
+        if (cxl == cxh && cyh - cyl < FMM_UNIFORM_ROWS) {
+            for (int dx = -1; dx <= 1; ++dx) {
+                const int xc = cxl + dx;
+                if (xc < 0 || xc >= G) continue;
+                const int64_t cl = coff + (int64_t)xc * G;
+                for (int row = max(cyl - 1, 0); row <= min(cyh + 1, G - 1); ++row) {
+                    const int a = uniform_int(A.offsets[cl + row]);
+                    const int b = uniform_int(A.offsets[cl + row + 1]);
+                    if (!(act && abs(row - cy) <= 1)) continue;
+                    cptr<FmmPart> E = as_const(A.pack);
+                    if (dx == 0 && row >= cyl && row <= cyh) {   // some lanes' own cell
+                        for (int j = a; j < b; j += 2) {
+                            const int j1 = min(j + 1, b - 1);
+                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j1].x, E[j1].y, E[j1].m,
+                                                  x, y, j != gi, j1 != gi && j1 != j, eps2, r2cut,
+                                                  sx, sy);
+                        }
+                    } else {
+                        int j = a;
+#pragma unroll 2
+                        for (; j + 1 < b; j += 2)
+                            pair_terms<LAW, false>(E[j].x, E[j].y, E[j].m, E[j + 1].x, E[j + 1].y,
+                                                   E[j + 1].m, x, y, true, true, eps2, r2cut, sx, sy);
+                        if (j < b)
+                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, E[j].m, x,
+                                                  y, true, false, eps2, r2cut, sx, sy);
+                    }
+                }
+            }
+        } else {
+            int ra[3], rb[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int xc = cx + k - 1;
+                ra[k] = 0;
+                rb[k] = 0;
+                if (act && xc >= 0 && xc < G) {
+                    const int64_t cl = coff + (int64_t)xc * G;
+                    ra[k] = A.offsets[cl + max(cy - 1, 0)];
+                    rb[k] = A.offsets[cl + min(cy + 1, G - 1) + 1];
+                }
+            }
+            const int n0 = rb[0] - ra[0], n1 = n0 + rb[1] - ra[1], n2 = n1 + rb[2] - ra[2];
+            const int s1 = ra[1] - n0, s2 = ra[2] - n1;
+#pragma unroll 2
+            for (int k = 0; k < n2; k += 2) {
+                const int ka = k, kb = min(k + 1, n2 - 1);
+                const int j0 = ka + (ka < n0 ? ra[0] : (ka < n1 ? s1 : s2));
+                const int j1 = kb + (kb < n0 ? ra[0] : (kb < n1 ? s1 : s2));
+                const FmmPart p0 = A.pack[j0], p1 = A.pack[j1];
+                pair_terms<LAW, true>(p0.x, p0.y, p0.m, p1.x, p1.y, p1.m, x, y, j0 != gi,
+                                      j1 != gi && kb != ka, eps2, r2cut, sx, sy);
+            }
+        }
+
+        // mid entries: 3x3 tiles, or every tile where the grouped part does not
+        // hold: a system of one tile, a cutoff that reaches past a tile, COMs
+        // outside their cells, particles moved since they were placed
+        const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
+        const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
+                         uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
+        const int nt = fs.n[0];
+        const int mx0 = all ? 0 : max(ttx - 1, 0), mx1 = all ? nt - 1 : min(ttx + 1, nt - 1);
+        const int my0 = all ? 0 : max(tty - 1, 0), my1 = all ? nt - 1 : min(tty + 1, nt - 1);
+        for (int mx = mx0; mx <= mx1; ++mx) {
+            for (int my = my0; my <= my1; ++my) {
+                const int mt = fs.off[0] + mx * nt + my;
+                const int e0 = uniform_int(A.tstart[mt]), ne = uniform_int(A.tne[mt]);
+                cptr<FmmCom> E = as_const(A.list) + e0;
+                for (int e = 0; e < ne; e += 4) {
+                    bool nr = false;   // some entry may lie in some lane's 3x3 cells
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        nr = nr || (E[e + u].kx >= cxl - 1 && E[e + u].kx <= cxh + 1 &&
+                                    E[e + u].ky >= cyl - 1 && E[e + u].ky <= cyh + 1);
+#pragma unroll
+                    for (int u = 0; u < 4; u += 2) {
+                        const cptr<FmmCom> f0 = E + e + u, f1 = f0 + 1;
+                        if (!nr)
+                            pair_terms<LAW, false>(f0->X, f0->Y, f0->M, f1->X, f1->Y, f1->M, x, y,
+                                                   true, true, eps2, r2cut, sx, sy);
+                        else
+                            pair_terms<LAW, true>(
+                                f0->X, f0->Y, f0->M, f1->X, f1->Y, f1->M, x, y,
+                                !(abs(f0->kx - cx) <= 1 && abs(f0->ky - cy) <= 1),
+                                !(abs(f1->kx - cx) <= 1 && abs(f1->ky - cy) <= 1), eps2, r2cut, sx,
+                                sy);
+                    }
+                }
+            }
+        }
+
+        // distant part: the tile's Chebyshev series
+        if (!all && act) {
+            double ty[P];
+            ty[0] = 1.0;
+            ty[1] = uy;
+#pragma unroll
+            for (int l = 2; l < P; ++l) ty[l] = fma(2.0 * uy, ty[l - 1], -ty[l - 2]);
+            cptr<double> L = as_const(A.loc) + (int64_t)t * (2 * Q);
+            double a0 = 1.0, a1 = ux;
+            for (int k = 0; k < P; ++k) {
+                double vx = 0.0, vy = 0.0;
+#pragma unroll
+                for (int l = 0; l < P; ++l) {
+                    vx = fma(L[k * P + l], ty[l], vx);
+                    vy = fma(L[Q + k * P + l], ty[l], vy);
+                }
+                fx = fma(a0, vx, fx);
+                fy = fma(a0, vy, fy);
+                const double an = fma(2.0 * ux, a1, -a0);
+                a0 = a1;
+                a1 = an;
+            }
+        }
+        if (act) {
+            A.ax[gi] += Gc * fma(sx, sig, fx);
+            A.ay[gi] += Gc * fma(sy, sig, fy);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- launches
+template <int P>
+static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int num_cu,
+                        hipStream_t st)
+{
+    const FmmTables& tb = P == 12 ? pl.tab[0] : pl.tab[1];
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt, (int64_t)(2 + A.S), 0);
+    hipLaunchKernelGGL(k_fmm_tiles, dim3((unsigned)((A.nleaf * 8 + 255) / 256)), dim3(256), 0, st,
+                       A);
+    const unsigned pg = (unsigned)((A.N + 255) / 256);
+    hipLaunchKernelGGL(k_fmm_pack, dim3(pg < (unsigned)num_cu * 16 ? pg : num_cu * 16), dim3(256),
+                       0, st, A);
+    hipLaunchKernelGGL(k_fmm_p2m<P>, dim3((unsigned)A.nleaf), dim3(256), 0, st, A, tb.cheb);
+    for (int l = 1; l < pl.nlev; ++l)
+        hipLaunchKernelGGL(k_fmm_m2m<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
+                           dim3(256), 0, st, A, tb.shift, l);
+    constexpr int W = M2LWaves<P>::value;
+    hipLaunchKernelGGL(k_fmm_m2l<P>, dim3((unsigned)pl.ngroups * (P * P / 16 / W)), dim3(64 * W),
+                       0, st, A, tb.nodes, eps2);
+    for (int l = pl.nlev - 1; l >= 0; --l)
+        hipLaunchKernelGGL(k_fmm_l2l<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
+                           dim3(256), 0, st, A, tb.shift, tb.cheb, l);
+}
+
+template <int P>
+static void fmm_force(const FmmArgs& A, double Gc, double eps2, double r2cut, int part, int nparts,
+                      int num_cu, hipStream_t st)
+{
+    const int64_t cap = A.max_chunks, most = (int64_t)num_cu * 256;
+    const unsigned g = (unsigned)(cap < most ? cap : most);
+    if (r2cut > 0.0)
+        hipLaunchKernelGGL((k_fmm_force<P, 1>), dim3(g), dim3(64), 0, st, A, Gc, eps2, r2cut, part,
+                           nparts);
+    else
+        hipLaunchKernelGGL((k_fmm_force<P, 0>), dim3(g), dim3(64), 0, st, A, Gc, eps2, r2cut, part,
+                           nparts);
+}
+
+void bh_fmm_pass(const FmmArgs& args, const FmmPlan& pl, bool fp64, double Gc, double eps2,
+                 double r2cut, int part, int nparts, int num_cu, hipStream_t st)
+{
+    FmmArgs A = args;
+    A.mult = pl.mult[fp64 ? 1 : 0];
+    if (part == 0) {
+        if (fp64) fmm_prepare<FMM_P64>(A, pl, eps2, num_cu, st);
+        else fmm_prepare<FMM_P32>(A, pl, eps2, num_cu, st);
+    }
+    if (fp64) fmm_force<FMM_P64>(A, Gc, eps2, r2cut, part, nparts, num_cu, st);
+    else fmm_force<FMM_P32>(A, Gc, eps2, r2cut, part, nparts, num_cu, st);
+}

@@ -64,6 +64,96 @@ struct PotArgs {
     double *u, *k;        // m_i phi_i and m_i |v_i|^2 per particle
 };
 
+// ---- grouped far field (bh_fmm.hip)
+#define FMM_TILE 8           // cells per side of a tile
+#define FMM_P32 12           // Chebyshev nodes per side, FP32 precision
+#define FMM_P64 20           // and FP64 precision
+#define FMM_LEVELS 13        // levels of squares (grid_dim <= 32767)
+#define FMM_MIN_GRID 32      // smaller grids are one tile, every COM taken on its own
+#define FMM_UNIFORM_ROWS 2   // rows a wave may span to walk its near candidates together
+
+// A system: T cells per tile side, nlev levels of squares (0: one tile, no
+// grouped part), n[l] squares per side at level l (level 0: the tiles), the
+// first of them at off[l] of the square index space.
+struct FmmSys {
+    int32_t T, nlev;
+    int32_t n[FMM_LEVELS];
+    int32_t off[FMM_LEVELS];
+    int64_t moff[FMM_LEVELS];   // first node-mass slot of the level (see fmm_slot)
+};
+struct FmmTile {
+    int32_t sys;
+    int16_t tx, ty;
+};
+struct FmmChunk {   // particles [64 k, 64 k + 64) of a tile
+    int32_t tile, k;
+};
+struct FmmGroup {   // targets t0 .. t0 + 63 of the squares (2 i + a, 2 j + b) of a level
+    int32_t sys, t0;
+    int16_t lev;
+    int8_t a, b;
+};
+struct alignas(32) FmmCom {   // COM in units of step_scale, tile order
+    double X, Y, M;
+    int32_t kx, ky;
+};
+struct alignas(32) FmmPart {
+    double x, y, m, pad;
+};
+
+struct FmmArgs {
+    const SysDev* sys;
+    const FmmSys* fsys;
+    const int32_t *sys_of, *offsets, *neprefix, *key_sorted;
+    const Com64* l64;
+    const double *x, *y, *m;
+    double *ax, *ay;
+    const FmmTile* tiles;      // every square, level by level
+    const FmmGroup* groups;
+    int32_t *tcnt;             // per square: particles
+    int32_t *tstart, *tne;     // per tile: its run of list
+    int32_t* cnt;              // chunks, list entries, then per system sbad
+    int32_t* sbad;             // != 0: a COM lies outside its cell
+    FmmChunk* chunks;
+    FmmCom* list;
+    FmmPart* pack;
+    double* mult;              // node masses, node-major (fmm_slot)
+    double* loc;               // per square: P^2 ax, P^2 ay
+    int32_t S;
+    int64_t N, nleaf, ntiles, max_chunks;
+    int64_t lev_off[FMM_LEVELS + 1];
+};
+
+// Node masses of a level of n^2 squares: node-major planes, so that the squares
+// a wave reads together are neighbours in memory.  A plane holds the squares by
+// child position (x & 1, y & 1), each class a (np + 2)^2 array with a border of
+// zeros (np = (n + 1) / 2) that stands for the squares outside the grid.
+__host__ __device__ inline int fmm_pitch(int n) { return (n + 1) / 2 + 2; }
+__host__ __device__ inline int64_t fmm_plane(int n)
+{
+    return 4 * (int64_t)fmm_pitch(n) * fmm_pitch(n);
+}
+// Slot of square (x, y) in a plane.
+__host__ __device__ inline int fmm_slot(int n, int x, int y)
+{
+    const int w = fmm_pitch(n);
+    return ((2 * (x & 1) + (y & 1)) * w + (x >> 1) + 1) * w + (y >> 1) + 1;
+}
+
+struct FmmTables {
+    const double *nodes;   // P Chebyshev nodes on [-1, 1]
+    const double *cheb;    // [k][i]: c_k T_k(node i), c_0 = 1 / P, c_k = 2 / P
+    const double *shift;   // [a][i][I]: cardinal i of a square at node I of its child half a
+};
+struct FmmPlan {
+    int nlev = 0;
+    int64_t ngroups = 0;
+    FmmTables tab[2];      // P = FMM_P32, FMM_P64
+    double* mult[2] = {nullptr, nullptr};   // their node masses (zero borders)
+};
+void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, double eps2,
+                 double r2cut, int part, int nparts, int num_cu, hipStream_t st);
+
 // m / q to FP64 accuracy without the IEEE division sequence: v_rcp_f64 gives
 // r0 with e = 1 - q r0 small (|e| < 2^-22), and 1/q = r0 (1 + e + e^2 + e^3 + ...),
 // so m r0 (1 + e + e^2) differs from m / q by the relative e^3 plus the
