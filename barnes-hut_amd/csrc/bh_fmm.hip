@@ -26,7 +26,7 @@
 #define FMM_IN 1.0001   // |coordinate| on a square up to which it counts as inside
 
 typedef double fd4 __attribute__((ext_vector_type(4)));
-typedef double fd2 __attribute__((ext_vector_type(2)));
+typedef double fd8 __attribute__((ext_vector_type(8)));
 
 // Wave-uniform reads through the constant address space: scalar loads, so
 // every lane gets the value from a scalar register.
@@ -312,22 +312,21 @@ __global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __rest
 }
 
 // ---------------------------------------------------------------- node to node
-// One wave per (64 targets of one level and child position, 16 target nodes);
-// the block's waves take neighbouring node rows of the same targets, so their
-// reads of the sources meet in the CU's cache.  For each of the 27 offsets a
-// wave forms its 16 x Q slice of the law between target and source nodes in
-// registers, one entry per lane and step (two components), and multiplies it
-// with the 64 sources' node masses on the FP64 matrix unit: A = 16 target
-// nodes x 4 source nodes, B = 4 source nodes x 16 squares, four B blocks per A.
-// Forming an entry costs ~11 issue slots per lane, the eight products it feeds
-// 8 x 16, so the matrix unit is the bound.  Softening enters relative to the
-// square's size, which differs by level and system; forming the slice on the
-// fly needs no table of them.
-template <int P>
-struct M2LWaves {
-    static constexpr int value = (P * P / 16) % 5 == 0 ? 5 : 3;
-};
-
+// One wave per (64 targets of one level and child position, 16 target nodes).
+// For each of the 27 offsets a wave forms its 16 x Q slice of the law between
+// target and source nodes in registers, one entry per lane and step (two
+// components), and multiplies it with the 64 sources' node masses on the FP64
+// matrix unit: A = 16 target nodes x 4 source nodes, B = 4 source nodes x 16
+// squares, four B blocks per A.  Forming an entry costs ~11 issue slots per
+// lane, the eight products it feeds 8 x 16, so the matrix unit is the bound.
+// Softening enters relative to the square's size, which differs by level and
+// system; forming the slice on the fly needs no table of them.
+// 4.2M particles, 1024^2 cells: P = 20 7.0 ms, 55 TFLOP/s (a large FP64 matrix
+// product reaches 73; the unit is busy 0.74 of the cycles, at 2.27 GHz), P = 12
+// 0.98 ms.  Tried: sources square-major (one line per 16 bytes read: 76 ms);
+// waves of several node rows sharing a workgroup (8.5 ms: its waves spread
+// unevenly over the SIMDs); node rows of a group kept on one XCD (6.8 ms, but
+// 4.3 instead of 2.8 ms on 512 systems, whose groups differ in size).
 // NB: blocks of 16 targets (no branch inside: a branch around a product would
 // copy its accumulators).
 template <int P, int NB>
@@ -433,15 +432,14 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
 }
 
 template <int P>
-__global__ __launch_bounds__(64 * M2LWaves<P>::value, 3) void k_fmm_m2l(
-    FmmArgs A, const double* __restrict__ nodes, double eps2)
+__global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, const double* __restrict__ nodes,
+                                                   double eps2)
 {
-    constexpr int W = M2LWaves<P>::value, RB = P * P / 16 / W;
+    constexpr int RB = P * P / 16;
     __shared__ double hn[P];   // nodes on [-1/2, 1/2]
     if (threadIdx.x < P) hn[threadIdx.x] = 0.5 * nodes[threadIdx.x];
     __syncthreads();
-    const int gi = blockIdx.x / RB;
-    const int rb = uniform_int((blockIdx.x - gi * RB) * W + (threadIdx.x >> 6));
+    const int gi = blockIdx.x / RB, rb = blockIdx.x - gi * RB;
     const FmmGroup gr = A.groups[gi];
     const int n = A.fsys[gr.sys].n[gr.lev];
     const int cnt = ((n - gr.a + 1) >> 1) * ((n - gr.b + 1) >> 1) - gr.t0;
@@ -575,13 +573,38 @@ __device__ __forceinline__ void pair_terms(double X0, double Y0, double m0, doub
     sy = fma(wy1, w1, sy);
 }
 
+// A lane's own near candidates in column xc (OWN: its own column, which holds
+// the particle itself).  gi < 0: no particle.
+template <int LAW, bool OWN>
+__device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G, int xc, int cy,
+                                           int gi, double x, double y, double eps2, double r2cut,
+                                           double& sx, double& sy)
+{
+    if (gi < 0 || xc < 0 || xc >= G) return;
+    const int64_t cl = coff + (int64_t)xc * G;
+    int j = A.offsets[cl + max(cy - 1, 0)];
+    const int b = A.offsets[cl + min(cy + 1, G - 1) + 1];
+    const FmmPart* E = A.pack + j;
+    for (; j < b; j += 2, E += 2) {
+        const bool two = j + 1 < b;
+        const FmmPart* E1 = two ? E + 1 : E;
+        const double m1 = two ? E1->m : 0.0;
+        pair_terms<LAW, OWN>(E->x, E->y, E->m, E1->x, E1->y, m1, x, y, j != gi,
+                             (two ? j + 1 : j) != gi, eps2, r2cut, sx, sy);
+    }
+}
+
 // One wave per chunk of 64 particles of one tile.  The tile's coefficients
-// and the mid entries are the same for every lane: scalar loads.  Near
+// and the mid entries are the same for every lane: scalar loads of whole quads
+// (128 bytes), no test in tiles that no lane's 3x3 cells touch.  Near
 // candidates: if the wave lies in one column and spans at most
 // FMM_UNIFORM_ROWS rows, the union of its lanes' ranges is walked with scalar
 // loads and a row test; otherwise each lane walks its own three ranges with
-// vector loads (a union would spend most of its pairs on the test).  Either
-// way a particle's terms come in the same order.
+// vector loads (a union would spend most of its pairs on the test).  Terms go
+// in pairs that share a reciprocal; only cells that hold the lanes themselves
+// are tested for the particle itself.  Bound by FP64 issue: ~12 slots a term,
+// 2.5e12 terms/s on 10M particles over 120^2 cells (6.7e10 near and mid terms,
+// 26.8 ms; 30.6 ms with entries loaded and tested one by one).
 template <int P, int LAW>
 __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2p,
                                                   double r2cutp, int qpart, int nqparts)
@@ -634,8 +657,8 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
         const double ux = 2.0 * ((x / sig - d.min_x) / h - ttx) - 1.0;
         const double uy = 2.0 * ((y / sig - d.min_y) / h - tty) - 1.0;
 
-        // near pairs, two at a time; the second of an odd count is the particle
-        // itself, not kept
+        // near pairs, two at a time; where a count is odd its last pair is the
+        // last particle and a copy of it without mass
         if (cxl == cxh && cyh - cyl < FMM_UNIFORM_ROWS) {
             for (int dx = -1; dx <= 1; ++dx) {
                 const int xc = cxl + dx;
@@ -645,50 +668,41 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                     const int a = uniform_int(A.offsets[cl + row]);
                     const int b = uniform_int(A.offsets[cl + row + 1]);
                     if (!(act && abs(row - cy) <= 1)) continue;
-                    cptr<FmmPart> E = as_const(A.pack);
+                    const cptr<FmmPart> E = as_const(A.pack);
+                    int j = a;
                     if (dx == 0 && row >= cyl && row <= cyh) {   // some lanes' own cell
-                        for (int j = a; j < b; j += 2) {
-                            const int j1 = min(j + 1, b - 1);
-                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j1].x, E[j1].y, E[j1].m,
-                                                  x, y, j != gi, j1 != gi && j1 != j, eps2, r2cut,
-                                                  sx, sy);
+                        for (; j + 1 < b; j += 2) {
+                            const fd8 f = *(cptr<fd8>)(E + j);
+                            pair_terms<LAW, true>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, j != gi,
+                                                  j + 1 != gi, eps2, r2cut, sx, sy);
                         }
-                    } else {
-                        int j = a;
-#pragma unroll 2
-                        for (; j + 1 < b; j += 2)
-                            pair_terms<LAW, false>(E[j].x, E[j].y, E[j].m, E[j + 1].x, E[j + 1].y,
-                                                   E[j + 1].m, x, y, true, true, eps2, r2cut, sx, sy);
                         if (j < b)
-                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, E[j].m, x,
-                                                  y, true, false, eps2, r2cut, sx, sy);
+                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, 0.0, x, y,
+                                                  j != gi, j != gi, eps2, r2cut, sx, sy);
+                    } else {
+                        for (; j + 3 < b; j += 4) {
+                            const fd8 f = *(cptr<fd8>)(E + j), h2 = *(cptr<fd8>)(E + j + 2);
+                            pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true,
+                                                   true, eps2, r2cut, sx, sy);
+                            pair_terms<LAW, false>(h2[0], h2[1], h2[2], h2[4], h2[5], h2[6], x, y,
+                                                   true, true, eps2, r2cut, sx, sy);
+                        }
+                        if (j + 1 < b) {
+                            const fd8 f = *(cptr<fd8>)(E + j);
+                            pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true,
+                                                   true, eps2, r2cut, sx, sy);
+                            j += 2;
+                        }
+                        if (j < b)
+                            pair_terms<LAW, false>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, 0.0, x, y,
+                                                   true, true, eps2, r2cut, sx, sy);
                     }
                 }
             }
         } else {
-            int ra[3], rb[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int xc = cx + k - 1;
-                ra[k] = 0;
-                rb[k] = 0;
-                if (act && xc >= 0 && xc < G) {
-                    const int64_t cl = coff + (int64_t)xc * G;
-                    ra[k] = A.offsets[cl + max(cy - 1, 0)];
-                    rb[k] = A.offsets[cl + min(cy + 1, G - 1) + 1];
-                }
-            }
-            const int n0 = rb[0] - ra[0], n1 = n0 + rb[1] - ra[1], n2 = n1 + rb[2] - ra[2];
-            const int s1 = ra[1] - n0, s2 = ra[2] - n1;
-#pragma unroll 2
-            for (int k = 0; k < n2; k += 2) {
-                const int ka = k, kb = min(k + 1, n2 - 1);
-                const int j0 = ka + (ka < n0 ? ra[0] : (ka < n1 ? s1 : s2));
-                const int j1 = kb + (kb < n0 ? ra[0] : (kb < n1 ? s1 : s2));
-                const FmmPart p0 = A.pack[j0], p1 = A.pack[j1];
-                pair_terms<LAW, true>(p0.x, p0.y, p0.m, p1.x, p1.y, p1.m, x, y, j0 != gi,
-                                      j1 != gi && kb != ka, eps2, r2cut, sx, sy);
-            }
+            near_range<LAW, false>(A, coff, G, cx - 1, cy, gi, x, y, eps2, r2cut, sx, sy);
+            near_range<LAW, true>(A, coff, G, cx, cy, gi, x, y, eps2, r2cut, sx, sy);
+            near_range<LAW, false>(A, coff, G, cx + 1, cy, gi, x, y, eps2, r2cut, sx, sy);
         }
 
         // mid entries: 3x3 tiles, or every tile where the grouped part does not
@@ -704,25 +718,29 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
             for (int my = my0; my <= my1; ++my) {
                 const int mt = fs.off[0] + mx * nt + my;
                 const int e0 = uniform_int(A.tstart[mt]), ne = uniform_int(A.tne[mt]);
-                cptr<FmmCom> E = as_const(A.list) + e0;
-                for (int e = 0; e < ne; e += 4) {
-                    bool nr = false;   // some entry may lie in some lane's 3x3 cells
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        nr = nr || (E[e + u].kx >= cxl - 1 && E[e + u].kx <= cxh + 1 &&
-                                    E[e + u].ky >= cyl - 1 && E[e + u].ky <= cyh + 1);
-#pragma unroll
-                    for (int u = 0; u < 4; u += 2) {
-                        const cptr<FmmCom> f0 = E + e + u, f1 = f0 + 1;
-                        if (!nr)
-                            pair_terms<LAW, false>(f0->X, f0->Y, f0->M, f1->X, f1->Y, f1->M, x, y,
-                                                   true, true, eps2, r2cut, sx, sy);
-                        else
-                            pair_terms<LAW, true>(
-                                f0->X, f0->Y, f0->M, f1->X, f1->Y, f1->M, x, y,
-                                !(abs(f0->kx - cx) <= 1 && abs(f0->ky - cy) <= 1),
-                                !(abs(f1->kx - cx) <= 1 && abs(f1->ky - cy) <= 1), eps2, r2cut, sx,
-                                sy);
+                const cptr<fd8> E = (cptr<fd8>)(as_const(A.list) + e0);
+                // a tile that some lane's 3x3 cells may touch: each entry is tested
+                const bool touch = mx * T <= cxh + 1 && mx * T + T > cxl - 1 &&
+                                   my * T <= cyh + 1 && my * T + T > cyl - 1;
+                if (!touch) {
+                    for (int e = 0; e < ne; e += 4) {
+                        const fd8 f = E[e >> 1], h2 = E[(e >> 1) + 1];
+                        pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true, true,
+                                               eps2, r2cut, sx, sy);
+                        pair_terms<LAW, false>(h2[0], h2[1], h2[2], h2[4], h2[5], h2[6], x, y, true,
+                                               true, eps2, r2cut, sx, sy);
+                    }
+                } else {
+                    for (int e = 0; e < ne; e += 2) {
+                        const fd8 f = E[e >> 1];
+                        const long long c0 = __double_as_longlong(f[3]);
+                        const long long c1 = __double_as_longlong(f[7]);
+                        const int kx0 = (int)c0, ky0 = (int)(c0 >> 32);
+                        const int kx1 = (int)c1, ky1 = (int)(c1 >> 32);
+                        pair_terms<LAW, true>(f[0], f[1], f[2], f[4], f[5], f[6], x, y,
+                                              (unsigned)(kx0 - cx + 1) > 2u || (unsigned)(ky0 - cy + 1) > 2u,
+                                              (unsigned)(kx1 - cx + 1) > 2u || (unsigned)(ky1 - cy + 1) > 2u,
+                                              eps2, r2cut, sx, sy);
                     }
                 }
             }
@@ -774,9 +792,8 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
     for (int l = 1; l < pl.nlev; ++l)
         hipLaunchKernelGGL(k_fmm_m2m<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
                            dim3(256), 0, st, A, tb.shift, l);
-    constexpr int W = M2LWaves<P>::value;
-    hipLaunchKernelGGL(k_fmm_m2l<P>, dim3((unsigned)pl.ngroups * (P * P / 16 / W)), dim3(64 * W),
-                       0, st, A, tb.nodes, eps2);
+    hipLaunchKernelGGL(k_fmm_m2l<P>, dim3((unsigned)pl.ngroups * (P * P / 16)), dim3(64), 0, st, A,
+                       tb.nodes, eps2);
     for (int l = pl.nlev - 1; l >= 0; --l)
         hipLaunchKernelGGL(k_fmm_l2l<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
                            dim3(256), 0, st, A, tb.shift, tb.cheb, l);
