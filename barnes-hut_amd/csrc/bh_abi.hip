@@ -100,6 +100,7 @@ struct bh_ctx_s {
     double* rc_blk = nullptr;      // per block: sum of M^2
     double* rc_bfar = nullptr;     // per block: its far-block part of the bound
     int64_t nblocks = 0;
+    int64_t nchunks = 0;           // chunks of 64 particles of one system
     // grouped far field (bh_fmm.hip): which passes take it is a rule on the
     // systems' sizes (fmm_wanted)
     bool fmm_on = false;
@@ -166,6 +167,7 @@ static int layout_systems(int32_t nsys, const int64_t* n, const int32_t* grid_di
 {
     sh.assign(nsys, SysDev{});
     N = C = cols = maxN = NB = 0;
+    int64_t chunks = 0;
     for (int s = 0; s < nsys; ++s) {
         if (n[s] < 1) return fail(BH_EINVAL, "system " + std::to_string(s) + " has n < 1");
         // the FP32 COM list packs column and row in 16 bits each (Com32::kxy)
@@ -178,6 +180,8 @@ static int layout_systems(int32_t nsys, const int64_t* n, const int32_t* grid_di
         d.col_off = cols;
         d.G = grid_dim[s];
         d.Gb = (int32_t)cdiv(grid_dim[s], RC_BLOCK);
+        d.k_off = chunks;
+        chunks += cdiv(n[s], 64);
         d.b_off = NB;
         NB += (int64_t)d.Gb * d.Gb;
         N += n[s];
@@ -384,7 +388,7 @@ static int for_each_buffer(Ctx* c, F&& f)
     B(bne, nb);
     B(stats, ST_COUNT);
     B(com_dense, 3 * C);
-    B(l64, C);
+    B(l64, C + 4);   // k_force64s reads whole quads
     B(l32, C);
     B(items, c->max_items);
     B(col_items, cols);
@@ -509,6 +513,7 @@ int bh_set_systems(void* ctx, int32_t nsys, const int64_t* n, const int32_t* gri
     free_all(c);
     unconfigure(c);
     c->sys_h = sh;
+    c->nchunks = sh.back().k_off + cdiv(sh.back().n, 64);
     int r = configure(c, nsys, N, C, cols, maxN, NB);
     if (r == BH_OK) r = ensure_part(c);
     if (r != BH_OK) {
@@ -844,6 +849,20 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     fa.eps2 = law->eps2;
     fa.r2cut = law->r2_cut;
     fa.cost_log = c->cost_log_on ? c->cost_log : nullptr;
+    if (precision == 0 && !c->cost_log_on) {
+        // chunks, not work items: the queue order does not enter (the cost log
+        // times the items, so it keeps k_force64)
+        fa.part_n = c->N;
+        fa.chunk0 = c->nchunks * part / nparts;
+        const int64_t end = c->nchunks * (part + 1) / nparts;
+        if (part == 0) c->rc_ready = 0;
+        if (end > fa.chunk0) bh_force64s(fa, lawi, c->S, end - fa.chunk0, st);
+        if (part == nparts - 1)
+            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
+                               (int64_t)2, 0);
+        LAUNCH_CHECK("evaluate");
+        return BH_OK;
+    }
     const bool fp32v = precision >= 1 && precision <= 3;
     fa.split = (fp32v && c->tune.tail_split > 1 && c->tune.tail_items > 0) ? c->tune.tail_split : 1;
     fa.n_tail = fa.split > 1 ? c->tune.tail_items : 0;
@@ -1392,6 +1411,7 @@ extern "C" int bh_step_noalloc(const bh_particles* a, const bh_particles* b, int
     c.num_cu = num_cu;
     const int64_t G = grid_dim, Gb = cdiv(G, RC_BLOCK);
     set_sizes(&c, 1, n, G * G, G, n, Gb * Gb);
+    c.nchunks = cdiv(n, 64);
     size_t off = 0;
     r = for_each_buffer(&c, [&](auto*& p, int64_t cnt) {
         using T = std::remove_reference_t<decltype(*p)>;

@@ -31,13 +31,14 @@ enum {
     ST_COUNT = 16
 };
 
-// Per-system parameters. Host fills p_off, n, c_off, col_off, b_off, G, Gb;
+// Per-system parameters. Host fills p_off, n, c_off, col_off, k_off, b_off, G, Gb;
 // the bounding-box kernels fill the FP64 box fields every step.
 struct SysDev {
     int64_t p_off;
     int64_t n;
     int64_t c_off;
     int64_t col_off;
+    int64_t k_off;   // first of the system's chunks of 64 particles
     int64_t b_off;   // first of the system's Gb x Gb blocks of RC_BLOCK x RC_BLOCK cells
     int32_t G;
     int32_t Gb;

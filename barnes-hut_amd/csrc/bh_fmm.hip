@@ -26,35 +26,6 @@
 #define FMM_IN 1.0001   // |coordinate| on a square up to which it counts as inside
 
 typedef double fd4 __attribute__((ext_vector_type(4)));
-typedef double fd8 __attribute__((ext_vector_type(8)));
-
-// Wave-uniform reads through the constant address space: scalar loads, so
-// every lane gets the value from a scalar register.
-template <typename T>
-using cptr = const T __attribute__((address_space(4)))*;
-
-template <typename T>
-__device__ __forceinline__ cptr<T> as_const(const T* p)
-{
-    return (cptr<T>)(uintptr_t)p;
-}
-
-// The power of two that brings the cell side into [1, 2): positions scaled by
-// it are exact, and a distance to another cell's COM is at least 1.
-__device__ __forceinline__ double step_scale(double step)
-{
-    if (!(step > 0.0) || !(step < __builtin_huge_val())) return 1.0;
-    int e2;
-    (void)frexp(step, &e2);
-    return ldexp(1.0, 1 - e2);
-}
-
-__device__ __forceinline__ double rcp64(double q)
-{
-    const double r0 = __builtin_amdgcn_rcp(q);
-    const double e = fma(-q, r0, 1.0);
-    return fma(r0, fma(e, e, e), r0);
-}
 
 // ---------------------------------------------------------------- tiles
 // Eight lanes per tile add up its columns' particles and non-empty cells; the
@@ -542,37 +513,6 @@ __global__ __launch_bounds__(256) void k_fmm_pack(FmmArgs A)
     }
 }
 
-// Two terms of the law from one reciprocal: Q = q0 q1, R = 1 / Q, so the
-// weights are (m0 R) q1 and (m1 R) q0.  An entry that the particle does not
-// keep enters as q = 1 with weight 0.
-template <int LAW, bool MASK>
-__device__ __forceinline__ void pair_terms(double X0, double Y0, double m0, double X1, double Y1,
-                                           double m1, double x, double y, bool k0, bool k1,
-                                           double eps2, double r2cut, double& sx, double& sy)
-{
-    const double wx0 = X0 - x, wy0 = Y0 - y, wx1 = X1 - x, wy1 = Y1 - y;
-    double q0 = fma(wx0, wx0, fma(wy0, wy0, eps2)), q1 = fma(wx1, wx1, fma(wy1, wy1, eps2));
-    if (LAW == 1) {
-        const bool c0 = fma(wx0, wx0, wy0 * wy0) > r2cut, c1 = fma(wx1, wx1, wy1 * wy1) > r2cut;
-        k0 = MASK ? k0 && c0 : c0;
-        k1 = MASK ? k1 && c1 : c1;
-    }
-    if (MASK || LAW == 1) {
-        q0 = k0 ? q0 : 1.0;
-        q1 = k1 ? q1 : 1.0;
-    }
-    const double R = rcp64(q0 * q1);
-    double w0 = (m0 * R) * q1, w1 = (m1 * R) * q0;
-    if (MASK || LAW == 1) {
-        w0 = k0 ? w0 : 0.0;
-        w1 = k1 ? w1 : 0.0;
-    }
-    sx = fma(wx0, w0, sx);
-    sy = fma(wy0, w0, sy);
-    sx = fma(wx1, w1, sx);
-    sy = fma(wy1, w1, sy);
-}
-
 // A lane's own near candidates in column xc (OWN: its own column, which holds
 // the particle itself).  gi < 0: no particle.
 template <int LAW, bool OWN>
@@ -589,7 +529,7 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
         const bool two = j + 1 < b;
         const FmmPart* E1 = two ? E + 1 : E;
         const double m1 = two ? E1->m : 0.0;
-        pair_terms<LAW, OWN>(E->x, E->y, E->m, E1->x, E1->y, m1, x, y, j != gi,
+        pair_terms<LAW, OWN>(E->x - x, E->y - y, E->m, E1->x - x, E1->y - y, m1, j != gi,
                              (two ? j + 1 : j) != gi, eps2, r2cut, sx, sy);
     }
 }
@@ -673,28 +613,28 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                     if (dx == 0 && row >= cyl && row <= cyh) {   // some lanes' own cell
                         for (; j + 1 < b; j += 2) {
                             const fd8 f = *(cptr<fd8>)(E + j);
-                            pair_terms<LAW, true>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, j != gi,
+                            pair_terms<LAW, true>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], j != gi,
                                                   j + 1 != gi, eps2, r2cut, sx, sy);
                         }
                         if (j < b)
-                            pair_terms<LAW, true>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, 0.0, x, y,
+                            pair_terms<LAW, true>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0,
                                                   j != gi, j != gi, eps2, r2cut, sx, sy);
                     } else {
                         for (; j + 3 < b; j += 4) {
                             const fd8 f = *(cptr<fd8>)(E + j), h2 = *(cptr<fd8>)(E + j + 2);
-                            pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true,
+                            pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true,
                                                    true, eps2, r2cut, sx, sy);
-                            pair_terms<LAW, false>(h2[0], h2[1], h2[2], h2[4], h2[5], h2[6], x, y,
+                            pair_terms<LAW, false>(h2[0] - x, h2[1] - y, h2[2], h2[4] - x, h2[5] - y, h2[6],
                                                    true, true, eps2, r2cut, sx, sy);
                         }
                         if (j + 1 < b) {
                             const fd8 f = *(cptr<fd8>)(E + j);
-                            pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true,
+                            pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true,
                                                    true, eps2, r2cut, sx, sy);
                             j += 2;
                         }
                         if (j < b)
-                            pair_terms<LAW, false>(E[j].x, E[j].y, E[j].m, E[j].x, E[j].y, 0.0, x, y,
+                            pair_terms<LAW, false>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0,
                                                    true, true, eps2, r2cut, sx, sy);
                     }
                 }
@@ -725,9 +665,9 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                 if (!touch) {
                     for (int e = 0; e < ne; e += 4) {
                         const fd8 f = E[e >> 1], h2 = E[(e >> 1) + 1];
-                        pair_terms<LAW, false>(f[0], f[1], f[2], f[4], f[5], f[6], x, y, true, true,
+                        pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true, true,
                                                eps2, r2cut, sx, sy);
-                        pair_terms<LAW, false>(h2[0], h2[1], h2[2], h2[4], h2[5], h2[6], x, y, true,
+                        pair_terms<LAW, false>(h2[0] - x, h2[1] - y, h2[2], h2[4] - x, h2[5] - y, h2[6], true,
                                                true, eps2, r2cut, sx, sy);
                     }
                 } else {
@@ -737,7 +677,7 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                         const long long c1 = __double_as_longlong(f[7]);
                         const int kx0 = (int)c0, ky0 = (int)(c0 >> 32);
                         const int kx1 = (int)c1, ky1 = (int)(c1 >> 32);
-                        pair_terms<LAW, true>(f[0], f[1], f[2], f[4], f[5], f[6], x, y,
+                        pair_terms<LAW, true>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6],
                                               (unsigned)(kx0 - cx + 1) > 2u || (unsigned)(ky0 - cy + 1) > 2u,
                                               (unsigned)(kx1 - cx + 1) > 2u || (unsigned)(ky1 - cy + 1) > 2u,
                                               eps2, r2cut, sx, sy);

@@ -421,6 +421,244 @@ __global__ __launch_bounds__(64) void k_force64(ForceArgs A)
     }
 }
 
+// ---------------------------------------------------------------- FP64, shared chunks
+// The terms of k_force64<.., FAST 1>, with the work of 64 particles shared by
+// the W waves of a block: each wave takes every W-th group of near candidates
+// and the w-th slice of the COM list, and the waves' sums are added in wave
+// order.  A pass has N / 64 W waves instead of N / 128 and each a W-th of the
+// chain, so small passes fill the chip; the terms come by scalar loads, so
+// they cost neither LDS reads nor a staging round per tile.  A chunk is 64
+// consecutive sorted particles of one system: a particle's terms and their
+// order depend on its system alone.
+//
+// Near candidates: if the chunk lies in one column and spans two rows at most
+// (dense cells), its waves walk the union of the lanes' cells, four candidates
+// at a time; else each lane walks its own three ranges with vector loads.
+//
+// Force pass against the one-wave kernel (uniform particles): 2,000 on 11^2
+// cells 90 -> 16 us, 16,384 on 32^2 152 -> 21 us, 262,144 on 256^2 10.4 -> 6.0 ms
+// (2.9e12 terms/s), 1M on 32^2 (8.8e9 near pairs) 7.3 -> 4.3 ms; no size was
+// slower, so only the cost log, which times work items, still takes k_force64.
+// Loading each quad one ahead of its use is worth 15 % and, where the
+// candidates of a cell exceed an XCD's L2, a third.  W = 4 and 16 are within
+// 10 % of W = 8 from 65k particles on and slower below (W = 4: 29 against 24 us
+// at 16,384) or above (W = 16).
+typedef double fd4a __attribute__((ext_vector_type(4), aligned(8)));
+
+struct Four {   // four candidates in scalar registers
+    double X[4], Y[4], M[4];
+};
+
+// Candidates j .. j + 3 of [j, b); those past b are copies of j without mass.
+__device__ __forceinline__ Four load_four(const double* x, const double* y, const double* m, int j,
+                                          int b, int N)
+{
+    Four f;
+    if (j + 4 <= N) {
+        const fd4a X = *(cptr<fd4a>)as_const(x + j), Y = *(cptr<fd4a>)as_const(y + j);
+        const fd4a M = *(cptr<fd4a>)as_const(m + j);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            f.X[u] = X[u];
+            f.Y[u] = Y[u];
+            f.M[u] = M[u];
+        }
+    } else {   // the last rows of the arrays
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = min(j + u, N - 1);
+            f.X[u] = as_const(x)[k];
+            f.Y[u] = as_const(y)[k];
+            f.M[u] = as_const(m)[k];
+        }
+    }
+#pragma unroll
+    for (int u = 1; u < 4; ++u)
+        if (j + u >= b) {
+            f.X[u] = f.X[0];
+            f.Y[u] = f.Y[0];
+            f.M[u] = 0.0;
+        }
+    return f;
+}
+
+template <int LAW, bool OWN>
+__device__ __forceinline__ void near_four(const Four& f, int j, int b, int gi, double x, double y,
+                                          double sig, double eps2, double r2cut, double& sx,
+                                          double& sy)
+{
+#pragma unroll
+    for (int u = 0; u < 4; u += 2)
+        pair_terms<LAW, OWN>(fma(f.X[u], sig, -x), fma(f.Y[u], sig, -y), f.M[u],
+                             fma(f.X[u + 1], sig, -x), fma(f.Y[u + 1], sig, -y), f.M[u + 1],
+                             (j + u < b ? j + u : j) != gi, (j + u + 1 < b ? j + u + 1 : j) != gi,
+                             eps2, r2cut, sx, sy);
+}
+
+// Every (4 W)-th group of four of [j, b), the next one loaded ahead.
+template <int W, int LAW, bool OWN>
+__device__ __forceinline__ void near_cell(const ForceArgs& A, int j, int b, int N, int gi, double x,
+                                          double y, double sig, double eps2, double r2cut,
+                                          double& sx, double& sy)
+{
+    if (j >= b) return;
+    Four f = load_four(A.x, A.y, A.m, j, b, N);
+    for (;;) {
+        const int jn = j + 4 * W;
+        Four n = f;
+        if (jn < b) n = load_four(A.x, A.y, A.m, jn, b, N);
+        near_four<LAW, OWN>(f, j, b, gi, x, y, sig, eps2, r2cut, sx, sy);
+        if (jn >= b) break;
+        f = n;
+        j = jn;
+    }
+}
+
+template <int W, int LAW>
+__global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
+{
+    __shared__ double part[2][W][BH_WAVE];
+    const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
+    const int64_t ci = A.chunk0 + blockIdx.x;
+    int s = 0;
+    if (S > 1) {   // the system of the chunk
+        int hi = S - 1;
+        while (s < hi) {
+            const int mid = (s + hi + 1) >> 1;
+            if (A.sys[mid].k_off <= ci) s = mid; else hi = mid - 1;
+        }
+        s = uniform_int(s);
+    }
+    const SysDev& d = A.sys[s];
+    const int G = d.G;
+    const int64_t coff = d.c_off;
+    const int rank = (int)(ci - d.k_off) * 64 + lane;
+    const bool act = rank < d.n;
+    const int gi = act ? (int)d.p_off + rank : -1;
+    const double sig = step_scale(d.step);
+    const double eps2 = A.eps2 * sig * sig, r2cut = A.r2cut * sig * sig;
+    double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0;
+    int cx = -100000, cy = -100000;
+    if (act) {
+        x = A.x[gi] * sig;
+        y = A.y[gi] * sig;
+        const int key = A.key_sorted[gi] - (int)coff;
+        cx = key / G;
+        cy = key - cx * G;
+    }
+    const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
+    const int cxh = uniform_int(wave_max(act ? cx : -1));
+    const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
+    const int cyh = uniform_int(wave_max(act ? cy : -1));
+
+    // near candidates
+    if (cxl == cxh && cyh - cyl < 2) {
+        int turn = 0;   // groups of four so far, dealt to the waves in turn
+        for (int dx = -1; dx <= 1; ++dx) {
+            const int xc = cxl + dx;
+            if (xc < 0 || xc >= G) continue;
+            const int64_t cl = coff + (int64_t)xc * G;
+            for (int row = max(cyl - 1, 0); row <= min(cyh + 1, G - 1); ++row) {
+                const int a = uniform_int(A.offsets[cl + row]);
+                const int b = uniform_int(A.offsets[cl + row + 1]);
+                const int first = (w - turn) & (W - 1);
+                turn += (b - a + 3) >> 2;
+                if (!(act && abs(row - cy) <= 1)) continue;
+                if (dx == 0 && row >= cyl && row <= cyh)   // some lanes' own cell
+                    near_cell<W, LAW, true>(A, a + 4 * first, b, (int)A.part_n, gi, x, y, sig, eps2,
+                                            r2cut, sx, sy);
+                else
+                    near_cell<W, LAW, false>(A, a + 4 * first, b, (int)A.part_n, gi, x, y, sig, eps2,
+                                             r2cut, sx, sy);
+            }
+        }
+    } else if (act) {
+        int n0 = 0, n1 = 0, n2 = 0, o0 = 0, o1 = 0, o2 = 0;   // the three ranges as one list
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int xc = cx + t - 1;
+            int a = 0, b = 0;
+            if (xc >= 0 && xc < G) {
+                const int64_t cl = coff + (int64_t)xc * G;
+                a = A.offsets[cl + max(cy - 1, 0)];
+                b = A.offsets[cl + min(cy + 1, G - 1) + 1];
+            }
+            if (t == 0) { o0 = a; n0 = b - a; }
+            if (t == 1) { o1 = a - n0; n1 = n0 + b - a; }
+            if (t == 2) { o2 = a - n1; n2 = n1 + b - a; }
+        }
+        for (int k = 2 * w; k < n2; k += 2 * W) {
+            const int k1 = min(k + 1, n2 - 1);
+            const int j0 = k + (k < n0 ? o0 : (k < n1 ? o1 : o2));
+            const int j1 = k1 + (k1 < n0 ? o0 : (k1 < n1 ? o1 : o2));
+            pair_terms<LAW, true>(fma(A.x[j0], sig, -x), fma(A.y[j0], sig, -y), A.m[j0],
+                                  fma(A.x[j1], sig, -x), fma(A.y[j1], sig, -y),
+                                  k + 1 < n2 ? A.m[j1] : 0.0, j0 != gi, j1 != gi, eps2, r2cut, sx,
+                                  sy);
+        }
+    }
+
+    // COM list: this wave's slice, a whole number of quads
+    const int ne0 = uniform_int(A.neprefix[coff]);
+    const int ne1 = uniform_int(A.neprefix[coff + (int64_t)G * G]);
+    const int mlo = uniform_int(A.neprefix[coff + (int64_t)max(cxl - 1, 0) * G]);
+    const int mhi = uniform_int(A.neprefix[coff + (int64_t)min(cxh + 2, G) * G]);
+    const int per = (((ne1 - ne0 + W - 1) / W) + 3) & ~3;
+    const int f0 = min(ne1, ne0 + w * per), f1 = min(ne1, f0 + per);
+    if (f0 < f1) {
+        // the list is padded by a quad, so whole quads are in bounds
+        fd8 p = *(cptr<fd8>)(as_const(A.l64) + f0), q = *(cptr<fd8>)(as_const(A.l64) + f0 + 2);
+        for (int e = f0; e < f1; e += 4) {
+            const int en = e + 4 < f1 ? e + 4 : e;
+            const fd8 pn = *(cptr<fd8>)(as_const(A.l64) + en);
+            const fd8 qn = *(cptr<fd8>)(as_const(A.l64) + en + 2);
+            if (e + 4 > f1) {   // past the slice: its first entry again, without mass
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (u != 2 && e + 1 >= f1) p[4 + u] = p[u];
+                    if (u != 2 && e + 2 >= f1) q[u] = p[u];
+                    if (u != 2 && e + 3 >= f1) q[4 + u] = p[u];
+                }
+                if (e + 1 >= f1) p[6] = 0.0;
+                if (e + 2 >= f1) q[2] = 0.0;
+                q[6] = 0.0;
+            }
+            const double wx0 = fma(p[0], sig, -x), wy0 = fma(p[1], sig, -y);
+            const double wx1 = fma(p[4], sig, -x), wy1 = fma(p[5], sig, -y);
+            const double wx2 = fma(q[0], sig, -x), wy2 = fma(q[1], sig, -y);
+            const double wx3 = fma(q[4], sig, -x), wy3 = fma(q[5], sig, -y);
+            if (e + 4 <= mlo || e >= mhi) {
+                pair_terms<LAW, false>(wx0, wy0, p[2], wx1, wy1, p[6], true, true, eps2, r2cut, sx,
+                                       sy);
+                pair_terms<LAW, false>(wx2, wy2, q[2], wx3, wy3, q[6], true, true, eps2, r2cut, sx,
+                                       sy);
+            } else {
+                auto far = [&](double kxy) {
+                    const long long c = __double_as_longlong(kxy);
+                    return (unsigned)((int)c - cx + 1) > 2u ||
+                           (unsigned)((int)(c >> 32) - cy + 1) > 2u;
+                };
+                pair_terms<LAW, true>(wx0, wy0, p[2], wx1, wy1, p[6], far(p[3]), far(p[7]), eps2,
+                                      r2cut, sx, sy);
+                pair_terms<LAW, true>(wx2, wy2, q[2], wx3, wy3, q[6], far(q[3]), far(q[7]), eps2,
+                                      r2cut, sx, sy);
+            }
+            p = pn;
+            q = qn;
+        }
+    }
+    part[0][w][lane] = sx;
+    part[1][w][lane] = sy;
+    __syncthreads();
+    if (w < 2 && act) {   // wave 0 adds x, wave 1 adds y
+        double t = 0.0;
+#pragma unroll
+        for (int v = 0; v < W; ++v) t += part[w][v][lane];
+        double* a = w ? A.ay : A.ax;
+        a[gi] += A.Gc * (t * sig);
+    }
+}
+
 // ---------------------------------------------------------------- FP32
 // Positions in cell units relative to the item origin (cx, oy), oy = the
 // item's middle row: the integer cell offsets are exact in FP32, so a far
@@ -1043,4 +1281,11 @@ const void* bh_force_kernel(int precision, int pidx, int law)
 {
     if (precision < 0 || precision > 5 || pidx < 0 || pidx > 2 || law < 0 || law > 1) return nullptr;
     return (const void*)g_force[precision][pidx][law];
+}
+
+void bh_force64s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_t st)
+{
+    const dim3 g((unsigned)nchunks), b(64 * F64S_WAVES);
+    if (law) hipLaunchKernelGGL((k_force64s<F64S_WAVES, 1>), g, b, 0, st, A, S);
+    else hipLaunchKernelGGL((k_force64s<F64S_WAVES, 0>), g, b, 0, st, A, S);
 }

@@ -46,7 +46,12 @@ struct ForceArgs {
     // FP32 or the FP64 result to the particles' accelerations.  A flag rather
     // than a third pointer keeps the kernel's scalar registers unchanged.
     int rc;
+    int64_t chunk0;   // k_force64s: first chunk of 64 particles of this launch
 };
+
+#define F64S_WAVES 8   // waves that share 64 particles (a power of two)
+// k_force64s over nchunks chunks from A.chunk0 on.
+void bh_force64s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_t st);
 
 // Arguments of the grid-method potential (bh_potential.hip).
 struct PotArgs {
@@ -192,6 +197,66 @@ __device__ __forceinline__ double near_w64(double wx, double wy, double m, doubl
     const double s2 = fma(wx, wx, wy * wy);
     if (LAW == 0) return qdiv64<FAST>(m, s2 + eps2);
     return (s2 > r2cut) ? qdiv64<FAST>(m, s2 + eps2) : 0.0;
+}
+
+// Wave-uniform reads through the constant address space: scalar loads, so
+// every lane gets the value from a scalar register.
+typedef double fd8 __attribute__((ext_vector_type(8)));
+template <typename T>
+using cptr = const T __attribute__((address_space(4)))*;
+
+template <typename T>
+__device__ __forceinline__ cptr<T> as_const(const T* p)
+{
+    return (cptr<T>)(uintptr_t)p;
+}
+
+// The power of two that brings the cell side into [1, 2): positions scaled by
+// it are exact, and a distance to another cell's COM is at least 1.
+__device__ __forceinline__ double step_scale(double step)
+{
+    if (!(step > 0.0) || !(step < __builtin_huge_val())) return 1.0;
+    int e2;
+    (void)frexp(step, &e2);
+    return ldexp(1.0, 1 - e2);
+}
+
+// 1 / q as in wdiv64.
+__device__ __forceinline__ double rcp64(double q)
+{
+    const double r0 = __builtin_amdgcn_rcp(q);
+    const double e = fma(-q, r0, 1.0);
+    return fma(r0, fma(e, e, e), r0);
+}
+
+// Two terms of the law from one reciprocal: Q = q0 q1, R = 1 / Q, so the
+// weights are (m0 R) q1 and (m1 R) q0.  An entry that the particle does not
+// keep enters as q = 1 with weight 0.  (wx, wy): from the particle.
+template <int LAW, bool MASK>
+__device__ __forceinline__ void pair_terms(double wx0, double wy0, double m0, double wx1,
+                                           double wy1, double m1, bool k0, bool k1, double eps2,
+                                           double r2cut, double& sx, double& sy)
+{
+    double q0 = fma(wx0, wx0, fma(wy0, wy0, eps2)), q1 = fma(wx1, wx1, fma(wy1, wy1, eps2));
+    if (LAW == 1) {
+        const bool c0 = fma(wx0, wx0, wy0 * wy0) > r2cut, c1 = fma(wx1, wx1, wy1 * wy1) > r2cut;
+        k0 = MASK ? k0 && c0 : c0;
+        k1 = MASK ? k1 && c1 : c1;
+    }
+    if (MASK || LAW == 1) {
+        q0 = k0 ? q0 : 1.0;
+        q1 = k1 ? q1 : 1.0;
+    }
+    const double R = rcp64(q0 * q1);
+    double w0 = (m0 * R) * q1, w1 = (m1 * R) * q0;
+    if (MASK || LAW == 1) {
+        w0 = k0 ? w0 : 0.0;
+        w1 = k1 ? w1 : 0.0;
+    }
+    sx = fma(wx0, w0, sx);
+    sy = fma(wy0, w0, sy);
+    sx = fma(wx1, w1, sx);
+    sy = fma(wy1, w1, sy);
 }
 
 // grid-method potential
