@@ -513,6 +513,33 @@ __global__ __launch_bounds__(256) void k_fmm_pack(FmmArgs A)
     }
 }
 
+// A cell's particles [j, b) as near candidates of the whole wave, by scalar
+// loads.  (Loading a quad ahead, as k_force64s does, is 5 % slower here: the
+// second set of registers spills scalars that the outer loops hold.)
+template <int LAW, bool OWN>
+__device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int gi, double x,
+                                          double y, double eps2, double r2cut, double& sx,
+                                          double& sy)
+{
+    const cptr<FmmPart> E = as_const(pack);
+    for (; j + 3 < b; j += 4) {
+        const fd8 p = *(cptr<fd8>)(E + j), q = *(cptr<fd8>)(E + j + 2);
+        pair_terms<LAW, OWN>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
+                             j + 1 != gi, eps2, r2cut, sx, sy);
+        pair_terms<LAW, OWN>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6], j + 2 != gi,
+                             j + 3 != gi, eps2, r2cut, sx, sy);
+    }
+    if (j + 1 < b) {
+        const fd8 p = *(cptr<fd8>)(E + j);
+        pair_terms<LAW, OWN>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
+                             j + 1 != gi, eps2, r2cut, sx, sy);
+        j += 2;
+    }
+    if (j < b)   // the last of an odd count, with a copy of itself without mass
+        pair_terms<LAW, OWN>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0, j != gi,
+                             j != gi, eps2, r2cut, sx, sy);
+}
+
 // A lane's own near candidates in column xc (OWN: its own column, which holds
 // the particle itself).  gi < 0: no particle.
 template <int LAW, bool OWN>
@@ -597,8 +624,7 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
         const double ux = 2.0 * ((x / sig - d.min_x) / h - ttx) - 1.0;
         const double uy = 2.0 * ((y / sig - d.min_y) / h - tty) - 1.0;
 
-        // near pairs, two at a time; where a count is odd its last pair is the
-        // last particle and a copy of it without mass
+        // near pairs
         if (cxl == cxh && cyh - cyl < FMM_UNIFORM_ROWS) {
             for (int dx = -1; dx <= 1; ++dx) {
                 const int xc = cxl + dx;
@@ -608,35 +634,10 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                     const int a = uniform_int(A.offsets[cl + row]);
                     const int b = uniform_int(A.offsets[cl + row + 1]);
                     if (!(act && abs(row - cy) <= 1)) continue;
-                    const cptr<FmmPart> E = as_const(A.pack);
-                    int j = a;
-                    if (dx == 0 && row >= cyl && row <= cyh) {   // some lanes' own cell
-                        for (; j + 1 < b; j += 2) {
-                            const fd8 f = *(cptr<fd8>)(E + j);
-                            pair_terms<LAW, true>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], j != gi,
-                                                  j + 1 != gi, eps2, r2cut, sx, sy);
-                        }
-                        if (j < b)
-                            pair_terms<LAW, true>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0,
-                                                  j != gi, j != gi, eps2, r2cut, sx, sy);
-                    } else {
-                        for (; j + 3 < b; j += 4) {
-                            const fd8 f = *(cptr<fd8>)(E + j), h2 = *(cptr<fd8>)(E + j + 2);
-                            pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true,
-                                                   true, eps2, r2cut, sx, sy);
-                            pair_terms<LAW, false>(h2[0] - x, h2[1] - y, h2[2], h2[4] - x, h2[5] - y, h2[6],
-                                                   true, true, eps2, r2cut, sx, sy);
-                        }
-                        if (j + 1 < b) {
-                            const fd8 f = *(cptr<fd8>)(E + j);
-                            pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true,
-                                                   true, eps2, r2cut, sx, sy);
-                            j += 2;
-                        }
-                        if (j < b)
-                            pair_terms<LAW, false>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0,
-                                                   true, true, eps2, r2cut, sx, sy);
-                    }
+                    if (dx == 0 && row >= cyl && row <= cyh)   // some lanes' own cell
+                        near_cell<LAW, true>(A.pack, a, b, gi, x, y, eps2, r2cut, sx, sy);
+                    else
+                        near_cell<LAW, false>(A.pack, a, b, gi, x, y, eps2, r2cut, sx, sy);
                 }
             }
         } else {
@@ -651,6 +652,8 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
         const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
         const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
                          uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
+        // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
+        const bool plain = LAW == 0 || r2cut < 0.99;
         const int nt = fs.n[0];
         const int mx0 = all ? 0 : max(ttx - 1, 0), mx1 = all ? nt - 1 : min(ttx + 1, nt - 1);
         const int my0 = all ? 0 : max(tty - 1, 0), my1 = all ? nt - 1 : min(tty + 1, nt - 1);
@@ -662,25 +665,24 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                 // a tile that some lane's 3x3 cells may touch: each entry is tested
                 const bool touch = mx * T <= cxh + 1 && mx * T + T > cxl - 1 &&
                                    my * T <= cyh + 1 && my * T + T > cyl - 1;
-                if (!touch) {
+                if (!touch && plain) {
                     for (int e = 0; e < ne; e += 4) {
-                        const fd8 f = E[e >> 1], h2 = E[(e >> 1) + 1];
-                        pair_terms<LAW, false>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6], true, true,
-                                               eps2, r2cut, sx, sy);
-                        pair_terms<LAW, false>(h2[0] - x, h2[1] - y, h2[2], h2[4] - x, h2[5] - y, h2[6], true,
-                                               true, eps2, r2cut, sx, sy);
+                        const fd8 p = E[e >> 1], q = E[(e >> 1) + 1];
+                        pair_terms<0, false>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
+                                             true, true, eps2, r2cut, sx, sy);
+                        pair_terms<0, false>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6],
+                                             true, true, eps2, r2cut, sx, sy);
                     }
                 } else {
+                    auto far = [&](double kxy) {
+                        const long long c = __double_as_longlong(kxy);
+                        return (unsigned)((int)c - cx + 1) > 2u ||
+                               (unsigned)((int)(c >> 32) - cy + 1) > 2u;
+                    };
                     for (int e = 0; e < ne; e += 2) {
-                        const fd8 f = E[e >> 1];
-                        const long long c0 = __double_as_longlong(f[3]);
-                        const long long c1 = __double_as_longlong(f[7]);
-                        const int kx0 = (int)c0, ky0 = (int)(c0 >> 32);
-                        const int kx1 = (int)c1, ky1 = (int)(c1 >> 32);
-                        pair_terms<LAW, true>(f[0] - x, f[1] - y, f[2], f[4] - x, f[5] - y, f[6],
-                                              (unsigned)(kx0 - cx + 1) > 2u || (unsigned)(ky0 - cy + 1) > 2u,
-                                              (unsigned)(kx1 - cx + 1) > 2u || (unsigned)(ky1 - cy + 1) > 2u,
-                                              eps2, r2cut, sx, sy);
+                        const fd8 p = E[e >> 1];
+                        pair_terms<LAW, true>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
+                                              far(p[3]), far(p[7]), eps2, r2cut, sx, sy);
                     }
                 }
             }

@@ -605,6 +605,8 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
     const int mhi = uniform_int(A.neprefix[coff + (int64_t)min(cxh + 2, G) * G]);
     const int per = (((ne1 - ne0 + W - 1) / W) + 3) & ~3;
     const int f0 = min(ne1, ne0 + w * per), f1 = min(ne1, f0 + per);
+    // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
+    const bool plain = LAW == 0 || r2cut < 0.99;
     if (f0 < f1) {
         // the list is padded by a quad, so whole quads are in bounds
         fd8 p = *(cptr<fd8>)(as_const(A.l64) + f0), q = *(cptr<fd8>)(as_const(A.l64) + f0 + 2);
@@ -627,11 +629,11 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
             const double wx1 = fma(p[4], sig, -x), wy1 = fma(p[5], sig, -y);
             const double wx2 = fma(q[0], sig, -x), wy2 = fma(q[1], sig, -y);
             const double wx3 = fma(q[4], sig, -x), wy3 = fma(q[5], sig, -y);
-            if (e + 4 <= mlo || e >= mhi) {
-                pair_terms<LAW, false>(wx0, wy0, p[2], wx1, wy1, p[6], true, true, eps2, r2cut, sx,
-                                       sy);
-                pair_terms<LAW, false>(wx2, wy2, q[2], wx3, wy3, q[6], true, true, eps2, r2cut, sx,
-                                       sy);
+            if (plain && (e + 4 <= mlo || e >= mhi)) {
+                pair_terms<0, false>(wx0, wy0, p[2], wx1, wy1, p[6], true, true, eps2, r2cut, sx,
+                                     sy);
+                pair_terms<0, false>(wx2, wy2, q[2], wx3, wy3, q[6], true, true, eps2, r2cut, sx,
+                                     sy);
             } else {
                 auto far = [&](double kxy) {
                     const long long c = __double_as_longlong(kxy);
