@@ -103,7 +103,7 @@ struct bh_ctx_s {
     int64_t nchunks = 0;           // chunks of 64 particles of one system
     // grouped far field (bh_fmm.hip): which passes take it is a rule on the
     // systems' sizes (fmm_wanted)
-    bool fmm_on = false;
+    int fmm_on = 0;          // bit 0: fp64 passes, bit 1: fp32 passes
     FmmPlan fmm;
     FmmArgs fa = {};         // device buffers and sizes; the per-pass fields are set by each pass
     hipStream_t cap_stream = nullptr;   // graph capture only; replays run on the caller's stream
@@ -207,17 +207,29 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 }
 
 // Far terms of a pass (at most N x cells) from which the grouped far field
-// (bh_fmm.hip) is used, by passes of the fp64 and fp32 precisions.  At the
-// line a term-by-term pass takes ~5 ms in FP32 and ~9 ms in FP64 and the
-// grouped one 1.1 and 2.4 ms (600,001 uniform particles, 193^2 cells: 2.2e10
-// terms); the two meet near 3e9 terms.  The line is above that because short
-// passes over many uneven systems are where a learned queue order shortens
-// the term-by-term pass, and because the allocation-free step (at most 1.7e10
-// terms) has no scratch for the squares and gives the bits of bh_step.
-static constexpr double FMM_MIN_TERMS = 2e10;
+// (bh_fmm.hip) is used, per precision.
+//
+// fp64: a term-by-term pass (k_force64s) and a grouped one took, on uniform and
+// on clustered particles,
+//   131,072 on  90^2 (1.1e9 terms)  0.50, 0.61 ms    0.53, 0.98 ms
+//   600,000 on  60^2 (2.2e9)        1.36, 4.12       1.40, 4.09
+//   262,144 on 128^2 (4.3e9)        1.63, 1.85       0.58, 1.20
+//   600,000 on 110^2 (7.3e9)        2.90, 3.96       0.80, 2.35
+//   1M      on 140^2 (2.0e10)       7.36, 9.17       1.20, 3.44
+// so they meet below the line.  The allocation-free step has no scratch for the
+// squares and gives the bits of bh_step, so single systems within its limits
+// stay term by term (at most 1.7e10 terms, 6 ms).
+// fp32: at 2.2e10 terms (600,001 particles, 193^2 cells) 4.5 and 1.1 ms.  The
+// line is above the crossing because short FP32 passes over many uneven
+// systems are where a learned queue order shortens the pass (it orders work
+// items, which grouped passes do not have), and because the recompute, whose
+// flags callers read, belongs to the term-by-term pass.
+static constexpr double FMM_MIN_TERMS_FP64 = 4e9;
+static constexpr double FMM_MIN_TERMS_FP32 = 2e10;
 static constexpr size_t FMM_MAX_BYTES = (size_t)48 << 30;
 
-static bool fmm_wanted(const std::vector<SysDev>& sh)
+// Bit 0: fp64 passes, bit 1: fp32 passes.
+static int fmm_wanted(const std::vector<SysDev>& sh)
 {
     double terms = 0.0, tiles = 0.0;
     int64_t side = 0;
@@ -228,10 +240,15 @@ static bool fmm_wanted(const std::vector<SysDev>& sh)
         tiles += n0 * n0 * (4.0 / 3.0);
         side = std::max(side, cdiv(d.G, FMM_TILE));
     }
-    // a nearly empty huge grid has more squares to serve than terms to save
-    return terms >= FMM_MIN_TERMS && terms >= 1e6 * tiles &&
-           tiles * 3.0 * FMM_P64 * FMM_P64 * sizeof(double) <= (double)FMM_MAX_BYTES &&
-           side <= 1024;   // a level's node masses are addressed with 32 bits
+    // a nearly empty huge grid has more squares to serve than terms to save;
+    // a level's node masses are addressed with 32 bits
+    if (terms < 1e6 * tiles || side > 1024 ||
+        tiles * 3.0 * FMM_P64 * FMM_P64 * sizeof(double) > (double)FMM_MAX_BYTES)
+        return 0;
+    const bool noalloc = sh.size() == 1 && sh[0].n <= BH_NOALLOC_MAX_N &&
+                         sh[0].G <= BH_NOALLOC_MAX_GRID;
+    return (terms >= FMM_MIN_TERMS_FP64 && !noalloc ? 1 : 0) |
+           (terms >= FMM_MIN_TERMS_FP32 ? 2 : 0);
 }
 
 // Chebyshev nodes, transform and parent-child interpolation for P nodes.
@@ -263,8 +280,9 @@ static std::vector<double> fmm_table(int P)
 // buffers (c->sys_h and the sizes are set).
 static int fmm_configure(Ctx* c)
 {
-    c->fmm_on = false;
-    if (!fmm_wanted(c->sys_h)) return BH_OK;
+    c->fmm_on = 0;
+    const int wanted = fmm_wanted(c->sys_h);
+    if (!wanted) return BH_OK;
     const int S = c->S;
     std::vector<FmmSys> fs(S);
     int nlev = 0;
@@ -286,6 +304,12 @@ static int fmm_configure(Ctx* c)
     std::vector<FmmTile> tiles;
     std::vector<FmmGroup> groups;
     int64_t slots = 0;
+    // 64 targets share a wave's slice of the law; where that leaves fewer waves
+    // than SIMDs, 16 (a wave then takes 0.3 instead of 0.8 ms at P = 20)
+    int64_t squares = 0;
+    for (const FmmSys& f : fs)
+        for (int l = 0; l < f.nlev; ++l) squares += (int64_t)f.n[l] * f.n[l];
+    const int gsize = squares < 64 * 48 ? 16 : 64;
     for (int l = 0; l < nlev; ++l) {
         a.lev_off[l] = (int64_t)tiles.size();
         for (int s = 0; s < S; ++s) {
@@ -301,8 +325,9 @@ static int fmm_configure(Ctx* c)
             for (int p = 0; p < 4; ++p) {
                 const int ga = p >> 1, gb = p & 1;
                 const int cnt = ((n - ga + 1) / 2) * ((n - gb + 1) / 2);
-                for (int t0 = 0; t0 < cnt; t0 += 64)
-                    groups.push_back({s, t0, (int16_t)l, (int8_t)ga, (int8_t)gb});
+                for (int t0 = 0; t0 < cnt; t0 += gsize)
+                    groups.push_back({s, t0, std::min(gsize, cnt - t0), (int16_t)l, (int8_t)ga,
+                                      (int8_t)gb});
             }
         }
     }
@@ -332,7 +357,7 @@ static int fmm_configure(Ctx* c)
     if ((r = dalloc(c, &dfs, S)) || (r = dalloc(c, &dt, a.ntiles)) ||
         (r = dalloc(c, &dg, (int64_t)groups.size())) || (r = dalloc(c, &a.tcnt, a.ntiles)) ||
         (r = dalloc(c, &a.tstart, a.nleaf)) || (r = dalloc(c, &a.tne, a.nleaf)) ||
-        (r = dalloc(c, &a.cnt, 2 + S)) || (r = dalloc(c, &a.chunks, a.max_chunks)) ||
+        (r = dalloc(c, &a.cnt, FMM_NCNT + S)) || (r = dalloc(c, &a.chunks, a.max_chunks)) ||
         (r = dalloc(c, &a.list, c->C + 4 * a.nleaf)) || (r = dalloc(c, &a.pack, c->N)) ||
         (r = dalloc(c, &a.loc, a.ntiles * 2 * Q)))
         return r;
@@ -344,7 +369,7 @@ static int fmm_configure(Ctx* c)
     HIP_TRY(hipMemcpy(dfs, fs.data(), sizeof(FmmSys) * S, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dt, tiles.data(), sizeof(FmmTile) * tiles.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dg, groups.data(), sizeof(FmmGroup) * groups.size(), hipMemcpyHostToDevice));
-    a.sbad = a.cnt + 2;
+    a.sbad = a.cnt + FMM_NCNT;
     a.fsys = dfs;
     a.tiles = dt;
     a.groups = dg;
@@ -354,7 +379,7 @@ static int fmm_configure(Ctx* c)
     a.neprefix = c->neprefix;
     a.key_sorted = c->key_sorted;
     a.l64 = c->l64;
-    c->fmm_on = true;
+    c->fmm_on = wanted;
     return BH_OK;
 }
 
@@ -423,7 +448,7 @@ static void unconfigure(Ctx* c)
     c->sys_h.clear();
     c->energy_buf = nullptr;
     c->rc_ready = 0;
-    c->fmm_on = false;
+    c->fmm_on = 0;
 }
 
 // Allocates and initialises the buffers for sizes already validated by
@@ -809,7 +834,7 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     const void* fn = bh_force_kernel(precision, pidx, lawi);
     if (!fn) return fail(BH_EINVAL, "no force kernel for this configuration");
     ForceArgs fa;
-    if (c->fmm_on && (precision == 0 || precision == 1) && !c->cost_log_on) {
+    if ((precision == 0 || precision == 1) && (c->fmm_on >> precision & 1) && !c->cost_log_on) {
         // Grouped far field: its chunks replace the work items, so the queue
         // order does not enter.  Near and mid terms are FP64 in both
         // precisions: nothing is left for the recompute to mend.

@@ -29,16 +29,19 @@ typedef double fd4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- tiles
 // Eight lanes per tile add up its columns' particles and non-empty cells; the
-// block reserves a run of the chunk list (64 particles of one tile each) and
-// of the tile-ordered COM list with one atomic.  The order of the runs varies
-// from launch to launch; no result depends on it.
+// block reserves runs of the chunk list (64 particles of one tile each) and of
+// the tile-ordered COM list with one atomic each.  Chunks of dense tiles, whose
+// particles have many near candidates, fill the chunk list from its start (a
+// block shares each of them), the others from its end (a wave each).  The
+// order of the runs varies from launch to launch; no result depends on it.
 __global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
 {
-    __shared__ int wc[4], we[4], base_c, base_e;
+    __shared__ int wc[4], we[4], wd[4], base_c, base_e, base_d;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int64_t t = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
     const int sub = threadIdx.x & 7;
     int np = 0, ne = 0;
+    float n2 = 0.0f;   // sum of squared cell counts
     FmmTile tl = {0, 0, 0};
     if (t < A.nleaf) {
         tl = A.tiles[t];
@@ -48,7 +51,13 @@ __global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
         const int x1 = min(x0 + T, d.G), y1 = min(y0 + T, d.G);
         for (int x = x0 + sub; x < x1; x += 8) {
             const int64_t cl = d.c_off + (int64_t)x * d.G;
-            np += A.offsets[cl + y1] - A.offsets[cl + y0];
+            int a = A.offsets[cl + y0];
+            for (int y = y0; y < y1; ++y) {
+                const int b = A.offsets[cl + y + 1];
+                n2 += (float)(b - a) * (float)(b - a);
+                np += b - a;
+                a = b;
+            }
             ne += A.neprefix[cl + y1] - A.neprefix[cl + y0];
         }
     }
@@ -56,49 +65,59 @@ __global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
     for (int o = 1; o < 8; o <<= 1) {
         np += __shfl_xor(np, o, BH_WAVE);
         ne += __shfl_xor(ne, o, BH_WAVE);
+        n2 += __shfl_xor(n2, o, BH_WAVE);
     }
-    const int nc = (np + 63) >> 6;
+    const bool dense = n2 > (float)FMM_DENSE * (float)np;
+    const int nch = (np + 63) >> 6;
+    const int nc = dense ? 0 : nch, nd = dense ? nch : 0;
     const int ner = (ne + 3) & ~3;   // a tile's run of the list is padded to whole quads
     // exclusive prefix over the wave's eight tiles
-    int pc = nc, pe = ner;
+    int pc = nc, pe = ner, pd = nd;
 #pragma unroll
     for (int o = 8; o < 64; o <<= 1) {
         const int a = __shfl_up(pc, o, BH_WAVE), b = __shfl_up(pe, o, BH_WAVE);
+        const int g = __shfl_up(pd, o, BH_WAVE);
         if (lane >= o) {
             pc += a;
             pe += b;
+            pd += g;
         }
     }
     if (lane == 63) {
         wc[wid] = pc;
         we[wid] = pe;
+        wd[wid] = pd;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int c = 0, e = 0;
+        int c = 0, e = 0, g = 0;
         for (int w = 0; w < 4; ++w) {
-            const int a = wc[w], b = we[w];
+            const int a = wc[w], b = we[w], v = wd[w];
             wc[w] = c;
             we[w] = e;
+            wd[w] = g;
             c += a;
             e += b;
+            g += v;
         }
-        base_c = c ? atomicAdd(&A.cnt[0], c) : 0;
-        base_e = e ? atomicAdd(&A.cnt[1], e) : 0;
+        base_c = c ? atomicAdd(&A.cnt[FMM_LIGHT], c) : 0;
+        base_e = e ? atomicAdd(&A.cnt[FMM_LIST], e) : 0;
+        base_d = g ? atomicAdd(&A.cnt[FMM_HEAVY], g) : 0;
     }
     __syncthreads();
     if (t >= A.nleaf) return;
-    const int c0 = base_c + wc[wid] + pc - nc, e0 = base_e + we[wid] + pe - ner;
+    const int c0 = base_c + wc[wid] + pc - nc, d0 = base_d + wd[wid] + pd - nd;
+    const int e0 = base_e + we[wid] + pe - ner;
     if (sub == 0) {
         A.tcnt[t] = np;
         A.tstart[t] = e0;
         A.tne[t] = ne;
     }
-    for (int k = sub; k < nc; k += 8) {
+    for (int k = sub; k < nch; k += 8) {
         FmmChunk c;
         c.tile = (int32_t)t;
         c.k = k;
-        A.chunks[c0 + k] = c;
+        A.chunks[dense ? d0 + k : A.max_chunks - 1 - (c0 + k)] = c;
     }
 }
 
@@ -308,7 +327,7 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const FmmSys& fs = A.fsys[gr.sys];
     const int lev = gr.lev, n = fs.n[lev], off = fs.off[lev];
-    const int nx = (n - gr.a + 1) >> 1, ny = (n - gr.b + 1) >> 1;   // targets of this child position
+    const int ny = (n - gr.b + 1) >> 1;   // targets of this child position: columns of ny
     const int w = fmm_pitch(n);
     const int64_t plane = fmm_plane(n);
     const double* M = A.mult + fs.moff[lev] * Q;
@@ -320,7 +339,7 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int t = gr.t0 + 16 * b + c;
-        const bool ok = t < nx * ny;
+        const bool ok = 16 * b + c < gr.cnt;
         const int i = ok ? t / ny : 0, j = ok ? t - i * ny : 0;
         tx[b] = 2 * i + gr.a;
         ty[b] = 2 * j + gr.b;
@@ -412,8 +431,7 @@ __global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, const double* __re
     __syncthreads();
     const int gi = blockIdx.x / RB, rb = blockIdx.x - gi * RB;
     const FmmGroup gr = A.groups[gi];
-    const int n = A.fsys[gr.sys].n[gr.lev];
-    const int cnt = ((n - gr.a + 1) >> 1) * ((n - gr.b + 1) >> 1) - gr.t0;
+    const int cnt = gr.cnt;
     if (cnt > 32) m2l_wave<P, 4>(A, gr, rb, eps2, hn);
     else if (cnt > 16) m2l_wave<P, 2>(A, gr, rb, eps2, hn);
     else m2l_wave<P, 1>(A, gr, rb, eps2, hn);
@@ -513,16 +531,16 @@ __global__ __launch_bounds__(256) void k_fmm_pack(FmmArgs A)
     }
 }
 
-// A cell's particles [j, b) as near candidates of the whole wave, by scalar
-// loads.  (Loading a quad ahead, as k_force64s does, is 5 % slower here: the
+// Quads of a cell's particles from j on, `step` apart, before b, as near
+// candidates of the whole wave, by scalar loads.  (Loading a quad ahead, as k_force64s does, is 5 % slower here: the
 // second set of registers spills scalars that the outer loops hold.)
 template <int LAW, bool OWN>
 __device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int gi, double x,
-                                          double y, double eps2, double r2cut, double& sx,
+                                          double y, double eps2, double r2cut, int step, double& sx,
                                           double& sy)
 {
     const cptr<FmmPart> E = as_const(pack);
-    for (; j + 3 < b; j += 4) {
+    for (; j + 3 < b; j += step) {
         const fd8 p = *(cptr<fd8>)(E + j), q = *(cptr<fd8>)(E + j + 2);
         pair_terms<LAW, OWN>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
                              j + 1 != gi, eps2, r2cut, sx, sy);
@@ -541,18 +559,18 @@ __device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int
 }
 
 // A lane's own near candidates in column xc (OWN: its own column, which holds
-// the particle itself).  gi < 0: no particle.
+// the particle itself), every W-th pair from the w-th on.  gi < 0: no particle.
 template <int LAW, bool OWN>
 __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G, int xc, int cy,
-                                           int gi, double x, double y, double eps2, double r2cut,
-                                           double& sx, double& sy)
+                                           int gi, int w, int W, double x, double y, double eps2,
+                                           double r2cut, double& sx, double& sy)
 {
     if (gi < 0 || xc < 0 || xc >= G) return;
     const int64_t cl = coff + (int64_t)xc * G;
-    int j = A.offsets[cl + max(cy - 1, 0)];
+    int j = A.offsets[cl + max(cy - 1, 0)] + 2 * w;
     const int b = A.offsets[cl + min(cy + 1, G - 1) + 1];
     const FmmPart* E = A.pack + j;
-    for (; j < b; j += 2, E += 2) {
+    for (; j < b; j += 2 * W, E += 2 * W) {
         const bool two = j + 1 < b;
         const FmmPart* E1 = two ? E + 1 : E;
         const double m1 = two ? E1->m : 0.0;
@@ -561,143 +579,143 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
     }
 }
 
-// One wave per chunk of 64 particles of one tile.  The tile's coefficients
-// and the mid entries are the same for every lane: scalar loads of whole quads
-// (128 bytes), no test in tiles that no lane's 3x3 cells touch.  Near
-// candidates: if the wave lies in one column and spans at most
+// The terms of chunk ci's particles that fall to wave w of the W that share it
+// (a power of two): gi is the lane's particle (-1: none), (rx, ry) its sum.  The
+// tile's coefficients and the mid entries are the same for every lane: scalar
+// loads of whole quads (128 bytes), no test in tiles that no lane's 3x3 cells
+// touch.  Near candidates: if the chunk lies in one column and spans at most
 // FMM_UNIFORM_ROWS rows, the union of its lanes' ranges is walked with scalar
 // loads and a row test; otherwise each lane walks its own three ranges with
 // vector loads (a union would spend most of its pairs on the test).  Terms go
 // in pairs that share a reciprocal; only cells that hold the lanes themselves
-// are tested for the particle itself.  Bound by FP64 issue: ~12 slots a term,
-// 2.5e12 terms/s on 10M particles over 120^2 cells (6.7e10 near and mid terms,
-// 26.8 ms; 30.6 ms with entries loaded and tested one by one).
+// are tested for the particle itself.
 template <int P, int LAW>
-__global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2p,
-                                                  double r2cutp, int qpart, int nqparts)
+__device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int W, double eps2p,
+                                            double r2cutp, int& gi, double& rx, double& ry)
 {
     constexpr int Q = P * P;
-    const int lane = threadIdx.x;
-    const int total = A.cnt[0];
-    const int qb = (int)(((int64_t)total * qpart) / nqparts);
-    const int qe = (int)(((int64_t)total * (qpart + 1)) / nqparts);
-    for (int ci = qb + blockIdx.x; ci < qe; ci += gridDim.x) {
-        const FmmChunk ch = A.chunks[ci];
-        const int t = uniform_int(ch.tile);
-        const FmmTile tl = A.tiles[t];
-        const int s = uniform_int(tl.sys);
-        const int ttx = uniform_int(tl.tx), tty = uniform_int(tl.ty);
-        const SysDev& d = A.sys[s];
-        const FmmSys& fs = A.fsys[s];
-        const int G = d.G, T = fs.T;
-        const int64_t coff = d.c_off;
-        const double step = d.step, sig = step_scale(step);
-        const double eps2 = eps2p * sig * sig, r2cut = r2cutp * sig * sig;
-        const double h = (double)T * step;
-        const int x0 = ttx * T, y0 = tty * T, x1 = min(x0 + T, G), y1 = min(y0 + T, G);
+    const int lane = threadIdx.x & 63;
+    const FmmChunk ch = A.chunks[ci];
+    const int t = uniform_int(ch.tile);
+    const FmmTile tl = A.tiles[t];
+    const int s = uniform_int(tl.sys);
+    const int ttx = uniform_int(tl.tx), tty = uniform_int(tl.ty);
+    const SysDev& d = A.sys[s];
+    const FmmSys& fs = A.fsys[s];
+    const int G = d.G, T = fs.T;
+    const int64_t coff = d.c_off;
+    const double step = d.step, sig = step_scale(step);
+    const double eps2 = eps2p * sig * sig, r2cut = r2cutp * sig * sig;
+    const double h = (double)T * step;
+    const int x0 = ttx * T, y0 = tty * T, x1 = min(x0 + T, G), y1 = min(y0 + T, G);
 
-        // lane -> particle: rank 64 k + lane in the tile, columns in order
-        int r = 64 * uniform_int(ch.k) + lane, gi = -1;
-        for (int x = x0; x < x1; ++x) {
-            const int64_t cl = coff + (int64_t)x * G;
-            const int a = A.offsets[cl + y0], b = A.offsets[cl + y1];
-            if (gi < 0 && r < b - a) gi = a + r;
-            r -= b - a;
-        }
-        const bool act = gi >= 0;
-        double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, fx = 0.0, fy = 0.0;
-        int cx = -100000, cy = -100000;
-        if (act) {
-            const FmmPart p = A.pack[gi];
-            x = p.x;
-            y = p.y;
-            const int key = A.key_sorted[gi] - (int)coff;
-            cx = key / G;
-            cy = key - cx * G;
-        }
-        const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
-        const int cxh = uniform_int(wave_max(act ? cx : -1));
-        const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
-        const int cyh = uniform_int(wave_max(act ? cy : -1));
+    // lane -> particle: rank 64 k + lane in the tile, columns in order
+    int r = 64 * uniform_int(ch.k) + lane;
+    gi = -1;
+    for (int x = x0; x < x1; ++x) {
+        const int64_t cl = coff + (int64_t)x * G;
+        const int a = A.offsets[cl + y0], b = A.offsets[cl + y1];
+        if (gi < 0 && r < b - a) gi = a + r;
+        r -= b - a;
+    }
+    const bool act = gi >= 0;
+    double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, fx = 0.0, fy = 0.0;
+    int cx = -100000, cy = -100000;
+    if (act) {
+        const FmmPart p = A.pack[gi];
+        x = p.x;
+        y = p.y;
+        const int key = A.key_sorted[gi] - (int)coff;
+        cx = key / G;
+        cy = key - cx * G;
+    }
+    const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
+    const int cxh = uniform_int(wave_max(act ? cx : -1));
+    const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
+    const int cyh = uniform_int(wave_max(act ? cy : -1));
 
-        // the particle on its tile, [-1, 1]^2
-        const double ux = 2.0 * ((x / sig - d.min_x) / h - ttx) - 1.0;
-        const double uy = 2.0 * ((y / sig - d.min_y) / h - tty) - 1.0;
+    // the particle on its tile, [-1, 1]^2
+    const double ux = 2.0 * ((x / sig - d.min_x) / h - ttx) - 1.0;
+    const double uy = 2.0 * ((y / sig - d.min_y) / h - tty) - 1.0;
 
-        // near pairs
-        if (cxl == cxh && cyh - cyl < FMM_UNIFORM_ROWS) {
-            for (int dx = -1; dx <= 1; ++dx) {
-                const int xc = cxl + dx;
-                if (xc < 0 || xc >= G) continue;
-                const int64_t cl = coff + (int64_t)xc * G;
-                for (int row = max(cyl - 1, 0); row <= min(cyh + 1, G - 1); ++row) {
-                    const int a = uniform_int(A.offsets[cl + row]);
-                    const int b = uniform_int(A.offsets[cl + row + 1]);
-                    if (!(act && abs(row - cy) <= 1)) continue;
-                    if (dx == 0 && row >= cyl && row <= cyh)   // some lanes' own cell
-                        near_cell<LAW, true>(A.pack, a, b, gi, x, y, eps2, r2cut, sx, sy);
-                    else
-                        near_cell<LAW, false>(A.pack, a, b, gi, x, y, eps2, r2cut, sx, sy);
-                }
-            }
-        } else {
-            near_range<LAW, false>(A, coff, G, cx - 1, cy, gi, x, y, eps2, r2cut, sx, sy);
-            near_range<LAW, true>(A, coff, G, cx, cy, gi, x, y, eps2, r2cut, sx, sy);
-            near_range<LAW, false>(A, coff, G, cx + 1, cy, gi, x, y, eps2, r2cut, sx, sy);
-        }
-
-        // mid entries: 3x3 tiles, or every tile where the grouped part does not
-        // hold: a system of one tile, a cutoff that reaches past a tile, COMs
-        // outside their cells, particles moved since they were placed
-        const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
-        const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
-                         uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
-        // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
-        const bool plain = LAW == 0 || r2cut < 0.99;
-        const int nt = fs.n[0];
-        const int mx0 = all ? 0 : max(ttx - 1, 0), mx1 = all ? nt - 1 : min(ttx + 1, nt - 1);
-        const int my0 = all ? 0 : max(tty - 1, 0), my1 = all ? nt - 1 : min(tty + 1, nt - 1);
-        for (int mx = mx0; mx <= mx1; ++mx) {
-            for (int my = my0; my <= my1; ++my) {
-                const int mt = fs.off[0] + mx * nt + my;
-                const int e0 = uniform_int(A.tstart[mt]), ne = uniform_int(A.tne[mt]);
-                const cptr<fd8> E = (cptr<fd8>)(as_const(A.list) + e0);
-                // a tile that some lane's 3x3 cells may touch: each entry is tested
-                const bool touch = mx * T <= cxh + 1 && mx * T + T > cxl - 1 &&
-                                   my * T <= cyh + 1 && my * T + T > cyl - 1;
-                if (!touch && plain) {
-                    for (int e = 0; e < ne; e += 4) {
-                        const fd8 p = E[e >> 1], q = E[(e >> 1) + 1];
-                        pair_terms<0, false>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
-                                             true, true, eps2, r2cut, sx, sy);
-                        pair_terms<0, false>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6],
-                                             true, true, eps2, r2cut, sx, sy);
-                    }
-                } else {
-                    auto far = [&](double kxy) {
-                        const long long c = __double_as_longlong(kxy);
-                        return (unsigned)((int)c - cx + 1) > 2u ||
-                               (unsigned)((int)(c >> 32) - cy + 1) > 2u;
-                    };
-                    for (int e = 0; e < ne; e += 2) {
-                        const fd8 p = E[e >> 1];
-                        pair_terms<LAW, true>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
-                                              far(p[3]), far(p[7]), eps2, r2cut, sx, sy);
-                    }
-                }
+    // near pairs
+    if (cxl == cxh && cyh - cyl < FMM_UNIFORM_ROWS) {
+        int turn = 0;   // quads so far, dealt to the waves in turn
+        for (int dx = -1; dx <= 1; ++dx) {
+            const int xc = cxl + dx;
+            if (xc < 0 || xc >= G) continue;
+            const int64_t cl = coff + (int64_t)xc * G;
+            for (int row = max(cyl - 1, 0); row <= min(cyh + 1, G - 1); ++row) {
+                const int a = uniform_int(A.offsets[cl + row]);
+                const int b = uniform_int(A.offsets[cl + row + 1]);
+                const int j = a + 4 * ((w - turn) & (W - 1));
+                turn += (b - a + 3) >> 2;
+                if (!(act && abs(row - cy) <= 1)) continue;
+                if (dx == 0 && row >= cyl && row <= cyh)   // some lanes' own cell
+                    near_cell<LAW, true>(A.pack, j, b, gi, x, y, eps2, r2cut, 4 * W, sx, sy);
+                else
+                    near_cell<LAW, false>(A.pack, j, b, gi, x, y, eps2, r2cut, 4 * W, sx, sy);
             }
         }
+    } else {
+        near_range<LAW, false>(A, coff, G, cx - 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
+        near_range<LAW, true>(A, coff, G, cx, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
+        near_range<LAW, false>(A, coff, G, cx + 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
+    }
 
-        // distant part: the tile's Chebyshev series
-        if (!all && act) {
-            double ty[P];
-            ty[0] = 1.0;
-            ty[1] = uy;
+    // mid entries: 3x3 tiles, or every tile where the grouped part does not
+    // hold: a system of one tile, a cutoff that reaches past a tile, COMs
+    // outside their cells, particles moved since they were placed
+    const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
+    const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
+                     uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
+    // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
+    const bool plain = LAW == 0 || r2cut < 0.99;
+    const int nt = fs.n[0];
+    const int mx0 = all ? 0 : max(ttx - 1, 0), mx1 = all ? nt - 1 : min(ttx + 1, nt - 1);
+    const int my0 = all ? 0 : max(tty - 1, 0), my1 = all ? nt - 1 : min(tty + 1, nt - 1);
+    for (int mx = mx0; mx <= mx1; ++mx) {
+        for (int my = my0; my <= my1; ++my) {
+            const int mt = fs.off[0] + mx * nt + my;
+            const int e0 = uniform_int(A.tstart[mt]), ne = uniform_int(A.tne[mt]);
+            const cptr<fd8> E = (cptr<fd8>)(as_const(A.list) + e0);
+            // a tile that some lane's 3x3 cells may touch: each entry is tested
+            const bool touch = mx * T <= cxh + 1 && mx * T + T > cxl - 1 &&
+                               my * T <= cyh + 1 && my * T + T > cyl - 1;
+            if (!touch && plain) {
+                for (int e = 4 * w; e < ne; e += 4 * W) {
+                    const fd8 p = E[e >> 1], q = E[(e >> 1) + 1];
+                    pair_terms<0, false>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
+                                         true, true, eps2, r2cut, sx, sy);
+                    pair_terms<0, false>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6],
+                                         true, true, eps2, r2cut, sx, sy);
+                }
+            } else {
+                auto far = [&](double kxy) {
+                    const long long c = __double_as_longlong(kxy);
+                    return (unsigned)((int)c - cx + 1) > 2u ||
+                           (unsigned)((int)(c >> 32) - cy + 1) > 2u;
+                };
+                for (int e = 2 * w; e < ne; e += 2 * W) {
+                    const fd8 p = E[e >> 1];
+                    pair_terms<LAW, true>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
+                                          far(p[3]), far(p[7]), eps2, r2cut, sx, sy);
+                }
+            }
+        }
+    }
+
+    // distant part: the tile's Chebyshev series
+    if (!all && act) {
+        double ty[P];
+        ty[0] = 1.0;
+        ty[1] = uy;
 #pragma unroll
-            for (int l = 2; l < P; ++l) ty[l] = fma(2.0 * uy, ty[l - 1], -ty[l - 2]);
-            cptr<double> L = as_const(A.loc) + (int64_t)t * (2 * Q);
-            double a0 = 1.0, a1 = ux;
-            for (int k = 0; k < P; ++k) {
+        for (int l = 2; l < P; ++l) ty[l] = fma(2.0 * uy, ty[l - 1], -ty[l - 2]);
+        cptr<double> L = as_const(A.loc) + (int64_t)t * (2 * Q);
+        double a0 = 1.0, a1 = ux;
+        for (int k = 0; k < P; ++k) {
+            if ((k & (W - 1)) == w) {
                 double vx = 0.0, vy = 0.0;
 #pragma unroll
                 for (int l = 0; l < P; ++l) {
@@ -706,14 +724,70 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
                 }
                 fx = fma(a0, vx, fx);
                 fy = fma(a0, vy, fy);
-                const double an = fma(2.0 * ux, a1, -a0);
-                a0 = a1;
-                a1 = an;
             }
+            const double an = fma(2.0 * ux, a1, -a0);
+            a0 = a1;
+            a1 = an;
         }
-        if (act) {
-            A.ax[gi] += Gc * fma(sx, sig, fx);
-            A.ay[gi] += Gc * fma(sy, sig, fy);
+    }
+    rx = fma(sx, sig, fx);
+    ry = fma(sy, sig, fy);
+}
+
+// Chunks of dense tiles, each shared by the eight waves of a block: a particle
+// of a cluster's core may have 10^4 near candidates where the others have a
+// hundred, and on a wave of its own such a chunk would outlast the rest of the
+// pass.  1M particles, 400^2 cells, cores of 10^3 a cell: 10.7 -> 7.9 ms.
+template <int P, int LAW>
+__global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double Gc, double eps2,
+                                                              double r2cut, int qpart, int nqparts)
+{
+    __shared__ double part[2][FMM_WAVES][BH_WAVE];
+    __shared__ int unit;
+    const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
+    const int64_t n = A.cnt[FMM_HEAVY];
+    const int q0 = (int)(n * qpart / nqparts), q1 = (int)(n * (qpart + 1) / nqparts);
+    if (q0 >= q1) return;
+    for (;;) {
+        if (threadIdx.x == 0) unit = q0 + atomicAdd(&A.cnt[FMM_QHEAVY], 1);
+        __syncthreads();
+        const int ci = uniform_int(unit);
+        if (ci >= q1) break;
+        int gi;
+        double rx, ry;
+        chunk_terms<P, LAW>(A, ci, w, FMM_WAVES, eps2, r2cut, gi, rx, ry);
+        part[0][w][lane] = rx;
+        part[1][w][lane] = ry;
+        __syncthreads();
+        if (w < 2 && gi >= 0) {   // wave 0 adds x, wave 1 adds y
+            double t = 0.0;
+#pragma unroll
+            for (int v = 0; v < FMM_WAVES; ++v) t += part[w][v][lane];
+            double* a = w ? A.ay : A.ax;
+            a[gi] += Gc * t;
+        }
+    }
+}
+
+// The other chunks, a wave each.  The chunks are left to the hardware's
+// dispatch: a queue cursor (one atomic on the same word every ~15 ns) took 4.2M
+// particles from 2.2 to 3.5 ms, a fixed deal 512 systems from 10.0 to 12.4 ms.
+// Bound by FP64 issue, ~12 slots a term: 2.5e12 terms/s on 10M particles over
+// 120^2 cells (6.7e10 near and mid terms, 26.8 ms; 30.6 ms with entries loaded
+// and tested one by one).
+template <int P, int LAW>
+__global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2, double r2cut,
+                                                  int qpart, int nqparts)
+{
+    const int64_t n = A.cnt[FMM_LIGHT];
+    const int q0 = (int)(n * qpart / nqparts), q1 = (int)(n * (qpart + 1) / nqparts);
+    for (int u = q0 + blockIdx.x; u < q1; u += gridDim.x) {
+        int gi;
+        double rx, ry;
+        chunk_terms<P, LAW>(A, (int)(A.max_chunks - 1 - u), 0, 1, eps2, r2cut, gi, rx, ry);
+        if (gi >= 0) {
+            A.ax[gi] += Gc * rx;
+            A.ay[gi] += Gc * ry;
         }
     }
 }
@@ -724,7 +798,8 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
                         hipStream_t st)
 {
     const FmmTables& tb = P == 12 ? pl.tab[0] : pl.tab[1];
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt, (int64_t)(2 + A.S), 0);
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt,
+                       (int64_t)(FMM_NCNT + A.S), 0);
     hipLaunchKernelGGL(k_fmm_tiles, dim3((unsigned)((A.nleaf * 8 + 255) / 256)), dim3(256), 0, st,
                        A);
     const unsigned pg = (unsigned)((A.N + 255) / 256);
@@ -745,14 +820,17 @@ template <int P>
 static void fmm_force(const FmmArgs& A, double Gc, double eps2, double r2cut, int part, int nparts,
                       int num_cu, hipStream_t st)
 {
+    if (part > 0)   // the queue of this launch
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt + FMM_QHEAVY, (int64_t)1, 0);
     const int64_t cap = A.max_chunks, most = (int64_t)num_cu * 256;
-    const unsigned g = (unsigned)(cap < most ? cap : most);
-    if (r2cut > 0.0)
-        hipLaunchKernelGGL((k_fmm_force<P, 1>), dim3(g), dim3(64), 0, st, A, Gc, eps2, r2cut, part,
-                           nparts);
-    else
-        hipLaunchKernelGGL((k_fmm_force<P, 0>), dim3(g), dim3(64), 0, st, A, Gc, eps2, r2cut, part,
-                           nparts);
+    const dim3 gd(num_cu * 4), bd(64 * FMM_WAVES), g((unsigned)(cap < most ? cap : most)), b(64);
+    if (r2cut > 0.0) {
+        hipLaunchKernelGGL((k_fmm_dense<P, 1>), gd, bd, 0, st, A, Gc, eps2, r2cut, part, nparts);
+        hipLaunchKernelGGL((k_fmm_force<P, 1>), g, b, 0, st, A, Gc, eps2, r2cut, part, nparts);
+    } else {
+        hipLaunchKernelGGL((k_fmm_dense<P, 0>), gd, bd, 0, st, A, Gc, eps2, r2cut, part, nparts);
+        hipLaunchKernelGGL((k_fmm_force<P, 0>), g, b, 0, st, A, Gc, eps2, r2cut, part, nparts);
+    }
 }
 
 void bh_fmm_pass(const FmmArgs& args, const FmmPlan& pl, bool fp64, double Gc, double eps2,

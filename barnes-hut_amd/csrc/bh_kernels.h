@@ -75,6 +75,8 @@ struct PotArgs {
 #define FMM_P64 20           // and FP64 precision
 #define FMM_LEVELS 13        // levels of squares (grid_dim <= 32767)
 #define FMM_MIN_GRID 32      // smaller grids are one tile, every COM taken on its own
+#define FMM_WAVES 8          // waves that share a chunk of a dense tile (a power of two)
+#define FMM_DENSE 512        // mean cell count a particle sees from which its tile is dense
 #define FMM_UNIFORM_ROWS 2   // rows a wave may span to walk its near candidates together
 
 // A system: T cells per tile side, nlev levels of squares (0: one tile, no
@@ -93,8 +95,8 @@ struct FmmTile {
 struct FmmChunk {   // particles [64 k, 64 k + 64) of a tile
     int32_t tile, k;
 };
-struct FmmGroup {   // targets t0 .. t0 + 63 of the squares (2 i + a, 2 j + b) of a level
-    int32_t sys, t0;
+struct FmmGroup {   // targets t0 .. t0 + cnt - 1 (at most 64) of a level's squares (2 i + a, 2 j + b)
+    int32_t sys, t0, cnt;
     int16_t lev;
     int8_t a, b;
 };
@@ -104,6 +106,14 @@ struct alignas(32) FmmCom {   // COM in units of step_scale, tile order
 };
 struct alignas(32) FmmPart {
     double x, y, m, pad;
+};
+
+enum {   // FmmArgs::cnt: chunks of dense tiles, of the others, list entries, dense queue cursor
+    FMM_HEAVY,
+    FMM_LIGHT,
+    FMM_LIST,
+    FMM_QHEAVY,
+    FMM_NCNT
 };
 
 struct FmmArgs {
@@ -117,7 +127,7 @@ struct FmmArgs {
     const FmmGroup* groups;
     int32_t *tcnt;             // per square: particles
     int32_t *tstart, *tne;     // per tile: its run of list
-    int32_t* cnt;              // chunks, list entries, then per system sbad
+    int32_t* cnt;              // FMM_HEAVY .. FMM_QHEAVY, then per system sbad
     int32_t* sbad;             // != 0: a COM lies outside its cell
     FmmChunk* chunks;
     FmmCom* list;
