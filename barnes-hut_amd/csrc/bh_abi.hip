@@ -257,22 +257,28 @@ static std::vector<double> fmm_table(int P)
     std::vector<double> v(P + 3 * P * P);
     double *nodes = v.data(), *cheb = nodes + P, *shift = cheb + P * P;
     const long double pi = 3.14159265358979323846264338327950288L;
-    auto T = [&](int k, long double u) { return cosl(k * acosl(u)); };
-    std::vector<long double> x(P);
+    std::vector<long double> x(P), t(P);
+    std::vector<long double> tn(P * P);   // T_k(node i)
+    auto chebyshev = [&](long double u, long double* T) {
+        T[0] = 1.0L;
+        T[1] = u;
+        for (int k = 2; k < P; ++k) T[k] = 2.0L * u * T[k - 1] - T[k - 2];
+    };
     for (int i = 0; i < P; ++i) {
         x[i] = cosl((2 * i + 1) * pi / (2 * P));
         nodes[i] = (double)x[i];
+        chebyshev(x[i], &tn[i * P]);
+        for (int k = 0; k < P; ++k) cheb[k * P + i] = (double)((k ? 2.0L : 1.0L) / P * tn[i * P + k]);
     }
-    for (int k = 0; k < P; ++k)
-        for (int i = 0; i < P; ++i) cheb[k * P + i] = (double)((k ? 2.0L : 1.0L) / P * T(k, x[i]));
     for (int a = 0; a < 2; ++a)
-        for (int i = 0; i < P; ++i)
-            for (int I = 0; I < P; ++I) {
-                const long double u = 0.5L * x[I] + (a ? 0.5L : -0.5L);
+        for (int I = 0; I < P; ++I) {
+            chebyshev(0.5L * x[I] + (a ? 0.5L : -0.5L), t.data());
+            for (int i = 0; i < P; ++i) {
                 long double c = 0.0L;
-                for (int k = 0; k < P; ++k) c += (k ? 2.0L : 1.0L) / P * T(k, x[i]) * T(k, u);
+                for (int k = 0; k < P; ++k) c += (k ? 2.0L : 1.0L) / P * tn[i * P + k] * t[k];
                 shift[(a * P + i) * P + I] = (double)c;
             }
+        }
     return v;
 }
 
