@@ -100,6 +100,7 @@ struct bh_ctx_s {
     double* rc_blk = nullptr;      // per block: sum of M^2
     double* rc_bfar = nullptr;     // per block: its far-block part of the bound
     int64_t nblocks = 0;
+    int maxG = 0;                  // largest grid side
     int64_t nchunks = 0;           // chunks of 64 particles of one system
     // grouped far field (bh_fmm.hip): which passes take it is a rule on the
     // systems' sizes (fmm_wanted)
@@ -545,6 +546,7 @@ int bh_set_systems(void* ctx, int32_t nsys, const int64_t* n, const int32_t* gri
     unconfigure(c);
     c->sys_h = sh;
     c->nchunks = sh.back().k_off + cdiv(sh.back().n, 64);
+    c->maxG = *std::max_element(grid_dim, grid_dim + nsys);
     int r = configure(c, nsys, N, C, cols, maxN, NB);
     if (r == BH_OK) r = ensure_part(c);
     if (r != BH_OK) {
@@ -642,25 +644,41 @@ int bh_place_particles(void* ctx, const bh_particles* p, void* stream)
     if (r) return r;
     hipStream_t st = (hipStream_t)stream;
     const int64_t N = c->N;
-    unsigned nchunk = (unsigned)cdiv(N, PLACE_CHUNK);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats, (int64_t)ST_COUNT, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c->C, 256, 4096)), dim3(256), 0, st, c->counts,
-                       c->C, 0);
-    hipLaunchKernelGGL(k_bbox_init, dim3(cdiv(c->S, 256)), dim3(256), 0, st, c->bb, c->S);
-    hipLaunchKernelGGL(k_bbox, dim3(nchunk), dim3(256), 0, st, (const double*)p->px,
-                       (const double*)p->py, (const int32_t*)c->sys_of, N, c->bb, c->stats);
-    hipLaunchKernelGGL(k_bbox_finalize, dim3(cdiv(c->S, 256)), dim3(256), 0, st, c->sys,
-                       (const uint64_t*)c->bb, c->S, c->stats);
-    hipLaunchKernelGGL(k_keys_hist, dim3(nchunk), dim3(256), 0, st, (const double*)p->px,
-                       (const double*)p->py, (const int32_t*)c->sys_of, (const SysDev*)c->sys, N,
-                       c->key, c->counts);
+    hipLaunchKernelGGL(k_place_init, dim3(grid_for(std::max<int64_t>(c->C, c->S), 256, 4096)),
+                       dim3(256), 0, st, c->stats, c->counts, c->C, c->bb, c->S);
+    const double *x = p->px, *y = p->py;
+    const int32_t* so = c->sys_of;
+    if (N < PLACE_SMALL) {
+        hipLaunchKernelGGL(k_bbox<4>, dim3(cdiv(N, 1024)), dim3(256), 0, st, x, y, so, N, c->bb,
+                           c->stats);
+        hipLaunchKernelGGL(k_keys_hist<2>, dim3(cdiv(N, 512)), dim3(256), 0, st, x, y, so, c->sys,
+                           (const uint64_t*)c->bb, N, c->key, c->counts, c->stats);
+    } else {
+        hipLaunchKernelGGL(k_bbox<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, N, c->bb,
+                           c->stats);
+        hipLaunchKernelGGL(k_keys_hist<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, c->sys,
+                           (const uint64_t*)c->bb, N, c->key, c->counts, c->stats);
+    }
     LAUNCH_CHECK("place");
     return BH_OK;
 }
 
+// Exclusive scan of the cells (cnt: offsets and non-empty prefix, and what the
+// later phases find cleared) or of the columns' item counts (the total to
+// stats[total_slot], at most max_total).
 static void run_scan(Ctx* c, bool cnt, const int32_t* in, int64_t n, int32_t* out_v,
-                     int32_t* out_f, int total_slot, hipStream_t st)
+                     int32_t* out_f, int total_slot, int64_t max_total, hipStream_t st)
 {
+    int32_t *nl = c->ne_list, *cur = c->cursor;
+    if (n <= SCAN_ONE) {
+        if (cnt)
+            hipLaunchKernelGGL(k_scan_one<true>, dim3(1), dim3(1024), 0, st, in, (int)n, out_v,
+                               out_f, nl, cur, c->com_dense, c->stats, total_slot, max_total);
+        else
+            hipLaunchKernelGGL(k_scan_one<false>, dim3(1), dim3(1024), 0, st, in, (int)n, out_v,
+                               out_f, nl, cur, c->com_dense, c->stats, total_slot, max_total);
+        return;
+    }
     unsigned nb = (unsigned)cdiv(n, SCAN_TILE);
     if (cnt) {
         hipLaunchKernelGGL(k_scan_reduce<true>, dim3(nb), dim3(256), 0, st, in, n, c->bsum, c->bne,
@@ -668,15 +686,19 @@ static void run_scan(Ctx* c, bool cnt, const int32_t* in, int64_t n, int32_t* ou
         hipLaunchKernelGGL(k_scan_blocks<true>, dim3(1), dim3(1024), 0, st, c->bsum, c->bne,
                            (int64_t)nb, c->stats, total_slot);
         hipLaunchKernelGGL(k_scan_final<true>, dim3(nb), dim3(256), 0, st, in, n,
-                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f);
+                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl, cur,
+                           c->com_dense);
     } else {
         hipLaunchKernelGGL(k_scan_reduce<false>, dim3(nb), dim3(256), 0, st, in, n, c->bsum,
                            c->bne, c->stats);
         hipLaunchKernelGGL(k_scan_blocks<false>, dim3(1), dim3(1024), 0, st, c->bsum, c->bne,
                            (int64_t)nb, c->stats, total_slot);
         hipLaunchKernelGGL(k_scan_final<false>, dim3(nb), dim3(256), 0, st, in, n,
-                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f);
+                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl, cur,
+                           c->com_dense);
     }
+    if (max_total >= 0)
+        hipLaunchKernelGGL(k_clamp_items, dim3(1), dim3(64), 0, st, c->stats, max_total);
 }
 
 int bh_calculate_box_cumm(void* ctx, void* stream)
@@ -684,7 +706,7 @@ int bh_calculate_box_cumm(void* ctx, void* stream)
     Ctx* c = (Ctx*)ctx;
     CTX_READY(c);
     hipStream_t st = (hipStream_t)stream;
-    run_scan(c, true, c->counts, c->C, c->offsets, c->neprefix, -1, st);
+    run_scan(c, true, c->counts, c->C, c->offsets, c->neprefix, -1, -1, st);
     LAUNCH_CHECK("scan");
     return BH_OK;
 }
@@ -717,7 +739,10 @@ static BhParticles dev_of(const bh_particles* p)
     return d;
 }
 
-int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
+// clear: the scatter's cursors, which the scan leaves at zero, may hold the
+// counts of an earlier sort of the same placement.
+static int sort_impl(void* ctx, const bh_particles* src, const bh_particles* dst, bool clear,
+                     void* stream)
 {
     Ctx* c = (Ctx*)ctx;
     CTX_READY(c);
@@ -728,25 +753,31 @@ int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* ds
     hipStream_t st = (hipStream_t)stream;
     const int64_t N = c->N;
     SortFields F = fields_of(src);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c->C, 256, 4096)), dim3(256), 0, st, c->cursor,
-                       c->C, 0);
-    hipLaunchKernelGGL(k_scatter, dim3(cdiv(N, PLACE_CHUNK)), dim3(256), 0, st,
-                       (const int32_t*)c->key, N, (const int32_t*)c->offsets, c->cursor, c->idx_a,
-                       c->key_sorted, (const double*)src->px, (const double*)src->py, c->pxkey,
-                       c->pykey);
+    if (clear)
+        hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c->C, 256, 4096)), dim3(256), 0, st, c->cursor,
+                           c->C, 0);
+    if (N < PLACE_SMALL)
+        hipLaunchKernelGGL(k_scatter<2>, dim3(cdiv(N, 512)), dim3(256), 0, st,
+                           (const int32_t*)c->key, N, (const int32_t*)c->offsets, c->cursor,
+                           c->idx_a, c->key_sorted, (const double*)src->px, (const double*)src->py,
+                           c->pxkey, c->pykey);
+    else
+        hipLaunchKernelGGL(k_scatter<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st,
+                           (const int32_t*)c->key, N, (const int32_t*)c->offsets, c->cursor,
+                           c->idx_a, c->key_sorted, (const double*)src->px, (const double*)src->py,
+                           c->pxkey, c->pykey);
     hipLaunchKernelGGL(k_sort_units, dim3(cdiv(N, SORT_W)), dim3(SORT_THREADS), 0, st, F, N,
                        (const int32_t*)c->idx_a, (const int32_t*)c->key_sorted,
                        (const uint64_t*)c->pxkey, (const uint64_t*)c->pykey,
                        (const int32_t*)c->offsets, c->idx_b);
     // merge passes for cells longer than SORT_W: b -> a -> b -> ...
-    int maxpass = 0;
-    while (((int64_t)SORT_W << maxpass) < c->maxN) ++maxpass;
     unsigned mgrid = grid_for(N, 256, (int64_t)c->num_cu * 8);
-    for (int L = 0; L < maxpass; ++L) {
+    int L = 0;
+    for (int64_t R = SORT_W; R < c->maxN; R *= SORT_WAYS, ++L) {
         const int32_t* in = (L & 1) ? c->idx_a : c->idx_b;
         int32_t* out = (L & 1) ? c->idx_b : c->idx_a;
         hipLaunchKernelGGL(k_sort_merge, dim3(mgrid), dim3(256), 0, st, F, N, in,
-                           (const int32_t*)c->key_sorted, (const int32_t*)c->offsets, out, L,
+                           (const int32_t*)c->key_sorted, (const int32_t*)c->offsets, out, R,
                            (const int32_t*)c->stats);
     }
     hipLaunchKernelGGL(k_gather, dim3(grid_for(N, 256, (int64_t)c->num_cu * 16)), dim3(256), 0, st,
@@ -757,6 +788,11 @@ int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* ds
     return BH_OK;
 }
 
+int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
+{
+    return sort_impl(ctx, src, dst, true, stream);
+}
+
 int bh_summarize(void* ctx, const bh_particles* p, void* stream)
 {
     Ctx* c = (Ctx*)ctx;
@@ -764,10 +800,6 @@ int bh_summarize(void* ctx, const bh_particles* p, void* stream)
     int r = check_parts(p, "particles");
     if (r) return r;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_ne_list, dim3(grid_for(c->C, 256, 8192)), dim3(256), 0, st,
-                       (const int32_t*)c->counts, (const int32_t*)c->neprefix, c->C, c->ne_list);
-    hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(3 * c->C, 256, 8192)), dim3(256), 0, st,
-                       c->com_dense, 3 * c->C, 0.0);
     // one wave per non-empty cell; the grid is sized for the worst case
     int64_t waves = std::min<int64_t>(c->C, (int64_t)c->num_cu * 64);
     hipLaunchKernelGGL(k_com, dim3(grid_for(waves * 64, 256)), dim3(256), 0, st,
@@ -785,12 +817,25 @@ int bh_build_items(void* ctx, void* stream)
     CTX_READY(c);
     hipStream_t st = (hipStream_t)stream;
     const int pitem = 64 * c->tune.p;
+    if (c->maxG <= c->tune.yspan && c->ncols <= SCAN_ONE) {
+        const int write = c->N <= ITEMS_ONE;
+        hipLaunchKernelGGL(k_items_runs, dim3(1), dim3(1024), 0, st, (const SysDev*)c->sys, c->S,
+                           (int)c->ncols, (const int32_t*)c->offsets, pitem, c->col_off, c->items,
+                           c->max_items, c->stats, write);
+        if (!write)
+            hipLaunchKernelGGL(k_items_fill, dim3(grid_for(cdiv(c->N, pitem) + c->ncols, 256,
+                                                           (int64_t)c->num_cu * 8)), dim3(256), 0,
+                               st, (const SysDev*)c->sys, c->S, (int)c->ncols,
+                               (const int32_t*)c->offsets, pitem, (const int32_t*)c->col_off,
+                               c->items, (const int32_t*)c->stats);
+        LAUNCH_CHECK("items");
+        return BH_OK;
+    }
     unsigned g = (unsigned)c->ncols;   // one wave per grid column
     hipLaunchKernelGGL(k_items<false>, dim3(g), dim3(64), 0, st, (const SysDev*)c->sys, c->S,
                        c->ncols, (const int32_t*)c->counts, (const int32_t*)c->offsets, pitem,
                        c->tune.yspan, c->col_items, c->items, c->max_items, c->stats);
-    run_scan(c, false, c->col_items, c->ncols, c->col_off, nullptr, ST_NITEMS, st);
-    hipLaunchKernelGGL(k_clamp_items, dim3(1), dim3(64), 0, st, c->stats, c->max_items);
+    run_scan(c, false, c->col_items, c->ncols, c->col_off, nullptr, ST_NITEMS, c->max_items, st);
     hipLaunchKernelGGL(k_items<true>, dim3(g), dim3(64), 0, st, (const SysDev*)c->sys, c->S,
                        c->ncols, (const int32_t*)c->counts, (const int32_t*)c->offsets, pitem,
                        c->tune.yspan, c->col_off, c->items, c->max_items, c->stats);
@@ -888,9 +933,6 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
         const int64_t end = c->nchunks * (part + 1) / nparts;
         if (part == 0) c->rc_ready = 0;
         if (end > fa.chunk0) bh_force64s(fa, lawi, c->S, end - fa.chunk0, st);
-        if (part == nparts - 1)
-            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
-                               (int64_t)2, 0);
         LAUNCH_CHECK("evaluate");
         return BH_OK;
     }
@@ -1033,7 +1075,7 @@ static int step_impl(void* ctx, const bh_particles* a, const bh_particles* b, co
     int r;
     if ((r = bh_place_particles(ctx, a, stream))) return r;
     if ((r = bh_calculate_box_cumm(ctx, stream))) return r;
-    if ((r = bh_sort_particles(ctx, a, b, stream))) return r;
+    if ((r = sort_impl(ctx, a, b, false, stream))) return r;
     if ((r = bh_summarize(ctx, b, stream))) return r;
     if ((r = bh_build_items(ctx, stream))) return r;
     const int32_t* ord = nullptr;
@@ -1443,6 +1485,7 @@ extern "C" int bh_step_noalloc(const bh_particles* a, const bh_particles* b, int
     const int64_t G = grid_dim, Gb = cdiv(G, RC_BLOCK);
     set_sizes(&c, 1, n, G * G, G, n, Gb * Gb);
     c.nchunks = cdiv(n, 64);
+    c.maxG = grid_dim;
     size_t off = 0;
     r = for_each_buffer(&c, [&](auto*& p, int64_t cnt) {
         using T = std::remove_reference_t<decltype(*p)>;

@@ -30,26 +30,25 @@
 // more rows below its first one, and at the end of the column.  Pass 1
 // (WRITE = false) counts items per column; pass 2 writes them at the scanned
 // column offsets.
+//
+// The column's counts and offsets are read 64 rows at a time, and the greedy
+// cut walks the non-empty rows with wave-uniform values (every lane holds the
+// same state; lane 0 writes).  A row's values come by v_readlane: through
+// shuffles the walk of a 1024-row column took 160 us, of which the chip idles
+// all but 1024 waves.
 template <bool WRITE>
-__global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, int S, int64_t ncols,
-                                              const int32_t* __restrict__ counts,
-                                              const int32_t* __restrict__ offsets, int pitem,
-                                              int yspan, int32_t* __restrict__ col_items,
-                                              Item* __restrict__ items, int64_t max_items,
-                                              int32_t* stats)
+__device__ __forceinline__ int column_items(const SysDev* __restrict__ sys, int S, int64_t col,
+                                            const int32_t* __restrict__ counts,
+                                            const int32_t* __restrict__ offsets, int pitem,
+                                            int yspan, int64_t out, Item* __restrict__ items,
+                                            int64_t max_items, int32_t* stats)
 {
-    // One wave per column: the column's counts and offsets are read 64 rows at
-    // a time, and the greedy cut walks the non-empty rows with wave-uniform
-    // values (every lane holds the same state; lane 0 writes).
-    const int64_t col = blockIdx.x;
-    if (col >= ncols) return;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     const int s = sys_of_col(sys, S, col);
     const SysDev& d = sys[s];
     const int G = d.G;
     const int x = (int)(col - d.col_off);
     const int64_t cb = d.c_off + (int64_t)x * G;
-    int64_t out = WRITE ? col_items[col] : 0;
     int n_out = 0;
     bool open = false;
     int p0 = 0, np = 0, y0 = 0, y1 = 0;
@@ -83,8 +82,8 @@ __global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, in
             const int l = __ffsll((long long)nz) - 1;
             nz &= nz - 1;
             const int yy = yb + l;
-            int nc = __shfl(ncl, l, BH_WAVE);
-            int pc = __shfl(pcl, l, BH_WAVE);
+            int nc = __builtin_amdgcn_readlane(ncl, l);
+            int pc = __builtin_amdgcn_readlane(pcl, l);
             if (open && yy - y0 >= yspan) emit();
             while (nc > 0) {
                 if (!open) {
@@ -103,13 +102,149 @@ __global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, in
         }
     }
     if (open) emit();
-    if (!WRITE && lane == 0) col_items[col] = n_out;
+    return n_out;
+}
+
+template <bool WRITE>
+__global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, int S, int64_t ncols,
+                                              const int32_t* __restrict__ counts,
+                                              const int32_t* __restrict__ offsets, int pitem,
+                                              int yspan, int32_t* __restrict__ col_items,
+                                              Item* __restrict__ items, int64_t max_items,
+                                              int32_t* stats)
+{
+    const int64_t col = blockIdx.x;
+    if (col >= ncols) return;
+    const int n = column_items<WRITE>(sys, S, col, counts, offsets, pitem, yspan,
+                                      WRITE ? col_items[col] : 0, items, max_items, stats);
+    if (!WRITE && threadIdx.x == 0) col_items[col] = n;
 }
 
 template __global__ void k_items<false>(const SysDev*, int, int64_t, const int32_t*, const int32_t*,
                                         int, int, int32_t*, Item*, int64_t, int32_t*);
 template __global__ void k_items<true>(const SysDev*, int, int64_t, const int32_t*, const int32_t*,
                                        int, int, int32_t*, Item*, int64_t, int32_t*);
+
+// Where no item can reach the row span (every grid at most yspan rows), a
+// column's items are its runs of pitem particles: item t of the pass, in column
+// col, starts pitem (t - at) particles into it (at: the column's first item).
+__device__ __forceinline__ void write_run(const SysDev* __restrict__ sys, int S, int col, int t,
+                                          int at, const int32_t* __restrict__ offsets, int pitem,
+                                          Item* __restrict__ items)
+{
+    const int s = sys_of_col(sys, S, col);
+    const SysDev& d = sys[s];
+    const int G = d.G, x = (int)(col - d.col_off);
+    const int32_t* o = offsets + d.c_off + (int64_t)x * G;
+    Item it;
+    it.p0 = o[0] + (t - at) * pitem;
+    it.np = min(pitem, o[G] - it.p0);
+    it.sys = s;
+    it.cx = x;
+    // rows of the first and last particle: the last row that starts at or before it
+    int y[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int p = u ? it.p0 + it.np - 1 : it.p0;
+        int lo = 0, hi = G - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (o[mid] <= p) lo = mid; else hi = mid - 1;
+        }
+        y[u] = lo;
+    }
+    it.y0 = y[0];
+    it.y1 = y[1];
+    it.pad0 = 0;
+    it.pad1 = 0;
+    items[t] = it;
+}
+
+__device__ __forceinline__ int col_of_item(const int32_t* col_off, int ncols, int t)
+{
+    int lo = 0, hi = ncols - 1;   // the last column whose first item is at or before t
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (col_off[mid] <= t) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Counts and scans the runs of ncols <= SCAN_ONE columns in one block, and
+// writes the items too where they are few (write != 0): the count, scan, clamp
+// and write of a 16,384-particle step were six launches and 24 us.
+__global__ __launch_bounds__(1024) void k_items_runs(const SysDev* __restrict__ sys, int S,
+                                                     int ncols, const int32_t* __restrict__ offsets,
+                                                     int pitem, int32_t* col_off,
+                                                     Item* __restrict__ items, int64_t max_items,
+                                                     int32_t* stats, int write)
+{
+    constexpr int R = SCAN_ONE / 1024;
+    __shared__ int32_t at[SCAN_ONE];
+    __shared__ int wsum[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int v[R], sum = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int col = threadIdx.x * R + r;
+        v[r] = 0;
+        if (col < ncols) {
+            const SysDev& d = sys[sys_of_col(sys, S, col)];
+            const int32_t* o = offsets + d.c_off + (int64_t)(col - d.col_off) * d.G;
+            v[r] = (o[d.G] - o[0] + pitem - 1) / pitem;
+        }
+        sum += v[r];
+    }
+    int inc = sum;
+#pragma unroll
+    for (int o = 1; o < BH_WAVE; o <<= 1) {
+        const int a = __shfl_up(inc, o, BH_WAVE);
+        if (lane >= o) inc += a;
+    }
+    if (lane == BH_WAVE - 1) wsum[w] = inc;
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (k < w) before += wsum[k];
+        total += wsum[k];
+    }
+    int e = before + inc - sum;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int col = threadIdx.x * R + r;
+        if (col < ncols) {
+            at[col] = e;
+            col_off[col] = e;
+        }
+        e += v[r];
+    }
+    const int n = (int)min((int64_t)total, max_items);
+    if (threadIdx.x == 0) {
+        col_off[ncols] = total;
+        stats[ST_NITEMS] = n;
+        if (total > max_items) atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
+    }
+    if (!write) return;
+    __syncthreads();
+    for (int t = threadIdx.x; t < n; t += 1024) {
+        const int col = col_of_item(at, ncols, t);
+        write_run(sys, S, col, t, at[col], offsets, pitem, items);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_items_fill(const SysDev* __restrict__ sys, int S,
+                                                    int ncols, const int32_t* __restrict__ offsets,
+                                                    int pitem, const int32_t* __restrict__ col_off,
+                                                    Item* __restrict__ items,
+                                                    const int32_t* __restrict__ stats)
+{
+    const int n = stats[ST_NITEMS];
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
+        const int col = col_of_item(col_off, ncols, t);
+        write_run(sys, S, col, t, col_off[col], offsets, pitem, items);
+    }
+}
 
 // Keeps the item count within the allocated capacity (flags the overflow).
 __global__ void k_clamp_items(int32_t* stats, int64_t max_items)
@@ -529,6 +664,7 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
         }
         s = uniform_int(s);
     }
+    if (blockIdx.x == 0 && threadIdx.x < 2) A.stats[ST_NRECOMP + threadIdx.x] = 0;
     const SysDev& d = A.sys[s];
     const int G = d.G;
     const int64_t coff = d.c_off;

@@ -2,9 +2,16 @@
 #pragma once
 #include "bh_common.h"
 
-#define PLACE_CHUNK 2048   // particles per block in bbox / keys / scatter
+// Particles per block in bbox / keys / scatter: 256 R.  Large sets take R = 8
+// (a block's rows share its histogram window); below PLACE_SMALL that leaves
+// too few blocks and each thread's rows come one after the other (k_bbox: 9.8
+// us for 16,384 particles in 8 blocks).
+#define PLACE_SMALL 262144
 #define HIST_BINS 8192     // LDS histogram window (keys) per block
 #define SCAN_TILE 2048     // elements per block in the scans
+#define SCAN_ONE 8192      // elements that one block scans in one launch
+#define SORT_WAYS 8        // runs that a merge pass joins
+#define ITEMS_ONE 65536    // particles up to which one block builds a step's items
 #define SORT_W 1024        // within-cell rank window (rows)
 #define SORT_THREADS 1024  // threads of a k_sort_units block (2 rows of the 2 SORT_W window each)
 
@@ -293,12 +300,14 @@ __global__ void k_potential(PotArgs A);
 // placement
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v);
 __global__ void k_fill_f64(double* p, int64_t n, double v);
-__global__ void k_bbox_init(uint64_t* bb, int S);
+__global__ void k_place_init(int32_t* stats, int32_t* counts, int64_t C, uint64_t* bb, int S);
+template <int R>
 __global__ void k_bbox(const double* px, const double* py, const int32_t* sys_of, int64_t N,
                        uint64_t* bb, int32_t* stats);
-__global__ void k_bbox_finalize(SysDev* sys, const uint64_t* bb, int S, int32_t* stats);
-__global__ void k_keys_hist(const double* px, const double* py, const int32_t* sys_of,
-                            const SysDev* sys, int64_t N, int32_t* key_out, int32_t* counts);
+template <int R>
+__global__ void k_keys_hist(const double* px, const double* py, const int32_t* sys_of, SysDev* sys,
+                            const uint64_t* bb, int64_t N, int32_t* key_out, int32_t* counts,
+                            int32_t* stats);
 template <bool CNT>
 __global__ void k_scan_reduce(const int32_t* in, int64_t n, int32_t* bsum, int32_t* bne,
                               int32_t* stats);
@@ -307,7 +316,13 @@ __global__ void k_scan_blocks(int32_t* bsum, int32_t* bne, int64_t nb, int32_t* 
                               int total_slot);
 template <bool CNT>
 __global__ void k_scan_final(const int32_t* in, int64_t n, const int32_t* bsum, const int32_t* bne,
-                             int32_t* out_v, int32_t* out_f);
+                             int32_t* out_v, int32_t* out_f, int32_t* ne_list, int32_t* cursor,
+                             double* com_dense);
+template <bool CNT>
+__global__ void k_scan_one(const int32_t* in, int n, int32_t* out_v, int32_t* out_f,
+                           int32_t* ne_list, int32_t* cursor, double* com_dense, int32_t* stats,
+                           int total_slot, int64_t max_total);
+template <int R>
 __global__ void k_scatter(const int32_t* key, int64_t N, const int32_t* offsets, int32_t* cursor,
                           int32_t* idx_out, int32_t* key_sorted, const double* px,
                           const double* py, uint64_t* pxkey_out, uint64_t* pykey_out);
@@ -316,14 +331,12 @@ __global__ void k_sort_units(SortFields F, int64_t N, const int32_t* idx_in,
                              const uint64_t* pykey, const int32_t* offsets, int32_t* idx_out);
 __global__ void k_sort_merge(SortFields F, int64_t N, const int32_t* idx_in,
                              const int32_t* key_sorted, const int32_t* offsets, int32_t* idx_out,
-                             int L, const int32_t* stats);
+                             int64_t R, const int32_t* stats);
 __global__ void k_gather(SortFields S, BhParticles D, int64_t N, const int32_t* idx_a,
                          const int32_t* idx_b, const int32_t* key_sorted, const int32_t* offsets,
                          const int32_t* stats, int32_t* perm_out);
 
 // summarize + tick
-__global__ void k_ne_list(const int32_t* counts, const int32_t* neprefix, int64_t C,
-                          int32_t* ne_list);
 __global__ void k_com(const SysDev* sys, int S, const int32_t* ne_list, const int32_t* stats,
                       const int32_t* offsets, const double* x, const double* y, const double* m,
                       double* com_dense, Com64* l64, Com32* l32);
@@ -372,3 +385,8 @@ template <bool WRITE>
 __global__ void k_items(const SysDev* sys, int S, int64_t ncols, const int32_t* counts,
                         const int32_t* offsets, int pitem, int yspan, int32_t* col_items,
                         Item* items, int64_t max_items, int32_t* stats);
+__global__ void k_items_runs(const SysDev* sys, int S, int ncols, const int32_t* offsets, int pitem,
+                             int32_t* col_off, Item* items, int64_t max_items, int32_t* stats,
+                             int write);
+__global__ void k_items_fill(const SysDev* sys, int S, int ncols, const int32_t* offsets, int pitem,
+                             const int32_t* col_off, Item* items, const int32_t* stats);

@@ -25,18 +25,24 @@ __global__ void k_fill_f64(double* p, int64_t n, double v)
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
-// ---------------------------------------------------------------- bbox
-__global__ void k_bbox_init(uint64_t* bb, int S)
+// Everything a placement clears: the stats block, the cell counts and the
+// bounding boxes (one launch).
+__global__ __launch_bounds__(256) void k_place_init(int32_t* stats, int32_t* counts, int64_t C,
+                                                    uint64_t* bb, int S)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    if (t < ST_COUNT) stats[t] = 0;
+    for (int64_t s = t; s < S; s += stride) {
         bb[4 * s + 0] = ~0ull;   // min x (ordered key)
         bb[4 * s + 1] = ~0ull;   // min y
         bb[4 * s + 2] = 0ull;    // max x
         bb[4 * s + 3] = 0ull;    // max y
     }
+    for (int64_t c = t; c < C; c += stride) counts[c] = 0;
 }
 
+// ---------------------------------------------------------------- bbox
 // Atomic min/max of the ordered keys; skipped when the stored value already
 // bounds ours (stored minima only fall and maxima only rise, so a stale read
 // can only cause an unneeded atomic, never a missed one).
@@ -52,106 +58,126 @@ __device__ __forceinline__ void bbox_flush(uint64_t* bb, int s, double mnx, doub
     if (k3 > __atomic_load_n(&b[3], __ATOMIC_RELAXED)) atomicMax(&b[3], k3);
 }
 
-// Each block covers PLACE_CHUNK consecutive particles; min/max are exact so
-// the reduction order does not matter.
+// Each wave covers 64 R consecutive particles, all of its loads issued before
+// the first is used; min/max are exact, so the reduction order does not matter.
+// Rows of one system are consecutive: a wave reduces when the system changes
+// (a block of one system reduces over the block).
+template <int R>
 __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
                                               const double* __restrict__ py,
                                               const int32_t* __restrict__ sys_of, int64_t N,
                                               uint64_t* bb, int32_t* stats)
 {
     const double inf = __longlong_as_double(0x7ff0000000000000ll);
-    int64_t base = (int64_t)blockIdx.x * PLACE_CHUNK;
-    int cur = -1;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int64_t base = ((int64_t)blockIdx.x * 4 + wid) * (64 * R);
+    int sv[R];
+    double xv[R], yv[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t i = base + 64 * r + lane;
+        const bool in = i < N;
+        sv[r] = in ? sys_of[i] : -1;
+        xv[r] = in ? px[i] : 0.0;
+        yv[r] = in ? py[i] : 0.0;
+    }
+    int cur = -1;   // system of the running extremes (wave-uniform)
     double mnx = inf, mny = inf, mxx = -inf, mxy = -inf;
     bool bad = false;
-    for (int r = 0; r < PLACE_CHUNK / 256; ++r) {
-        int64_t i = base + r * 256 + threadIdx.x;
-        if (i >= N) break;
-        int s = sys_of[i];
-        if (s != cur) {
-            if (cur >= 0) bbox_flush(bb, cur, mnx, mny, mxx, mxy);
-            cur = s;
-            mnx = inf; mny = inf; mxx = -inf; mxy = -inf;
-        }
-        double x = px[i], y = py[i];
-        if (!isfinite(x) || !isfinite(y)) {
-            bad = true;
-            continue;
-        }
-        mnx = fmin(mnx, x);
-        mxx = fmax(mxx, x);
-        mny = fmin(mny, y);
-        mxy = fmax(mxy, y);
-    }
-    // Reduce over the block when all its rows belong to one system (one
-    // flush per block), else per wave, else per lane.
-    __shared__ double red[4][4];
-    __shared__ int wsys[4];
-    const int wid = threadIdx.x >> 6;
-    int c0 = __shfl(cur, 0, BH_WAVE);
-    bool uni = __all(cur == c0);
-    if (uni && c0 >= 0) {
+    auto reduce = [&]() {
         mnx = wave_min(mnx);
         mny = wave_min(mny);
         mxx = wave_max(mxx);
         mxy = wave_max(mxy);
+    };
+    auto flush = [&]() {
+        if (cur < 0) return;
+        reduce();
+        if (lane == 0) bbox_flush(bb, cur, mnx, mny, mxx, mxy);
+        mnx = inf; mny = inf; mxx = -inf; mxy = -inf;
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool fin = isfinite(xv[r]) && isfinite(yv[r]);
+        if (sv[r] >= 0 && !fin) bad = true;
+        unsigned long long todo = __ballot(sv[r] >= 0);
+        while (todo) {   // the systems of these 64 rows, nearly always one
+            const int s = __builtin_amdgcn_readlane(sv[r], __ffsll((long long)todo) - 1);
+            if (s != cur) {
+                flush();
+                cur = s;
+            }
+            if (sv[r] == s && fin) {
+                mnx = fmin(mnx, xv[r]);
+                mxx = fmax(mxx, xv[r]);
+                mny = fmin(mny, yv[r]);
+                mxy = fmax(mxy, yv[r]);
+            }
+            todo &= ~__ballot(sv[r] == s);
+        }
     }
-    if ((threadIdx.x & 63) == 0) {
-        wsys[wid] = (uni && c0 >= 0) ? c0 : -1;
+    __shared__ double red[4][4];
+    __shared__ int wsys[4];
+    if (cur >= 0) reduce();
+    if (lane == 0) {
+        wsys[wid] = cur;
         red[wid][0] = mnx;
         red[wid][1] = mny;
         red[wid][2] = mxx;
         red[wid][3] = mxy;
     }
+    if (__any(bad) && lane == 0) atomicOr(&stats[ST_ERR], BH_ERR_NONFINITE);
     __syncthreads();
-    const int nwv = (int)(blockDim.x >> 6);
-    bool block_uni = true;
-    for (int v = 0; v < nwv; ++v) block_uni = block_uni && wsys[v] >= 0 && wsys[v] == wsys[0];
-    if (block_uni) {
-        if (threadIdx.x == 0) {
-            for (int v = 1; v < nwv; ++v) {
-                mnx = fmin(mnx, red[v][0]);
-                mny = fmin(mny, red[v][1]);
-                mxx = fmax(mxx, red[v][2]);
-                mxy = fmax(mxy, red[v][3]);
+    if (threadIdx.x == 0) {   // waves of one system meet here
+        for (int v = 0; v < 4; ++v) {
+            if (wsys[v] < 0) continue;
+            if (v + 1 < 4 && wsys[v + 1] == wsys[v]) {
+                red[v + 1][0] = fmin(red[v + 1][0], red[v][0]);
+                red[v + 1][1] = fmin(red[v + 1][1], red[v][1]);
+                red[v + 1][2] = fmax(red[v + 1][2], red[v][2]);
+                red[v + 1][3] = fmax(red[v + 1][3], red[v][3]);
+            } else {
+                bbox_flush(bb, wsys[v], red[v][0], red[v][1], red[v][2], red[v][3]);
             }
-            bbox_flush(bb, wsys[0], mnx, mny, mxx, mxy);
         }
-    } else if (uni && c0 >= 0) {
-        if ((threadIdx.x & 63) == 0) bbox_flush(bb, c0, mnx, mny, mxx, mxy);
-    } else if (cur >= 0) {
-        bbox_flush(bb, cur, mnx, mny, mxx, mxy);
     }
-    if (bad) atomicOr(&stats[ST_ERR], BH_ERR_NONFINITE);
 }
 
-// helpers/grid.py:15-22 square-up, base.py:237 step, exactly in FP64.
-__global__ void k_bbox_finalize(SysDev* sys, const uint64_t* bb, int S, int32_t* stats)
-{
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) return;
-    double mnx = bh_ord_val(bb[4 * s + 0]);
-    double mny = bh_ord_val(bb[4 * s + 1]);
-    double mxx = bh_ord_val(bb[4 * s + 2]);
-    double mxy = bh_ord_val(bb[4 * s + 3]);
-    double xe = mxx - mnx, ye = mxy - mny;
-    if (xe > ye) {
-        mxy += (xe - ye);
-    } else if (ye > xe) {
-        mxx += (ye - xe);
-    }
-    double step = (mxx - mnx) / (double)sys[s].G;
-    sys[s].min_x = mnx;
-    sys[s].min_y = mny;
-    sys[s].max_x = mxx;
-    sys[s].max_y = mxy;
-    sys[s].step = step;
-    if (!(step > 0.0) || !isfinite(step)) atomicOr(&stats[ST_ERR], BH_ERR_DEGENERATE);
-}
+template __global__ void k_bbox<4>(const double*, const double*, const int32_t*, int64_t, uint64_t*,
+                                   int32_t*);
+template __global__ void k_bbox<8>(const double*, const double*, const int32_t*, int64_t, uint64_t*,
+                                   int32_t*);
 
 // ---------------------------------------------------------------- keys + histogram
+struct Box {
+    double min_x, min_y, max_x, max_y, step;
+    int64_t c_off;
+    int32_t G;
+};
+
+// A system's box from its extremes: helpers/grid.py:15-22 square-up,
+// base.py:237 step, exactly in FP64.
+__device__ __forceinline__ Box box_of(const SysDev* sys, const uint64_t* bb, int s)
+{
+    Box d;
+    d.min_x = bh_ord_val(bb[4 * s + 0]);
+    d.min_y = bh_ord_val(bb[4 * s + 1]);
+    d.max_x = bh_ord_val(bb[4 * s + 2]);
+    d.max_y = bh_ord_val(bb[4 * s + 3]);
+    const double xe = d.max_x - d.min_x, ye = d.max_y - d.min_y;
+    if (xe > ye) {
+        d.max_y += (xe - ye);
+    } else if (ye > xe) {
+        d.max_x += (ye - xe);
+    }
+    d.G = sys[s].G;
+    d.c_off = sys[s].c_off;
+    d.step = (d.max_x - d.min_x) / (double)d.G;
+    return d;
+}
+
 // sequential.py:32-34: g = clip(floor((p - min) / step), 0, G-1), IEEE division.
-__device__ __forceinline__ int32_t cell_key(double x, double y, const SysDev& d)
+__device__ __forceinline__ int32_t cell_key(double x, double y, const Box& d)
 {
     double fx = floor((x - d.min_x) / d.step);
     double fy = floor((y - d.min_y) / d.step);
@@ -180,30 +206,53 @@ __device__ __forceinline__ void block_minmax(int& kmin, int& kmax, int* red)
     __syncthreads();
 }
 
-// Keys for PLACE_CHUNK consecutive particles per block, then an LDS
+// Keys for 256 R consecutive particles per block, then an LDS
 // histogram over the block's key window when it fits (the input is the
 // previous step's sorted order, so a block's keys are nearly contiguous);
-// only non-zero bins go to global atomics.
+// only non-zero bins go to global atomics.  Each row's box comes straight from
+// the extremes; the thread of a system's first row stores it (a kernel of its
+// own, or a last block behind a device fence, costs more than the division).
+template <int R>
 __global__ __launch_bounds__(256) void k_keys_hist(const double* __restrict__ px,
                                                    const double* __restrict__ py,
                                                    const int32_t* __restrict__ sys_of,
-                                                   const SysDev* __restrict__ sys, int64_t N,
-                                                   int32_t* __restrict__ key_out,
-                                                   int32_t* __restrict__ counts)
+                                                   SysDev* sys, const uint64_t* __restrict__ bb,
+                                                   int64_t N, int32_t* __restrict__ key_out,
+                                                   int32_t* __restrict__ counts, int32_t* stats)
 {
     __shared__ int32_t hist[HIST_BINS];
     __shared__ int red[8];
-    constexpr int R = PLACE_CHUNK / 256;
-    int64_t base = (int64_t)blockIdx.x * PLACE_CHUNK;
-    int kk[R];
+    int64_t base = (int64_t)blockIdx.x * (256 * R);
+    int kk[R], sr[R];
+    double xr[R], yr[R];
     int kmin = INT_MAX, kmax = INT_MIN;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t i = min(base + r * 256 + threadIdx.x, N - 1);
+        sr[r] = sys_of[i];
+        xr[r] = px[i];
+        yr[r] = py[i];
+    }
+    int cur = sr[0];
+    Box d = box_of(sys, bb, cur);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         int64_t i = base + r * 256 + threadIdx.x;
         kk[r] = -1;
         if (i < N) {
-            const SysDev& d = sys[sys_of[i]];
-            int k = cell_key(px[i], py[i], d);
+            if (sr[r] != cur) {
+                cur = sr[r];
+                d = box_of(sys, bb, cur);
+            }
+            if (i == sys[cur].p_off) {
+                sys[cur].min_x = d.min_x;
+                sys[cur].min_y = d.min_y;
+                sys[cur].max_x = d.max_x;
+                sys[cur].max_y = d.max_y;
+                sys[cur].step = d.step;
+                if (!(d.step > 0.0) || !isfinite(d.step)) atomicOr(&stats[ST_ERR], BH_ERR_DEGENERATE);
+            }
+            int k = cell_key(xr[r], yr[r], d);
             key_out[i] = k;
             kk[r] = k;
             kmin = min(kmin, k);
@@ -228,6 +277,11 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double* __restrict__ px
             if (kk[r] >= 0) atomicAdd(&counts[kk[r]], 1);
     }
 }
+
+template __global__ void k_keys_hist<2>(const double*, const double*, const int32_t*, SysDev*,
+                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*);
+template __global__ void k_keys_hist<8>(const double*, const double*, const int32_t*, SysDev*,
+                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*);
 
 // ---------------------------------------------------------------- scan
 // Block-wide exclusive scan of two int sequences (256 or 1024 threads).
@@ -336,11 +390,27 @@ __global__ __launch_bounds__(1024) void k_scan_blocks(int32_t* bsum, int32_t* bn
     }
 }
 
+// What the cells' scan leaves for the phases after it, besides the prefixes:
+// the list of non-empty cells, zeros in the dense COM array (k_com writes the
+// non-empty cells) and in the scatter's cursors.
+struct CellOut {
+    int32_t *ne_list, *cursor;
+    double* com_dense;
+};
+
+__device__ __forceinline__ void clear_cells(const CellOut& o, int64_t c0, int64_t n, int threads)
+{
+    for (int64_t i = c0 + threadIdx.x; i < n; i += threads) o.cursor[i] = 0;
+    for (int64_t i = 3 * c0 + threadIdx.x; i < 3 * n; i += threads) o.com_dense[i] = 0.0;
+}
+
 // Phase 3: exclusive prefix per element; out has n + 1 entries.
 template <bool CNT>
 __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ in, int64_t n,
                                                     const int32_t* bsum, const int32_t* bne,
-                                                    int32_t* out_v, int32_t* out_f)
+                                                    int32_t* out_v, int32_t* out_f,
+                                                    int32_t* ne_list, int32_t* cursor,
+                                                    double* com_dense)
 {
     __shared__ int sh[40];
     constexpr int R = SCAN_TILE / 256;
@@ -363,7 +433,10 @@ __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ 
         int64_t i = base + r;
         if (i < n) {
             out_v[i] = av;
-            if (CNT) out_f[i] = af;
+            if (CNT) {
+                out_f[i] = af;
+                if (cv[r] > 0) ne_list[af] = (int32_t)i;
+            }
             av += cv[r];
             af += cv[r] > 0;
             if (i == n - 1) {
@@ -372,6 +445,67 @@ __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ 
             }
         }
     }
+    if (CNT) {
+        const int64_t c0 = (int64_t)blockIdx.x * SCAN_TILE;
+        clear_cells({ne_list, cursor, com_dense}, c0, min(n, c0 + SCAN_TILE), 256);
+    }
+}
+
+// The three phases in one block, for n <= SCAN_ONE (three launches cost more
+// than the scan).  max_total >= 0: the total is kept within it, BH_ERR_ITEMS
+// raised beyond.
+template <bool CNT>
+__global__ __launch_bounds__(1024) void k_scan_one(const int32_t* __restrict__ in, int n,
+                                                   int32_t* out_v, int32_t* out_f, int32_t* ne_list,
+                                                   int32_t* cursor, double* com_dense,
+                                                   int32_t* stats, int total_slot,
+                                                   int64_t max_total)
+{
+    __shared__ int sh[40];
+    constexpr int R = SCAN_ONE / 1024;
+    const int base = threadIdx.x * R;
+    int cv[R];
+    int v = 0, f = 0, mx = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = base + r;
+        cv[r] = i < n ? in[i] : 0;
+        v += cv[r];
+        f += cv[r] > 0;
+        mx = max(mx, cv[r]);
+    }
+    int av, af, tv, tf;
+    block_excl_scan2(v, f, av, af, tv, tf, sh);
+    if (CNT) {
+        mx = wave_max(mx);
+        if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&stats[ST_MAXCOUNT], mx);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = base + r;
+        if (i < n) {
+            out_v[i] = av;
+            if (CNT) {
+                out_f[i] = af;
+                if (cv[r] > 0) ne_list[af] = i;
+            }
+            av += cv[r];
+            af += cv[r] > 0;
+        }
+    }
+    if (threadIdx.x == 0) {
+        out_v[n] = tv;
+        if (CNT) {
+            out_f[n] = tf;
+            stats[ST_NCELLS_NE] = tf;
+        }
+        if (total_slot >= 0) {
+            const bool over = max_total >= 0 && tv > max_total;
+            stats[total_slot] = over ? (int32_t)max_total : tv;
+            if (over) atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
+        }
+    }
+    if (CNT) clear_cells({ne_list, cursor, com_dense}, 0, n, 1024);
 }
 
 template __global__ void k_scan_reduce<true>(const int32_t*, int64_t, int32_t*, int32_t*, int32_t*);
@@ -379,9 +513,14 @@ template __global__ void k_scan_reduce<false>(const int32_t*, int64_t, int32_t*,
 template __global__ void k_scan_blocks<true>(int32_t*, int32_t*, int64_t, int32_t*, int);
 template __global__ void k_scan_blocks<false>(int32_t*, int32_t*, int64_t, int32_t*, int);
 template __global__ void k_scan_final<true>(const int32_t*, int64_t, const int32_t*, const int32_t*,
-                                            int32_t*, int32_t*);
+                                            int32_t*, int32_t*, int32_t*, int32_t*, double*);
 template __global__ void k_scan_final<false>(const int32_t*, int64_t, const int32_t*,
-                                             const int32_t*, int32_t*, int32_t*);
+                                             const int32_t*, int32_t*, int32_t*, int32_t*, int32_t*,
+                                             double*);
+template __global__ void k_scan_one<true>(const int32_t*, int, int32_t*, int32_t*, int32_t*,
+                                          int32_t*, double*, int32_t*, int, int64_t);
+template __global__ void k_scan_one<false>(const int32_t*, int, int32_t*, int32_t*, int32_t*,
+                                           int32_t*, double*, int32_t*, int, int64_t);
 
 // 64-bit key ordered as numpy orders doubles: -0.0 equals +0.0, every NaN is
 // equal to every other NaN and sorts after all numbers.
@@ -397,6 +536,7 @@ __device__ __forceinline__ uint64_t sort_key(double d)
 // cursor); the order inside a cell is fixed afterwards by k_sort_units.
 // Each row's px and py sort keys travel with it, so that pass reads them
 // contiguously (rows clipped to the box edge tie in px by the thousand).
+template <int R>
 __global__ __launch_bounds__(256) void k_scatter(const int32_t* __restrict__ key, int64_t N,
                                                  const int32_t* __restrict__ offsets,
                                                  int32_t* __restrict__ cursor,
@@ -409,8 +549,7 @@ __global__ __launch_bounds__(256) void k_scatter(const int32_t* __restrict__ key
 {
     __shared__ int32_t hist[HIST_BINS];
     __shared__ int red[8];
-    constexpr int R = PLACE_CHUNK / 256;
-    int64_t base = (int64_t)blockIdx.x * PLACE_CHUNK;
+    int64_t base = (int64_t)blockIdx.x * (256 * R);
     int kk[R];
     int kmin = INT_MAX, kmax = INT_MIN;
 #pragma unroll
@@ -463,6 +602,11 @@ __global__ __launch_bounds__(256) void k_scatter(const int32_t* __restrict__ key
         }
     }
 }
+
+template __global__ void k_scatter<2>(const int32_t*, int64_t, const int32_t*, int32_t*, int32_t*,
+                                      int32_t*, const double*, const double*, uint64_t*, uint64_t*);
+template __global__ void k_scatter<8>(const int32_t*, int64_t, const int32_t*, int32_t*, int32_t*,
+                                      int32_t*, const double*, const double*, uint64_t*, uint64_t*);
 
 // ---------------------------------------------------------------- within-cell order
 // numpy's structured-sort tie rule after (gx, gy): px, py, mass, vx, vy, ax,
@@ -587,46 +731,42 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_units(SortFields F, int64
     }
 }
 
-// Merge pass for cells longer than SORT_W: runs of length R = SORT_W << L,
-// counted from the cell start, are merged pairwise by binary search.  Only
-// rows of such cells are touched; the pass is a no-op once R >= max count.
+// Merge pass for cells longer than SORT_W: runs of length R = SORT_W *
+// SORT_WAYS^L, counted from the cell start, are merged SORT_WAYS at a time: a
+// row's place is its place in its own run plus, by binary search, the rows
+// before it in each of the others.  Only rows of such cells are touched; the
+// pass is a no-op once R >= max count.  (Pairwise merging searches less per row
+// but takes three times the launches, and most of them find nothing to do: 12
+// at 4.5 us on 4.2M particles.)
 __global__ __launch_bounds__(256) void k_sort_merge(SortFields F, int64_t N,
                                                     const int32_t* __restrict__ idx_in,
                                                     const int32_t* __restrict__ key_sorted,
                                                     const int32_t* __restrict__ offsets,
-                                                    int32_t* __restrict__ idx_out, int L,
+                                                    int32_t* __restrict__ idx_out, int64_t R,
                                                     const int32_t* __restrict__ stats)
 {
-    const int64_t R = (int64_t)SORT_W << L;
     if (R >= stats[ST_MAXCOUNT]) return;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < N; q += stride) {
         int k = key_sorted[q];
         int64_t a = offsets[k], b = offsets[k + 1];
         if (b - a <= SORT_W) continue;
-        int e = idx_in[q];
-        int64_t W0 = a + ((q - a) / (2 * R)) * (2 * R);
-        int64_t mid = W0 + R, hi = min(b, W0 + 2 * R);
-        int64_t own0, p0, p1;
-        if (q < mid) {
-            own0 = W0;
-            p0 = mid;
-            p1 = hi;
-        } else {
-            own0 = mid;
-            p0 = W0;
-            p1 = mid;
+        const int e = idx_in[q];
+        const int64_t W0 = a + ((q - a) / (SORT_WAYS * R)) * (SORT_WAYS * R);
+        const int own = (int)((q - W0) / R);
+        int64_t place = q - (W0 + own * R);
+        for (int r = 0; r < SORT_WAYS; ++r) {
+            if (r == own) continue;
+            const int64_t p0 = W0 + r * R, p1 = min(b, p0 + R);
+            if (p0 >= b) break;
+            int64_t lo = p0, hi = p1;
+            while (lo < hi) {
+                const int64_t m = (lo + hi) >> 1;
+                if (row_less(F, idx_in[m], e)) lo = m + 1; else hi = m;
+            }
+            place += lo - p0;
         }
-        if (p0 >= p1) {
-            idx_out[q] = e;
-            continue;
-        }
-        int64_t lo2 = p0, hi2 = p1;
-        while (lo2 < hi2) {
-            int64_t m2 = (lo2 + hi2) >> 1;
-            if (row_less(F, idx_in[m2], e)) lo2 = m2 + 1; else hi2 = m2;
-        }
-        idx_out[W0 + (q - own0) + (lo2 - p0)] = e;
+        idx_out[W0 + place] = e;
     }
 }
 
@@ -643,7 +783,7 @@ __global__ __launch_bounds__(256) void k_gather(SortFields S, BhParticles D, int
 {
     int mc = stats[ST_MAXCOUNT];
     int npass = 0;
-    while (((int64_t)SORT_W << npass) < mc) ++npass;
+    for (int64_t R = SORT_W; R < mc; R *= SORT_WAYS) ++npass;
     const int32_t* big = (npass & 1) ? idx_a : idx_b;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < N; q += stride) {

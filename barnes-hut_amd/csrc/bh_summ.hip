@@ -6,15 +6,6 @@
 #include "bh_common.h"
 #include "bh_kernels.h"
 
-// Compact list of non-empty cells in global cell order.
-__global__ void k_ne_list(const int32_t* __restrict__ counts, const int32_t* __restrict__ neprefix,
-                          int64_t C, int32_t* __restrict__ ne_list)
-{
-    int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < C; c += stride)
-        if (counts[c] > 0) ne_list[neprefix[c]] = (int32_t)c;
-}
-
 // FP64 sums of m*x, m*y, m over each non-empty cell's sorted particles.
 // Writes the dense G*G x 3 array of the reference layout (empty cells were
 // zero-filled) and the two compact lists the force kernels stream.

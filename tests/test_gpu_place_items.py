@@ -1,0 +1,102 @@
+"""Placement, merge passes and work items at the sizes where their launches
+change: sets below and above the small-set limit, systems that end inside a
+wave, cells of one run, of eight runs and beyond (merge passes), columns whose
+items are plain runs and columns cut by the row span.  Everything is an integer
+or an order: exact."""
+import numpy as np
+import pytest
+
+from conftest import gpu_available
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
+
+from barneshut import inputs  # noqa: E402
+from oracle import oracle as orc  # noqa: E402
+
+
+def _greedy_items(counts, offsets, sizes, grids, pitem, yspan):
+    """Runs of pitem particles of a column, closed yspan rows below their first."""
+    out, c0 = [], 0
+    for s, G in enumerate(grids):
+        for x in range(G):
+            it = None
+            for y in range(G):
+                c = c0 + x * G + y
+                n, p = int(counts[c]), int(offsets[c])
+                if n and it is not None and y - it[4] >= yspan:
+                    out.append(it)
+                    it = None
+                while n:
+                    if it is None:
+                        it = [p, 0, s, x, y, y]
+                    t = min(n, pitem - it[1])
+                    it[1] += t
+                    it[5] = y
+                    p += t
+                    n -= t
+                    if it[1] == pitem:
+                        out.append(it)
+                        it = None
+            if it is not None:
+                out.append(it)
+        c0 += G * G
+    return np.array(out, np.int32).reshape(-1, 6)
+
+
+@pytest.mark.parametrize("sizes,grids,p,yspan", [
+    ([1000], [7], 1, 512), ([1000], [7], 1, 3), ([5000], [40], 2, 40), ([5000], [40], 2, 39),
+    ([70001], [50], 4, 512), ([3, 900, 64, 5000, 2], [2, 11, 1, 30, 9], 1, 512),
+    ([300, 20000], [600, 20], 2, 512), ([300001], [300], 2, 16)])
+def test_items_and_placement(sizes, grids, p, yspan):
+    from barneshut.engine import Engine
+    d = inputs.batched_uniform(sizes, seed=71)
+    eng = Engine(sizes, grids, tuning=dict(p=p, yspan=yspan, waves_per_cu=8, tail_split=1,
+                                           tail_items=0))
+    eng.load(d)
+    for _ in range(2):   # the second time from the sorted rows
+        src = eng.fetch()
+        eng.create_tree()
+        eng.summarize()
+        eng.ctx.build_items()
+        eng.check()
+    counts, offsets, items = eng.counts(), eng.offsets(), eng.items()
+    np.testing.assert_array_equal(items[:, :6],
+                                  _greedy_items(counts, offsets, sizes, grids, 64 * p, yspan))
+    h, com, box = eng.fetch(), eng.com(), eng.bbox()
+    p0 = c0 = 0
+    for s, (n, G) in enumerate(zip(sizes, grids)):
+        sl = slice(p0, p0 + n)
+        bb = orc.bbox(src["px"][sl], src["py"][sl], G)
+        assert tuple(box[s][[0, 1, 2, 4]]) == (bb[0], bb[1], bb[2], bb[4])
+        _, _, key = orc.place(src["px"][sl], src["py"][sl], bb[0], bb[1], bb[4], G)
+        np.testing.assert_array_equal(counts[c0:c0 + G * G], np.bincount(key, minlength=G * G))
+        order = orc.sort_perm(key, [src[k][sl] for k in ("px", "py", "mass", "vx", "vy", "ax", "ay",
+                                                         "pid")])
+        np.testing.assert_array_equal(h["pid"][sl], src["pid"][sl][order])
+        empty = counts[c0:c0 + G * G] == 0
+        assert (com[c0:c0 + G * G][empty] == 0.0).all()
+        p0 += n
+        c0 += G * G
+    eng.close()
+
+
+@pytest.mark.parametrize("n,G", [(1024, 1), (1025, 1), (8192, 1), (8193, 1), (30000, 1),
+                                 (70000, 1), (200000, 2), (300000, 1)])
+def test_merge_passes(n, G):
+    """One or four cells of up to 300,000 rows, many of them tied in px and py."""
+    from barneshut.engine import Engine
+    rng = np.random.default_rng(n)
+    d = inputs.uniform(n, seed=72)
+    d["px"] = np.round(d["px"], 2)
+    d["py"] = np.round(d["py"], 1)
+    d["mass"] = rng.integers(1, 4, n).astype(np.float64)
+    eng = Engine([n], [G])
+    eng.load(d)
+    eng.create_tree()
+    eng.check()
+    h, keys = eng.fetch(), eng.keys()
+    o = np.lexsort((h["pid"], h["mass"], h["py"], h["px"], keys))
+    np.testing.assert_array_equal(o, np.arange(n))
+    np.testing.assert_array_equal(np.sort(h["pid"]), np.arange(n))
+    eng.close()
