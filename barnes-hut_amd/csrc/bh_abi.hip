@@ -101,6 +101,7 @@ struct bh_ctx_s {
     double* rc_bfar = nullptr;     // per block: its far-block part of the bound
     int64_t nblocks = 0;
     int maxG = 0;                  // largest grid side
+    double terms = 0.0;            // far terms of a pass: sum of n min(n, cells)
     int64_t nchunks = 0;           // chunks of 64 particles of one system
     // grouped far field (bh_fmm.hip): which passes take it is a rule on the
     // systems' sizes (fmm_wanted)
@@ -157,6 +158,12 @@ static unsigned persistent_grid(const Ctx* c, int split)
     const int64_t want = (int64_t)c->num_cu * c->tune.waves_per_cu;
     const int64_t queue = (cdiv(c->N, 64LL * c->tune.p) + 2 * c->ncols) * split;
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, queue));
+}
+
+// Far terms of a system, at most.
+static double far_terms(int64_t n, int32_t G)
+{
+    return (double)n * std::min((double)n, (double)G * G);
 }
 
 // Checks the system sizes and lays the systems out in the global particle,
@@ -225,6 +232,7 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 // systems are where a learned queue order shortens the pass (it orders work
 // items, which grouped passes do not have), and because the recompute, whose
 // flags callers read, belongs to the term-by-term pass.
+static constexpr double FP32_SHARED_TERMS = 4e9;
 static constexpr double FMM_MIN_TERMS_FP64 = 4e9;
 static constexpr double FMM_MIN_TERMS_FP32 = 2e10;
 static constexpr size_t FMM_MAX_BYTES = (size_t)48 << 30;
@@ -236,7 +244,7 @@ static int fmm_wanted(const std::vector<SysDev>& sh)
     int64_t side = 0;
     for (const SysDev& d : sh) {
         if (d.G < FMM_MIN_GRID) continue;
-        terms += (double)d.n * std::min((double)d.n, (double)d.G * d.G);
+        terms += far_terms(d.n, d.G);
         const double n0 = (double)cdiv(d.G, FMM_TILE);
         tiles += n0 * n0 * (4.0 / 3.0);
         side = std::max(side, cdiv(d.G, FMM_TILE));
@@ -547,6 +555,8 @@ int bh_set_systems(void* ctx, int32_t nsys, const int64_t* n, const int32_t* gri
     c->sys_h = sh;
     c->nchunks = sh.back().k_off + cdiv(sh.back().n, 64);
     c->maxG = *std::max_element(grid_dim, grid_dim + nsys);
+    c->terms = 0.0;
+    for (const SysDev& d : sh) c->terms += far_terms(d.n, d.G);
     int r = configure(c, nsys, N, C, cols, maxN, NB);
     if (r == BH_OK) r = ensure_part(c);
     if (r != BH_OK) {
@@ -866,6 +876,17 @@ int bh_force_pass(void* ctx, const bh_particles* p, const bh_law* law, int32_t p
     return bh_force_pass_part(ctx, p, law, precision, order, 0, 1, stream);
 }
 
+// Whether an FP32 pass goes by shared chunks (k_force32s) or by the queue of
+// work items (k_force32).  Chunks were faster on all of 28 single systems from
+// 2,000 to 4M particles but the densest (4M clustered particles on 30^2 cells,
+// 378 against 395 ms).  Batches of several systems keep the queue from 4e9 far
+// terms on (~1.5 ms): there the learned order, which sorts the queue's items,
+// shortens the pass by 1 to 11 %.
+static bool fp32_shared(const Ctx* c)
+{
+    return c->S == 1 || c->terms <= FP32_SHARED_TERMS;
+}
+
 int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int32_t precision,
                        const int32_t* order, int32_t part, int32_t nparts, void* stream)
 {
@@ -947,17 +968,26 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     fa.rc = rc ? 1 : 0;
     fa.qpart = part;
     fa.nqparts = nparts;
+    const bool shared = precision == 1 && !c->cost_log_on && fp32_shared(c);
     if (rc) {   // the FP32 result goes to scratch; the recompute adds it (or the FP64 one)
-        if (part == 0)
+        if (part == 0 && !shared)
             hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(2 * c->N, 256, 8192)), dim3(256), 0, st,
                                c->rc_a32, 2 * c->N, 0.0);
         fa.ax = c->rc_a32;
         fa.ay = c->rc_a32 + c->N;
     }
     if (part == 0) c->rc_ready = 0;   // until the last part: no recompute of a partial pass
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_QUEUE, (int64_t)1, 0);
-    void* args[] = {&fa};
-    HIP_TRY(hipLaunchKernel(fn, dim3(persistent_grid(c, fa.split)), dim3(64), args, 0, st));
+    if (shared) {
+        fa.chunk0 = c->nchunks * part / nparts;
+        const int64_t end = c->nchunks * (part + 1) / nparts;
+        if (end > fa.chunk0) bh_force32s(fa, lawi, c->S, end - fa.chunk0, st);
+        fa.split = 1;   // no slices to add
+    } else {
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_QUEUE, (int64_t)1,
+                           0);
+        void* args[] = {&fa};
+        HIP_TRY(hipLaunchKernel(fn, dim3(persistent_grid(c, fa.split)), dim3(64), args, 0, st));
+    }
     if (part < nparts - 1) {   // the slice combine and the recompute follow the last part
         LAUNCH_CHECK("evaluate");
         return BH_OK;
@@ -1486,6 +1516,7 @@ extern "C" int bh_step_noalloc(const bh_particles* a, const bh_particles* b, int
     set_sizes(&c, 1, n, G * G, G, n, Gb * Gb);
     c.nchunks = cdiv(n, 64);
     c.maxG = grid_dim;
+    c.terms = far_terms(n, grid_dim);
     size_t off = 0;
     r = for_each_buffer(&c, [&](auto*& p, int64_t cnt) {
         using T = std::remove_reference_t<decltype(*p)>;

@@ -1162,6 +1162,268 @@ __global__ __launch_bounds__(256) void k_force_combine(const Item* __restrict__ 
     }
 }
 
+// ---------------------------------------------------------------- FP32, shared chunks
+// The terms of k_force32 (tile sums carried in FP64 instead of Kahan pairs),
+// with the work of 64 particles shared by the W waves of a block, as in
+// k_force64s.  Near separations are formed in FP64 in units of 1 / sig and
+// rounded once; far entries are staged per wave in LDS in mass-scaled,
+// cell-relative form (origin: the chunk's first cell), 64 at a time, the next
+// 64 on their way.
+// Force pass with the recompute against k_force32 (default launch shape):
+// 2,000 particles on 11^2 cells 165 -> 70 us, 16,384 on 32^2 210 -> 72 us, in
+// clusters 486 -> 143 us; 262,144 on 256^2 3.47 -> 3.31 ms, 1M on 100^2 2.74 ->
+// 2.46 ms and 14.2 -> 7.6 ms in clusters.
+template <int LAW, bool OWN>
+__device__ __forceinline__ void near_four32(const Four& f, int j, int b, int gi, double x, double y,
+                                            double sig, double inv_msc, float eps2, float r2cut,
+                                            double& sx, double& sy, float& s2n)
+{
+    float tx = 0.0f, ty = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float wx = (float)fma(f.X[u], sig, -x), wy = (float)fma(f.Y[u], sig, -y);
+        const float fm = (float)(f.M[u] * inv_msc);
+        float q;
+        bool keep = true;
+        if (LAW == 1) {
+            const float s2 = fmaf(wx, wx, wy * wy);
+            keep = s2 > r2cut;
+            q = s2 + eps2;
+        } else {
+            q = fmaf(wx, wx, fmaf(wy, wy, eps2));
+        }
+        float t = fm * __builtin_amdgcn_rcpf(q);
+        if (OWN) keep = keep && (j + u < b ? j + u : j) != gi;
+        // past the end: a copy of the first without mass
+        if (LAW == 1 || OWN) t = keep ? t : 0.0f;
+        s2n = fmaf(fm, t, s2n);
+        tx = fmaf(wx, t, tx);
+        ty = fmaf(wy, t, ty);
+    }
+    sx += (double)tx;
+    sy += (double)ty;
+}
+
+template <int W, int LAW, bool OWN>
+__device__ __forceinline__ void near_cell32(const ForceArgs& A, int j, int b, int N, int gi,
+                                            double x, double y, double sig, double inv_msc,
+                                            float eps2, float r2cut, double& sx, double& sy,
+                                            float& s2n)
+{
+    if (j >= b) return;
+    Four f = load_four(A.x, A.y, A.m, j, b, N);
+    for (;;) {
+        const int jn = j + 4 * W;
+        Four n = f;
+        if (jn < b) n = load_four(A.x, A.y, A.m, jn, b, N);
+        near_four32<LAW, OWN>(f, j, b, gi, x, y, sig, inv_msc, eps2, r2cut, sx, sy, s2n);
+        if (jn >= b) break;
+        f = n;
+        j = jn;
+    }
+}
+
+template <int W, int LAW>
+__global__ __launch_bounds__(64 * W) void k_force32s(ForceArgs A, int S)
+{
+    __shared__ float4 ftile[W][BH_WAVE];
+    __shared__ int32_t ktile[W][BH_WAVE];
+    __shared__ double part[2][W][BH_WAVE];
+    __shared__ float part2[W][BH_WAVE];
+    const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
+    const int64_t ci = A.chunk0 + blockIdx.x;
+    int s = 0;
+    if (S > 1) {   // the system of the chunk
+        int hi = S - 1;
+        while (s < hi) {
+            const int mid = (s + hi + 1) >> 1;
+            if (A.sys[mid].k_off <= ci) s = mid; else hi = mid - 1;
+        }
+        s = uniform_int(s);
+    }
+    const SysDev& d = A.sys[s];
+    const int G = d.G;
+    const int64_t coff = d.c_off;
+    const int rank = (int)(ci - d.k_off) * 64 + lane;
+    const bool act = rank < d.n;
+    const int gi = act ? (int)d.p_off + rank : -1;
+    const double step = d.step, inv_step = 1.0 / step, sig = step_scale(step);
+    const float eps2n = (float)(A.eps2 * sig * sig), r2cn = (float)(A.r2cut * sig * sig);
+    const float eps2c = (float)(A.eps2 * inv_step * inv_step);
+    const float r2c = (float)(A.r2cut * inv_step * inv_step);
+    double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, fx = 0.0, fy = 0.0;
+    float s2n = 0.0f, ux = 0.0f, uy = 0.0f;
+    int cx = -100000, cy = -100000, key = 0;
+    if (act) {
+        x = A.x[gi];
+        y = A.y[gi];
+        key = A.key_sorted[gi] - (int)coff;
+        cx = key / G;
+        cy = key - cx * G;
+    }
+    const int ox = __builtin_amdgcn_readfirstlane(cx), oy = __builtin_amdgcn_readfirstlane(cy);
+    const int own = __builtin_amdgcn_readfirstlane(key);
+    // mass scale, as in k_force32: the power of two at or above the own cell's mass
+    float msc = 1.0f;
+    {
+        const float r0 = fabsf(A.l32[A.neprefix[coff + own]].rM);
+        const float p2 = __int_as_float(__float_as_int(r0) & 0x7f800000);
+        if (p2 >= 1.0e-37f && p2 <= 1.0e37f) msc = 1.0f / p2;
+    }
+    const double inv_msc = 1.0 / (double)msc;
+    if (act) {
+        ux = (float)((x - d.min_x) * inv_step - (double)ox);
+        uy = (float)((y - d.min_y) * inv_step - (double)oy);
+        x *= sig;
+        y *= sig;
+    }
+    const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
+    const int cxh = uniform_int(wave_max(act ? cx : -1));
+    const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
+    const int cyh = uniform_int(wave_max(act ? cy : -1));
+
+    // near candidates
+    if (cxl == cxh && cyh - cyl < 2) {
+        int turn = 0;   // groups of four so far, dealt to the waves in turn
+        for (int dx = -1; dx <= 1; ++dx) {
+            const int xc = cxl + dx;
+            if (xc < 0 || xc >= G) continue;
+            const int64_t cl = coff + (int64_t)xc * G;
+            for (int row = max(cyl - 1, 0); row <= min(cyh + 1, G - 1); ++row) {
+                const int a = uniform_int(A.offsets[cl + row]);
+                const int b = uniform_int(A.offsets[cl + row + 1]);
+                const int first = (w - turn) & (W - 1);
+                turn += (b - a + 3) >> 2;
+                if (!(act && abs(row - cy) <= 1)) continue;
+                if (dx == 0 && row >= cyl && row <= cyh)   // some lanes' own cell
+                    near_cell32<W, LAW, true>(A, a + 4 * first, b, (int)A.part_n, gi, x, y, sig,
+                                              inv_msc, eps2n, r2cn, sx, sy, s2n);
+                else
+                    near_cell32<W, LAW, false>(A, a + 4 * first, b, (int)A.part_n, gi, x, y, sig,
+                                               inv_msc, eps2n, r2cn, sx, sy, s2n);
+            }
+        }
+    } else if (act) {
+        int n0 = 0, n1 = 0, n2 = 0, o0 = 0, o1 = 0, o2 = 0;   // the three ranges as one list
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int xc = cx + t - 1;
+            int a = 0, b = 0;
+            if (xc >= 0 && xc < G) {
+                const int64_t cl = coff + (int64_t)xc * G;
+                a = A.offsets[cl + max(cy - 1, 0)];
+                b = A.offsets[cl + min(cy + 1, G - 1) + 1];
+            }
+            if (t == 0) { o0 = a; n0 = b - a; }
+            if (t == 1) { o1 = a - n0; n1 = n0 + b - a; }
+            if (t == 2) { o2 = a - n1; n2 = n1 + b - a; }
+        }
+#pragma unroll 2
+        for (int k = w; k < n2; k += W) {
+            const int j = k + (k < n0 ? o0 : (k < n1 ? o1 : o2));
+            const float wx = (float)fma(A.x[j], sig, -x), wy = (float)fma(A.y[j], sig, -y);
+            const float fm = (float)(A.m[j] * inv_msc);
+            const float s2 = fmaf(wx, wx, wy * wy);
+            float t = fm * __builtin_amdgcn_rcpf(s2 + eps2n);
+            const bool keep = j != gi && (LAW == 0 || s2 > r2cn);
+            t = keep ? t : 0.0f;
+            s2n = fmaf(fm, t, s2n);
+            sx += (double)(wx * t);
+            sy += (double)(wy * t);
+        }
+    }
+
+    // COM list: this wave's slice
+    const int ne0 = uniform_int(A.neprefix[coff]);
+    const int ne1 = uniform_int(A.neprefix[coff + (int64_t)G * G]);
+    const int mlo = uniform_int(A.neprefix[coff + (int64_t)max(cxl - 1, 0) * G]);
+    const int mhi = uniform_int(A.neprefix[coff + (int64_t)min(cxh + 2, G) * G]);
+    const int per = (((ne1 - ne0 + W - 1) / W) + 7) & ~7;
+    const int f0 = min(ne1, ne0 + w * per), f1 = min(ne1, f0 + per);
+    auto fetch = [&](int e) {
+        Com32 c;
+        if (e < f1) {
+            c = A.l32[e];
+        } else {
+            c.fx = 1e18f; c.fy = 1e18f; c.rM = __builtin_huge_valf(); c.kxy = 0x7fff7fff;
+        }
+        return c;
+    };
+    Com32 nxt = fetch(f0 + lane);
+    for (int base = f0; base < f1; base += BH_WAVE) {
+        const int kx = nxt.kxy >> 16, ky = nxt.kxy & 0xffff;
+        const float ex = (float)(kx - ox) + nxt.fx, ey = (float)(ky - oy) + nxt.fy;
+        float4 v;
+        if (LAW == 0) {
+            v.x = 1e30f; v.y = 1e30f; v.z = 0.0f; v.w = 0.0f;
+            if (fabsf(nxt.rM) != __builtin_huge_valf()) {   // M != 0 (NaN passes)
+                const float c = msc * nxt.rM;
+                v.x = ex * c;
+                v.y = ey * c;
+                v.z = -c;
+                v.w = (c * c) * eps2c;
+            }
+        } else {
+            v.x = ex; v.y = ey; v.z = nxt.rM; v.w = 0.0f;
+        }
+        ftile[w][lane] = v;
+        ktile[w][lane] = nxt.kxy;
+        __builtin_amdgcn_wave_barrier();
+        nxt = fetch(base + BH_WAVE + lane);
+        const int cnt = min(BH_WAVE, (f1 - base + 7) & ~7);   // padded with nothing
+        float tx = 0.0f, ty = 0.0f;
+        auto term = [&](const float4& f, bool keep) {
+            float wx, wy, t;
+            if (LAW == 0) {
+                wx = fmaf(ux, f.z, f.x);
+                wy = fmaf(uy, f.z, f.y);
+                t = __builtin_amdgcn_rcpf(fmaf(wx, wx, fmaf(wy, wy, f.w)));
+            } else {
+                wx = f.x - ux;
+                wy = f.y - uy;
+                t = far_t32<LAW>(wx, wy, f.z, eps2c, r2c);
+            }
+            t = keep ? t : 0.0f;
+            tx = fmaf(wx, t, tx);
+            ty = fmaf(wy, t, ty);
+        };
+        if (!meets(base, base + BH_WAVE, mlo, mhi)) {
+#pragma unroll 8
+            for (int j = 0; j < cnt; ++j) term(ftile[w][j], true);
+        } else {
+            for (int j = 0; j < cnt; ++j) {
+                const int k = ktile[w][j];
+                term(ftile[w][j], (unsigned)((k >> 16) - cx + 1) > 2u ||
+                                      (unsigned)((k & 0xffff) - cy + 1) > 2u);
+            }
+        }
+        fx += (double)tx;
+        fy += (double)ty;
+        __builtin_amdgcn_wave_barrier();
+    }
+    // near sums are in units of msc / (1 / sig), far ones of msc / step (LAW 0) or 1 / step
+    const double fs = LAW == 0 ? inv_step * (double)msc : inv_step;
+    part[0][w][lane] = sx * (sig * (double)msc) + fx * fs;
+    part[1][w][lane] = sy * (sig * (double)msc) + fy * fs;
+    part2[w][lane] = s2n;
+    __syncthreads();
+    if (!act) return;
+    if (w < 2) {   // wave 0 adds x, wave 1 adds y
+        double t = 0.0;
+#pragma unroll
+        for (int v = 0; v < W; ++v) t += part[w][v][lane];
+        double* a = w ? A.ay : A.ax;
+        if (A.rc) a[gi] = A.Gc * t;   // a scratch plane: the recompute adds it
+        else a[gi] += A.Gc * t;
+    } else if (w == 2 && A.rc) {   // sum of (m / r)^2, r in cells
+        double t = 0.0;
+#pragma unroll
+        for (int v = 0; v < W; ++v) t += (double)part2[v][lane];
+        const double ms = (double)msc * (step * sig);
+        A.ay[A.part_n + gi] = t * (ms * ms);
+    }
+}
+
 // ---------------------------------------------------------------- FP32 + matrix cores
 // Same decomposition and coordinates as k_force32, with the far-field sum
 // split as  sum_k M_k r_k (a_k - u) = sum_k r_k (M_k a_k) - u sum_k r_k M_k,
@@ -1426,4 +1688,11 @@ void bh_force64s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_
     const dim3 g((unsigned)nchunks), b(64 * F64S_WAVES);
     if (law) hipLaunchKernelGGL((k_force64s<F64S_WAVES, 1>), g, b, 0, st, A, S);
     else hipLaunchKernelGGL((k_force64s<F64S_WAVES, 0>), g, b, 0, st, A, S);
+}
+
+void bh_force32s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_t st)
+{
+    const dim3 g((unsigned)nchunks), b(64 * F32S_WAVES);
+    if (law) hipLaunchKernelGGL((k_force32s<F32S_WAVES, 1>), g, b, 0, st, A, S);
+    else hipLaunchKernelGGL((k_force32s<F32S_WAVES, 0>), g, b, 0, st, A, S);
 }

@@ -53,10 +53,12 @@ struct ForceArgs {
     // FP32 or the FP64 result to the particles' accelerations.  A flag rather
     // than a third pointer keeps the kernel's scalar registers unchanged.
     int rc;
-    int64_t chunk0;   // k_force64s: first chunk of 64 particles of this launch
+    int64_t chunk0;   // k_force64s: first chunk of 64 particles of this launch (k_force32s too)
 };
 
 #define F64S_WAVES 8   // waves that share 64 particles (a power of two)
+#define F32S_WAVES 8
+void bh_force32s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_t st);
 // k_force64s over nchunks chunks from A.chunk0 on.
 void bh_force64s(const ForceArgs& A, int law, int S, int64_t nchunks, hipStream_t st);
 
