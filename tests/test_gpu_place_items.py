@@ -100,3 +100,37 @@ def test_merge_passes(n, G):
     np.testing.assert_array_equal(o, np.arange(n))
     np.testing.assert_array_equal(np.sort(h["pid"]), np.arange(n))
     eng.close()
+
+
+@pytest.mark.parametrize("kind", ["px", "px_pairs", "px_py", "rows"])
+def test_equal_keys_by_cell_size(kind):
+    """One cell a system, of 2 to 1,026 rows, whose px, px and py or whole rows
+    tie; a first row elsewhere gives the box an extent."""
+    from barneshut.engine import Engine
+    rng = np.random.default_rng(5)
+    sizes = [2, 3, 7, 8, 9, 10, 15, 16, 17, 18, 64, 66, 1023, 1024, 1025, 1026]
+    d = inputs.batched_uniform(sizes, seed=73)
+    if kind == "px_pairs":
+        d["px"] = np.round(d["px"] * 64) / 64
+    else:
+        d["px"][:] = 0.25
+    if kind in ("px_py", "rows"):
+        d["py"][:] = 0.5
+    first = np.cumsum([0] + sizes[:-1])
+    d["px"][first] = d["py"][first] = 1.0
+    d["mass"][:] = 1.0 if kind == "rows" else rng.integers(1, 9, len(d["px"]))
+    eng = Engine(sizes, [1] * len(sizes))
+    eng.load(d)
+    src = eng.fetch()
+    eng.create_tree()
+    eng.check()
+    h = eng.fetch()
+    p0 = 0
+    for n in sizes:
+        sl = slice(p0, p0 + n)
+        order = orc.sort_perm(np.zeros(n, np.int64), [src[k][sl] for k in (
+            "px", "py", "mass", "vx", "vy", "ax", "ay", "pid")])
+        for k in ("pid", "px", "py", "mass"):
+            np.testing.assert_array_equal(h[k][sl], src[k][sl][order])
+        p0 += n
+    eng.close()
