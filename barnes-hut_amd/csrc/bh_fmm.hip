@@ -209,13 +209,13 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
         }
         __syncthreads();
     }
-    if (tid < (-ne & 3)) {   // padding: no mass, far from everything
+    if (tid < (-ne & 3)) {   // padding: no mass, far away (three in a product of four)
         FmmCom f;
-        f.X = 1e60;
-        f.Y = 1e60;
+        f.X = 1e30;
+        f.Y = 1e30;
         f.M = 0.0;
-        f.kx = -100000;
-        f.ky = -100000;
+        f.kx = 0x3fffffff;   // after the last column
+        f.ky = 0x3fffffff;
         A.list[e0 + ne + tid] = f;
     }
     if (!up) return;
@@ -542,10 +542,9 @@ __device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int
     const cptr<FmmPart> E = as_const(pack);
     for (; j + 3 < b; j += step) {
         const fd8 p = *(cptr<fd8>)(E + j), q = *(cptr<fd8>)(E + j + 2);
-        pair_terms<LAW, OWN>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
-                             j + 1 != gi, eps2, r2cut, sx, sy);
-        pair_terms<LAW, OWN>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6], j + 2 != gi,
-                             j + 3 != gi, eps2, r2cut, sx, sy);
+        quad_terms<LAW, OWN>({p[0] - x, p[4] - x, q[0] - x, q[4] - x},
+                             {p[1] - y, p[5] - y, q[1] - y, q[5] - y}, {p[2], p[6], q[2], q[6]},
+                             {j != gi, j + 1 != gi, j + 2 != gi, j + 3 != gi}, eps2, r2cut, sx, sy);
     }
     if (j + 1 < b) {
         const fd8 p = *(cptr<fd8>)(E + j);
@@ -582,13 +581,14 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
 // The terms of chunk ci's particles that fall to wave w of the W that share it
 // (a power of two): gi is the lane's particle (-1: none), (rx, ry) its sum.  The
 // tile's coefficients and the mid entries are the same for every lane: scalar
-// loads of whole quads (128 bytes), no test in tiles that no lane's 3x3 cells
-// touch.  Near candidates: if the chunk lies in one column and spans at most
+// loads of whole quads (128 bytes), no test per lane in quads that no lane's 3x3
+// cells touch (a test and its selects double a quad's instructions).  Near
+// candidates: if the chunk lies in one column and spans at most
 // FMM_UNIFORM_ROWS rows, the union of its lanes' ranges is walked with scalar
 // loads and a row test; otherwise each lane walks its own three ranges with
-// vector loads (a union would spend most of its pairs on the test).  Terms go
-// in pairs that share a reciprocal; only cells that hold the lanes themselves
-// are tested for the particle itself.
+// vector loads (a union would spend most of its terms on the test).  Terms go in
+// quads, or a lane's own in pairs, that share a reciprocal; only cells that hold
+// the lanes themselves are tested for the particle itself.
 template <int P, int LAW>
 __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int W, double eps2p,
                                             double r2cutp, int& gi, double& rx, double& ry)
@@ -685,10 +685,10 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
             if (!touch && plain) {
                 for (int e = 4 * w; e < ne; e += 4 * W) {
                     const fd8 p = E[e >> 1], q = E[(e >> 1) + 1];
-                    pair_terms<0, false>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
-                                         true, true, eps2, r2cut, sx, sy);
-                    pair_terms<0, false>(q[0] - x, q[1] - y, q[2], q[4] - x, q[5] - y, q[6],
-                                         true, true, eps2, r2cut, sx, sy);
+                    quad_terms<0, false>({p[0] - x, p[4] - x, q[0] - x, q[4] - x},
+                                         {p[1] - y, p[5] - y, q[1] - y, q[5] - y},
+                                         {p[2], p[6], q[2], q[6]}, {true, true, true, true}, eps2,
+                                         r2cut, sx, sy);
                 }
             } else {
                 auto far = [&](double kxy) {
@@ -696,10 +696,26 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
                     return (unsigned)((int)c - cx + 1) > 2u ||
                            (unsigned)((int)(c >> 32) - cy + 1) > 2u;
                 };
-                for (int e = 2 * w; e < ne; e += 2 * W) {
-                    const fd8 p = E[e >> 1];
-                    pair_terms<LAW, true>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6],
-                                          far(p[3]), far(p[7]), eps2, r2cut, sx, sy);
+                for (int e = 4 * w; e < ne; e += 4 * W) {
+                    const fd8 p = E[e >> 1], q = E[(e >> 1) + 1];
+                    // the quad's cells, in column order: does one of them lie
+                    // in some lane's 3x3?
+                    const long long c0 = __double_as_longlong(p[3]);
+                    const long long c3 = __double_as_longlong(q[7]);
+                    const int kx0 = (int)c0, kx3 = (int)c3, ky0 = (int)(c0 >> 32),
+                              ky3 = (int)(c3 >> 32);
+                    const bool meet = kx3 >= cxl - 1 && kx0 <= cxh + 1 &&
+                                      (kx0 != kx3 || (ky3 >= cyl - 1 && ky0 <= cyh + 1));
+                    const double wx[4] = {p[0] - x, p[4] - x, q[0] - x, q[4] - x};
+                    const double wy[4] = {p[1] - y, p[5] - y, q[1] - y, q[5] - y};
+                    const double m[4] = {p[2], p[6], q[2], q[6]};
+                    if (plain && !meet)
+                        quad_terms<0, false>(wx, wy, m, {true, true, true, true}, eps2, r2cut, sx,
+                                             sy);
+                    else
+                        quad_terms<LAW, true>(wx, wy, m,
+                                              {far(p[3]), far(p[7]), far(q[3]), far(q[7])}, eps2,
+                                              r2cut, sx, sy);
                 }
             }
         }
@@ -772,9 +788,10 @@ __global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double 
 // The other chunks, a wave each.  The chunks are left to the hardware's
 // dispatch: a queue cursor (one atomic on the same word every ~15 ns) took 4.2M
 // particles from 2.2 to 3.5 ms, a fixed deal 512 systems from 10.0 to 12.4 ms.
-// Bound by FP64 issue, ~12 slots a term: 2.5e12 terms/s on 10M particles over
-// 120^2 cells (6.7e10 near and mid terms, 26.8 ms; 30.6 ms with entries loaded
-// and tested one by one).
+// Bound by FP64 issue (the vector units are busy 91 % of the time on 4.2M
+// clustered particles over 1024^2 cells): 2.02 ms there, 8.8 ms on 512 systems;
+// 2.16 and 9.9 ms with terms in pairs and every entry of a tile that the 3x3
+// cells touch tested, 2.8 and 12.8 ms with entries loaded one by one.
 template <int P, int LAW>
 __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2, double r2cut,
                                                   int qpart, int nqparts)

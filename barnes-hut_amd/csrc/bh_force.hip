@@ -572,7 +572,7 @@ __global__ __launch_bounds__(64) void k_force64(ForceArgs A)
 //
 // Force pass against the one-wave kernel (uniform particles): 2,000 on 11^2
 // cells 90 -> 16 us, 16,384 on 32^2 152 -> 21 us, 262,144 on 256^2 10.4 -> 6.0 ms
-// (2.9e12 terms/s), 1M on 32^2 (8.8e9 near pairs) 7.3 -> 4.3 ms; no size was
+// (2.9e12 terms/s, with terms in pairs; quads save 2 to 4 % more), 1M on 32^2 (8.8e9 near pairs) 7.3 -> 4.3 ms; no size was
 // slower, so only the cost log, which times work items, still takes k_force64.
 // Loading each quad one ahead of its use is worth 15 % and, where the
 // candidates of a cell exceed an XCD's L2, a third.  W = 4 and 16 are within
@@ -622,12 +622,15 @@ __device__ __forceinline__ void near_four(const Four& f, int j, int b, int gi, d
                                           double sig, double eps2, double r2cut, double& sx,
                                           double& sy)
 {
+    double wx[4], wy[4];
+    bool keep[4];
 #pragma unroll
-    for (int u = 0; u < 4; u += 2)
-        pair_terms<LAW, OWN>(fma(f.X[u], sig, -x), fma(f.Y[u], sig, -y), f.M[u],
-                             fma(f.X[u + 1], sig, -x), fma(f.Y[u + 1], sig, -y), f.M[u + 1],
-                             (j + u < b ? j + u : j) != gi, (j + u + 1 < b ? j + u + 1 : j) != gi,
-                             eps2, r2cut, sx, sy);
+    for (int u = 0; u < 4; ++u) {
+        wx[u] = fma(f.X[u], sig, -x);
+        wy[u] = fma(f.Y[u], sig, -y);
+        keep[u] = (j + u < b ? j + u : j) != gi;
+    }
+    quad_terms<LAW, OWN>(wx, wy, f.M, keep, eps2, r2cut, sx, sy);
 }
 
 // Every (4 W)-th group of four of [j, b), the next one loaded ahead.
@@ -761,25 +764,21 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
                 if (e + 2 >= f1) q[2] = 0.0;
                 q[6] = 0.0;
             }
-            const double wx0 = fma(p[0], sig, -x), wy0 = fma(p[1], sig, -y);
-            const double wx1 = fma(p[4], sig, -x), wy1 = fma(p[5], sig, -y);
-            const double wx2 = fma(q[0], sig, -x), wy2 = fma(q[1], sig, -y);
-            const double wx3 = fma(q[4], sig, -x), wy3 = fma(q[5], sig, -y);
+            const double wx[4] = {fma(p[0], sig, -x), fma(p[4], sig, -x), fma(q[0], sig, -x),
+                                  fma(q[4], sig, -x)};
+            const double wy[4] = {fma(p[1], sig, -y), fma(p[5], sig, -y), fma(q[1], sig, -y),
+                                  fma(q[5], sig, -y)};
+            const double m[4] = {p[2], p[6], q[2], q[6]};
             if (plain && (e + 4 <= mlo || e >= mhi)) {
-                pair_terms<0, false>(wx0, wy0, p[2], wx1, wy1, p[6], true, true, eps2, r2cut, sx,
-                                     sy);
-                pair_terms<0, false>(wx2, wy2, q[2], wx3, wy3, q[6], true, true, eps2, r2cut, sx,
-                                     sy);
+                quad_terms<0, false>(wx, wy, m, {true, true, true, true}, eps2, r2cut, sx, sy);
             } else {
                 auto far = [&](double kxy) {
                     const long long c = __double_as_longlong(kxy);
                     return (unsigned)((int)c - cx + 1) > 2u ||
                            (unsigned)((int)(c >> 32) - cy + 1) > 2u;
                 };
-                pair_terms<LAW, true>(wx0, wy0, p[2], wx1, wy1, p[6], far(p[3]), far(p[7]), eps2,
-                                      r2cut, sx, sy);
-                pair_terms<LAW, true>(wx2, wy2, q[2], wx3, wy3, q[6], far(q[3]), far(q[7]), eps2,
-                                      r2cut, sx, sy);
+                quad_terms<LAW, true>(wx, wy, m, {far(p[3]), far(p[7]), far(q[3]), far(q[7])},
+                                      eps2, r2cut, sx, sy);
             }
             p = pn;
             q = qn;

