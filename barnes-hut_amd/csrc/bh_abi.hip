@@ -235,7 +235,7 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 static constexpr double FP32_SHARED_TERMS = 4e9;
 static constexpr double FMM_MIN_TERMS_FP64 = 4e9;
 static constexpr double FMM_MIN_TERMS_FP32 = 2e10;
-static constexpr size_t FMM_MAX_BYTES = (size_t)48 << 30;
+static constexpr size_t FMM_MAX_BYTES = (size_t)80 << 30;
 
 // Bit 0: fp64 passes, bit 1: fp32 passes.
 static int fmm_wanted(const std::vector<SysDev>& sh)
@@ -250,9 +250,10 @@ static int fmm_wanted(const std::vector<SysDev>& sh)
         side = std::max(side, cdiv(d.G, FMM_TILE));
     }
     // a nearly empty huge grid has more squares to serve than terms to save;
-    // a level's node masses are addressed with 32 bits
+    // a level's node masses are addressed with 32 bits; masses and fields at the
+    // nodes are 3 (P^2 + F^2) numbers a square
     if (terms < 1e6 * tiles || side > 1024 ||
-        tiles * 3.0 * FMM_P64 * FMM_P64 * sizeof(double) > (double)FMM_MAX_BYTES)
+        tiles * 2000.0 * sizeof(double) > (double)FMM_MAX_BYTES)
         return 0;
     const bool noalloc = sh.size() == 1 && sh[0].n <= BH_NOALLOC_MAX_N &&
                          sh[0].G <= BH_NOALLOC_MAX_GRID;
@@ -260,11 +261,14 @@ static int fmm_wanted(const std::vector<SysDev>& sh)
            (terms >= FMM_MIN_TERMS_FP32 ? 2 : 0);
 }
 
-// Chebyshev nodes, transform and parent-child interpolation for P nodes.
+// Chebyshev nodes, transform and parent-child interpolation for P nodes, then the
+// nodes for far offsets and the interpolation from them.
 static std::vector<double> fmm_table(int P)
 {
-    std::vector<double> v(P + 3 * P * P);
+    const int F = fmm_far(P);
+    std::vector<double> v(P + 3 * P * P + F + F * P);
     double *nodes = v.data(), *cheb = nodes + P, *shift = cheb + P * P;
+    double *fnodes = shift + 2 * P * P, *fine = fnodes + F;
     const long double pi = 3.14159265358979323846264338327950288L;
     std::vector<long double> x(P), t(P);
     std::vector<long double> tn(P * P);   // T_k(node i)
@@ -288,6 +292,19 @@ static std::vector<double> fmm_table(int P)
                 shift[(a * P + i) * P + I] = (double)c;
             }
         }
+    std::vector<long double> fn(F);   // T_k of a coarser node
+    for (int I = 0; I < F; ++I) {
+        const long double u = cosl((2 * I + 1) * pi / (2 * F));
+        fnodes[I] = (double)u;
+        fn[0] = 1.0L;
+        fn[1] = u;
+        for (int k = 2; k < F; ++k) fn[k] = 2.0L * u * fn[k - 1] - fn[k - 2];
+        for (int i = 0; i < P; ++i) {
+            long double c = 0.0L;
+            for (int k = 0; k < F; ++k) c += (k ? 2.0L : 1.0L) / F * fn[k] * tn[i * P + k];
+            fine[I * P + i] = (double)c;
+        }
+    }
     return v;
 }
 
@@ -367,18 +384,23 @@ static int fmm_configure(Ctx* c)
         c->fmm.tab[i].nodes = d;
         c->fmm.tab[i].cheb = d + P[i];
         c->fmm.tab[i].shift = d + P[i] + P[i] * P[i];
+        c->fmm.tab[i].fnodes = d + P[i] + 3 * P[i] * P[i];
+        c->fmm.tab[i].fine = c->fmm.tab[i].fnodes + fmm_far(P[i]);
     }
-    const int64_t Q = FMM_P64 * FMM_P64;
+    const int64_t Q = FMM_P64 * FMM_P64, QF = fmm_far(FMM_P64) * fmm_far(FMM_P64);
     if ((r = dalloc(c, &dfs, S)) || (r = dalloc(c, &dt, a.ntiles)) ||
         (r = dalloc(c, &dg, (int64_t)groups.size())) || (r = dalloc(c, &a.tcnt, a.ntiles)) ||
         (r = dalloc(c, &a.tstart, a.nleaf)) || (r = dalloc(c, &a.tne, a.nleaf)) ||
         (r = dalloc(c, &a.cnt, FMM_NCNT + S)) || (r = dalloc(c, &a.chunks, a.max_chunks)) ||
         (r = dalloc(c, &a.list, c->C + 4 * a.nleaf)) || (r = dalloc(c, &a.pack, c->N)) ||
-        (r = dalloc(c, &a.loc, a.ntiles * 2 * Q)))
+        (r = dalloc(c, &a.loc, a.ntiles * 2 * Q)) || (r = dalloc(c, &a.locf, a.ntiles * 2 * QF)))
         return r;
     for (int i = 0; i < 2; ++i) {   // the borders stay zero
-        const int64_t cnt = slots * P[i] * P[i];
+        if (!(wanted >> (1 - i) & 1)) continue;
+        const int F = fmm_far(P[i]);
+        const int64_t cnt = slots * (P[i] * P[i] + F * F);
         if ((r = dalloc(c, &c->fmm.mult[i], cnt))) return r;
+        c->fmm.multf[i] = c->fmm.mult[i] + slots * P[i] * P[i];
         HIP_TRY(hipMemset(c->fmm.mult[i], 0, sizeof(double) * cnt));
     }
     HIP_TRY(hipMemcpy(dfs, fs.data(), sizeof(FmmSys) * S, hipMemcpyHostToDevice));
@@ -482,7 +504,15 @@ static int configure(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, i
     HIP_TRY(hipMemset(c->stats, 0, sizeof(int32_t) * ST_COUNT));
     HIP_TRY(hipMemset(c->offsets, 0, sizeof(int32_t) * (C + 1)));
     HIP_TRY(hipMemset(c->neprefix, 0, sizeof(int32_t) * (C + 1)));
-    if ((r = fmm_configure(c)) != BH_OK) return r;
+    const size_t held = c->allocs.size();
+    if (fmm_configure(c) != BH_OK) {   // no room: every pass stays term by term
+        while (c->allocs.size() > held) {
+            (void)hipFree(c->allocs.back());
+            c->allocs.pop_back();
+        }
+        (void)hipGetLastError();
+        c->fmm_on = 0;
+    }
     HIP_TRY(hipDeviceSynchronize());
     return BH_OK;
 }

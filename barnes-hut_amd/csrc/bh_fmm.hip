@@ -15,11 +15,13 @@
 // Interpolating across a gap of one square converges as 5.8^-P: P = 12 leaves
 // 1.3e-10 of the far field (the FP32 precision's own rounding was 4e-8), and
 // P = 20 leaves 1e-15, below the rounding of a term-by-term FP64 sum over
-// 10^4 cells and more.  Everything here is FP64.
+// 10^4 cells and more.  Across a gap of two squares, or past a corner, it
+// converges as 9.9^-F or 8.6^-F, so these 15 of a square's 27 take F = 10 or 16
+// nodes a side for the same remainder.  Everything here is FP64.
 //
-// Work per pass: 27 node-to-node products of (2 P^2) x P^2 per square instead
-// of one term per (particle, cell): 4.2M particles on 1024^2 cells go from
-// 2.0e12 far terms to ~4e9 terms and ~4.4e5 products.
+// Work per pass: 12 node-to-node products of (2 P^2) x P^2 and 15 of (2 F^2) x
+// F^2 per square instead of one term per (particle, cell): 4.2M particles on
+// 1024^2 cells go from 2.0e12 far terms to ~4e9 terms and ~4.4e5 products.
 #include "bh_common.h"
 #include "bh_kernels.h"
 
@@ -122,13 +124,41 @@ __global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
 }
 
 // ---------------------------------------------------------------- sources up
+// A square's node masses C (P^2, in LDS) anterpolated to its F x F coarser nodes
+// (fine[I][i]: the coarse cardinal I at node i); V: scratch for F P.  By the
+// whole block.
+template <int P, int F>
+__device__ __forceinline__ void coarse_masses(const double* C, double* V,
+                                              const double* __restrict__ fine, double* M,
+                                              int64_t plane)
+{
+    const int tid = threadIdx.x;
+    __syncthreads();
+    for (int q = tid; q < F * P; q += 256) {   // V[I][j] = sum_i fine[I][i] C[i][j]
+        const int I = q / P, j = q - I * P;
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < P; ++i) s = fma(fine[I * P + i], C[i * P + j], s);
+        V[q] = s;
+    }
+    __syncthreads();
+    for (int q = tid; q < F * F; q += 256) {
+        const int I = q / F, J = q - I * F;
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < P; ++j) s = fma(V[I * P + j], fine[J * P + j], s);
+        M[q * plane] = s;
+    }
+}
+
 // One block per tile: the tile's COMs into the tile-ordered list, and their
 // masses anterpolated to the tile's nodes: Chebyshev moments
 // W_kl = sum M T_k(x) T_l(y) over the entries, then nodes = C^T W C.
 template <int P>
-__global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __restrict__ ctab)
+__global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __restrict__ ctab,
+                                                 const double* __restrict__ fine)
 {
-    constexpr int Q = P * P;
+    constexpr int Q = P * P, F = fmm_far(P);
     constexpr int PER = (Q + 255) / 256;
     __shared__ double tx[32][P], ty[32][P], mm[32], W[Q], V[Q], ct[Q];
     const int tid = threadIdx.x;
@@ -140,11 +170,12 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
     const int x0 = tl.tx * T, y0 = tl.ty * T;
     const int x1 = min(x0 + T, d.G), y1 = min(y0 + T, d.G);
     const double sig = step_scale(d.step);
-    double* M = nullptr;   // node q's mass goes to M[q * plane]
+    double *M = nullptr, *MF = nullptr;   // node q's mass goes to M[q * plane]
     int64_t plane = 0;
     if (fs.nlev > 0) {
         plane = fmm_plane(fs.n[0]);
         M = A.mult + fs.moff[0] * Q + fmm_slot(fs.n[0], tl.tx, tl.ty);
+        MF = A.multf + fs.moff[0] * (F * F) + fmm_slot(fs.n[0], tl.tx, tl.ty);
     }
     const bool up = fs.nlev > 0;
     for (int i = tid; i < Q; i += 256) ct[i] = ctab[i];
@@ -221,6 +252,7 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
     if (!up) return;
     if (ne == 0) {   // uniform over the block
         for (int q = tid; q < Q; q += 256) M[q * plane] = 0.0;
+        for (int q = tid; q < F * F; q += 256) MF[q * plane] = 0.0;
         return;
     }
 #pragma unroll
@@ -241,16 +273,18 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
 #pragma unroll
         for (int l = 0; l < P; ++l) s = fma(V[i * P + l], ct[l * P + j], s);
         M[q * plane] = s;
+        W[q] = s;
     }
+    coarse_masses<P, F>(W, V, fine, MF, plane);
 }
 
 // One block per square of level lev: its children's node masses anterpolated
 // to its own nodes (shift[a][i][I]: the parent's cardinal i at child node I).
 template <int P>
 __global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __restrict__ shift,
-                                                 int lev)
+                                                 const double* __restrict__ fine, int lev)
 {
-    constexpr int Q = P * P;
+    constexpr int Q = P * P, F = fmm_far(P);
     constexpr int PER = (Q + 255) / 256;
     __shared__ double S[2 * Q], C[Q], V[Q];
     const int tid = threadIdx.x;
@@ -296,41 +330,53 @@ __global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __rest
     }
     if (tid == 0) A.tcnt[t] = np;
     double* M = A.mult + fs.moff[lev] * Q + fmm_slot(fs.n[lev], tl.tx, tl.ty);
+    __syncthreads();
 #pragma unroll
     for (int p = 0; p < PER; ++p)
-        if (tid + 256 * p < Q) M[(tid + 256 * p) * plane] = acc[p];
+        if (tid + 256 * p < Q) {
+            M[(tid + 256 * p) * plane] = acc[p];
+            C[tid + 256 * p] = acc[p];
+        }
+    coarse_masses<P, F>(C, V, fine,
+                        A.multf + fs.moff[lev] * (F * F) + fmm_slot(fs.n[lev], tl.tx, tl.ty),
+                        plane);
 }
 
 // ---------------------------------------------------------------- node to node
-// One wave per (64 targets of one level and child position, 16 target nodes).
-// For each of the 27 offsets a wave forms its 16 x Q slice of the law between
-// target and source nodes in registers, one entry per lane and step (two
-// components), and multiplies it with the 64 sources' node masses on the FP64
-// matrix unit: A = 16 target nodes x 4 source nodes, B = 4 source nodes x 16
-// squares, four B blocks per A.  Forming an entry costs ~11 issue slots per
-// lane, the eight products it feeds 8 x 16, so the matrix unit is the bound.
-// Softening enters relative to the square's size, which differs by level and
-// system; forming the slice on the fly needs no table of them.
-// 4.2M particles, 1024^2 cells: P = 20 7.0 ms, 55 TFLOP/s (a large FP64 matrix
-// product reaches 73; the unit is busy 0.74 of the cycles, at 2.27 GHz), P = 12
-// 0.98 ms.  Tried: sources square-major (one line per 16 bytes read: 76 ms);
+// One wave per (64 targets of one level and child position, 16 target nodes,
+// near or far offsets).  For each of its 12 or 15 offsets a wave forms its 16 x Q
+// slice of the law between target and source nodes in registers, one entry per
+// lane and step (two components), and multiplies it with the 64 sources' node
+// masses on the FP64 matrix unit: A = 16 target nodes x 4 source nodes, B = 4
+// source nodes x 16 squares, four B blocks per A.  Forming an entry costs ~11
+// issue slots per lane, the eight products it feeds 8 x 16, so the matrix unit is
+// the bound.  Softening enters relative to the square's size, which differs by
+// level and system; forming the slice on the fly needs no table of them.
+// 4.2M particles, 1024^2 cells: P = 20 4.6 ms (7.0 with all 27 offsets at P), 55
+// TFLOP/s (a large FP64 matrix product reaches 73; the unit is busy 0.74 of the
+// cycles, at 2.27 GHz), P = 12 0.76 ms (0.98); 512 systems 2.3 ms (2.7).  F = 8
+// for P = 12 would take 0.56 and 1.6 ms but leaves 1e-9 of the far field, and
+// single particles whose terms cancel up to 6e-6.  Tried: sources square-major
+// (one line per 16 bytes read: 76 ms at P = 20 with 27 offsets, against 7.0);
 // waves of several node rows sharing a workgroup (8.5 ms: its waves spread
 // unevenly over the SIMDs); node rows of a group kept on one XCD (6.8 ms, but
 // 4.3 instead of 2.8 ms on 512 systems, whose groups differ in size).
 // NB: blocks of 16 targets (no branch inside: a branch around a product would
 // copy its accumulators).
-template <int P, int NB>
+template <int P, int NB, bool FAR>
 __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, int rb, double eps2,
                                          const double* hn)
 {
     constexpr int Q = P * P, QP = P / 4;
+    constexpr int U = P % 4 == 0 ? 2 : 1;   // products between loads
+    static_assert(Q % 4 == 0, "a lane group takes a quarter of the nodes");
     const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
     const FmmSys& fs = A.fsys[gr.sys];
     const int lev = gr.lev, n = fs.n[lev], off = fs.off[lev];
     const int ny = (n - gr.b + 1) >> 1;   // targets of this child position: columns of ny
     const int w = fmm_pitch(n);
     const int64_t plane = fmm_plane(n);
-    const double* M = A.mult + fs.moff[lev] * Q;
+    const double* M = (FAR ? A.multf : A.mult) + fs.moff[lev] * Q;
     const double h = (double)fs.T * A.sys[gr.sys].step * (double)(1 << lev);
     const double e2 = eps2 / (h * h);
     int tx[NB], ty[NB], tg[NB];
@@ -349,13 +395,14 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
         any = any || tg[b] >= 0;
     }
     if (!__any(any)) return;
-    const int row = 16 * rb + c;
+    const int row = min(16 * rb + c, Q - 1);   // the last block may repeat the last node
     const double xt = hn[row / P], yt = hn[row % P];
     fd4 ax[NB] = {}, ay[NB] = {};
     for (int o = 0; o < 36; ++o) {
         const int pi = o / 12 - 1, ca = (o / 6) & 1, pj = (o % 6) / 2 - 1, cb = o & 1;
         const int ox = 2 * pi + ca - gr.a, oy = 2 * pj + cb - gr.b;
         if (abs(ox) <= 1 && abs(oy) <= 1) continue;
+        if (fmm_is_far(ox, oy) != FAR) continue;
         bool act = false;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
@@ -367,44 +414,61 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
         // the sources' class, shifted by (pi, pj)
         const char* mp = (const char*)(M + ((2 * ca + cb) * w + pi) * w + pj);
         const double dy0 = (double)oy - yt;
-        double m[2][NB];   // the next step's node masses, on their way
+        double m[U][NB];   // the next step's node masses, on their way
+        auto load = [&]() {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < U; ++u) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) m[u][b] = *(const double*)(mp + pos[b]);
-            mp += plane * sizeof(double);
-        }
-#pragma unroll 1
-        for (int k = 0; k < QP; ++k) {
-            const double dx = ((double)ox - xt) + hn[g * QP + k];
-            const double dx2 = fma(dx, dx, e2);
-#pragma unroll 1
-            for (int j = 0; j < P; j += 2) {
-                double mc[2][NB], kx[2], ky[2];
+                for (int b = 0; b < NB; ++b) m[u][b] = *(const double*)(mp + pos[b]);
+                mp += plane * sizeof(double);
+            }
+        };
+        auto products = [&](const double (&mc)[U][NB], const double (&kx)[U],
+                            const double (&ky)[U]) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < U; ++u)
 #pragma unroll
-                    for (int b = 0; b < NB; ++b) mc[u][b] = m[u][b];
-                    const double dy = hn[j + u] + dy0;
-                    const double r = rcp64(fma(dy, dy, dx2));
-                    kx[u] = dx * r;
-                    ky[u] = dy * r;
+                for (int b = 0; b < NB; ++b) {
+                    ax[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(kx[u], mc[u][b], ax[b], 0, 0, 0);
+                    ay[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ky[u], mc[u][b], ay[b], 0, 0, 0);
                 }
-                if (k < QP - 1 || j + 2 < P) {
+        };
+        load();
+        double mc[U][NB], kx[U], ky[U];
+        if (P % 4 == 0) {   // a lane's quarter is whole columns of nodes
+#pragma unroll 1
+            for (int k = 0; k < QP; ++k) {
+                const double dx = ((double)ox - xt) + hn[g * QP + k];
+                const double dx2 = fma(dx, dx, e2);
+#pragma unroll 1
+                for (int j = 0; j < P; j += U) {
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
+                    for (int u = 0; u < U; ++u) {
 #pragma unroll
-                        for (int b = 0; b < NB; ++b) m[u][b] = *(const double*)(mp + pos[b]);
-                        mp += plane * sizeof(double);
+                        for (int b = 0; b < NB; ++b) mc[u][b] = m[u][b];
+                        const double dy = hn[j + u] + dy0;
+                        const double r = rcp64(fma(dy, dy, dx2));
+                        kx[u] = dx * r;
+                        ky[u] = dy * r;
                     }
+                    if (k < QP - 1 || j + U < P) load();
+                    products(mc, kx, ky);
                 }
+            }
+        } else {
+            int i = g * (Q / 4) / P, j = g * (Q / 4) % P;
+#pragma unroll 1
+            for (int k = 0; k < Q / 4; ++k) {
+                const double dx = ((double)ox - xt) + hn[i], dy = hn[j] + dy0;
+                const double r = rcp64(fma(dy, dy, fma(dx, dx, e2)));
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) {
-                        ax[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(kx[u], mc[u][b], ax[b], 0, 0, 0);
-                        ay[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ky[u], mc[u][b], ay[b], 0, 0, 0);
-                    }
+                for (int b = 0; b < NB; ++b) mc[0][b] = m[0][b];
+                kx[0] = dx * r;
+                ky[0] = dy * r;
+                j = j + 1 < P ? j + 1 : 0;
+                i += j == 0;
+                if (k + 1 < Q / 4) load();
+                products(mc, kx, ky);
             }
         }
     }
@@ -412,29 +476,45 @@ __device__ __forceinline__ void m2l_wave(const FmmArgs& A, const FmmGroup& gr, i
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         if (tg[b] < 0) continue;
-        double* L = A.loc + (int64_t)tg[b] * (2 * Q) + 16 * rb;
+        double* L = (FAR ? A.locf : A.loc) + (int64_t)tg[b] * (2 * Q) + 16 * rb;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {   // register v of lane (c, g): row 4 v + g, column c
+            if (Q % 16 && 16 * rb + 4 * v + g >= Q) continue;
             L[4 * v + g] = ax[b][v] * inv_h;
             L[Q + 4 * v + g] = ay[b][v] * inv_h;
         }
     }
 }
 
-template <int P>
-__global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, const double* __restrict__ nodes,
-                                                   double eps2)
+// Blocks of 16 target nodes of a square with P^2.
+__host__ __device__ constexpr int m2l_rows(int P) { return (P * P + 15) / 16; }
+
+template <int P, bool FAR>
+__device__ __forceinline__ void m2l_group(const FmmArgs& A, int64_t blk, const double* __restrict__ nodes, double eps2,
+                                          double* hn)
 {
-    constexpr int RB = P * P / 16;
-    __shared__ double hn[P];   // nodes on [-1/2, 1/2]
+    constexpr int RB = m2l_rows(P);
     if (threadIdx.x < P) hn[threadIdx.x] = 0.5 * nodes[threadIdx.x];
     __syncthreads();
-    const int gi = blockIdx.x / RB, rb = blockIdx.x - gi * RB;
+    const int gi = (int)(blk / RB), rb = (int)(blk - (int64_t)gi * RB);
     const FmmGroup gr = A.groups[gi];
     const int cnt = gr.cnt;
-    if (cnt > 32) m2l_wave<P, 4>(A, gr, rb, eps2, hn);
-    else if (cnt > 16) m2l_wave<P, 2>(A, gr, rb, eps2, hn);
-    else m2l_wave<P, 1>(A, gr, rb, eps2, hn);
+    if (cnt > 32) m2l_wave<P, 4, FAR>(A, gr, rb, eps2, hn);
+    else if (cnt > 16) m2l_wave<P, 2, FAR>(A, gr, rb, eps2, hn);
+    else m2l_wave<P, 1, FAR>(A, gr, rb, eps2, hn);
+}
+
+// The longer waves, those of the near offsets, come first.
+template <int P>
+__global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, int ngroups,
+                                                   const double* __restrict__ nodes,
+                                                   const double* __restrict__ fnodes, double eps2)
+{
+    constexpr int F = fmm_far(P);
+    __shared__ double hn[P];   // nodes on [-1/2, 1/2]
+    const int64_t near = (int64_t)ngroups * m2l_rows(P);
+    if (blockIdx.x < near) m2l_group<P, false>(A, blockIdx.x, nodes, eps2, hn);
+    else m2l_group<F, true>(A, blockIdx.x - near, fnodes, eps2, hn);
 }
 
 // ---------------------------------------------------------------- field down
@@ -442,9 +522,10 @@ __global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, const double* __re
 // the square's nodes; on tiles (lev 0) the sum becomes Chebyshev coefficients.
 template <int P>
 __global__ __launch_bounds__(256) void k_fmm_l2l(FmmArgs A, const double* __restrict__ shift,
-                                                 const double* __restrict__ ctab, int lev)
+                                                 const double* __restrict__ ctab,
+                                                 const double* __restrict__ fine, int lev)
 {
-    constexpr int Q = P * P;
+    constexpr int Q = P * P, F = fmm_far(P), QF = F * F;
     constexpr int PER = (2 * Q + 255) / 256;
     __shared__ double S[2 * Q], C[2 * Q], V[2 * Q];
     const int tid = threadIdx.x;
@@ -454,11 +535,34 @@ __global__ __launch_bounds__(256) void k_fmm_l2l(FmmArgs A, const double* __rest
     const FmmSys& fs = A.fsys[tl.sys];
     if (fs.nlev <= lev) return;
     const bool par = lev + 1 < fs.nlev;
-    if (!par && lev > 0) return;
     double* L = A.loc + t * (int64_t)(2 * Q);
     double acc[PER];
 #pragma unroll
     for (int p = 0; p < PER; ++p) acc[p] = tid + 256 * p < 2 * Q ? L[tid + 256 * p] : 0.0;
+    // the far offsets' field, from the coarser nodes
+    for (int q = tid; q < F * P; q += 256) S[q] = fine[q];
+    for (int q = tid; q < 2 * QF; q += 256) C[q] = A.locf[t * (2 * QF) + q];
+    __syncthreads();
+    for (int q = tid; q < 2 * P * F; q += 256) {   // V[i][J] = sum_I fine[I][i] C[I][J]
+        const int z = q >= P * F, r = q - z * P * F, i = r / F, J = r - i * F;
+        double v = 0.0;
+#pragma unroll
+        for (int I = 0; I < F; ++I) v = fma(S[I * P + i], C[z * QF + I * F + J], v);
+        V[q] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int q = tid + 256 * p;
+        if (q < 2 * Q) {
+            const int z = q >= Q, r = q - z * Q, i = r / P, j = r - i * P;
+            double v = 0.0;
+#pragma unroll
+            for (int J = 0; J < F; ++J) v = fma(V[z * P * F + i * F + J], S[J * P + j], v);
+            acc[p] += v;
+        }
+    }
+    __syncthreads();
     if (par) {
         const int64_t pt = fs.off[lev + 1] + (int64_t)(tl.tx >> 1) * fs.n[lev + 1] + (tl.ty >> 1);
         const int a = tl.tx & 1, b = tl.ty & 1;
@@ -822,15 +926,17 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
     const unsigned pg = (unsigned)((A.N + 255) / 256);
     hipLaunchKernelGGL(k_fmm_pack, dim3(pg < (unsigned)num_cu * 16 ? pg : num_cu * 16), dim3(256),
                        0, st, A);
-    hipLaunchKernelGGL(k_fmm_p2m<P>, dim3((unsigned)A.nleaf), dim3(256), 0, st, A, tb.cheb);
+    hipLaunchKernelGGL(k_fmm_p2m<P>, dim3((unsigned)A.nleaf), dim3(256), 0, st, A, tb.cheb,
+                       tb.fine);
     for (int l = 1; l < pl.nlev; ++l)
         hipLaunchKernelGGL(k_fmm_m2m<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
-                           dim3(256), 0, st, A, tb.shift, l);
-    hipLaunchKernelGGL(k_fmm_m2l<P>, dim3((unsigned)pl.ngroups * (P * P / 16)), dim3(64), 0, st, A,
-                       tb.nodes, eps2);
+                           dim3(256), 0, st, A, tb.shift, tb.fine, l);
+    constexpr int F = fmm_far(P);
+    hipLaunchKernelGGL(k_fmm_m2l<P>, dim3((unsigned)pl.ngroups * (m2l_rows(P) + m2l_rows(F))),
+                       dim3(64), 0, st, A, (int)pl.ngroups, tb.nodes, tb.fnodes, eps2);
     for (int l = pl.nlev - 1; l >= 0; --l)
         hipLaunchKernelGGL(k_fmm_l2l<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
-                           dim3(256), 0, st, A, tb.shift, tb.cheb, l);
+                           dim3(256), 0, st, A, tb.shift, tb.cheb, tb.fine, l);
 }
 
 template <int P>
@@ -855,6 +961,7 @@ void bh_fmm_pass(const FmmArgs& args, const FmmPlan& pl, bool fp64, double Gc, d
 {
     FmmArgs A = args;
     A.mult = pl.mult[fp64 ? 1 : 0];
+    A.multf = pl.multf[fp64 ? 1 : 0];
     if (part == 0) {
         if (fp64) fmm_prepare<FMM_P64>(A, pl, eps2, num_cu, st);
         else fmm_prepare<FMM_P32>(A, pl, eps2, num_cu, st);

@@ -142,11 +142,24 @@ struct FmmArgs {
     FmmCom* list;
     FmmPart* pack;
     double* mult;              // node masses, node-major (fmm_slot)
+    double* multf;             // the same on the coarser nodes of far offsets
     double* loc;               // per square: P^2 ax, P^2 ay
+    double* locf;              // the part of far offsets, F^2 ax, F^2 ay
     int32_t S;
     int64_t N, nleaf, ntiles, max_chunks;
     int64_t lev_off[FMM_LEVELS + 1];
 };
+
+// Of the 27 squares that a square takes directly, the 15 with a gap of two
+// squares or past a corner converge faster and take fewer nodes per side: across
+// (3, 0) and (2, 2), 16 leave 4e-15 (20 across (2, 0) 2e-15) and 10 leave 4e-11
+// and 2e-10 (12 across (2, 0) 6e-10).
+__host__ __device__ constexpr int fmm_far(int P) { return P == FMM_P64 ? 16 : 10; }
+__host__ __device__ inline bool fmm_is_far(int ox, int oy)
+{
+    const int a = ox < 0 ? -ox : ox, b = oy < 0 ? -oy : oy;
+    return a + b >= 4 || a > 2 || b > 2;
+}
 
 // Node masses of a level of n^2 squares: node-major planes, so that the squares
 // a wave reads together are neighbours in memory.  A plane holds the squares by
@@ -168,12 +181,15 @@ struct FmmTables {
     const double *nodes;   // P Chebyshev nodes on [-1, 1]
     const double *cheb;    // [k][i]: c_k T_k(node i), c_0 = 1 / P, c_k = 2 / P
     const double *shift;   // [a][i][I]: cardinal i of a square at node I of its child half a
+    const double *fnodes;  // F = fmm_far(P) nodes
+    const double *fine;    // [I][i]: cardinal I of the F nodes at node i of the P
 };
 struct FmmPlan {
     int nlev = 0;
     int64_t ngroups = 0;
     FmmTables tab[2];      // P = FMM_P32, FMM_P64
-    double* mult[2] = {nullptr, nullptr};   // their node masses (zero borders)
+    double* mult[2] = {nullptr, nullptr};    // their node masses (zero borders)
+    double* multf[2] = {nullptr, nullptr};
 };
 void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, double eps2,
                  double r2cut, int part, int nparts, int num_cu, hipStream_t st);
