@@ -371,41 +371,67 @@ static int fmm_configure(Ctx* c)
     a.max_chunks = cdiv(c->N, 64) + a.nleaf;
     c->fmm.nlev = nlev;
     c->fmm.ngroups = (int64_t)groups.size();
-    const std::vector<double> tab[2] = {fmm_table(FMM_P32), fmm_table(FMM_P64)};
+    static const std::vector<double> tab[2] = {fmm_table(FMM_P32), fmm_table(FMM_P64)};
     const int P[2] = {FMM_P32, FMM_P64};
+    const int pl = wanted & 1 ? FMM_P64 : FMM_P32;   // the larger one in use
+    const int64_t Q = pl * pl, QF = fmm_far(pl) * fmm_far(pl);
+    // one allocation (each costs ~50 us): first what the host fills in, then the
+    // node masses, whose borders stay zero, then the rest
     FmmSys* dfs = nullptr;
     FmmTile* dt = nullptr;
     FmmGroup* dg = nullptr;
-    int r;
+    double *dtab[2] = {nullptr, nullptr}, *mult[2] = {nullptr, nullptr};
+    size_t size = 0, host = 0, zero = 0;
+    unsigned char* base = nullptr;
+    auto carve = [&](auto*& p, int64_t count) {
+        p = base ? (std::remove_reference_t<decltype(p)>)(base + size) : nullptr;
+        size += ((size_t)std::max<int64_t>(count, 1) * sizeof(*p) + 255) & ~(size_t)255;
+    };
+    auto layout = [&] {
+        size = 0;
+        for (int i = 0; i < 2; ++i) carve(dtab[i], (int64_t)tab[i].size());
+        carve(dfs, S);
+        carve(dt, a.ntiles);
+        carve(dg, (int64_t)groups.size());
+        host = size;
+        for (int i = 0; i < 2; ++i)
+            if (wanted >> (1 - i) & 1)
+                carve(mult[i], slots * (P[i] * P[i] + fmm_far(P[i]) * fmm_far(P[i])));
+        zero = size;
+        carve(a.tcnt, a.ntiles);
+        carve(a.tstart, a.nleaf);
+        carve(a.tne, a.nleaf);
+        carve(a.cnt, FMM_NCNT + S);
+        carve(a.chunks, a.max_chunks);
+        carve(a.list, c->C + 4 * a.nleaf);
+        carve(a.pack, c->N);
+        carve(a.loc, a.ntiles * 2 * Q);
+        carve(a.locf, a.ntiles * 2 * QF);
+    };
+    layout();
+    int r = dalloc(c, &base, (int64_t)size);
+    if (r) return r;
+    layout();
+    std::vector<unsigned char> up(host);
+    auto fill = [&](const void* dst, const void* src, size_t bytes) {
+        std::memcpy(up.data() + ((const unsigned char*)dst - base), src, bytes);
+    };
     for (int i = 0; i < 2; ++i) {
-        double* d = nullptr;
-        if ((r = dalloc(c, &d, (int64_t)tab[i].size()))) return r;
-        HIP_TRY(hipMemcpy(d, tab[i].data(), tab[i].size() * sizeof(double), hipMemcpyHostToDevice));
+        fill(dtab[i], tab[i].data(), tab[i].size() * sizeof(double));
+        const double* d = dtab[i];
         c->fmm.tab[i].nodes = d;
         c->fmm.tab[i].cheb = d + P[i];
         c->fmm.tab[i].shift = d + P[i] + P[i] * P[i];
         c->fmm.tab[i].fnodes = d + P[i] + 3 * P[i] * P[i];
         c->fmm.tab[i].fine = c->fmm.tab[i].fnodes + fmm_far(P[i]);
+        c->fmm.mult[i] = mult[i];
+        c->fmm.multf[i] = mult[i] ? mult[i] + slots * P[i] * P[i] : nullptr;
     }
-    const int64_t Q = FMM_P64 * FMM_P64, QF = fmm_far(FMM_P64) * fmm_far(FMM_P64);
-    if ((r = dalloc(c, &dfs, S)) || (r = dalloc(c, &dt, a.ntiles)) ||
-        (r = dalloc(c, &dg, (int64_t)groups.size())) || (r = dalloc(c, &a.tcnt, a.ntiles)) ||
-        (r = dalloc(c, &a.tstart, a.nleaf)) || (r = dalloc(c, &a.tne, a.nleaf)) ||
-        (r = dalloc(c, &a.cnt, FMM_NCNT + S)) || (r = dalloc(c, &a.chunks, a.max_chunks)) ||
-        (r = dalloc(c, &a.list, c->C + 4 * a.nleaf)) || (r = dalloc(c, &a.pack, c->N)) ||
-        (r = dalloc(c, &a.loc, a.ntiles * 2 * Q)) || (r = dalloc(c, &a.locf, a.ntiles * 2 * QF)))
-        return r;
-    for (int i = 0; i < 2; ++i) {   // the borders stay zero
-        if (!(wanted >> (1 - i) & 1)) continue;
-        const int F = fmm_far(P[i]);
-        const int64_t cnt = slots * (P[i] * P[i] + F * F);
-        if ((r = dalloc(c, &c->fmm.mult[i], cnt))) return r;
-        c->fmm.multf[i] = c->fmm.mult[i] + slots * P[i] * P[i];
-        HIP_TRY(hipMemset(c->fmm.mult[i], 0, sizeof(double) * cnt));
-    }
-    HIP_TRY(hipMemcpy(dfs, fs.data(), sizeof(FmmSys) * S, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dt, tiles.data(), sizeof(FmmTile) * tiles.size(), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dg, groups.data(), sizeof(FmmGroup) * groups.size(), hipMemcpyHostToDevice));
+    fill(dfs, fs.data(), sizeof(FmmSys) * S);
+    fill(dt, tiles.data(), sizeof(FmmTile) * tiles.size());
+    fill(dg, groups.data(), sizeof(FmmGroup) * groups.size());
+    HIP_TRY(hipMemcpy(base, up.data(), host, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemset(base + host, 0, zero - host));
     a.sbad = a.cnt + FMM_NCNT;
     a.fsys = dfs;
     a.tiles = dt;
