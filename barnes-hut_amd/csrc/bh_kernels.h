@@ -12,6 +12,7 @@
 #define SCAN_ONE 8192      // elements that one block scans in one launch
 #define SORT_WAYS 8        // runs that a merge pass joins
 #define ITEMS_ONE 65536    // particles up to which one block builds a step's items
+#define COM_BIG 1024       // rows from which a cell's sums are a block's work (k_com)
 #define SORT_W 1024        // within-cell rank window (rows)
 #define SORT_THREADS 1024  // threads of a k_sort_units block (2 rows of the 2 SORT_W window each)
 

@@ -134,3 +134,36 @@ def test_equal_keys_by_cell_size(kind):
             np.testing.assert_array_equal(h[k][sl], src[k][sl][order])
         p0 += n
     eng.close()
+
+
+@pytest.mark.parametrize("big", [1023, 1024, 1025, 5000])
+def test_com_of_large_cells(big):
+    """Cells of a few and of `big` rows side by side.  Any order of adding n
+    positive numbers is off by at most n ulp, so the quotients by 2 n."""
+    from barneshut.engine import Engine
+    rng = np.random.default_rng(big)
+    G = 9
+    cnt = np.where(rng.random(G * G) < 0.2, big, rng.integers(0, 40, G * G))
+    cnt[0] = cnt[-1] = 3
+    cell = np.repeat(np.arange(G * G), cnt)
+    n = len(cell)
+    x, y = cell // G + 0.1 + 0.8 * rng.random(n), cell % G + 0.1 + 0.8 * rng.random(n)
+    x[0] = y[0] = 0.0
+    x[-1] = y[-1] = G   # the box
+    d = inputs._pack(x, y, rng.uniform(1, 2, n))
+    eng = Engine([n], [G])
+    eng.load(d)
+    eng.create_tree()
+    eng.summarize()
+    eng.check()
+    h, com, off = eng.fetch(), eng.com(), eng.offsets()
+    eng.close()
+    np.testing.assert_array_equal(np.diff(off), cnt)
+    for c in np.nonzero(cnt)[0]:
+        sl = slice(off[c], off[c + 1])
+        m = h["mass"][sl].astype(np.longdouble)
+        tol = 2 * (cnt[c] + 3) * 2.0 ** -52
+        for k, f in ((0, "px"), (1, "py")):
+            ref = float((m * h[f][sl]).sum() / m.sum())
+            assert abs(com[c][k] - ref) <= tol * abs(ref)
+        assert abs(com[c][2] - float(m.sum())) <= tol * float(m.sum())
