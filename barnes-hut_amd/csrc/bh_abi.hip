@@ -63,7 +63,8 @@ struct bh_ctx_s {
     SysDev* sys = nullptr;
     int32_t* sys_of = nullptr;
     uint64_t* bb = nullptr;
-    int32_t *key = nullptr, *key_sorted = nullptr, *counts = nullptr, *cursor = nullptr;
+    int32_t *key = nullptr, *key_sorted = nullptr, *counts = nullptr;
+    int32_t* rank = nullptr;   // of a row among its cell's, as placed
     int32_t *offsets = nullptr, *neprefix = nullptr, *ne_list = nullptr;
     int32_t *idx_a = nullptr, *idx_b = nullptr, *perm = nullptr;
     uint64_t *pxkey = nullptr, *pykey = nullptr;   // sort keys of the scattered rows
@@ -463,7 +464,7 @@ static int for_each_buffer(Ctx* c, F&& f)
     B(key, N);
     B(key_sorted, N);
     B(counts, C);
-    B(cursor, C);
+    B(rank, N);
     B(offsets, C + 1);
     B(neprefix, C + 1);
     B(ne_list, C);
@@ -718,12 +719,14 @@ int bh_place_particles(void* ctx, const bh_particles* p, void* stream)
         hipLaunchKernelGGL(k_bbox<4>, dim3(cdiv(N, 1024)), dim3(256), 0, st, x, y, so, N, c->bb,
                            c->stats);
         hipLaunchKernelGGL(k_keys_hist<2>, dim3(cdiv(N, 512)), dim3(256), 0, st, x, y, so, c->sys,
-                           (const uint64_t*)c->bb, N, c->key, c->counts, c->stats);
+                           (const uint64_t*)c->bb, N, c->key, c->rank, c->counts,
+                           c->stats);
     } else {
         hipLaunchKernelGGL(k_bbox<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, N, c->bb,
                            c->stats);
         hipLaunchKernelGGL(k_keys_hist<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, c->sys,
-                           (const uint64_t*)c->bb, N, c->key, c->counts, c->stats);
+                           (const uint64_t*)c->bb, N, c->key, c->rank, c->counts,
+                           c->stats);
     }
     LAUNCH_CHECK("place");
     return BH_OK;
@@ -735,14 +738,14 @@ int bh_place_particles(void* ctx, const bh_particles* p, void* stream)
 static void run_scan(Ctx* c, bool cnt, const int32_t* in, int64_t n, int32_t* out_v,
                      int32_t* out_f, int total_slot, int64_t max_total, hipStream_t st)
 {
-    int32_t *nl = c->ne_list, *cur = c->cursor;
+    int32_t* nl = c->ne_list;
     if (n <= SCAN_ONE) {
         if (cnt)
             hipLaunchKernelGGL(k_scan_one<true>, dim3(1), dim3(1024), 0, st, in, (int)n, out_v,
-                               out_f, nl, cur, c->com_dense, c->stats, total_slot, max_total);
+                               out_f, nl, c->com_dense, c->stats, total_slot, max_total);
         else
             hipLaunchKernelGGL(k_scan_one<false>, dim3(1), dim3(1024), 0, st, in, (int)n, out_v,
-                               out_f, nl, cur, c->com_dense, c->stats, total_slot, max_total);
+                               out_f, nl, c->com_dense, c->stats, total_slot, max_total);
         return;
     }
     unsigned nb = (unsigned)cdiv(n, SCAN_TILE);
@@ -752,7 +755,7 @@ static void run_scan(Ctx* c, bool cnt, const int32_t* in, int64_t n, int32_t* ou
         hipLaunchKernelGGL(k_scan_blocks<true>, dim3(1), dim3(1024), 0, st, c->bsum, c->bne,
                            (int64_t)nb, c->stats, total_slot);
         hipLaunchKernelGGL(k_scan_final<true>, dim3(nb), dim3(256), 0, st, in, n,
-                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl, cur,
+                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl,
                            c->com_dense);
     } else {
         hipLaunchKernelGGL(k_scan_reduce<false>, dim3(nb), dim3(256), 0, st, in, n, c->bsum,
@@ -760,7 +763,7 @@ static void run_scan(Ctx* c, bool cnt, const int32_t* in, int64_t n, int32_t* ou
         hipLaunchKernelGGL(k_scan_blocks<false>, dim3(1), dim3(1024), 0, st, c->bsum, c->bne,
                            (int64_t)nb, c->stats, total_slot);
         hipLaunchKernelGGL(k_scan_final<false>, dim3(nb), dim3(256), 0, st, in, n,
-                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl, cur,
+                           (const int32_t*)c->bsum, (const int32_t*)c->bne, out_v, out_f, nl,
                            c->com_dense);
     }
     if (max_total >= 0)
@@ -805,10 +808,7 @@ static BhParticles dev_of(const bh_particles* p)
     return d;
 }
 
-// clear: the scatter's cursors, which the scan leaves at zero, may hold the
-// counts of an earlier sort of the same placement.
-static int sort_impl(void* ctx, const bh_particles* src, const bh_particles* dst, bool clear,
-                     void* stream)
+int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
 {
     Ctx* c = (Ctx*)ctx;
     CTX_READY(c);
@@ -819,19 +819,11 @@ static int sort_impl(void* ctx, const bh_particles* src, const bh_particles* dst
     hipStream_t st = (hipStream_t)stream;
     const int64_t N = c->N;
     SortFields F = fields_of(src);
-    if (clear)
-        hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c->C, 256, 4096)), dim3(256), 0, st, c->cursor,
-                           c->C, 0);
-    if (N < PLACE_SMALL)
-        hipLaunchKernelGGL(k_scatter<2>, dim3(cdiv(N, 512)), dim3(256), 0, st,
-                           (const int32_t*)c->key, N, (const int32_t*)c->offsets, c->cursor,
-                           c->idx_a, c->key_sorted, (const double*)src->px, (const double*)src->py,
-                           c->pxkey, c->pykey);
-    else
-        hipLaunchKernelGGL(k_scatter<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st,
-                           (const int32_t*)c->key, N, (const int32_t*)c->offsets, c->cursor,
-                           c->idx_a, c->key_sorted, (const double*)src->px, (const double*)src->py,
-                           c->pxkey, c->pykey);
+    const int sr = N < PLACE_SMALL ? 1 : 8;
+    hipLaunchKernelGGL(sr == 1 ? k_scatter<1> : k_scatter<8>, dim3(cdiv(N, 256 * sr)), dim3(256), 0,
+                       st, (const int32_t*)c->key, N, (const int32_t*)c->offsets,
+                       (const int32_t*)c->rank, c->idx_a, c->key_sorted, (const double*)src->px,
+                       (const double*)src->py, c->pxkey, c->pykey);
     hipLaunchKernelGGL(k_sort_units, dim3(cdiv(N, SORT_W)), dim3(SORT_THREADS), 0, st, F, N,
                        (const int32_t*)c->idx_a, (const int32_t*)c->key_sorted,
                        (const uint64_t*)c->pxkey, (const uint64_t*)c->pykey,
@@ -852,11 +844,6 @@ static int sort_impl(void* ctx, const bh_particles* src, const bh_particles* dst
                        (const int32_t*)c->stats, c->perm);
     LAUNCH_CHECK("sort");
     return BH_OK;
-}
-
-int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
-{
-    return sort_impl(ctx, src, dst, true, stream);
 }
 
 int bh_summarize(void* ctx, const bh_particles* p, void* stream)
@@ -1161,7 +1148,7 @@ static int step_impl(void* ctx, const bh_particles* a, const bh_particles* b, co
     int r;
     if ((r = bh_place_particles(ctx, a, stream))) return r;
     if ((r = bh_calculate_box_cumm(ctx, stream))) return r;
-    if ((r = sort_impl(ctx, a, b, false, stream))) return r;
+    if ((r = bh_sort_particles(ctx, a, b, stream))) return r;
     if ((r = bh_summarize(ctx, b, stream))) return r;
     if ((r = bh_build_items(ctx, stream))) return r;
     const int32_t* ord = nullptr;
@@ -1614,11 +1601,6 @@ int bh_ctx_S(void* ctx) { return ((Ctx*)ctx)->S; }
 const int32_t* bh_ctx_offsets(void* ctx) { return ((Ctx*)ctx)->offsets; }
 const int32_t* bh_ctx_neprefix(void* ctx) { return ((Ctx*)ctx)->neprefix; }
 const Com64* bh_ctx_l64(void* ctx) { return ((Ctx*)ctx)->l64; }
-int32_t* bh_ctx_scratch_i32(void* ctx, int which)
-{
-    Ctx* c = (Ctx*)ctx;
-    return which == 0 ? c->bsum : (which == 1 ? c->bne : c->cursor);
-}
 int32_t* bh_ctx_cost_scratch(void* ctx) { return ((Ctx*)ctx)->cost_scratch; }
 float* bh_ctx_feat(void* ctx) { return ((Ctx*)ctx)->feat; }
 float* bh_ctx_pred(void* ctx) { return ((Ctx*)ctx)->pred; }

@@ -374,8 +374,8 @@ __global__ void k_bbox(const double* px, const double* py, const int32_t* sys_of
                        uint64_t* bb, int32_t* stats);
 template <int R>
 __global__ void k_keys_hist(const double* px, const double* py, const int32_t* sys_of, SysDev* sys,
-                            const uint64_t* bb, int64_t N, int32_t* key_out, int32_t* counts,
-                            int32_t* stats);
+                            const uint64_t* bb, int64_t N, int32_t* key_out, int32_t* rank_out,
+                            int32_t* counts, int32_t* stats);
 template <bool CNT>
 __global__ void k_scan_reduce(const int32_t* in, int64_t n, int32_t* bsum, int32_t* bne,
                               int32_t* stats);
@@ -384,15 +384,14 @@ __global__ void k_scan_blocks(int32_t* bsum, int32_t* bne, int64_t nb, int32_t* 
                               int total_slot);
 template <bool CNT>
 __global__ void k_scan_final(const int32_t* in, int64_t n, const int32_t* bsum, const int32_t* bne,
-                             int32_t* out_v, int32_t* out_f, int32_t* ne_list, int32_t* cursor,
-                             double* com_dense);
+                             int32_t* out_v, int32_t* out_f, int32_t* ne_list, double* com_dense);
 template <bool CNT>
 __global__ void k_scan_one(const int32_t* in, int n, int32_t* out_v, int32_t* out_f,
-                           int32_t* ne_list, int32_t* cursor, double* com_dense, int32_t* stats,
-                           int total_slot, int64_t max_total);
+                           int32_t* ne_list, double* com_dense, int32_t* stats, int total_slot,
+                           int64_t max_total);
 template <int R>
-__global__ void k_scatter(const int32_t* key, int64_t N, const int32_t* offsets, int32_t* cursor,
-                          int32_t* idx_out, int32_t* key_sorted, const double* px,
+__global__ void k_scatter(const int32_t* key, int64_t N, const int32_t* offsets,
+                          const int32_t* rank, int32_t* idx_out, int32_t* key_sorted, const double* px,
                           const double* py, uint64_t* pxkey_out, uint64_t* pykey_out);
 __global__ void k_sort_units(SortFields F, int64_t N, const int32_t* idx_in,
                              const int32_t* key_sorted, const uint64_t* pxkey,

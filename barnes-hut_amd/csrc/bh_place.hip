@@ -206,18 +206,24 @@ __device__ __forceinline__ void block_minmax(int& kmin, int& kmax, int* red)
     __syncthreads();
 }
 
-// Keys for 256 R consecutive particles per block, then an LDS
-// histogram over the block's key window when it fits (the input is the
-// previous step's sorted order, so a block's keys are nearly contiguous);
-// only non-zero bins go to global atomics.  Each row's box comes straight from
-// the extremes; the thread of a system's first row stores it (a kernel of its
-// own, or a last block behind a device fence, costs more than the division).
+// Keys of 256 R consecutive particles per block, the cells' counts, and each
+// row's rank among its cell's rows (in no fixed order; the scatter places rows
+// by it, so that it needs no counters of its own).  Rows are counted in LDS first
+// and each cell goes to global memory once a block: in a window of keys when the
+// block's fit one (the input is the previous step's sorted order, so they are
+// nearly contiguous), else in a hash table (unsorted input; rows that find no
+// place in four probes go to global memory by themselves).  Bound by latency and,
+// unsorted, by additions to the same words: 262,144 unsorted particles with 9,900
+// in one cell 202 -> 44 us with k_scatter; 10M sorted ones 370 -> 333 us.  Each row's box comes straight from the
+// extremes; the thread of a system's first row stores it (a kernel of its own, or
+// a last block behind a device fence, costs more than the division).
 template <int R>
 __global__ __launch_bounds__(256) void k_keys_hist(const double* __restrict__ px,
                                                    const double* __restrict__ py,
                                                    const int32_t* __restrict__ sys_of,
                                                    SysDev* sys, const uint64_t* __restrict__ bb,
                                                    int64_t N, int32_t* __restrict__ key_out,
+                                                   int32_t* __restrict__ rank_out,
                                                    int32_t* __restrict__ counts, int32_t* stats)
 {
     __shared__ int32_t hist[HIST_BINS];
@@ -261,27 +267,59 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double* __restrict__ px
     }
     block_minmax(kmin, kmax, red);
     if (kmax < kmin) return;   // empty block
+    int slot[R], lr[R];
     if ((int64_t)kmax - kmin < HIST_BINS) {
         int span = kmax - kmin + 1;
         for (int b = threadIdx.x; b < span; b += 256) hist[b] = 0;
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (kk[r] >= 0) atomicAdd(&hist[kk[r] - kmin], 1);
+        for (int r = 0; r < R; ++r) lr[r] = kk[r] >= 0 ? atomicAdd(&hist[kk[r] - kmin], 1) : 0;
         __syncthreads();
         for (int b = threadIdx.x; b < span; b += 256)
-            if (hist[b]) atomicAdd(&counts[kmin + b], hist[b]);
-    } else {
+            if (hist[b]) hist[b] = atomicAdd(&counts[kmin + b], hist[b]);
+        __syncthreads();
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            if (kk[r] >= 0) atomicAdd(&counts[kk[r]], 1);
+            if (kk[r] >= 0) rank_out[base + r * 256 + threadIdx.x] = hist[kk[r] - kmin] + lr[r];
+    } else {
+        // hist holds HASH keys, then their counts
+        constexpr int HASH = R > 2 ? HIST_BINS / 2 : HIST_BINS / 8;
+        int32_t* hk = hist;
+        int32_t* hc = hist + HASH;
+        for (int b = threadIdx.x; b < HASH; b += 256) {
+            hk[b] = -1;
+            hc[b] = 0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            slot[r] = -1;
+            if (kk[r] < 0) continue;
+            unsigned h = ((unsigned)kk[r] * 2654435761u) >> 16;
+            for (int t = 0; t < 4 && slot[r] < 0; ++t, ++h) {
+                const int old = atomicCAS(&hk[h & (HASH - 1)], -1, kk[r]);
+                if (old == -1 || old == kk[r]) slot[r] = h & (HASH - 1);
+            }
+            if (slot[r] >= 0) lr[r] = atomicAdd(&hc[slot[r]], 1);
+        }
+        __syncthreads();
+        for (int b = threadIdx.x; b < HASH; b += 256)
+            if (hc[b]) hc[b] = atomicAdd(&counts[hk[b]], hc[b]);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (kk[r] >= 0)
+                rank_out[base + r * 256 + threadIdx.x] =
+                    slot[r] >= 0 ? hc[slot[r]] + lr[r] : atomicAdd(&counts[kk[r]], 1);
     }
 }
 
 template __global__ void k_keys_hist<2>(const double*, const double*, const int32_t*, SysDev*,
-                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*);
+                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*,
+                                        int32_t*);
 template __global__ void k_keys_hist<8>(const double*, const double*, const int32_t*, SysDev*,
-                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*);
+                                        const uint64_t*, int64_t, int32_t*, int32_t*, int32_t*,
+                                        int32_t*);
 
 // ---------------------------------------------------------------- scan
 // Block-wide exclusive scan of two int sequences (256 or 1024 threads).
@@ -391,17 +429,11 @@ __global__ __launch_bounds__(1024) void k_scan_blocks(int32_t* bsum, int32_t* bn
 }
 
 // What the cells' scan leaves for the phases after it, besides the prefixes:
-// the list of non-empty cells, zeros in the dense COM array (k_com writes the
-// non-empty cells) and in the scatter's cursors.
-struct CellOut {
-    int32_t *ne_list, *cursor;
-    double* com_dense;
-};
-
-__device__ __forceinline__ void clear_cells(const CellOut& o, int64_t c0, int64_t n, int threads)
+// the list of non-empty cells and zeros in the dense COM array (k_com writes the
+// non-empty cells).
+__device__ __forceinline__ void clear_com(double* com_dense, int64_t c0, int64_t c1, int threads)
 {
-    for (int64_t i = c0 + threadIdx.x; i < n; i += threads) o.cursor[i] = 0;
-    for (int64_t i = 3 * c0 + threadIdx.x; i < 3 * n; i += threads) o.com_dense[i] = 0.0;
+    for (int64_t i = 3 * c0 + threadIdx.x; i < 3 * c1; i += threads) com_dense[i] = 0.0;
 }
 
 // Phase 3: exclusive prefix per element; out has n + 1 entries.
@@ -409,8 +441,7 @@ template <bool CNT>
 __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ in, int64_t n,
                                                     const int32_t* bsum, const int32_t* bne,
                                                     int32_t* out_v, int32_t* out_f,
-                                                    int32_t* ne_list, int32_t* cursor,
-                                                    double* com_dense)
+                                                    int32_t* ne_list, double* com_dense)
 {
     __shared__ int sh[40];
     constexpr int R = SCAN_TILE / 256;
@@ -447,7 +478,7 @@ __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ 
     }
     if (CNT) {
         const int64_t c0 = (int64_t)blockIdx.x * SCAN_TILE;
-        clear_cells({ne_list, cursor, com_dense}, c0, min(n, c0 + SCAN_TILE), 256);
+        clear_com(com_dense, c0, min(n, c0 + SCAN_TILE), 256);
     }
 }
 
@@ -457,8 +488,7 @@ __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ 
 template <bool CNT>
 __global__ __launch_bounds__(1024) void k_scan_one(const int32_t* __restrict__ in, int n,
                                                    int32_t* out_v, int32_t* out_f, int32_t* ne_list,
-                                                   int32_t* cursor, double* com_dense,
-                                                   int32_t* stats, int total_slot,
+                                                   double* com_dense, int32_t* stats, int total_slot,
                                                    int64_t max_total)
 {
     __shared__ int sh[40];
@@ -505,7 +535,7 @@ __global__ __launch_bounds__(1024) void k_scan_one(const int32_t* __restrict__ i
             if (over) atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
         }
     }
-    if (CNT) clear_cells({ne_list, cursor, com_dense}, 0, n, 1024);
+    if (CNT) clear_com(com_dense, 0, n, 1024);
 }
 
 template __global__ void k_scan_reduce<true>(const int32_t*, int64_t, int32_t*, int32_t*, int32_t*);
@@ -513,14 +543,13 @@ template __global__ void k_scan_reduce<false>(const int32_t*, int64_t, int32_t*,
 template __global__ void k_scan_blocks<true>(int32_t*, int32_t*, int64_t, int32_t*, int);
 template __global__ void k_scan_blocks<false>(int32_t*, int32_t*, int64_t, int32_t*, int);
 template __global__ void k_scan_final<true>(const int32_t*, int64_t, const int32_t*, const int32_t*,
-                                            int32_t*, int32_t*, int32_t*, int32_t*, double*);
+                                            int32_t*, int32_t*, int32_t*, double*);
 template __global__ void k_scan_final<false>(const int32_t*, int64_t, const int32_t*,
-                                             const int32_t*, int32_t*, int32_t*, int32_t*, int32_t*,
-                                             double*);
+                                             const int32_t*, int32_t*, int32_t*, int32_t*, double*);
 template __global__ void k_scan_one<true>(const int32_t*, int, int32_t*, int32_t*, int32_t*,
-                                          int32_t*, double*, int32_t*, int, int64_t);
+                                          double*, int32_t*, int, int64_t);
 template __global__ void k_scan_one<false>(const int32_t*, int, int32_t*, int32_t*, int32_t*,
-                                           int32_t*, double*, int32_t*, int, int64_t);
+                                           double*, int32_t*, int, int64_t);
 
 // 64-bit key ordered as numpy orders doubles: -0.0 equals +0.0, every NaN is
 // equal to every other NaN and sorts after all numbers.
@@ -531,15 +560,15 @@ __device__ __forceinline__ uint64_t sort_key(double d)
 }
 
 // ---------------------------------------------------------------- scatter
-// Counting-sort scatter into cell order.  A block reserves one contiguous
-// range per distinct key with a single global atomic (LDS-privatised
-// cursor); the order inside a cell is fixed afterwards by k_sort_units.
+// Counting-sort scatter into cell order: a row's place is its cell's first plus
+// its rank among the cell's rows, which k_keys_hist kept; the order inside a
+// cell is fixed afterwards by k_sort_units.
 // Each row's px and py sort keys travel with it, so that pass reads them
 // contiguously (rows clipped to the box edge tie in px by the thousand).
 template <int R>
 __global__ __launch_bounds__(256) void k_scatter(const int32_t* __restrict__ key, int64_t N,
                                                  const int32_t* __restrict__ offsets,
-                                                 int32_t* __restrict__ cursor,
+                                                 const int32_t* __restrict__ rank,
                                                  int32_t* __restrict__ idx_out,
                                                  int32_t* __restrict__ key_sorted,
                                                  const double* __restrict__ px,
@@ -547,66 +576,35 @@ __global__ __launch_bounds__(256) void k_scatter(const int32_t* __restrict__ key
                                                  uint64_t* __restrict__ pxkey_out,
                                                  uint64_t* __restrict__ pykey_out)
 {
-    __shared__ int32_t hist[HIST_BINS];
-    __shared__ int red[8];
-    int64_t base = (int64_t)blockIdx.x * (256 * R);
-    int kk[R];
-    int kmin = INT_MAX, kmax = INT_MIN;
+    const int64_t base = (int64_t)blockIdx.x * (256 * R) + threadIdx.x;
+    int kr[R], rr[R];
+    double xr[R], yr[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {   // clamped, so that all loads are under way at once
+        const int64_t i = min(base + r * 256, N - 1);
+        kr[r] = key[i];
+        rr[r] = rank[i];
+        xr[r] = px[i];
+        yr[r] = py[i];
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        int64_t i = base + r * 256 + threadIdx.x;
-        kk[r] = i < N ? key[i] : -1;
-        if (kk[r] >= 0) {
-            kmin = min(kmin, kk[r]);
-            kmax = max(kmax, kk[r]);
-        }
-    }
-    block_minmax(kmin, kmax, red);
-    if (kmax < kmin) return;
-    if ((int64_t)kmax - kmin < HIST_BINS) {
-        int span = kmax - kmin + 1;
-        int lr[R];
-        for (int b = threadIdx.x; b < span; b += 256) hist[b] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            lr[r] = kk[r] >= 0 ? atomicAdd(&hist[kk[r] - kmin], 1) : 0;
-        __syncthreads();
-        for (int b = threadIdx.x; b < span; b += 256) {
-            int c = hist[b];
-            if (c) hist[b] = offsets[kmin + b] + atomicAdd(&cursor[kmin + b], c);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (kk[r] >= 0) {
-                int pos = hist[kk[r] - kmin] + lr[r];
-                const int64_t i = base + r * 256 + threadIdx.x;
-                idx_out[pos] = (int32_t)i;
-                key_sorted[pos] = kk[r];
-                pxkey_out[pos] = sort_key(px[i]);
-                pykey_out[pos] = sort_key(py[i]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (kk[r] >= 0) {
-                int pos = offsets[kk[r]] + atomicAdd(&cursor[kk[r]], 1);
-                const int64_t i = base + r * 256 + threadIdx.x;
-                idx_out[pos] = (int32_t)i;
-                key_sorted[pos] = kk[r];
-                pxkey_out[pos] = sort_key(px[i]);
-                pykey_out[pos] = sort_key(py[i]);
-            }
-        }
+        const int64_t i = base + r * 256;
+        if (i >= N) break;
+        const int64_t pos = (int64_t)offsets[kr[r]] + rr[r];
+        idx_out[pos] = (int32_t)i;
+        key_sorted[pos] = kr[r];
+        pxkey_out[pos] = sort_key(xr[r]);
+        pykey_out[pos] = sort_key(yr[r]);
     }
 }
 
-template __global__ void k_scatter<2>(const int32_t*, int64_t, const int32_t*, int32_t*, int32_t*,
-                                      int32_t*, const double*, const double*, uint64_t*, uint64_t*);
-template __global__ void k_scatter<8>(const int32_t*, int64_t, const int32_t*, int32_t*, int32_t*,
-                                      int32_t*, const double*, const double*, uint64_t*, uint64_t*);
+template __global__ void k_scatter<1>(const int32_t*, int64_t, const int32_t*, const int32_t*,
+                                      int32_t*, int32_t*, const double*, const double*, uint64_t*,
+                                      uint64_t*);
+template __global__ void k_scatter<8>(const int32_t*, int64_t, const int32_t*, const int32_t*,
+                                      int32_t*, int32_t*, const double*, const double*, uint64_t*,
+                                      uint64_t*);
 
 // ---------------------------------------------------------------- within-cell order
 // numpy's structured-sort tie rule after (gx, gy): px, py, mass, vx, vy, ax,

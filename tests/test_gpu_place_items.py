@@ -167,3 +167,26 @@ def test_com_of_large_cells(big):
             ref = float((m * h[f][sl]).sum() / m.sum())
             assert abs(com[c][k] - ref) <= tol * abs(ref)
         assert abs(com[c][2] - float(m.sum())) <= tol * float(m.sum())
+
+
+@pytest.mark.parametrize("n", [2, 511, 513, 2049, 262143, 262145])
+def test_unsorted_rows_over_many_cells(n):
+    """Every second row in one of three cells, the others over 512^2 cells."""
+    from barneshut.engine import Engine
+    G = 512
+    rng = np.random.default_rng(n)
+    x, y = rng.random(n), rng.random(n)
+    x[::2] = (rng.integers(0, 3, len(x[::2])) * 100 + 50.2 + 0.6 * rng.random(len(x[::2]))) / G
+    y[::2] = (77.2 + 0.6 * rng.random(len(x[::2]))) / G
+    eng = Engine([n], [G])
+    eng.load(inputs._pack(x, y, rng.uniform(1, 2, n)))
+    src = eng.fetch()
+    eng.create_tree()
+    eng.check()
+    bb = orc.bbox(src["px"], src["py"], G)
+    _, _, key = orc.place(src["px"], src["py"], bb[0], bb[1], bb[4], G)
+    order = orc.sort_perm(key, [src[k] for k in ("px", "py", "mass", "vx", "vy", "ax", "ay",
+                                                 "pid")])
+    np.testing.assert_array_equal(eng.counts(), np.bincount(key, minlength=G * G))
+    np.testing.assert_array_equal(eng.fetch()["pid"], src["pid"][order])
+    eng.close()
