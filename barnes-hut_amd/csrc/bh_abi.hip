@@ -1088,8 +1088,12 @@ int bh_recompute(void* ctx, const bh_particles* p, const bh_law* law, void* stre
     hipLaunchKernelGGL(k_rc_blockfar, dim3(grid_for(c->nblocks, 1, (int64_t)c->num_cu * 16)),
                        dim3(64), 0, st, (const SysDev*)c->sys, c->S, c->nblocks,
                        (const double*)c->rc_blk, c->rc_bfar);
-    hipLaunchKernelGGL(k_rc_flag, dim3(grid_for(c->max_items, 1, (int64_t)c->num_cu * 32)),
-                       dim3(64), 0, st, (const Item*)c->items, (const SysDev*)c->sys,
+    // four waves an item where items of 64 P particles span 16 rows and more on
+    // average and do not fill the chip by themselves (k_rc_flag)
+    const bool wide = c->C * 64 * c->tune.p >= 16 * c->N && c->N <= (int64_t)c->num_cu * 4096;
+    hipLaunchKernelGGL(wide ? k_rc_flag<4> : k_rc_flag<1>,
+                       dim3(grid_for(c->max_items, 1, (int64_t)c->num_cu * 32)),
+                       dim3(wide ? 256 : 64), 0, st, (const Item*)c->items, (const SysDev*)c->sys,
                        (const int32_t*)c->key_sorted, (const int32_t*)c->neprefix,
                        (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
                        (const double*)c->com_dense, (const double*)c->rc_tiles,

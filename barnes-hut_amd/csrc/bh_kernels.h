@@ -429,6 +429,7 @@ __global__ void k_rc_tiles(const SysDev* sys, int S, int64_t ntiles, const doubl
                            double* tl);
 __global__ void k_rc_blockfar(const SysDev* sys, int S, int64_t nblocks, const double* blk,
                               double* bfar);
+template <int W>
 __global__ void k_rc_flag(const Item* items, const SysDev* sys, const int32_t* key_sorted,
                           const int32_t* neprefix, const Com64* l64, const double* x,
                           const double* y, const double* com, const double* tl,
