@@ -107,8 +107,8 @@ struct bh_ctx_s {
     // grouped far field (bh_fmm.hip): which passes take it is a rule on the
     // systems' sizes (fmm_wanted)
     int fmm_on = 0;          // bit 0: fp64 passes, bit 1: fp32 passes
-    FmmPlan fmm;
-    FmmArgs fa = {};         // device buffers and sizes; the per-pass fields are set by each pass
+    FmmPlan fmm[2];          // per precision (0: fp64, 1: fp32)
+    FmmArgs fa[2] = {};      // device buffers and sizes; the per-pass fields are set by each pass
     hipStream_t cap_stream = nullptr;   // graph capture only; replays run on the caller's stream
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     GraphKey gkey[2];
@@ -236,12 +236,30 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 static constexpr double FP32_SHARED_TERMS = 4e9;
 static constexpr double FMM_MIN_TERMS_FP64 = 4e9;
 static constexpr double FMM_MIN_TERMS_FP32 = 2e10;
-static constexpr size_t FMM_MAX_BYTES = (size_t)80 << 30;
+static constexpr double FMM_MAX_BYTES = 48.0 * (1 << 30);
+
+// Cells per tile side of a system.  A tile of T^2 cells costs its particles 9 T^2
+// mid terms each and one set of node-to-node products, so the sum is least at
+// T^4 = c G^2 / n with c the ratio of the two costs, measured with every T from 4
+// to 24 on 300k to 10M particles (times of a pass, T = 8 first, then the best):
+//   fp64: 2.0M on 1000^2 7.3, 4.5 ms (T = 16); 1M on 300^2 1.60, 1.50 (12); 2M on
+//         200^2 2.2 (8); 10M on 120^2 26.6, 25.9 (4)
+//   fp32: 2.0M on 1000^2 2.8, 2.7 ms (10); 1M on 300^2 0.98 (7 and 8); 2M on 200^2
+//         1.90, 1.74 (5); 512 systems of 16 a cell 14.9, 14.8 (6)
+// and clustered particles within 5 % of their best.
+static int fmm_tile(int64_t n, int G, int P)
+{
+    if (G < FMM_MIN_GRID) return G;
+    const double c = P == FMM_P64 ? 130000.0 : 22000.0;
+    const int T = (int)std::lround(std::pow(c * G * G / (double)n, 0.25));
+    return (int)std::max<int64_t>(std::min(std::max(T, FMM_TILE_MIN), FMM_TILE_MAX),
+                                  cdiv(G, FMM_SIDE_MAX));
+}
 
 // Bit 0: fp64 passes, bit 1: fp32 passes.
 static int fmm_wanted(const std::vector<SysDev>& sh)
 {
-    double terms = 0.0, tiles = 0.0;
+    double terms = 0.0, tiles = 0.0, bytes[2] = {0.0, 0.0};
     int64_t side = 0;
     for (const SysDev& d : sh) {
         if (d.G < FMM_MIN_GRID) continue;
@@ -249,17 +267,18 @@ static int fmm_wanted(const std::vector<SysDev>& sh)
         const double n0 = (double)cdiv(d.G, FMM_TILE);
         tiles += n0 * n0 * (4.0 / 3.0);
         side = std::max(side, cdiv(d.G, FMM_TILE));
+        for (int i = 0; i < 2; ++i) {   // 3 numbers per square and node: mass, ax, ay
+            const int P = i ? FMM_P32 : FMM_P64;
+            const double n = (double)cdiv(d.G, fmm_tile(d.n, d.G, P));
+            bytes[i] += n * n * 4.0 * (P * P + fmm_far(P) * fmm_far(P)) * sizeof(double);
+        }
     }
-    // a nearly empty huge grid has more squares to serve than terms to save;
-    // a level's node masses are addressed with 32 bits; masses and fields at the
-    // nodes are 3 (P^2 + F^2) numbers a square
-    if (terms < 1e6 * tiles || side > 1024 ||
-        tiles * 2000.0 * sizeof(double) > (double)FMM_MAX_BYTES)
-        return 0;
+    // a nearly empty huge grid has more squares to serve than terms to save
+    if (terms < 1e6 * tiles || side > FMM_SIDE_MAX) return 0;
     const bool noalloc = sh.size() == 1 && sh[0].n <= BH_NOALLOC_MAX_N &&
                          sh[0].G <= BH_NOALLOC_MAX_GRID;
-    return (terms >= FMM_MIN_TERMS_FP64 && !noalloc ? 1 : 0) |
-           (terms >= FMM_MIN_TERMS_FP32 ? 2 : 0);
+    return (terms >= FMM_MIN_TERMS_FP64 && !noalloc && bytes[0] <= FMM_MAX_BYTES ? 1 : 0) |
+           (terms >= FMM_MIN_TERMS_FP32 && bytes[1] <= FMM_MAX_BYTES ? 2 : 0);
 }
 
 // Chebyshev nodes, transform and parent-child interpolation for P nodes, then the
@@ -309,13 +328,11 @@ static std::vector<double> fmm_table(int P)
     return v;
 }
 
-// Lays out the squares of every system and allocates the grouped far field's
-// buffers (c->sys_h and the sizes are set).
-static int fmm_configure(Ctx* c)
+// Lays out the squares of every system for one precision and allocates the
+// grouped far field's buffers (c->sys_h and the sizes are set).
+static int fmm_configure(Ctx* c, int precision)
 {
-    c->fmm_on = 0;
-    const int wanted = fmm_wanted(c->sys_h);
-    if (!wanted) return BH_OK;
+    const int P = precision == 0 ? FMM_P64 : FMM_P32, F = fmm_far(P);
     const int S = c->S;
     std::vector<FmmSys> fs(S);
     int nlev = 0;
@@ -323,7 +340,7 @@ static int fmm_configure(Ctx* c)
         const int G = c->sys_h[s].G;
         FmmSys& f = fs[s];
         std::memset(&f, 0, sizeof(f));
-        f.T = G < FMM_MIN_GRID ? G : FMM_TILE;
+        f.T = fmm_tile(c->sys_h[s].n, G, P);
         f.n[0] = (int32_t)cdiv(G, f.T);
         f.nlev = f.n[0] > 1 ? 1 : 0;
         while (f.nlev && f.n[f.nlev - 1] > 4) {
@@ -332,7 +349,8 @@ static int fmm_configure(Ctx* c)
         }
         nlev = std::max(nlev, std::max(f.nlev, 1));
     }
-    FmmArgs& a = c->fa;
+    FmmPlan& plan = c->fmm[precision];
+    FmmArgs& a = c->fa[precision];
     a = FmmArgs{};
     std::vector<FmmTile> tiles;
     std::vector<FmmGroup> groups;
@@ -370,18 +388,16 @@ static int fmm_configure(Ctx* c)
     a.nleaf = a.lev_off[1];
     a.ntiles = (int64_t)tiles.size();
     a.max_chunks = cdiv(c->N, 64) + a.nleaf;
-    c->fmm.nlev = nlev;
-    c->fmm.ngroups = (int64_t)groups.size();
-    static const std::vector<double> tab[2] = {fmm_table(FMM_P32), fmm_table(FMM_P64)};
-    const int P[2] = {FMM_P32, FMM_P64};
-    const int pl = wanted & 1 ? FMM_P64 : FMM_P32;   // the larger one in use
-    const int64_t Q = pl * pl, QF = fmm_far(pl) * fmm_far(pl);
+    plan.nlev = nlev;
+    plan.ngroups = (int64_t)groups.size();
+    static const std::vector<double> tabs[2] = {fmm_table(FMM_P64), fmm_table(FMM_P32)};
+    const std::vector<double>& tab = tabs[precision];
     // one allocation (each costs ~50 us): first what the host fills in, then the
     // node masses, whose borders stay zero, then the rest
     FmmSys* dfs = nullptr;
     FmmTile* dt = nullptr;
     FmmGroup* dg = nullptr;
-    double *dtab[2] = {nullptr, nullptr}, *mult[2] = {nullptr, nullptr};
+    double* dtab = nullptr;
     size_t size = 0, host = 0, zero = 0;
     unsigned char* base = nullptr;
     auto carve = [&](auto*& p, int64_t count) {
@@ -390,14 +406,13 @@ static int fmm_configure(Ctx* c)
     };
     auto layout = [&] {
         size = 0;
-        for (int i = 0; i < 2; ++i) carve(dtab[i], (int64_t)tab[i].size());
+        carve(dtab, (int64_t)tab.size());
         carve(dfs, S);
         carve(dt, a.ntiles);
         carve(dg, (int64_t)groups.size());
         host = size;
-        for (int i = 0; i < 2; ++i)
-            if (wanted >> (1 - i) & 1)
-                carve(mult[i], slots * (P[i] * P[i] + fmm_far(P[i]) * fmm_far(P[i])));
+        carve(a.mult, slots * P * P);
+        carve(a.multf, slots * F * F);
         zero = size;
         carve(a.tcnt, a.ntiles);
         carve(a.tstart, a.nleaf);
@@ -406,8 +421,8 @@ static int fmm_configure(Ctx* c)
         carve(a.chunks, a.max_chunks);
         carve(a.list, c->C + 4 * a.nleaf);
         carve(a.pack, c->N);
-        carve(a.loc, a.ntiles * 2 * Q);
-        carve(a.locf, a.ntiles * 2 * QF);
+        carve(a.loc, a.ntiles * 2 * P * P);
+        carve(a.locf, a.ntiles * 2 * F * F);
     };
     layout();
     int r = dalloc(c, &base, (int64_t)size);
@@ -417,17 +432,12 @@ static int fmm_configure(Ctx* c)
     auto fill = [&](const void* dst, const void* src, size_t bytes) {
         std::memcpy(up.data() + ((const unsigned char*)dst - base), src, bytes);
     };
-    for (int i = 0; i < 2; ++i) {
-        fill(dtab[i], tab[i].data(), tab[i].size() * sizeof(double));
-        const double* d = dtab[i];
-        c->fmm.tab[i].nodes = d;
-        c->fmm.tab[i].cheb = d + P[i];
-        c->fmm.tab[i].shift = d + P[i] + P[i] * P[i];
-        c->fmm.tab[i].fnodes = d + P[i] + 3 * P[i] * P[i];
-        c->fmm.tab[i].fine = c->fmm.tab[i].fnodes + fmm_far(P[i]);
-        c->fmm.mult[i] = mult[i];
-        c->fmm.multf[i] = mult[i] ? mult[i] + slots * P[i] * P[i] : nullptr;
-    }
+    fill(dtab, tab.data(), tab.size() * sizeof(double));
+    plan.tab.nodes = dtab;
+    plan.tab.cheb = dtab + P;
+    plan.tab.shift = plan.tab.cheb + P * P;
+    plan.tab.fnodes = plan.tab.shift + 2 * P * P;
+    plan.tab.fine = plan.tab.fnodes + F;
     fill(dfs, fs.data(), sizeof(FmmSys) * S);
     fill(dt, tiles.data(), sizeof(FmmTile) * tiles.size());
     fill(dg, groups.data(), sizeof(FmmGroup) * groups.size());
@@ -443,7 +453,7 @@ static int fmm_configure(Ctx* c)
     a.neprefix = c->neprefix;
     a.key_sorted = c->key_sorted;
     a.l64 = c->l64;
-    c->fmm_on = wanted;
+    c->fmm_on |= 1 << precision;
     return BH_OK;
 }
 
@@ -531,14 +541,16 @@ static int configure(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, i
     HIP_TRY(hipMemset(c->stats, 0, sizeof(int32_t) * ST_COUNT));
     HIP_TRY(hipMemset(c->offsets, 0, sizeof(int32_t) * (C + 1)));
     HIP_TRY(hipMemset(c->neprefix, 0, sizeof(int32_t) * (C + 1)));
-    const size_t held = c->allocs.size();
-    if (fmm_configure(c) != BH_OK) {   // no room: every pass stays term by term
-        while (c->allocs.size() > held) {
+    c->fmm_on = 0;
+    const int wanted = fmm_wanted(c->sys_h);
+    for (int precision = 0; precision < 2; ++precision) {
+        const size_t held = c->allocs.size();
+        if (!(wanted >> precision & 1) || fmm_configure(c, precision) == BH_OK) continue;
+        while (c->allocs.size() > held) {   // no room: these passes stay term by term
             (void)hipFree(c->allocs.back());
             c->allocs.pop_back();
         }
         (void)hipGetLastError();
-        c->fmm_on = 0;
     }
     HIP_TRY(hipDeviceSynchronize());
     return BH_OK;
@@ -953,7 +965,7 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
         // Grouped far field: its chunks replace the work items, so the queue
         // order does not enter.  Near and mid terms are FP64 in both
         // precisions: nothing is left for the recompute to mend.
-        FmmArgs A = c->fa;
+        FmmArgs A = c->fa[precision];
         A.x = p->px;
         A.y = p->py;
         A.m = p->mass;
@@ -961,7 +973,7 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
         A.ay = p->ay;
         const bool rc = precision == 1 && c->rc_kappa > 0.0;
         if (part == 0) c->rc_ready = 0;
-        bh_fmm_pass(A, c->fmm, precision == 0, law->G, law->eps2, law->r2_cut, part, nparts,
+        bh_fmm_pass(A, c->fmm[precision], precision == 0, law->G, law->eps2, law->r2_cut, part, nparts,
                     c->num_cu, st);
         if (part == nparts - 1) {
             hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,

@@ -1,11 +1,11 @@
 // Grouped far field: the same sums as the term-by-term force kernels, with
 // the COMs of distant cells taken in groups.
 //
-// A system's grid is covered by square tiles of FMM_TILE cells per side.  A
+// A system's grid is covered by square tiles of T cells per side (fmm_tile).  A
 // particle's terms split into
 //   near     the particles of its 3x3 cells, one by one;
 //   mid      the COMs of the other non-empty cells of its 3x3 tiles, one by one;
-//   distant  the COMs of all other cells, at least FMM_TILE cells away.
+//   distant  the COMs of all other cells, at least T cells away.
 // The law's weight 1 / (r^2 + eps2) is smooth over the distant part (softening
 // only makes it smoother), so that part is interpolated: on each tile, and on
 // each square of 2^l tiles per side, a P x P Chebyshev grid carries the
@@ -918,7 +918,7 @@ template <int P>
 static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int num_cu,
                         hipStream_t st)
 {
-    const FmmTables& tb = P == 12 ? pl.tab[0] : pl.tab[1];
+    const FmmTables& tb = pl.tab;
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt,
                        (int64_t)(FMM_NCNT + A.S), 0);
     hipLaunchKernelGGL(k_fmm_tiles, dim3((unsigned)((A.nleaf * 8 + 255) / 256)), dim3(256), 0, st,
@@ -956,12 +956,9 @@ static void fmm_force(const FmmArgs& A, double Gc, double eps2, double r2cut, in
     }
 }
 
-void bh_fmm_pass(const FmmArgs& args, const FmmPlan& pl, bool fp64, double Gc, double eps2,
+void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, double eps2,
                  double r2cut, int part, int nparts, int num_cu, hipStream_t st)
 {
-    FmmArgs A = args;
-    A.mult = pl.mult[fp64 ? 1 : 0];
-    A.multf = pl.multf[fp64 ? 1 : 0];
     if (part == 0) {
         if (fp64) fmm_prepare<FMM_P64>(A, pl, eps2, num_cu, st);
         else fmm_prepare<FMM_P32>(A, pl, eps2, num_cu, st);

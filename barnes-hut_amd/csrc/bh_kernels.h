@@ -80,7 +80,10 @@ struct PotArgs {
 };
 
 // ---- grouped far field (bh_fmm.hip)
-#define FMM_TILE 8           // cells per side of a tile
+#define FMM_TILE 8           // cells per side of a tile at ~4 (fp32) or 30 (fp64) particles a cell
+#define FMM_TILE_MIN 4       // and its range (fmm_tile)
+#define FMM_TILE_MAX 24
+#define FMM_SIDE_MAX 1024    // most tiles a side: a level's node masses are addressed with 32 bits
 #define FMM_P32 12           // Chebyshev nodes per side, FP32 precision
 #define FMM_P64 20           // and FP64 precision
 #define FMM_LEVELS 13        // levels of squares (grid_dim <= 32767)
@@ -188,9 +191,7 @@ struct FmmTables {
 struct FmmPlan {
     int nlev = 0;
     int64_t ngroups = 0;
-    FmmTables tab[2];      // P = FMM_P32, FMM_P64
-    double* mult[2] = {nullptr, nullptr};    // their node masses (zero borders)
-    double* multf[2] = {nullptr, nullptr};
+    FmmTables tab;
 };
 void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, double eps2,
                  double r2cut, int part, int nparts, int num_cu, hipStream_t st);

@@ -53,7 +53,7 @@ def _against_oracle(h, G, off, keys, law, prec, seed=3, count=1500):
 
 
 def _input(kind):
-    n, G = 600001, 193            # 25 tiles per side, the last one a cell wide
+    n, G = 600001, 193            # a last tile of fewer cells
     if kind == "sparse_columns":   # most tiles empty, some of one cell, a few dense
         rng = np.random.default_rng(41)
         x = np.floor(rng.random(n) * 24) / 24 + 1e-4 * rng.random(n)
@@ -97,6 +97,24 @@ def test_grouped_pass_against_oracle(kind, eps2, r2_cut):
         # signed masses cancel in every particle: FP64 sums of 2e4 terms
         assert norm <= (1e-11 if kind == "signed" else NORM[prec])
         assert each <= (1e-5 if kind == "signed" else EACH[prec])
+    eng.close()
+
+
+@pytest.mark.parametrize("n,G,precisions", [
+    (70001, 600, "64"),          # 0.2 particles a cell: tiles of 24 cells
+    (150001, 500, "64 32"),      # 0.6: 22 and 14
+    (400001, 301, "64 32"),      # 4.4: 13 and 8
+    (1000003, 97, "64"),         # 106: 6
+    (2500001, 90, "64 32")])     # 309: 4 and 4, a last tile of two cells
+def test_tile_sizes(n, G, precisions):
+    """The tile side follows from particles per cell, by precision."""
+    d = inputs.uniform(n, seed=47)
+    eng = _engine([n], [G], d)
+    off, keys = eng.offsets().astype(np.int64), eng.keys().astype(np.int64)
+    for prec in ("fp" + p for p in precisions.split()):
+        law = (1e-6, 1e-10, 0.0)
+        norm, each = _against_oracle(_pass(eng, law, prec), G, off, keys, law, prec, count=700)
+        assert norm <= NORM[prec] and each <= EACH[prec]
     eng.close()
 
 
