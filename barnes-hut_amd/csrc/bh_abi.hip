@@ -728,14 +728,15 @@ int bh_place_particles(void* ctx, const bh_particles* p, void* stream)
     const double *x = p->px, *y = p->py;
     const int32_t* so = c->sys_of;
     if (N < PLACE_SMALL) {
-        hipLaunchKernelGGL(k_bbox<4>, dim3(cdiv(N, 1024)), dim3(256), 0, st, x, y, so, N, c->bb,
+        hipLaunchKernelGGL(k_bbox<4>, dim3(cdiv(N, 1024)), dim3(256), 0, st, x, y, so, N, 1, c->bb,
                            c->stats);
         hipLaunchKernelGGL(k_keys_hist<2>, dim3(cdiv(N, 512)), dim3(256), 0, st, x, y, so, c->sys,
                            (const uint64_t*)c->bb, N, c->key, c->rank, c->counts,
                            c->stats);
     } else {
-        hipLaunchKernelGGL(k_bbox<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, N, c->bb,
-                           c->stats);
+        const int rounds = (int)cdiv(N, (int64_t)c->num_cu * 2 * 2048);
+        hipLaunchKernelGGL(k_bbox<8>, dim3(cdiv(N, 2048 * (int64_t)rounds)), dim3(256), 0, st, x, y,
+                           so, N, rounds, c->bb, c->stats);
         hipLaunchKernelGGL(k_keys_hist<8>, dim3(cdiv(N, 2048)), dim3(256), 0, st, x, y, so, c->sys,
                            (const uint64_t*)c->bb, N, c->key, c->rank, c->counts,
                            c->stats);

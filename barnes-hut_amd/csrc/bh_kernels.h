@@ -371,7 +371,7 @@ __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v);
 __global__ void k_fill_f64(double* p, int64_t n, double v);
 __global__ void k_place_init(int32_t* stats, int32_t* counts, int64_t C, uint64_t* bb, int S);
 template <int R>
-__global__ void k_bbox(const double* px, const double* py, const int32_t* sys_of, int64_t N,
+__global__ void k_bbox(const double* px, const double* py, const int32_t* sys_of, int64_t N, int rounds,
                        uint64_t* bb, int32_t* stats);
 template <int R>
 __global__ void k_keys_hist(const double* px, const double* py, const int32_t* sys_of, SysDev* sys,

@@ -58,29 +58,22 @@ __device__ __forceinline__ void bbox_flush(uint64_t* bb, int s, double mnx, doub
     if (k3 > __atomic_load_n(&b[3], __ATOMIC_RELAXED)) atomicMax(&b[3], k3);
 }
 
-// Each wave covers 64 R consecutive particles, all of its loads issued before
-// the first is used; min/max are exact, so the reduction order does not matter.
+// Each wave covers `rounds` runs of 64 R consecutive particles, all of a run's
+// loads issued before the first is used; min/max are exact, so the reduction
+// order does not matter.  Two blocks a CU with as many rounds as it takes: a
+// block's look at the stored extremes costs ~15 ns of one cache line's time, so a
+// block per 2048 rows took 157 us on 10M particles, 116 on 4.2M and 245 on 512
+// systems, against 58, 40 and 181 (the rows: 43, 18 and 115 at copy rate).
 // Rows of one system are consecutive: a wave reduces when the system changes
 // (a block of one system reduces over the block).
 template <int R>
 __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
                                               const double* __restrict__ py,
                                               const int32_t* __restrict__ sys_of, int64_t N,
-                                              uint64_t* bb, int32_t* stats)
+                                              int rounds, uint64_t* bb, int32_t* stats)
 {
     const double inf = __longlong_as_double(0x7ff0000000000000ll);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int64_t base = ((int64_t)blockIdx.x * 4 + wid) * (64 * R);
-    int sv[R];
-    double xv[R], yv[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int64_t i = base + 64 * r + lane;
-        const bool in = i < N;
-        sv[r] = in ? sys_of[i] : -1;
-        xv[r] = in ? px[i] : 0.0;
-        yv[r] = in ? py[i] : 0.0;
-    }
     int cur = -1;   // system of the running extremes (wave-uniform)
     double mnx = inf, mny = inf, mxx = -inf, mxy = -inf;
     bool bad = false;
@@ -96,24 +89,38 @@ __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
         if (lane == 0) bbox_flush(bb, cur, mnx, mny, mxx, mxy);
         mnx = inf; mny = inf; mxx = -inf; mxy = -inf;
     };
+    // a wave's rows: `rounds` runs of 64 R, one after the other
+    int64_t base = ((int64_t)blockIdx.x * 4 + wid) * (64 * R) * rounds;
+    for (int k = 0; k < rounds && base < N; ++k, base += 64 * R) {
+        int sv[R];
+        double xv[R], yv[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const bool fin = isfinite(xv[r]) && isfinite(yv[r]);
-        if (sv[r] >= 0 && !fin) bad = true;
-        unsigned long long todo = __ballot(sv[r] >= 0);
-        while (todo) {   // the systems of these 64 rows, nearly always one
-            const int s = __builtin_amdgcn_readlane(sv[r], __ffsll((long long)todo) - 1);
-            if (s != cur) {
-                flush();
-                cur = s;
+        for (int r = 0; r < R; ++r) {
+            const int64_t i = base + 64 * r + lane;
+            const bool in = i < N;
+            sv[r] = in ? sys_of[i] : -1;
+            xv[r] = in ? px[i] : 0.0;
+            yv[r] = in ? py[i] : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool fin = isfinite(xv[r]) && isfinite(yv[r]);
+            if (sv[r] >= 0 && !fin) bad = true;
+            unsigned long long todo = __ballot(sv[r] >= 0);
+            while (todo) {   // the systems of these 64 rows, nearly always one
+                const int s = __builtin_amdgcn_readlane(sv[r], __ffsll((long long)todo) - 1);
+                if (s != cur) {
+                    flush();
+                    cur = s;
+                }
+                if (sv[r] == s && fin) {
+                    mnx = fmin(mnx, xv[r]);
+                    mxx = fmax(mxx, xv[r]);
+                    mny = fmin(mny, yv[r]);
+                    mxy = fmax(mxy, yv[r]);
+                }
+                todo &= ~__ballot(sv[r] == s);
             }
-            if (sv[r] == s && fin) {
-                mnx = fmin(mnx, xv[r]);
-                mxx = fmax(mxx, xv[r]);
-                mny = fmin(mny, yv[r]);
-                mxy = fmax(mxy, yv[r]);
-            }
-            todo &= ~__ballot(sv[r] == s);
         }
     }
     __shared__ double red[4][4];
@@ -143,10 +150,10 @@ __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
     }
 }
 
-template __global__ void k_bbox<4>(const double*, const double*, const int32_t*, int64_t, uint64_t*,
-                                   int32_t*);
-template __global__ void k_bbox<8>(const double*, const double*, const int32_t*, int64_t, uint64_t*,
-                                   int32_t*);
+template __global__ void k_bbox<4>(const double*, const double*, const int32_t*, int64_t, int,
+                                   uint64_t*, int32_t*);
+template __global__ void k_bbox<8>(const double*, const double*, const int32_t*, int64_t, int,
+                                   uint64_t*, int32_t*);
 
 // ---------------------------------------------------------------- keys + histogram
 struct Box {
