@@ -821,7 +821,9 @@ static BhParticles dev_of(const bh_particles* p)
     return d;
 }
 
-int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
+// scattered: k_place_one has put the rows into cell order.
+static int sort_impl(void* ctx, const bh_particles* src, const bh_particles* dst, bool scattered,
+                     void* stream)
 {
     Ctx* c = (Ctx*)ctx;
     CTX_READY(c);
@@ -833,10 +835,11 @@ int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* ds
     const int64_t N = c->N;
     SortFields F = fields_of(src);
     const int sr = N < PLACE_SMALL ? 1 : 8;
-    hipLaunchKernelGGL(sr == 1 ? k_scatter<1> : k_scatter<8>, dim3(cdiv(N, 256 * sr)), dim3(256), 0,
-                       st, (const int32_t*)c->key, N, (const int32_t*)c->offsets,
-                       (const int32_t*)c->rank, c->idx_a, c->key_sorted, (const double*)src->px,
-                       (const double*)src->py, c->pxkey, c->pykey);
+    if (!scattered)
+        hipLaunchKernelGGL(sr == 1 ? k_scatter<1> : k_scatter<8>, dim3(cdiv(N, 256 * sr)), dim3(256), 0,
+                           st, (const int32_t*)c->key, N, (const int32_t*)c->offsets,
+                           (const int32_t*)c->rank, c->idx_a, c->key_sorted, (const double*)src->px,
+                           (const double*)src->py, c->pxkey, c->pykey);
     hipLaunchKernelGGL(k_sort_units, dim3(cdiv(N, SORT_W)), dim3(SORT_THREADS), 0, st, F, N,
                        (const int32_t*)c->idx_a, (const int32_t*)c->key_sorted,
                        (const uint64_t*)c->pxkey, (const uint64_t*)c->pykey,
@@ -859,6 +862,11 @@ int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* ds
     return BH_OK;
 }
 
+int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream)
+{
+    return sort_impl(ctx, src, dst, false, stream);
+}
+
 int bh_summarize(void* ctx, const bh_particles* p, void* stream)
 {
     Ctx* c = (Ctx*)ctx;
@@ -877,6 +885,15 @@ int bh_summarize(void* ctx, const bh_particles* p, void* stream)
     return BH_OK;
 }
 
+static void fill_items(Ctx* c, hipStream_t st)
+{
+    const int pitem = 64 * c->tune.p;
+    hipLaunchKernelGGL(k_items_fill, dim3(grid_for(cdiv(c->N, pitem) + c->ncols, 256,
+                                                   (int64_t)c->num_cu * 8)), dim3(256), 0, st,
+                       (const SysDev*)c->sys, c->S, (int)c->ncols, (const int32_t*)c->offsets, pitem,
+                       (const int32_t*)c->col_off, c->items, (const int32_t*)c->stats);
+}
+
 int bh_build_items(void* ctx, void* stream)
 {
     Ctx* c = (Ctx*)ctx;
@@ -888,12 +905,7 @@ int bh_build_items(void* ctx, void* stream)
         hipLaunchKernelGGL(k_items_runs, dim3(1), dim3(1024), 0, st, (const SysDev*)c->sys, c->S,
                            (int)c->ncols, (const int32_t*)c->offsets, pitem, c->col_off, c->items,
                            c->max_items, c->stats, write);
-        if (!write)
-            hipLaunchKernelGGL(k_items_fill, dim3(grid_for(cdiv(c->N, pitem) + c->ncols, 256,
-                                                           (int64_t)c->num_cu * 8)), dim3(256), 0,
-                               st, (const SysDev*)c->sys, c->S, (int)c->ncols,
-                               (const int32_t*)c->offsets, pitem, (const int32_t*)c->col_off,
-                               c->items, (const int32_t*)c->stats);
+        if (!write) fill_items(c, st);
         LAUNCH_CHECK("items");
         return BH_OK;
     }
@@ -1163,18 +1175,41 @@ static int step_impl(void* ctx, const bh_particles* a, const bh_particles* b, co
                      int32_t* order, void* stream)
 {
     int r;
-    if ((r = bh_place_particles(ctx, a, stream))) return r;
-    if ((r = bh_calculate_box_cumm(ctx, stream))) return r;
-    if ((r = bh_sort_particles(ctx, a, b, stream))) return r;
-    if ((r = bh_summarize(ctx, b, stream))) return r;
-    if ((r = bh_build_items(ctx, stream))) return r;
+    Ctx* c = (Ctx*)ctx;
+    CTX_READY(c);
+    if ((r = check_parts(a, "particles")) || (r = check_parts(b, "dst"))) return r;
+    hipStream_t st = (hipStream_t)stream;
+    const bool one = c->S == 1 && c->N <= PLACE_ONE && c->C <= SCAN_ONE;
+    if (one) {
+        hipLaunchKernelGGL(k_place_one, dim3(1), dim3(1024), 0, st, (const double*)a->px,
+                           (const double*)a->py, c->sys, (int)c->N, (int)c->C, c->key, c->rank,
+                           c->counts, c->offsets, c->neprefix, c->ne_list, c->com_dense, c->idx_a,
+                           c->key_sorted, c->pxkey, c->pykey, c->stats);
+    } else {
+        if ((r = bh_place_particles(ctx, a, stream))) return r;
+        if ((r = bh_calculate_box_cumm(ctx, stream))) return r;
+    }
+    if ((r = sort_impl(ctx, a, b, one, stream))) return r;
+    if (c->maxG <= c->tune.yspan && c->ncols <= ITEMS_COLS) {
+        const int write = c->N <= ITEMS_ONE;
+        const int64_t waves = std::min<int64_t>(c->C, (int64_t)c->num_cu * 64);
+        hipLaunchKernelGGL(k_com_items, dim3(grid_for(waves * 64, 256) + 1), dim3(256), 0, st,
+                           (const SysDev*)c->sys, c->S, (const int32_t*)c->ne_list, c->stats,
+                           (const int32_t*)c->offsets, (const double*)b->px, (const double*)b->py,
+                           (const double*)b->mass, c->com_dense, c->l64, c->l32, (int)c->ncols,
+                           64 * c->tune.p, c->col_off, c->items, c->max_items, write);
+        if (!write) fill_items(c, st);
+        LAUNCH_CHECK("summarize");
+    } else {
+        if ((r = bh_summarize(ctx, b, stream))) return r;
+        if ((r = bh_build_items(ctx, stream))) return r;
+    }
     const int32_t* ord = nullptr;
     if (params) {
         if ((r = bh_learned_order(ctx, params, order, stream))) return r;
         ord = order;
     }
     if ((r = bh_force_pass(ctx, b, law, precision, ord, stream))) return r;
-    Ctx* c = (Ctx*)ctx;
     if (c->rc_ready && c->rc_deferred && (r = bh_recompute(ctx, b, law, stream))) return r;
     if (do_tick && (r = bh_tick_particles(ctx, b, dt, stream))) return r;
     return BH_OK;

@@ -10,7 +10,9 @@
 #define HIST_BINS 8192     // LDS histogram window (keys) per block
 #define SCAN_TILE 2048     // elements per block in the scans
 #define SCAN_ONE 8192      // elements that one block scans in one launch
-#define SORT_WAYS 8        // runs that a merge pass joins
+#define PLACE_ONE 4096     // rows of a system that one block places (k_place_one)
+#define SORT_WAYS 16       // runs that a merge pass joins
+#define ITEMS_COLS 1024    // columns whose items a block of k_com_items builds
 #define ITEMS_ONE 65536    // particles up to which one block builds a step's items
 #define COM_BIG 1024       // rows from which a cell's sums are a block's work (k_com)
 #define SORT_W 1024        // within-cell rank window (rows)
@@ -394,6 +396,11 @@ template <int R>
 __global__ void k_scatter(const int32_t* key, int64_t N, const int32_t* offsets,
                           const int32_t* rank, int32_t* idx_out, int32_t* key_sorted, const double* px,
                           const double* py, uint64_t* pxkey_out, uint64_t* pykey_out);
+__global__ void k_place_one(const double* px, const double* py, SysDev* sys, int N, int C,
+                            int32_t* key_out, int32_t* rank_out, int32_t* counts, int32_t* offsets,
+                            int32_t* neprefix, int32_t* ne_list, double* com_dense,
+                            int32_t* idx_out, int32_t* key_sorted, uint64_t* pxkey,
+                            uint64_t* pykey, int32_t* stats);
 __global__ void k_sort_units(SortFields F, int64_t N, const int32_t* idx_in,
                              const int32_t* key_sorted, const uint64_t* pxkey,
                              const uint64_t* pykey, const int32_t* offsets, int32_t* idx_out);
@@ -408,6 +415,11 @@ __global__ void k_gather(SortFields S, BhParticles D, int64_t N, const int32_t* 
 __global__ void k_com(const SysDev* sys, int S, const int32_t* ne_list, const int32_t* stats,
                       const int32_t* offsets, const double* x, const double* y, const double* m,
                       double* com_dense, Com64* l64, Com32* l32);
+// k_com, and in its last block the items (k_items_runs) of at most ITEMS_COLS columns
+__global__ void k_com_items(const SysDev* sys, int S, const int32_t* ne_list, int32_t* stats,
+                            const int32_t* offsets, const double* x, const double* y,
+                            const double* m, double* com_dense, Com64* l64, Com32* l32, int ncols,
+                            int pitem, int32_t* col_off, Item* items, int64_t max_items, int write);
 __global__ void k_tick(double* x, double* y, double* vx, double* vy, double* ax, double* ay,
                        int64_t N, double dt);
 __global__ void k_interactions(const SysDev* sys, int S, const int32_t* counts,

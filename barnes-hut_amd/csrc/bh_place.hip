@@ -164,23 +164,41 @@ struct Box {
 
 // A system's box from its extremes: helpers/grid.py:15-22 square-up,
 // base.py:237 step, exactly in FP64.
-__device__ __forceinline__ Box box_of(const SysDev* sys, const uint64_t* bb, int s)
+__device__ __forceinline__ Box square_box(const SysDev& sys, double min_x, double min_y,
+                                          double max_x, double max_y)
 {
     Box d;
-    d.min_x = bh_ord_val(bb[4 * s + 0]);
-    d.min_y = bh_ord_val(bb[4 * s + 1]);
-    d.max_x = bh_ord_val(bb[4 * s + 2]);
-    d.max_y = bh_ord_val(bb[4 * s + 3]);
+    d.min_x = min_x;
+    d.min_y = min_y;
+    d.max_x = max_x;
+    d.max_y = max_y;
     const double xe = d.max_x - d.min_x, ye = d.max_y - d.min_y;
     if (xe > ye) {
         d.max_y += (xe - ye);
     } else if (ye > xe) {
         d.max_x += (ye - xe);
     }
-    d.G = sys[s].G;
-    d.c_off = sys[s].c_off;
+    d.G = sys.G;
+    d.c_off = sys.c_off;
     d.step = (d.max_x - d.min_x) / (double)d.G;
     return d;
+}
+
+__device__ __forceinline__ Box box_of(const SysDev* sys, const uint64_t* bb, int s)
+{
+    return square_box(sys[s], bh_ord_val(bb[4 * s + 0]), bh_ord_val(bb[4 * s + 1]),
+                      bh_ord_val(bb[4 * s + 2]), bh_ord_val(bb[4 * s + 3]));
+}
+
+// Whether the box has an extent.
+__device__ __forceinline__ bool store_box(SysDev& sys, const Box& d)
+{
+    sys.min_x = d.min_x;
+    sys.min_y = d.min_y;
+    sys.max_x = d.max_x;
+    sys.max_y = d.max_y;
+    sys.step = d.step;
+    return d.step > 0.0 && isfinite(d.step);
 }
 
 // sequential.py:32-34: g = clip(floor((p - min) / step), 0, G-1), IEEE division.
@@ -258,12 +276,7 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double* __restrict__ px
                 d = box_of(sys, bb, cur);
             }
             if (i == sys[cur].p_off) {
-                sys[cur].min_x = d.min_x;
-                sys[cur].min_y = d.min_y;
-                sys[cur].max_x = d.max_x;
-                sys[cur].max_y = d.max_y;
-                sys[cur].step = d.step;
-                if (!(d.step > 0.0) || !isfinite(d.step)) atomicOr(&stats[ST_ERR], BH_ERR_DEGENERATE);
+                if (!store_box(sys[cur], d)) atomicOr(&stats[ST_ERR], BH_ERR_DEGENERATE);
             }
             int k = cell_key(xr[r], yr[r], d);
             key_out[i] = k;
@@ -613,6 +626,130 @@ template __global__ void k_scatter<8>(const int32_t*, int64_t, const int32_t*, c
                                       int32_t*, int32_t*, const double*, const double*, uint64_t*,
                                       uint64_t*);
 
+// ---------------------------------------------------------------- small systems
+// Box, keys, counts, scan and scatter of one system of at most PLACE_ONE rows and
+// SCAN_ONE cells in one block: five launches of 2 to 5 us each otherwise, most of
+// it latency.  2,000 particles on 11^2 cells: 10 us instead of 16; 16,384 on 32^2
+// would take 32 instead of 20.
+__global__ __launch_bounds__(1024) void k_place_one(
+    const double* __restrict__ px, const double* __restrict__ py, SysDev* sys, int N, int C,
+    int32_t* __restrict__ key_out, int32_t* __restrict__ rank_out, int32_t* __restrict__ counts,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ neprefix, int32_t* __restrict__ ne_list,
+    double* __restrict__ com_dense, int32_t* __restrict__ idx_out, int32_t* __restrict__ key_sorted,
+    uint64_t* __restrict__ pxkey, uint64_t* __restrict__ pykey, int32_t* __restrict__ stats)
+{
+    constexpr int RP = PLACE_ONE / 1024, RC = SCAN_ONE / 1024;
+    __shared__ int32_t cell[SCAN_ONE];   // counts, then offsets
+    __shared__ double red[4][16];
+    __shared__ int sh[40], err, mxc[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const double inf = __longlong_as_double(0x7ff0000000000000ll);
+    double x[RP], y[RP], mnx = inf, mny = inf, mxx = -inf, mxy = -inf;
+    if (tid == 0) err = 0;
+    for (int c = tid; c < C; c += 1024) cell[c] = 0;
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {   // clamped: a row past the end repeats the last
+        const int i = min(tid + 1024 * r, N - 1);
+        x[r] = px[i];
+        y[r] = py[i];
+    }
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {
+        if (!isfinite(x[r]) || !isfinite(y[r])) {
+            bad = true;
+            continue;
+        }
+        mnx = fmin(mnx, x[r]);
+        mxx = fmax(mxx, x[r]);
+        mny = fmin(mny, y[r]);
+        mxy = fmax(mxy, y[r]);
+    }
+    mnx = wave_min(mnx);
+    mny = wave_min(mny);
+    mxx = wave_max(mxx);
+    mxy = wave_max(mxy);
+    __syncthreads();
+    if (lane == 0) {
+        red[0][w] = mnx;
+        red[1][w] = mny;
+        red[2][w] = mxx;
+        red[3][w] = mxy;
+    }
+    if (bad) atomicOr(&err, BH_ERR_NONFINITE);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        mnx = fmin(mnx, red[0][k]);
+        mny = fmin(mny, red[1][k]);
+        mxx = fmax(mxx, red[2][k]);
+        mxy = fmax(mxy, red[3][k]);
+    }
+    const Box d = square_box(sys[0], mnx, mny, mxx, mxy);
+    int key[RP], lr[RP];
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {
+        const int i = tid + 1024 * r;
+        if (i >= N) continue;
+        key[r] = cell_key(x[r], y[r], d);
+        lr[r] = atomicAdd(&cell[key[r]], 1);
+        key_out[i] = key[r];
+        rank_out[i] = lr[r];
+    }
+    __syncthreads();
+    if (tid == 0 && !store_box(sys[0], d)) atomicOr(&err, BH_ERR_DEGENERATE);
+    int cv[RC], v = 0, f = 0, mx = 0;
+#pragma unroll
+    for (int r = 0; r < RC; ++r) {
+        const int i = tid * RC + r;
+        cv[r] = i < C ? cell[i] : 0;
+        v += cv[r];
+        f += cv[r] > 0;
+        mx = max(mx, cv[r]);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) mxc[w] = mx;
+    int av, af, tv, tf;
+    block_excl_scan2(v, f, av, af, tv, tf, sh);
+#pragma unroll
+    for (int r = 0; r < RC; ++r) {
+        const int i = tid * RC + r;
+        if (i < C) {
+            counts[i] = cv[r];
+            offsets[i] = av;
+            neprefix[i] = af;
+            cell[i] = av;
+            if (cv[r] > 0) ne_list[af] = i;
+            av += cv[r];
+            af += cv[r] > 0;
+        }
+    }
+    clear_com(com_dense, 0, C, 1024);
+    __syncthreads();
+    if (tid < ST_COUNT) {
+        int st = 0;
+        if (tid == ST_ERR) st = err;
+        if (tid == ST_NCELLS_NE) st = tf;
+        if (tid == ST_MAXCOUNT)
+            for (int k = 0; k < 16; ++k) st = max(st, mxc[k]);
+        stats[tid] = st;
+    }
+    if (tid == 0) {
+        offsets[C] = tv;
+        neprefix[C] = tf;
+    }
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {
+        const int i = tid + 1024 * r;
+        if (i >= N) continue;
+        const int pos = cell[key[r]] + lr[r];
+        idx_out[pos] = i;
+        key_sorted[pos] = key[r];
+        pxkey[pos] = sort_key(x[r]);
+        pykey[pos] = sort_key(y[r]);
+    }
+}
+
 // ---------------------------------------------------------------- within-cell order
 // numpy's structured-sort tie rule after (gx, gy): px, py, mass, vx, vy, ax,
 // ay, pid (internals/particle.py:3-9); equal rows keep input order (stable).
@@ -764,8 +901,10 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort_units(SortFields F, int64
 // row's place is its place in its own run plus, by binary search, the rows
 // before it in each of the others.  Only rows of such cells are touched; the
 // pass is a no-op once R >= max count.  (Pairwise merging searches less per row
-// but takes three times the launches, and most of them find nothing to do: 12
-// at 4.5 us on 4.2M particles.)
+// but takes four times the launches, and most of them find nothing to do: 12 at
+// 4.5 us on 4.2M particles.  8 at a time: one launch more at 16,384, 262,144 and
+// 4.2M particles, 2 to 5 us each; 32 saves one more at 1M but searches twice as
+// many runs per row of the largest cells.)
 __global__ __launch_bounds__(256) void k_sort_merge(SortFields F, int64_t N,
                                                     const int32_t* __restrict__ idx_in,
                                                     const int32_t* __restrict__ key_sorted,

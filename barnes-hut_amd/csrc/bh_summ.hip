@@ -4,6 +4,7 @@
 //   calc_COM          python-bh/barneshut/internals/cloud.py:9-17
 //   g_tick_particles  python-bh/barneshut/kernels/grid_decomposition/gpu/grid.py:159-174
 #include "bh_common.h"
+#include "bh_items.h"
 #include "bh_kernels.h"
 
 // Entry w of the lists and cell c's place in the dense array, from its sums.
@@ -48,22 +49,18 @@ __device__ __forceinline__ void com_out(const SysDev& d, int64_t w, int c, doubl
 // not: cells of more than COM_BIG rows are left to the whole block, after its
 // others.  262,144 particles in 16 clusters on 256^2 cells (up to 9,900 in a
 // cell): 144 -> 20 us; 4.2M on 1024^2 99 -> 89 us.
-__global__ __launch_bounds__(256) void k_com(const SysDev* __restrict__ sys, int S,
-                                             const int32_t* __restrict__ ne_list,
-                                             const int32_t* __restrict__ stats,
-                                             const int32_t* __restrict__ offsets,
-                                             const double* __restrict__ x,
-                                             const double* __restrict__ y,
-                                             const double* __restrict__ m,
-                                             double* __restrict__ com_dense,
-                                             Com64* __restrict__ l64, Com32* __restrict__ l32)
+__device__ __forceinline__ void com_cells(
+    const SysDev* __restrict__ sys, int S, const int32_t* __restrict__ ne_list,
+    const int32_t* __restrict__ stats, const int32_t* __restrict__ offsets,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ m,
+    double* __restrict__ com_dense, Com64* __restrict__ l64, Com32* __restrict__ l32, int nblocks,
+    double (*part)[4])
 {
     constexpr int QW = 16;
-    __shared__ double part[3][4];
     const int lane = threadIdx.x & 63;
     const int q = lane >> 4, ql = lane & (QW - 1);
     const int64_t wv = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    const int64_t nw = ((int64_t)nblocks * blockDim.x) >> 6;
     const int nne = stats[ST_NCELLS_NE];
     // each wave takes a contiguous run of the non-empty list, so it crosses
     // few system boundaries and looks its system up only when it does
@@ -131,6 +128,40 @@ __global__ __launch_bounds__(256) void k_com(const SysDev* __restrict__ sys, int
             com_out(sys[sys_of_cell(sys, S, c)], w, c, t[0], t[1], t[2], com_dense, l64, l32);
         }
     }
+}
+
+__global__ __launch_bounds__(256) void k_com(const SysDev* __restrict__ sys, int S,
+                                             const int32_t* __restrict__ ne_list,
+                                             const int32_t* __restrict__ stats,
+                                             const int32_t* __restrict__ offsets,
+                                             const double* __restrict__ x,
+                                             const double* __restrict__ y,
+                                             const double* __restrict__ m,
+                                             double* __restrict__ com_dense,
+                                             Com64* __restrict__ l64, Com32* __restrict__ l32)
+{
+    __shared__ double part[3][4];
+    com_cells(sys, S, ne_list, stats, offsets, x, y, m, com_dense, l64, l32, gridDim.x, part);
+}
+
+// The last block builds the work items meanwhile: a launch of its own for them is
+// 5 us of a 2,000-particle step, 11 us of one of 40 small systems.
+__global__ __launch_bounds__(256) void k_com_items(
+    const SysDev* __restrict__ sys, int S, const int32_t* __restrict__ ne_list, int32_t* stats,
+    const int32_t* __restrict__ offsets, const double* __restrict__ x,
+    const double* __restrict__ y, const double* __restrict__ m, double* __restrict__ com_dense,
+    Com64* __restrict__ l64, Com32* __restrict__ l32, int ncols, int pitem, int32_t* col_off,
+    Item* __restrict__ items, int64_t max_items, int write)
+{
+    __shared__ double part[3][4];
+    __shared__ int32_t at[ITEMS_COLS];
+    __shared__ int wsum[4];
+    if (blockIdx.x + 1 < gridDim.x)
+        com_cells(sys, S, ne_list, stats, offsets, x, y, m, com_dense, l64, l32, gridDim.x - 1,
+                  part);
+    else
+        items_runs<256, ITEMS_COLS>(sys, S, ncols, offsets, pitem, col_off, items, max_items, stats,
+                                    write, at, wsum);
 }
 
 // v += a*dt; a = 0; x += v*dt  (separate multiply and add; the library is

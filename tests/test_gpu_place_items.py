@@ -190,3 +190,34 @@ def test_unsorted_rows_over_many_cells(n):
     np.testing.assert_array_equal(eng.counts(), np.bincount(key, minlength=G * G))
     np.testing.assert_array_equal(eng.fetch()["pid"], src["pid"][order])
     eng.close()
+
+
+@pytest.mark.parametrize("sizes,grids", [
+    ([2], [1]), ([2], [90]), ([1023], [11]), ([1025], [11]), ([4095], [1]), ([4096], [90]),
+    ([4097], [90]), ([4096], [91]), ([3000], [600]), ([70001], [40]), ([500, 9000, 2], [1000, 31, 1]),
+    ([500, 66000, 2], [400, 500, 130])])
+def test_steps_equal_their_phases(sizes, grids):
+    """A step joins the placement of a small system and the items of few columns
+    with their neighbours; the phases one by one give the same bits."""
+    from barneshut.engine import Engine
+    d = inputs.batched_uniform(sizes, seed=74)
+    law = (1e-6, 1e-10, 0.0)
+    runs = []
+    for whole in (True, False):
+        eng = Engine(sizes, grids)
+        eng.load(d)
+        for _ in range(3):
+            if whole:
+                eng.step(*law, precision="fp64", dt=1e-4)
+            else:
+                eng.create_tree()
+                eng.summarize()
+                eng.evaluate(*law, "fp64")
+                eng.timestep(1e-4)
+            st = eng.check()
+        runs.append(dict(eng.fetch(), counts=eng.counts(), offsets=eng.offsets(), com=eng.com(),
+                         keys=eng.keys(), items=eng.items(), perm=eng.perm(), box=eng.bbox(),
+                         stats=np.array([st[1], st[2], st[4]])))
+        eng.close()
+    for k, v in runs[0].items():
+        np.testing.assert_array_equal(v, runs[1][k])
