@@ -1099,17 +1099,16 @@ int bh_recompute(void* ctx, const bh_particles* p, const bh_law* law, void* stre
     if (!c->rc_ready) return fail(BH_ESTATE, "no FP32 force pass prepared a recompute");
     if (c->rc_ready == 2) return BH_OK;   // the pass formed its sums in FP64: nothing flagged
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP, (int64_t)2, 0);
-    if (law->G == 0.0) return BH_OK;   // every term, and so the FP32 result, is zero
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(c->S, 64, 1024)), dim3(64), 0, st, c->rc_cnt,
-                       (int64_t)c->S, 0);
-    hipLaunchKernelGGL(k_rc_blocks, dim3(grid_for(c->nblocks, 1, (int64_t)c->num_cu * 16)),
-                       dim3(64), 0, st, (const SysDev*)c->sys, c->S, c->nblocks,
-                       (const double*)c->com_dense, c->rc_blk);
+    if (law->G == 0.0) {   // every term, and so the FP32 result, is zero
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP, (int64_t)2,
+                           0);
+        return BH_OK;
+    }
     const int64_t ntiles = c->nblocks * (RC_BLOCK / RC_TILE) * (RC_BLOCK / RC_TILE);
-    hipLaunchKernelGGL(k_rc_tiles, dim3(grid_for(ntiles, 256, (int64_t)c->num_cu * 8)), dim3(256),
-                       0, st, (const SysDev*)c->sys, c->S, ntiles, (const double*)c->com_dense,
-                       c->rc_tiles);
+    const unsigned nb = grid_for(c->nblocks, 4, (int64_t)c->num_cu * 4);
+    hipLaunchKernelGGL(k_rc_sums, dim3(nb + grid_for(ntiles, 256, (int64_t)c->num_cu * 8)),
+                       dim3(256), 0, st, (const SysDev*)c->sys, c->S, c->nblocks, ntiles, (int)nb,
+                       (const double*)c->com_dense, c->rc_blk, c->rc_tiles, c->rc_cnt, c->stats);
     hipLaunchKernelGGL(k_rc_blockfar, dim3(grid_for(c->nblocks, 1, (int64_t)c->num_cu * 16)),
                        dim3(64), 0, st, (const SysDev*)c->sys, c->S, c->nblocks,
                        (const double*)c->rc_blk, c->rc_bfar);
@@ -1179,7 +1178,7 @@ static int step_impl(void* ctx, const bh_particles* a, const bh_particles* b, co
     CTX_READY(c);
     if ((r = check_parts(a, "particles")) || (r = check_parts(b, "dst"))) return r;
     hipStream_t st = (hipStream_t)stream;
-    const bool one = c->S == 1 && c->N <= PLACE_ONE && c->C <= SCAN_ONE;
+    const bool one = c->S == 1 && c->N <= PLACE_ONE && c->C <= PLACE_CELLS;
     if (one) {
         hipLaunchKernelGGL(k_place_one, dim3(1), dim3(1024), 0, st, (const double*)a->px,
                            (const double*)a->py, c->sys, (int)c->N, (int)c->C, c->key, c->rank,
@@ -1646,6 +1645,14 @@ extern "C" int bh_step_noalloc(const bh_particles* a, const bh_particles* b, int
 Item* bh_ctx_items(void* ctx) { return ((Ctx*)ctx)->items; }
 int32_t* bh_ctx_stats(void* ctx) { return ((Ctx*)ctx)->stats; }
 int64_t bh_ctx_max_items(void* ctx) { return ((Ctx*)ctx)->max_items; }
+// The most items a pass can have: whole runs and a rest per column where no run
+// reaches the row span.
+int64_t bh_ctx_item_bound(void* ctx)
+{
+    Ctx* c = (Ctx*)ctx;
+    if (c->maxG > c->tune.yspan) return c->max_items;
+    return std::min(c->max_items, cdiv(c->N, 64 * c->tune.p) + c->ncols);
+}
 int bh_ctx_num_cu(void* ctx) { return ((Ctx*)ctx)->num_cu; }
 int bh_ctx_p(void* ctx) { return ((Ctx*)ctx)->tune.p; }
 const SysDev* bh_ctx_sys(void* ctx) { return ((Ctx*)ctx)->sys; }

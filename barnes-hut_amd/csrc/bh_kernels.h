@@ -9,7 +9,8 @@
 #define PLACE_SMALL 262144
 #define HIST_BINS 8192     // LDS histogram window (keys) per block
 #define SCAN_TILE 2048     // elements per block in the scans
-#define SCAN_ONE 8192      // elements that one block scans in one launch
+#define SCAN_ONE 16384     // elements that one block scans in one launch
+#define PLACE_CELLS 8192   // cells of a system that one block places (k_place_one)
 #define PLACE_ONE 4096     // rows of a system that one block places (k_place_one)
 #define SORT_WAYS 16       // runs that a merge pass joins
 #define ITEMS_COLS 1024    // columns whose items a block of k_com_items builds
@@ -436,10 +437,9 @@ __global__ void k_force_combine(const Item* items, const int32_t* order, const i
                                 int64_t part_n, double* ax, double* ay);
 // FP64 recompute of the particles whose FP32 rounding-error estimate is
 // large against their acceleration
-__global__ void k_rc_blocks(const SysDev* sys, int S, int64_t nblocks, const double* com_dense,
-                            double* blk);
-__global__ void k_rc_tiles(const SysDev* sys, int S, int64_t ntiles, const double* com_dense,
-                           double* tl);
+__global__ void k_rc_sums(const SysDev* sys, int S, int64_t nblocks, int64_t ntiles, int nb,
+                          const double* com_dense, double* blk, double* tl, int32_t* rc_cnt,
+                          int32_t* stats);
 __global__ void k_rc_blockfar(const SysDev* sys, int S, int64_t nblocks, const double* blk,
                               double* bfar);
 template <int W>

@@ -502,56 +502,107 @@ __global__ __launch_bounds__(256) void k_scan_final(const int32_t* __restrict__ 
     }
 }
 
+// Exclusive scan of n <= 1024 R counts and of their non-empty flags by one block:
+// get(i) gives count i, put(i, count, before, non-empty before) takes its place.
+// A wave's elements are R rows of 64, so that both ends are contiguous across the
+// lanes.  Returns the totals and the largest count.
+struct ScanTotals {
+    int v, f, mx;
+};
+
+template <int R, typename Get, typename Put>
+__device__ __forceinline__ ScanTotals scan_block(int n, int* sh /* 48 ints */, Get&& get, Put&& put)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, base = w * (64 * R) + lane;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int cv[R], inc[R], v = 0, f = 0, mx = 0;
+    unsigned long long ne[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) cv[r] = base + 64 * r < n ? get(base + 64 * r) : 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        inc[r] = cv[r];
+        mx = max(mx, cv[r]);
+        ne[r] = __ballot(cv[r] > 0);
+        f += __popcll(ne[r]);
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int a = __shfl_up(inc[r], o, BH_WAVE);
+            if (lane >= o) inc[r] += a;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) v += __builtin_amdgcn_readlane(inc[r], 63);
+    mx = wave_max(mx);
+    if (lane == 0) {
+        sh[w] = v;
+        sh[16 + w] = f;
+        sh[32 + w] = mx;
+    }
+    __syncthreads();
+    ScanTotals t = {0, 0, 0};
+    int av = 0, af = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (k == w) {
+            av = t.v;
+            af = t.f;
+        }
+        t.v += sh[k];
+        t.f += sh[16 + k];
+        t.mx = max(t.mx, sh[32 + k]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = base + 64 * r;
+        if (i < n) put(i, cv[r], av + inc[r] - cv[r], af + __popcll(ne[r] & below));
+        av += __builtin_amdgcn_readlane(inc[r], 63);
+        af += __popcll(ne[r]);
+    }
+    return t;
+}
+
+// scan_block with as few rows as hold n.
+template <int RMAX, typename Get, typename Put>
+__device__ __forceinline__ ScanTotals scan_fit(int n, int* sh, Get&& get, Put&& put)
+{
+    if (n <= 1024) return scan_block<1>(n, sh, get, put);
+    if (n <= 4096) return scan_block<4>(n, sh, get, put);
+    return scan_block<RMAX>(n, sh, get, put);
+}
+
 // The three phases in one block, for n <= SCAN_ONE (three launches cost more
-// than the scan).  max_total >= 0: the total is kept within it, BH_ERR_ITEMS
-// raised beyond.
+// than the scan: 13,603 cells 16 us, in one block 13.5; 1,024 cells 3.0).  max_total >= 0: the total is kept within it,
+// BH_ERR_ITEMS raised beyond.
 template <bool CNT>
 __global__ __launch_bounds__(1024) void k_scan_one(const int32_t* __restrict__ in, int n,
                                                    int32_t* out_v, int32_t* out_f, int32_t* ne_list,
-                                                   double* com_dense, int32_t* stats, int total_slot,
-                                                   int64_t max_total)
+                                                   double* com_dense, int32_t* stats,
+                                                   int total_slot, int64_t max_total)
 {
-    __shared__ int sh[40];
-    constexpr int R = SCAN_ONE / 1024;
-    const int base = threadIdx.x * R;
-    int cv[R];
-    int v = 0, f = 0, mx = 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int i = base + r;
-        cv[r] = i < n ? in[i] : 0;
-        v += cv[r];
-        f += cv[r] > 0;
-        mx = max(mx, cv[r]);
-    }
-    int av, af, tv, tf;
-    block_excl_scan2(v, f, av, af, tv, tf, sh);
-    if (CNT) {
-        mx = wave_max(mx);
-        if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&stats[ST_MAXCOUNT], mx);
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int i = base + r;
-        if (i < n) {
+    __shared__ int sh[48];
+    const ScanTotals t = scan_fit<SCAN_ONE / 1024>(
+        n, sh, [&](int i) { return in[i]; },
+        [&](int i, int c, int av, int af) {
             out_v[i] = av;
             if (CNT) {
                 out_f[i] = af;
-                if (cv[r] > 0) ne_list[af] = i;
+                if (c > 0) ne_list[af] = i;
             }
-            av += cv[r];
-            af += cv[r] > 0;
-        }
-    }
+        });
     if (threadIdx.x == 0) {
-        out_v[n] = tv;
+        out_v[n] = t.v;
         if (CNT) {
-            out_f[n] = tf;
-            stats[ST_NCELLS_NE] = tf;
+            out_f[n] = t.f;
+            stats[ST_NCELLS_NE] = t.f;
+            if (t.mx > 0) atomicMax(&stats[ST_MAXCOUNT], t.mx);
         }
         if (total_slot >= 0) {
-            const bool over = max_total >= 0 && tv > max_total;
-            stats[total_slot] = over ? (int32_t)max_total : tv;
+            const bool over = max_total >= 0 && t.v > max_total;
+            stats[total_slot] = over ? (int32_t)max_total : t.v;
             if (over) atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
         }
     }
@@ -628,8 +679,8 @@ template __global__ void k_scatter<8>(const int32_t*, int64_t, const int32_t*, c
 
 // ---------------------------------------------------------------- small systems
 // Box, keys, counts, scan and scatter of one system of at most PLACE_ONE rows and
-// SCAN_ONE cells in one block: five launches of 2 to 5 us each otherwise, most of
-// it latency.  2,000 particles on 11^2 cells: 10 us instead of 16; 16,384 on 32^2
+// PLACE_CELLS cells in one block: five launches of 2 to 5 us each otherwise, most of
+// it latency.  2,000 particles on 11^2 cells: 9.6 us instead of 16; 16,384 on 32^2
 // would take 32 instead of 20.
 __global__ __launch_bounds__(1024) void k_place_one(
     const double* __restrict__ px, const double* __restrict__ py, SysDev* sys, int N, int C,
@@ -638,10 +689,10 @@ __global__ __launch_bounds__(1024) void k_place_one(
     double* __restrict__ com_dense, int32_t* __restrict__ idx_out, int32_t* __restrict__ key_sorted,
     uint64_t* __restrict__ pxkey, uint64_t* __restrict__ pykey, int32_t* __restrict__ stats)
 {
-    constexpr int RP = PLACE_ONE / 1024, RC = SCAN_ONE / 1024;
-    __shared__ int32_t cell[SCAN_ONE];   // counts, then offsets
+    constexpr int RP = PLACE_ONE / 1024;
+    __shared__ int32_t cell[PLACE_CELLS];   // counts, then offsets
     __shared__ double red[4][16];
-    __shared__ int sh[40], err, mxc[16];
+    __shared__ int sh[48], err;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const double inf = __longlong_as_double(0x7ff0000000000000ll);
     double x[RP], y[RP], mnx = inf, mny = inf, mxx = -inf, mxy = -inf;
@@ -698,45 +749,27 @@ __global__ __launch_bounds__(1024) void k_place_one(
     }
     __syncthreads();
     if (tid == 0 && !store_box(sys[0], d)) atomicOr(&err, BH_ERR_DEGENERATE);
-    int cv[RC], v = 0, f = 0, mx = 0;
-#pragma unroll
-    for (int r = 0; r < RC; ++r) {
-        const int i = tid * RC + r;
-        cv[r] = i < C ? cell[i] : 0;
-        v += cv[r];
-        f += cv[r] > 0;
-        mx = max(mx, cv[r]);
-    }
-    mx = wave_max(mx);
-    if (lane == 0) mxc[w] = mx;
-    int av, af, tv, tf;
-    block_excl_scan2(v, f, av, af, tv, tf, sh);
-#pragma unroll
-    for (int r = 0; r < RC; ++r) {
-        const int i = tid * RC + r;
-        if (i < C) {
-            counts[i] = cv[r];
+    const ScanTotals t = scan_fit<PLACE_CELLS / 1024>(
+        C, sh, [&](int i) { return cell[i]; },
+        [&](int i, int c, int av, int af) {
+            counts[i] = c;
             offsets[i] = av;
             neprefix[i] = af;
             cell[i] = av;
-            if (cv[r] > 0) ne_list[af] = i;
-            av += cv[r];
-            af += cv[r] > 0;
-        }
-    }
+            if (c > 0) ne_list[af] = i;
+        });
     clear_com(com_dense, 0, C, 1024);
     __syncthreads();
     if (tid < ST_COUNT) {
         int st = 0;
         if (tid == ST_ERR) st = err;
-        if (tid == ST_NCELLS_NE) st = tf;
-        if (tid == ST_MAXCOUNT)
-            for (int k = 0; k < 16; ++k) st = max(st, mxc[k]);
+        if (tid == ST_NCELLS_NE) st = t.f;
+        if (tid == ST_MAXCOUNT) st = t.mx;
         stats[tid] = st;
     }
     if (tid == 0) {
-        offsets[C] = tv;
-        neprefix[C] = tf;
+        offsets[C] = t.v;
+        neprefix[C] = t.f;
     }
 #pragma unroll
     for (int r = 0; r < RP; ++r) {

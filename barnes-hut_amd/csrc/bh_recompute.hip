@@ -46,13 +46,12 @@
 
 // Sum of M^2 over each RC_BLOCK x RC_BLOCK block of cells (one wave per block;
 // fixed summation order, so the bound is the same on every run).
-__global__ __launch_bounds__(64) void k_rc_blocks(const SysDev* __restrict__ sys, int S,
-                                                  int64_t nblocks,
-                                                  const double* __restrict__ com_dense,
-                                                  double* __restrict__ blk)
+__device__ __forceinline__ void rc_blocks(const SysDev* __restrict__ sys, int S, int64_t nblocks,
+                                          const double* __restrict__ com_dense,
+                                          double* __restrict__ blk, int blk0, int nblk)
 {
-    const int lane = threadIdx.x;
-    for (int64_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const int lane = threadIdx.x & (BH_WAVE - 1);
+    for (int64_t b = (int64_t)blk0 * 4 + threadIdx.x / BH_WAVE; b < nblocks; b += (int64_t)nblk * 4) {
         int lo = 0, hi = S - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -79,14 +78,13 @@ __global__ __launch_bounds__(64) void k_rc_blocks(const SysDev* __restrict__ sys
 // Sum of M^2 over each RC_TILE x RC_TILE tile of cells (one thread per tile,
 // fixed order); system s's tiles start at b_off * (RC_BLOCK / RC_TILE)^2, in
 // a Gb * RC_BLOCK / RC_TILE square.
-__global__ __launch_bounds__(256) void k_rc_tiles(const SysDev* __restrict__ sys, int S,
-                                                  int64_t ntiles,
-                                                  const double* __restrict__ com_dense,
-                                                  double* __restrict__ tl)
+__device__ __forceinline__ void rc_tiles(const SysDev* __restrict__ sys, int S, int64_t ntiles,
+                                         const double* __restrict__ com_dense,
+                                         double* __restrict__ tl, int blk0, int nblk)
 {
     constexpr int TPB = RC_BLOCK / RC_TILE;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < ntiles; q += stride) {
+    const int64_t stride = (int64_t)nblk * 256;
+    for (int64_t q = (int64_t)blk0 * 256 + threadIdx.x; q < ntiles; q += stride) {
         int lo = 0, hi = S - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -109,6 +107,23 @@ __global__ __launch_bounds__(256) void k_rc_tiles(const SysDev* __restrict__ sys
         }
         tl[q] = acc;
     }
+}
+
+// What the flags need of the cells, in one launch: the first nb workgroups take
+// the blocks, the others the tiles; the first also clears the counts.
+__global__ __launch_bounds__(256) void k_rc_sums(const SysDev* __restrict__ sys, int S,
+                                                 int64_t nblocks, int64_t ntiles, int nb,
+                                                 const double* __restrict__ com_dense,
+                                                 double* __restrict__ blk, double* __restrict__ tl,
+                                                 int32_t* __restrict__ rc_cnt,
+                                                 int32_t* __restrict__ stats)
+{
+    if (blockIdx.x == 0) {
+        for (int s = threadIdx.x; s < S; s += 256) rc_cnt[s] = 0;
+        if (threadIdx.x < 2) stats[ST_NRECOMP + threadIdx.x] = 0;
+    }
+    if ((int)blockIdx.x < nb) rc_blocks(sys, S, nblocks, com_dense, blk, blockIdx.x, nb);
+    else rc_tiles(sys, S, ntiles, com_dense, tl, blockIdx.x - nb, gridDim.x - nb);
 }
 
 // Per block b: sum over the blocks outside b's 3 x 3 block neighbourhood of

@@ -221,3 +221,31 @@ def test_steps_equal_their_phases(sizes, grids):
         eng.close()
     for k, v in runs[0].items():
         np.testing.assert_array_equal(v, runs[1][k])
+
+
+@pytest.mark.parametrize("n,G", [(500, 5), (524000, 3), (524800, 3)])
+def test_cost_order_of_few_and_many_items(n, G):
+    """Orders of up to 8,192 items (one block) and of more: a permutation by
+    falling cost, to within a bin of the range; the static order if a cost is
+    not finite."""
+    import torch
+    from barneshut.engine import Engine
+    eng = Engine([n], [G], tuning=dict(p=1, yspan=512, waves_per_cu=8, tail_split=1, tail_items=0))
+    eng.load(inputs.uniform(n, seed=75))
+    eng.create_tree()
+    eng.ctx.build_items()
+    items = int(eng.check()[2])
+    cap = eng.ctx.query(4)
+    cost = np.random.default_rng(n).normal(size=cap).astype(np.float32)
+    cost[:items][:: max(items // 50, 1)] = 0.25   # ties
+    order = torch.full((cap,), -1, dtype=torch.int32, device="cuda")
+    eng.ctx.order_by_cost(torch.as_tensor(cost, device="cuda"), order)
+    o = order.cpu().numpy()
+    np.testing.assert_array_equal(np.sort(o[:items]), np.arange(items))
+    assert (o[items:] == -1).all()
+    c = cost[:items][o[:items]]
+    assert (np.diff(c) <= np.ptp(cost[:items]) / 4095 * 1.001).all()
+    cost[items // 2] = np.nan
+    eng.ctx.order_by_cost(torch.as_tensor(cost, device="cuda"), order)
+    np.testing.assert_array_equal(order.cpu().numpy()[:items], np.arange(items))
+    eng.close()
