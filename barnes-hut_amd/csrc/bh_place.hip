@@ -46,16 +46,18 @@ __global__ __launch_bounds__(256) void k_place_init(int32_t* stats, int32_t* cou
 // Atomic min/max of the ordered keys; skipped when the stored value already
 // bounds ours (stored minima only fall and maxima only rise, so a stale read
 // can only cause an unneeded atomic, never a missed one).
+// By lanes 0 to 3, an extreme each: one after the other they made k_bbox 6.8 instead
+// of 5.2 us on 16,384 particles, 11 instead of 6.5 us on 40 systems.
 __device__ __forceinline__ void bbox_flush(uint64_t* bb, int s, double mnx, double mny, double mxx,
                                            double mxy)
 {
-    unsigned long long* b = (unsigned long long*)&bb[4 * s];
-    const unsigned long long k0 = bh_ord_key(mnx), k1 = bh_ord_key(mny);
-    const unsigned long long k2 = bh_ord_key(mxx), k3 = bh_ord_key(mxy);
-    if (k0 < __atomic_load_n(&b[0], __ATOMIC_RELAXED)) atomicMin(&b[0], k0);
-    if (k1 < __atomic_load_n(&b[1], __ATOMIC_RELAXED)) atomicMin(&b[1], k1);
-    if (k2 > __atomic_load_n(&b[2], __ATOMIC_RELAXED)) atomicMax(&b[2], k2);
-    if (k3 > __atomic_load_n(&b[3], __ATOMIC_RELAXED)) atomicMax(&b[3], k3);
+    const int k = threadIdx.x & 63;
+    if (k >= 4) return;
+    unsigned long long* b = (unsigned long long*)&bb[4 * s + k];
+    const unsigned long long key = bh_ord_key(k == 0 ? mnx : k == 1 ? mny : k == 2 ? mxx : mxy);
+    const unsigned long long had = __atomic_load_n(b, __ATOMIC_RELAXED);
+    if (k < 2 && key < had) atomicMin(b, key);
+    if (k >= 2 && key > had) atomicMax(b, key);
 }
 
 // Each wave covers `rounds` runs of 64 R consecutive particles, all of a run's
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
     auto flush = [&]() {
         if (cur < 0) return;
         reduce();
-        if (lane == 0) bbox_flush(bb, cur, mnx, mny, mxx, mxy);
+        bbox_flush(bb, cur, mnx, mny, mxx, mxy);
         mnx = inf; mny = inf; mxx = -inf; mxy = -inf;
     };
     // a wave's rows: `rounds` runs of 64 R, one after the other
@@ -135,17 +137,16 @@ __global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ px,
     }
     if (__any(bad) && lane == 0) atomicOr(&stats[ST_ERR], BH_ERR_NONFINITE);
     __syncthreads();
-    if (threadIdx.x == 0) {   // waves of one system meet here
-        for (int v = 0; v < 4; ++v) {
-            if (wsys[v] < 0) continue;
-            if (v + 1 < 4 && wsys[v + 1] == wsys[v]) {
-                red[v + 1][0] = fmin(red[v + 1][0], red[v][0]);
-                red[v + 1][1] = fmin(red[v + 1][1], red[v][1]);
-                red[v + 1][2] = fmax(red[v + 1][2], red[v][2]);
-                red[v + 1][3] = fmax(red[v + 1][3], red[v][3]);
-            } else {
-                bbox_flush(bb, wsys[v], red[v][0], red[v][1], red[v][2], red[v][3]);
-            }
+    if (wid > 0) return;
+    for (int v = 0; v < 4; ++v) {   // waves of one system meet here
+        if (wsys[v] < 0) continue;
+        if (v + 1 < 4 && wsys[v + 1] == wsys[v]) {
+            if (lane < 4)
+                red[v + 1][lane] = lane < 2 ? fmin(red[v + 1][lane], red[v][lane])
+                                            : fmax(red[v + 1][lane], red[v][lane]);
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            bbox_flush(bb, wsys[v], red[v][0], red[v][1], red[v][2], red[v][3]);
         }
     }
 }
