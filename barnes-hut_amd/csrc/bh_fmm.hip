@@ -123,44 +123,103 @@ __global__ __launch_bounds__(256) void k_fmm_tiles(FmmArgs A)
     }
 }
 
+// ---------------------------------------------------------------- small products
+#define FMM_THREADS 128   // of the kernels that take a square per block
+
+// For NF pairs A_z (M x K, at A + z az) and B_z (K x N, at B + z bz), row-major in
+// LDS on 16 bytes: C_z[m][n] = sum_k A_z[m][k] B_z[k][n], handed to put(z, m, n, C)
+// in pieces of 2 x NB.  A thread's piece takes 6 bytes of LDS reads a multiply-add
+// (16 with an element per thread); these reads bound the kernels below.  One
+// element per thread, 256 threads: 4.2M FP64 particles on 1024^2 cells p2m 181, m2m
+// 5 x 24.7, l2l 6 x 39 us; in pieces 129, 5 x 23 and 6 x 22.  512 systems: 413, 3 x
+// 60, 4 x 80; 382, 3 x 64 and 4 x 55.
+template <int N>
+constexpr int piece() { return N % 4 == 0 ? 4 : 2; }
+
+template <int M, int N, int K, int NF, int TH = FMM_THREADS, typename Put>
+__device__ __forceinline__ void products(const double* A, int az, const double* B, int bz,
+                                         Put&& put)
+{
+    constexpr int NB = piece<N>(), PM = M / 2, PN = N / NB;
+    static_assert(M % 2 == 0 && N % NB == 0 && K % 2 == 0, "whole pieces");
+    for (int u = threadIdx.x; u < NF * PM * PN; u += TH) {
+        const int z = u / (PM * PN), r = u - z * (PM * PN);
+        const int m = 2 * (r / PN), n = NB * (r % PN);
+        const double *a = A + z * az + m * K, *b = B + z * bz + n;
+        double c[2][NB] = {};
+#pragma unroll
+        for (int k = 0; k < K; k += 2) {
+            const double2 a0 = *(const double2*)(a + k);
+            const double2 a1 = *(const double2*)(a + K + k);
+#pragma unroll
+            for (int v = 0; v < NB; v += 2) {
+                const double2 b0 = *(const double2*)(b + k * N + v);
+                const double2 b1 = *(const double2*)(b + (k + 1) * N + v);
+                c[0][v] = fma(a0.y, b1.x, fma(a0.x, b0.x, c[0][v]));
+                c[0][v + 1] = fma(a0.y, b1.y, fma(a0.x, b0.y, c[0][v + 1]));
+                c[1][v] = fma(a1.y, b1.x, fma(a1.x, b0.x, c[1][v]));
+                c[1][v + 1] = fma(a1.y, b1.y, fma(a1.x, b0.y, c[1][v + 1]));
+            }
+        }
+        put(z, m, n, c);
+    }
+}
+
+// A piece into a row-major N-wide matrix in LDS.
+template <int N, int NB>
+__device__ __forceinline__ void put_lds(double* D, int m, int n, const double (&c)[2][NB])
+{
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int v = 0; v < NB; ++v) D[(m + w) * N + n + v] = c[w][v];
+}
+
+// An R x C table from global memory, and its transpose.
+template <int R, int C, int TH = FMM_THREADS>
+__device__ __forceinline__ void load_table(const double* __restrict__ g, double* t, double* tt)
+{
+    for (int q = threadIdx.x; q < R * C; q += TH) {
+        const double v = g[q];
+        if (t) t[q] = v;
+        if (tt) tt[(q % C) * R + q / C] = v;
+    }
+}
+
 // ---------------------------------------------------------------- sources up
 // A square's node masses C (P^2, in LDS) anterpolated to its F x F coarser nodes
-// (fine[I][i]: the coarse cardinal I at node i); V: scratch for F P.  By the
-// whole block.
-template <int P, int F>
-__device__ __forceinline__ void coarse_masses(const double* C, double* V,
-                                              const double* __restrict__ fine, double* M,
-                                              int64_t plane)
+// (fine[I][i]: the coarse cardinal I at node i; fineT its transpose); V: scratch
+// for F P.  By the whole block.
+template <int P, int F, int TH = FMM_THREADS>
+__device__ __forceinline__ void coarse_masses(const double* C, double* V, const double* fine,
+                                              const double* fineT, double* M, int64_t plane)
 {
-    const int tid = threadIdx.x;
     __syncthreads();
-    for (int q = tid; q < F * P; q += 256) {   // V[I][j] = sum_i fine[I][i] C[i][j]
-        const int I = q / P, j = q - I * P;
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < P; ++i) s = fma(fine[I * P + i], C[i * P + j], s);
-        V[q] = s;
-    }
+    products<F, P, P, 1, TH>(fine, 0, C, 0, [&](int, int m, int n, const auto& c) {
+        put_lds<P>(V, m, n, c);
+    });
     __syncthreads();
-    for (int q = tid; q < F * F; q += 256) {
-        const int I = q / F, J = q - I * F;
-        double s = 0.0;
+    products<F, F, P, 1, TH>(V, 0, fineT, 0, [&](int, int m, int n, const auto& c) {
 #pragma unroll
-        for (int j = 0; j < P; ++j) s = fma(V[I * P + j], fine[J * P + j], s);
-        M[q * plane] = s;
-    }
+        for (int w = 0; w < 2; ++w)
+#pragma unroll
+            for (int v = 0; v < piece<F>(); ++v) M[((m + w) * F + n + v) * plane] = c[w][v];
+    });
 }
 
 // One block per tile: the tile's COMs into the tile-ordered list, and their
 // masses anterpolated to the tile's nodes: Chebyshev moments
 // W_kl = sum M T_k(x) T_l(y) over the entries, then nodes = C^T W C.
 template <int P>
-__global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __restrict__ ctab,
-                                                 const double* __restrict__ fine)
+__global__ __launch_bounds__(FMM_THREADS) void k_fmm_p2m(FmmArgs A,
+                                                         const double* __restrict__ ctab,
+                                                         const double* __restrict__ ftab)
 {
-    constexpr int Q = P * P, F = fmm_far(P);
-    constexpr int PER = (Q + 255) / 256;
-    __shared__ double tx[32][P], ty[32][P], mm[32], W[Q], V[Q], ct[Q];
+    constexpr int Q = P * P, F = fmm_far(P), EB = 32, NB = piece<P>();
+    // tx, ty: T_k of the entries; afterwards scratch and the coarser nodes' tables
+    __shared__ alignas(16) double tx[P * EB], ty[EB * P], W[Q], ct[Q], ctT[Q];
+    static_assert(Q <= P * EB && 2 * F * P <= P * EB, "room in tx and ty");
+    double *V = tx, *fine = ty, *fineT = ty + F * P;
     const int tid = threadIdx.x;
     const int64_t t = blockIdx.x;
     const FmmTile tl = A.tiles[t];
@@ -172,21 +231,25 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
     const double sig = step_scale(d.step);
     double *M = nullptr, *MF = nullptr;   // node q's mass goes to M[q * plane]
     int64_t plane = 0;
-    if (fs.nlev > 0) {
+    const bool up = fs.nlev > 0;
+    if (up) {
         plane = fmm_plane(fs.n[0]);
         M = A.mult + fs.moff[0] * Q + fmm_slot(fs.n[0], tl.tx, tl.ty);
         MF = A.multf + fs.moff[0] * (F * F) + fmm_slot(fs.n[0], tl.tx, tl.ty);
+        if (ne > 0) load_table<P, P>(ctab, ct, ctT);
     }
-    const bool up = fs.nlev > 0;
-    for (int i = tid; i < Q; i += 256) ct[i] = ctab[i];
-    double acc[PER] = {};
     const double h = (double)T * d.step;
+    // a thread's piece of the moments, over all entries
+    constexpr int PN = P / NB;
+    const int pm = 2 * (tid / PN), pn = NB * (tid % PN);
+    double acc[2][NB] = {};
     int cx = x0, cb = A.neprefix[d.c_off + (int64_t)x0 * d.G + y0];
     int cn = A.neprefix[d.c_off + (int64_t)x0 * d.G + y1] - cb, cpre = 0;
-    for (int b = 0; b < ne; b += 32) {
-        const int nb = min(32, ne - b);
-        if (tid < nb) {
-            const int r = b + tid;   // entry rank in the tile, columns in order
+    for (int b = 0; b < ne; b += EB) {
+        const int nb = min(EB, ne - b);
+        const int el = tid & (EB - 1);   // threads 0 .. 31 take x, 32 .. 63 y
+        if (tid < 2 * EB && el < nb) {
+            const int r = b + el;   // entry rank in the tile, columns in order
             while (r - cpre >= cn && cx + 1 < x1) {
                 cpre += cn;
                 ++cx;
@@ -195,46 +258,56 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
                 cn = A.neprefix[cl + y1] - cb;
             }
             const Com64 c = A.l64[cb + (r - cpre)];
-            FmmCom f;
-            f.X = c.X * sig;
-            f.Y = c.Y * sig;
-            f.M = c.M;
-            f.kx = c.kx;
-            f.ky = c.ky;
-            if (c.M == 0.0) {   // no COM: any point of the cell, at weight 0
-                f.X = fma((double)c.kx + 0.5, d.step, d.min_x) * sig;
-                f.Y = fma((double)c.ky + 0.5, d.step, d.min_y) * sig;
-            }
-            A.list[e0 + r] = f;
-            if (up) {
-                const double ux = 2.0 * ((c.X - d.min_x) / h - tl.tx) - 1.0;
-                const double uy = 2.0 * ((c.Y - d.min_y) / h - tl.ty) - 1.0;
+            const double ux = 2.0 * ((c.X - d.min_x) / h - tl.tx) - 1.0;
+            const double uy = 2.0 * ((c.Y - d.min_y) / h - tl.ty) - 1.0;
+            if (tid < EB) {
+                FmmCom f;
+                f.X = c.X * sig;
+                f.Y = c.Y * sig;
+                f.M = c.M;
+                f.kx = c.kx;
+                f.ky = c.ky;
+                if (c.M == 0.0) {   // no COM: any point of the cell, at weight 0
+                    f.X = fma((double)c.kx + 0.5, d.step, d.min_x) * sig;
+                    f.Y = fma((double)c.ky + 0.5, d.step, d.min_y) * sig;
+                }
+                A.list[e0 + r] = f;
                 // masses of both signs can put a COM outside its cell, where
                 // the interpolation does not hold: that system goes term by term
-                if (c.M != 0.0 && !(fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN)) A.sbad[tl.sys] = 1;
-                mm[tid] = c.M;
-                double a0 = 1.0, a1 = ux, b0 = 1.0, b1 = uy;
-                if (c.M == 0.0) a0 = a1 = b0 = b1 = 0.0;
+                if (up && c.M != 0.0 && !(fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN))
+                    A.sbad[tl.sys] = 1;
+            }
+            // T_k(x) M and T_k(y)
+            const double u = tid < EB ? ux : uy;
+            double t0 = tid < EB ? c.M : 1.0, t1 = t0 * u;
+            if (c.M == 0.0) t0 = t1 = 0.0;
+            double* dst = tid < EB ? tx + el : ty + el * P;
+            const int step = tid < EB ? EB : 1;
 #pragma unroll
-                for (int k = 0; k < P; ++k) {
-                    tx[tid][k] = a0;
-                    ty[tid][k] = b0;
-                    const double an = fma(2.0 * ux, a1, -a0), bn = fma(2.0 * uy, b1, -b0);
-                    a0 = a1;
-                    a1 = c.M == 0.0 ? 0.0 : an;
-                    b0 = b1;
-                    b1 = c.M == 0.0 ? 0.0 : bn;
-                }
+            for (int k = 0; k < P; ++k) {
+                dst[k * step] = t0;
+                const double tn = fma(2.0 * u, t1, -t0);
+                t0 = t1;
+                t1 = c.M == 0.0 ? 0.0 : tn;
+            }
+        } else if (tid < 2 * EB && el == nb) {   // past an odd last entry: nothing
+            for (int k = 0; k < P; ++k) {
+                if (tid < EB) tx[k * EB + el] = 0.0;
+                else ty[el * P + k] = 0.0;
             }
         }
+        if (!up) continue;
         __syncthreads();
-        if (up) {
+        if (pm < P) {
+#pragma unroll 4
+            for (int e = 0; e < nb; e += 2) {
+                const double2 a0 = *(const double2*)(tx + pm * EB + e);
+                const double2 a1 = *(const double2*)(tx + (pm + 1) * EB + e);
 #pragma unroll
-            for (int p = 0; p < PER; ++p) {
-                const int q = tid + 256 * p;
-                if (q < Q) {
-                    const int k = q / P, l = q - (q / P) * P;
-                    for (int e = 0; e < nb; ++e) acc[p] = fma(mm[e] * tx[e][k], ty[e][l], acc[p]);
+                for (int v = 0; v < NB; ++v) {
+                    const double b0 = ty[e * P + pn + v], b1 = ty[(e + 1) * P + pn + v];
+                    acc[0][v] = fma(a0.y, b1, fma(a0.x, b0, acc[0][v]));
+                    acc[1][v] = fma(a1.y, b1, fma(a1.x, b0, acc[1][v]));
                 }
             }
         }
@@ -251,95 +324,91 @@ __global__ __launch_bounds__(256) void k_fmm_p2m(FmmArgs A, const double* __rest
     }
     if (!up) return;
     if (ne == 0) {   // uniform over the block
-        for (int q = tid; q < Q; q += 256) M[q * plane] = 0.0;
-        for (int q = tid; q < F * F; q += 256) MF[q * plane] = 0.0;
+        for (int q = tid; q < Q; q += FMM_THREADS) M[q * plane] = 0.0;
+        for (int q = tid; q < F * F; q += FMM_THREADS) MF[q * plane] = 0.0;
         return;
     }
-#pragma unroll
-    for (int p = 0; p < PER; ++p)
-        if (tid + 256 * p < Q) W[tid + 256 * p] = acc[p];
+    if (pm < P) put_lds<P>(W, pm, pn, acc);
+    load_table<F, P>(ftab, fine, fineT);
     __syncthreads();
-    for (int q = tid; q < Q; q += 256) {   // V[i][l] = sum_k ct[k][i] W[k][l]
-        const int i = q / P, l = q - i * P;
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < P; ++k) s = fma(ct[k * P + i], W[k * P + l], s);
-        V[q] = s;
-    }
+    products<P, P, P, 1>(ctT, 0, W, 0, [&](int, int m, int n, const auto& c) {
+        put_lds<P>(V, m, n, c);
+    });
     __syncthreads();
-    for (int q = tid; q < Q; q += 256) {
-        const int i = q / P, j = q - i * P;
-        double s = 0.0;
+    products<P, P, P, 1>(V, 0, ct, 0, [&](int, int m, int n, const auto& c) {
+        put_lds<P>(W, m, n, c);
 #pragma unroll
-        for (int l = 0; l < P; ++l) s = fma(V[i * P + l], ct[l * P + j], s);
-        M[q * plane] = s;
-        W[q] = s;
-    }
-    coarse_masses<P, F>(W, V, fine, MF, plane);
+        for (int w = 0; w < 2; ++w)
+#pragma unroll
+            for (int v = 0; v < NB; ++v) M[((m + w) * P + n + v) * plane] = c[w][v];
+    });
+    coarse_masses<P, F>(W, V, fine, fineT, MF, plane);
 }
 
 // One block per square of level lev: its children's node masses anterpolated
-// to its own nodes (shift[a][i][I]: the parent's cardinal i at child node I).
+// to its own nodes (shift[a][i][I]: the parent's cardinal i at child node I).  The
+// four children are read and taken through the first product together: the few
+// squares of the upper levels are a chain of latencies.
 template <int P>
 __global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __restrict__ shift,
-                                                 const double* __restrict__ fine, int lev)
+                                                 const double* __restrict__ ftab, int lev)
 {
-    constexpr int Q = P * P, F = fmm_far(P);
-    constexpr int PER = (Q + 255) / 256;
-    __shared__ double S[2 * Q], C[Q], V[Q];
+    constexpr int Q = P * P, F = fmm_far(P), TH = 256;
+    __shared__ alignas(16) double S[2 * Q], ST[2 * Q], C[4 * Q], V[4 * Q];
     const int tid = threadIdx.x;
     const int64_t t = A.lev_off[lev] + blockIdx.x;
     const FmmTile tl = A.tiles[t];
     const FmmSys& fs = A.fsys[tl.sys];
     const int nc = fs.n[lev - 1];
     const int64_t cplane = fmm_plane(nc), plane = fmm_plane(fs.n[lev]);
-    for (int i = tid; i < 2 * Q; i += 256) S[i] = shift[i];
-    double acc[PER] = {};
     int np = 0;
+    bool has[4];
+#pragma unroll
     for (int ch = 0; ch < 4; ++ch) {
-        const int a = ch >> 1, b = ch & 1;
-        const int cx = 2 * tl.tx + a, cy = 2 * tl.ty + b;
-        if (cx >= nc || cy >= nc) continue;
-        const int64_t c = fs.off[lev - 1] + (int64_t)cx * nc + cy;
-        const int n = A.tcnt[c];
-        if (n == 0) continue;
+        const int cx = 2 * tl.tx + (ch >> 1), cy = 2 * tl.ty + (ch & 1);
+        int n = 0;
+        if (cx < nc && cy < nc) n = A.tcnt[fs.off[lev - 1] + (int64_t)cx * nc + cy];
+        has[ch] = n != 0;
         np += n;
-        __syncthreads();
-        const double* src = A.mult + fs.moff[lev - 1] * Q + fmm_slot(nc, cx, cy);
-        for (int q = tid; q < Q; q += 256) C[q] = src[q * cplane];
-        __syncthreads();
-        for (int q = tid; q < Q; q += 256) {
-            const int i = q / P, J = q - i * P;
-            double s = 0.0;
-#pragma unroll
-            for (int I = 0; I < P; ++I) s = fma(S[a * Q + i * P + I], C[I * P + J], s);
-            V[q] = s;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int q = tid + 256 * p;
-            if (q < Q) {
-                const int i = q / P, j = q - (q / P) * P;
-                double s = acc[p];
-#pragma unroll
-                for (int J = 0; J < P; ++J) s = fma(V[i * P + J], S[b * Q + j * P + J], s);
-                acc[p] = s;
-            }
-        }
     }
     if (tid == 0) A.tcnt[t] = np;
     double* M = A.mult + fs.moff[lev] * Q + fmm_slot(fs.n[lev], tl.tx, tl.ty);
-    __syncthreads();
+    double* MF = A.multf + fs.moff[lev] * (F * F) + fmm_slot(fs.n[lev], tl.tx, tl.ty);
+    if (np == 0) {   // uniform over the block
+        for (int q = tid; q < Q; q += TH) M[q * plane] = 0.0;
+        for (int q = tid; q < F * F; q += TH) MF[q * plane] = 0.0;
+        return;
+    }
 #pragma unroll
-    for (int p = 0; p < PER; ++p)
-        if (tid + 256 * p < Q) {
-            M[(tid + 256 * p) * plane] = acc[p];
-            C[tid + 256 * p] = acc[p];
-        }
-    coarse_masses<P, F>(C, V, fine,
-                        A.multf + fs.moff[lev] * (F * F) + fmm_slot(fs.n[lev], tl.tx, tl.ty),
-                        plane);
+    for (int ch = 0; ch < 4; ++ch) {
+        const double* src = A.mult + fs.moff[lev - 1] * Q +
+                            fmm_slot(nc, 2 * tl.tx + (ch >> 1), 2 * tl.ty + (ch & 1));
+        for (int q = tid; q < Q; q += TH) C[ch * Q + q] = has[ch] ? src[q * cplane] : 0.0;
+    }
+    load_table<P, P, TH>(shift, S, ST);
+    load_table<P, P, TH>(shift + Q, S + Q, ST + Q);
+    __syncthreads();
+    auto in_V = [&](int c, int m, int n, const auto& v) { put_lds<P>(V + c * Q, m, n, v); };
+    products<P, P, P, 2, TH>(S, 0, C, Q, in_V);
+    products<P, P, P, 2, TH>(S + Q, 0, C + 2 * Q, Q, [&](int c, int m, int n, const auto& v) {
+        put_lds<P>(V + (c + 2) * Q, m, n, v);
+    });
+    __syncthreads();
+    // children (0, b) and (1, b) by the shift of b, then the four are added
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        products<P, P, P, 2, TH>(V + b * Q, 2 * Q, ST + b * Q, 0,
+                                 [&](int a, int m, int n, const auto& v) {
+                                     put_lds<P>(C + (2 * a + b) * Q, m, n, v);
+                                 });
+    __syncthreads();
+    for (int q = tid; q < Q; q += TH) {
+        const double s = ((C[q] + C[Q + q]) + C[2 * Q + q]) + C[3 * Q + q];
+        V[q] = s;
+        M[q * plane] = s;
+    }
+    load_table<F, P, TH>(ftab, S, S + Q);
+    coarse_masses<P, F, TH>(V, V + Q, S, S + Q, MF, plane);
 }
 
 // ---------------------------------------------------------------- node to node
@@ -518,16 +587,19 @@ __global__ __launch_bounds__(64, 3) void k_fmm_m2l(FmmArgs A, int ngroups,
 }
 
 // ---------------------------------------------------------------- field down
-// One block per square of level lev: adds the parent's field, interpolated at
-// the square's nodes; on tiles (lev 0) the sum becomes Chebyshev coefficients.
+// One block per square of level lev: adds the far offsets' field, from the coarser
+// nodes, and the parent's, interpolated at the square's nodes; on tiles (lev 0)
+// the sum becomes Chebyshev coefficients.
 template <int P>
-__global__ __launch_bounds__(256) void k_fmm_l2l(FmmArgs A, const double* __restrict__ shift,
-                                                 const double* __restrict__ ctab,
-                                                 const double* __restrict__ fine, int lev)
+__global__ __launch_bounds__(FMM_THREADS) void k_fmm_l2l(FmmArgs A,
+                                                         const double* __restrict__ shift,
+                                                         const double* __restrict__ ctab,
+                                                         const double* __restrict__ ftab, int lev)
 {
-    constexpr int Q = P * P, F = fmm_far(P), QF = F * F;
-    constexpr int PER = (2 * Q + 255) / 256;
-    __shared__ double S[2 * Q], C[2 * Q], V[2 * Q];
+    constexpr int Q = P * P, F = fmm_far(P), QF = F * F, NB = piece<P>();
+    constexpr int PM = P / 2, PN = P / NB;
+    static_assert(2 * PM * PN <= FMM_THREADS && F * P <= Q, "a piece per thread; room in S");
+    __shared__ alignas(16) double S[2 * Q], C[2 * Q], V[2 * Q];
     const int tid = threadIdx.x;
     const int64_t t = A.lev_off[lev] + blockIdx.x;
     if (A.tcnt[t] == 0) return;
@@ -536,88 +608,62 @@ __global__ __launch_bounds__(256) void k_fmm_l2l(FmmArgs A, const double* __rest
     if (fs.nlev <= lev) return;
     const bool par = lev + 1 < fs.nlev;
     double* L = A.loc + t * (int64_t)(2 * Q);
-    double acc[PER];
+    // this thread's piece of the field
+    const int z = tid / (PM * PN), r = tid - z * (PM * PN);
+    const int at = z * Q + 2 * (r / PN) * P + NB * (r % PN);
+    double acc[2][NB];
+    auto add = [&](int, int, int, const auto& c) {
 #pragma unroll
-    for (int p = 0; p < PER; ++p) acc[p] = tid + 256 * p < 2 * Q ? L[tid + 256 * p] : 0.0;
-    // the far offsets' field, from the coarser nodes
-    for (int q = tid; q < F * P; q += 256) S[q] = fine[q];
-    for (int q = tid; q < 2 * QF; q += 256) C[q] = A.locf[t * (2 * QF) + q];
+        for (int w = 0; w < 2; ++w)
+#pragma unroll
+            for (int v = 0; v < NB; ++v) acc[w][v] += c[w][v];
+    };
+    auto in_V = [&](int f, int m, int n, const auto& c) { put_lds<P>(V + f * Q, m, n, c); };
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int v = 0; v < NB; ++v) acc[w][v] = z < 2 ? L[at + w * P + v] : 0.0;
+    load_table<F, P>(ftab, S, S + Q);
+    for (int q = tid; q < 2 * QF; q += FMM_THREADS) C[q] = A.locf[t * (2 * QF) + q];
     __syncthreads();
-    for (int q = tid; q < 2 * P * F; q += 256) {   // V[i][J] = sum_I fine[I][i] C[I][J]
-        const int z = q >= P * F, r = q - z * P * F, i = r / F, J = r - i * F;
-        double v = 0.0;
-#pragma unroll
-        for (int I = 0; I < F; ++I) v = fma(S[I * P + i], C[z * QF + I * F + J], v);
-        V[q] = v;
-    }
+    // V[i][J] = sum_I fine[I][i] C[I][J], then over J
+    products<P, F, F, 2>(S + Q, 0, C, QF, [&](int f, int m, int n, const auto& c) {
+        put_lds<F>(V + f * P * F, m, n, c);
+    });
     __syncthreads();
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-        const int q = tid + 256 * p;
-        if (q < 2 * Q) {
-            const int z = q >= Q, r = q - z * Q, i = r / P, j = r - i * P;
-            double v = 0.0;
-#pragma unroll
-            for (int J = 0; J < F; ++J) v = fma(V[z * P * F + i * F + J], S[J * P + j], v);
-            acc[p] += v;
-        }
-    }
+    products<P, P, F, 2>(V, P * F, S, 0, add);
     __syncthreads();
     if (par) {
         const int64_t pt = fs.off[lev + 1] + (int64_t)(tl.tx >> 1) * fs.n[lev + 1] + (tl.ty >> 1);
-        const int a = tl.tx & 1, b = tl.ty & 1;
-        for (int q = tid; q < 2 * Q; q += 256) {
-            S[q] = shift[q];
-            C[q] = A.loc[pt * (2 * Q) + q];
-        }
+        load_table<P, P>(shift + (tl.tx & 1) * Q, nullptr, S);
+        load_table<P, P>(shift + (tl.ty & 1) * Q, S + Q, nullptr);
+        for (int q = tid; q < 2 * Q; q += FMM_THREADS) C[q] = A.loc[pt * (2 * Q) + q];
         __syncthreads();
-        for (int q = tid; q < 2 * Q; q += 256) {   // V[I][j] = sum_i shift_a[i][I] C[i][j]
-            const int z = q >= Q ? Q : 0, I = (q - z) / P, j = (q - z) - I * P;
-            double s = 0.0;
-#pragma unroll
-            for (int i = 0; i < P; ++i) s = fma(S[a * Q + i * P + I], C[z + i * P + j], s);
-            V[q] = s;
-        }
+        products<P, P, P, 2>(S, 0, C, Q, in_V);   // V[I][j] = sum_i shift_a[i][I] C[i][j]
         __syncthreads();
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int q = tid + 256 * p;
-            if (q < 2 * Q) {
-                const int z = q >= Q ? Q : 0, I = (q - z) / P, J = (q - z) - I * P;
-                double s = acc[p];
-#pragma unroll
-                for (int j = 0; j < P; ++j) s = fma(V[z + I * P + j], S[b * Q + j * P + J], s);
-                acc[p] = s;
-            }
-        }
+        products<P, P, P, 2>(V, Q, S + Q, 0, add);
+        __syncthreads();
     }
-    if (lev > 0) {
+    if (lev == 0) {
+        if (z < 2)
 #pragma unroll
-        for (int p = 0; p < PER; ++p)
-            if (tid + 256 * p < 2 * Q) L[tid + 256 * p] = acc[p];
-        return;
+            for (int w = 0; w < 2; ++w)
+#pragma unroll
+                for (int v = 0; v < NB; ++v) {
+                    C[at + w * P + v] = acc[w][v];
+                    acc[w][v] = 0.0;
+                }
+        load_table<P, P>(ctab, S, S + Q);
+        __syncthreads();
+        products<P, P, P, 2>(S, 0, C, Q, in_V);   // V[k][J] = sum_I ct[k][I] C[I][J]
+        __syncthreads();
+        products<P, P, P, 2>(V, Q, S + Q, 0, add);
     }
-    __syncthreads();
+    if (z < 2)
 #pragma unroll
-    for (int p = 0; p < PER; ++p)
-        if (tid + 256 * p < 2 * Q) C[tid + 256 * p] = acc[p];
-    for (int q = tid; q < Q; q += 256) S[q] = ctab[q];
-    __syncthreads();
-    for (int q = tid; q < 2 * Q; q += 256) {   // V[k][J] = sum_I ct[k][I] C[I][J]
-        const int z = q >= Q ? Q : 0, k = (q - z) / P, J = (q - z) - k * P;
-        double s = 0.0;
+        for (int w = 0; w < 2; ++w)
 #pragma unroll
-        for (int I = 0; I < P; ++I) s = fma(S[k * P + I], C[z + I * P + J], s);
-        V[q] = s;
-    }
-    __syncthreads();
-    for (int q = tid; q < 2 * Q; q += 256) {
-        const int z = q >= Q ? Q : 0, k = (q - z) / P, l = (q - z) - k * P;
-        double s = 0.0;
-#pragma unroll
-        for (int J = 0; J < P; ++J) s = fma(V[z + k * P + J], S[l * P + J], s);
-        L[q] = s;
-    }
+            for (int v = 0; v < NB; ++v) L[at + w * P + v] = acc[w][v];
 }
 
 // ---------------------------------------------------------------- particles
@@ -926,7 +972,7 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
     const unsigned pg = (unsigned)((A.N + 255) / 256);
     hipLaunchKernelGGL(k_fmm_pack, dim3(pg < (unsigned)num_cu * 16 ? pg : num_cu * 16), dim3(256),
                        0, st, A);
-    hipLaunchKernelGGL(k_fmm_p2m<P>, dim3((unsigned)A.nleaf), dim3(256), 0, st, A, tb.cheb,
+    hipLaunchKernelGGL(k_fmm_p2m<P>, dim3((unsigned)A.nleaf), dim3(FMM_THREADS), 0, st, A, tb.cheb,
                        tb.fine);
     for (int l = 1; l < pl.nlev; ++l)
         hipLaunchKernelGGL(k_fmm_m2m<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
@@ -936,7 +982,7 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
                        dim3(64), 0, st, A, (int)pl.ngroups, tb.nodes, tb.fnodes, eps2);
     for (int l = pl.nlev - 1; l >= 0; --l)
         hipLaunchKernelGGL(k_fmm_l2l<P>, dim3((unsigned)(A.lev_off[l + 1] - A.lev_off[l])),
-                           dim3(256), 0, st, A, tb.shift, tb.cheb, tb.fine, l);
+                           dim3(FMM_THREADS), 0, st, A, tb.shift, tb.cheb, tb.fine, l);
 }
 
 template <int P>
