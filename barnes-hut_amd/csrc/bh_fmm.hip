@@ -421,9 +421,9 @@ __global__ __launch_bounds__(256) void k_fmm_m2m(FmmArgs A, const double* __rest
 // issue slots per lane, the eight products it feeds 8 x 16, so the matrix unit is
 // the bound.  Softening enters relative to the square's size, which differs by
 // level and system; forming the slice on the fly needs no table of them.
-// 4.2M particles, 1024^2 cells: P = 20 4.6 ms (7.0 with all 27 offsets at P), 55
-// TFLOP/s (a large FP64 matrix product reaches 73; the unit is busy 0.74 of the
-// cycles, at 2.27 GHz), P = 12 0.76 ms (0.98); 512 systems 2.3 ms (2.7).  F = 8
+// 4.2M particles, 1024^2 cells, tiles of 8: P = 20 4.6 ms (7.0 with all 27 offsets
+// at P), 55 TFLOP/s (a large FP64 matrix product reaches 73; the unit is busy 0.74
+// of the cycles, at 2.27 GHz), P = 12 0.76 ms (0.98); 512 systems 2.3 ms (2.7).  F = 8
 // for P = 12 would take 0.56 and 1.6 ms but leaves 1e-9 of the far field, and
 // single particles whose terms cancel up to 6e-6.  Tried: sources square-major
 // (one line per 16 bytes read: 76 ms at P = 20 with 27 offsets, against 7.0);
@@ -862,6 +862,9 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
                     if (plain && !meet)
                         quad_terms<0, false>(wx, wy, m, {true, true, true, true}, eps2, r2cut, sx,
                                              sy);
+                    else if (LAW == 1 && !meet)   // a wide cutoff: one test a quad
+                        quad_terms<LAW, false>(wx, wy, m, {true, true, true, true}, eps2, r2cut,
+                                               sx, sy);
                     else
                         quad_terms<LAW, true>(wx, wy, m,
                                               {far(p[3]), far(p[7]), far(q[3]), far(q[7])}, eps2,
@@ -939,9 +942,10 @@ __global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double 
 // dispatch: a queue cursor (one atomic on the same word every ~15 ns) took 4.2M
 // particles from 2.2 to 3.5 ms, a fixed deal 512 systems from 10.0 to 12.4 ms.
 // Bound by FP64 issue (the vector units are busy 91 % of the time on 4.2M
-// clustered particles over 1024^2 cells): 2.02 ms there, 8.8 ms on 512 systems;
-// 2.16 and 9.9 ms with terms in pairs and every entry of a tile that the 3x3
-// cells touch tested, 2.8 and 12.8 ms with entries loaded one by one.
+// clustered particles over 1024^2 cells): with tiles of 8 cells 2.02 ms there, 8.8
+// ms on 512 systems (7.1 with tiles of 6); 2.16 and 9.9 ms with terms in pairs
+// and every entry of a tile that the 3x3 cells touch tested, 2.8 and 12.8 ms with
+// entries loaded one by one.
 template <int P, int LAW>
 __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2, double r2cut,
                                                   int qpart, int nqparts)
