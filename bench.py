@@ -17,18 +17,27 @@ time units, < 1 % of the clusters' free-fall time of ~0.03) particles move
 same interactions (1.99e12 per step), whatever --steps and --warmup are.
 Softening costs nothing: the kernels add eps^2 to r^2 either way.
 
+Passes of many far terms group the far field (FP64 interpolation on squares of
+cells), so `interactions` counts what the step's forces sum over, and
+`interactions_per_s` goes past what a kernel could evaluate one by one; the
+operations that a grouped pass does carry out are in `grouped`, and `achieved`
+counts those.
+
 A "step" is one full round: bounding box + placement + ordered permutation,
 per-cell COM, forces, tick.  Paths on the same input:
   * plain FP64, static work-queue order -- the rebuilt reference path, each
     weight m / r^2 from the hardware reciprocal plus one third-order
     refinement (within about one ulp of the quotient);
   * the same with the IEEE division per weight (`fp64_ieee`, secondary);
-  * FP32 cell-relative forces, Kahan-compensated tile sums, static order;
-  * the same FP32 path with the learned work-queue order (the cost model in
-    barnes-hut_amd/costmodels/clusters256.npz; --cost-model none disables).
-The FP32 paths include the FP64 recompute of the particles whose FP32 terms
-nearly cancel (kappa 1.5, --recompute-kappa 0 disables); it is timed apart from
-the force kernel.  `value` is the FP32 + learned-order path's whole-job
+  * the FP32 precision, static order: at this size its pass is grouped and in
+    FP64, to a remainder of 1e-9 (term by term, below 2e10 far terms, it is FP32
+    cell-relative forces with FP64 tile sums);
+  * the same with the learned work-queue order (the cost model in
+    barnes-hut_amd/costmodels/clusters256.npz; --cost-model none disables), which
+    is formed but orders nothing where the pass is grouped.
+Term-by-term FP32 paths include the FP64 recompute of the particles whose FP32
+terms nearly cancel (kappa 1.5, --recompute-kappa 0 disables), timed apart from
+the force kernel; a grouped pass has none.  `value` is the FP32 + learned-order path's whole-job
 throughput.
 
 Secondary blocks (not in `value`): the cost-model workload (256 clusters,
@@ -71,23 +80,14 @@ C4_CLUSTERS, C4_SIGMA, C4_SEED = 256, (0.001, 0.03), 91
 FP32_PEAK_TFLOPS = 157.3
 FP64_PEAK_TFLOPS = 78.6
 FLOP_PER_INTERACTION = 11
-# HBM bytes per FP32 force-kernel launch on this workload: rocprofv3 --pmc
-# FETCH_SIZE and WRITE_SIZE (KiB per dispatch), scaled by the readings of a
-# 1 GiB device copy (FETCH x2.0, WRITE x1.0), measured on the first two
-# steps of this workload with the default launch shape
-# (profiles/force32_gauss64_n4M_g1024_hbm_traffic.md).
-TRAFFIC = 5.09e9
-# Issue-limited ceiling of the FP32 far-field term: 6 VALU instructions per
-# interaction (v_rcp_f32 co-issued), no packed FP32, 256 CUs x 4 SIMDs x 16
-# lanes x 2.4 GHz = 39.3e12 lane-instructions/s -> 6.55e12 interactions/s.
+# Issue-limited ceiling of the FP64 near and mid terms of a grouped pass, four to a
+# reciprocal: 40 VALU instructions a quad and a v_rcp_f64 of 4 issue slots, no packed
+# arithmetic, 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz.
 LANE_OPS = 256 * 4 * 16 * 2.4e9
-ISSUE_CEILING_TFLOPS = LANE_OPS / 6 * FLOP_PER_INTERACTION / 1e12
-# FP64 far-field term, two entries per reciprocal: 10.5 VALU instructions
-# (2 differences, 2 fma for r^2, half of Q = q0 q1 and of its 3-instruction
-# refinement, 2 products for the weight, 2 fma into the sums) + half a
-# v_rcp_f64, which occupies 4 issue slots: 12.5 slots per term
-# (profiles/force64_gauss64_n4M_g1024_valu_issue.md)
-ISSUE_CEILING64_TFLOPS = LANE_OPS / 12.5 * FLOP_PER_INTERACTION / 1e12
+ISSUE_CEILING64_TFLOPS = LANE_OPS / 11 * FLOP_PER_INTERACTION / 1e12
+# From these many far terms a pass groups its far field (library rule), in all
+# precisions in FP64 (see grouped_work)
+GROUPED_TERMS = {"fp64": 4e9, "fp32": 2e10}
 # FP64 recompute threshold of the FP32 paths (--recompute-kappa)
 RECOMPUTE_KAPPA = 1.5
 
@@ -149,6 +149,43 @@ def run_path(eng, d, precision, steps, warmup, order_fn=None, kappa=RECOMPUTE_KA
     return (t1 - t0) / steps, kms, rms, near, far
 
 
+def grouped_work(counts, precision):
+    """FP64 operations of a grouped pass over G x G cells with these counts: near
+    and mid terms one by one (11 each), and per square with particles the products
+    of the nodes' masses with the law between nodes (2 components, a multiply and an
+    add each; 12 offsets at P^2 x P^2 nodes, 15 at F^2 x F^2).  None where the pass
+    is not grouped."""
+    G = counts.shape[0]
+    n, ne = int(counts.sum()), int((counts > 0).sum())
+    if precision not in GROUPED_TERMS or n * min(n, ne) < GROUPED_TERMS[precision]:
+        return None
+    P, F, c = (20, 16, 130000.0) if precision == "fp64" else (12, 10, 22000.0)
+    T = min(max(round((c * G * G / n) ** 0.25), 4), 24)   # cells per tile side
+    nt = -(-G // T)
+
+    def around(a):   # sums over 3 x 3
+        p = np.pad(a, 1)
+        return sum(p[i:i + a.shape[0], j:j + a.shape[1]] for i in range(3) for j in range(3))
+    pad = np.zeros((nt * T, nt * T), np.int64)
+    pad[:G, :G] = counts
+    tiles = pad.reshape(nt, T, nt, T)
+    near = int((counts * around(counts)).sum()) - n
+    mid = int((tiles.sum((1, 3)) * around((tiles > 0).sum((1, 3)))).sum()) \
+        - int((counts * around((counts > 0).astype(np.int64))).sum())
+    squares, occ = 0, tiles.sum((1, 3)) > 0
+    while True:
+        squares += int(occ.sum())
+        if occ.shape[0] <= 4:
+            break
+        m = (occ.shape[0] + 1) // 2
+        q = np.zeros((2 * m, 2 * m), bool)
+        q[:occ.shape[0], :occ.shape[0]] = occ
+        occ = q.reshape(m, 2, m, 2).any((1, 3))
+    node = 4 * (12 * P ** 4 + 15 * F ** 4) * squares
+    return {"tile_side": T, "near_terms": near, "mid_terms": mid, "squares": squares,
+            "node_product_flop": node, "flop": FLOP_PER_INTERACTION * (near + mid) + node}
+
+
 def measure(d, G, precision, tuning, steps, warmup, model=None, kappa=RECOMPUTE_KAPPA,
             autotune_first=False):
     """One path on workload `d` (G x G grid): see run_path."""
@@ -173,12 +210,15 @@ def measure(d, G, precision, tuning, steps, warmup, model=None, kappa=RECOMPUTE_
     sec, kms, rms, near, far = run_path(eng, d, precision, steps, warmup, order_fn, kappa)
     st = eng.ctx.stats()
     n_items, n_rc = int(st[2]), int(st[6])
+    grouped = grouped_work(eng.counts().reshape(G, G).astype(np.int64), precision)
     eng.close()
-    flops = FLOP_PER_INTERACTION * (near + far).astype(np.float64)
+    inter = (near + far).astype(np.float64)
+    flops = FLOP_PER_INTERACTION * inter if grouped is None else np.full(steps, grouped["flop"])
     return dict(seconds_per_step=sec, value=n / sec / 1e6, kms=kms,
                 force_kernel_ms=float(kms.mean()), recompute_ms=float(rms.mean()),
                 recomputed_last_step=n_rc, near=near, far=far,
-                flop_per_launch=float(flops.mean()),
+                flop_per_launch=float(flops.mean()), grouped=grouped,
+                interactions_per_s=float(inter.sum() / (kms.sum() * 1e-3)),
                 achieved=float(flops.sum() / (kms.sum() * 1e-3) / 1e12), tuning=tuning,
                 work_items=n_items, steps=steps)
 
@@ -187,7 +227,8 @@ def path_summary(r, peak):
     return {"value": r["value"], "ms_per_step": r["seconds_per_step"] * 1e3,
             "steps": r["steps"], "tuning": r["tuning"], "force_kernel_ms": r["force_kernel_ms"],
             "recompute_ms": r["recompute_ms"], "achieved_tflops": r["achieved"],
-            "frac_of_peak": r["achieved"] / peak,
+            "frac_of_peak": r["achieved"] / (peak if r["grouped"] is None else FP64_PEAK_TFLOPS),
+            "interactions_per_s": r["interactions_per_s"], "grouped": r["grouped"],
             "interactions_first_last": [float(r["near"][0] + r["far"][0]),
                                         float(r["near"][-1] + r["far"][-1])]}
 
@@ -382,7 +423,7 @@ def batched_line(steps, model_path, seed=0):
         inter = b.eng.interactions()[-1].astype(np.float64)    # placement of the last step
         out[name] = {"ms_per_step": sec * 1e3, "value": float(sizes.sum()) / sec / 1e6,
                      "interactions_last_step": float(inter.sum()),
-                     "tflops_whole_step": FLOP_PER_INTERACTION * float(inter.sum()) / sec / 1e12}
+                     "interactions_per_s": float(inter.sum()) / sec}
         b.close()
     return out
 
@@ -646,22 +687,25 @@ def main():
         "recompute": {"kappa": kappa, "ms_per_step": res["recompute_ms"],
                       "share_of_step": res["recompute_ms"] / (res["seconds_per_step"] * 1e3),
                       "particles_last_step": res["recomputed_last_step"]},
-        "roofline": {"bound": "valu", "achieved": res["achieved"], "peak": FP32_PEAK_TFLOPS,
-                     "unit": "TFLOP/s", "frac": res["achieved"] / FP32_PEAK_TFLOPS,
-                     "traffic": TRAFFIC, "kernel": "k_force32<P,0,1>",
+        "roofline": {"bound": "valu", "achieved": res["achieved"],
+                     "peak": FP64_PEAK_TFLOPS if res["grouped"] else FP32_PEAK_TFLOPS,
+                     "unit": "TFLOP/s",
+                     "frac": res["achieved"] / (FP64_PEAK_TFLOPS if res["grouped"]
+                                                else FP32_PEAK_TFLOPS),
+                     "kernel": "grouped far field: k_fmm_force and k_fmm_m2l (FP64)"
+                               if res["grouped"] else "k_force32",
                      "force_kernel_ms": res["force_kernel_ms"],
-                     "flop_per_launch": res["flop_per_launch"],
-                     "issue_ceiling": ISSUE_CEILING_TFLOPS,
-                     "frac_of_issue_ceiling": res["achieved"] / ISSUE_CEILING_TFLOPS},
+                     "flop_per_launch": res["flop_per_launch"], "grouped": res["grouped"],
+                     "interactions_per_s": res["interactions_per_s"]},
     }
     if res_static is not None:
         out["fp32_static"] = path_summary(res_static, FP32_PEAK_TFLOPS)
         out["learned_vs_static"] = res_static["seconds_per_step"] / res["seconds_per_step"]
     if res64 is not None:
         out["fp64_plain"] = path_summary(res64, FP64_PEAK_TFLOPS)
-        out["fp64_plain"]["kernel"] = "k_force64<P,0,1> (refined hardware reciprocal)"
+        out["fp64_plain"]["kernel"] = ("grouped far field: k_fmm_force and k_fmm_m2l"
+                                       if res64["grouped"] else "k_force64s")
         out["fp64_plain"]["issue_ceiling"] = ISSUE_CEILING64_TFLOPS
-        out["fp64_plain"]["frac_of_issue_ceiling"] = res64["achieved"] / ISSUE_CEILING64_TFLOPS
         out["speedup_vs_fp64"] = res64["seconds_per_step"] / res["seconds_per_step"]
     if res64i is not None:
         out["fp64_ieee"] = path_summary(res64i, FP64_PEAK_TFLOPS)

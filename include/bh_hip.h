@@ -41,10 +41,14 @@ enum {
 #define BH_DEVERR_ITEMS 4       /* work-item capacity exceeded */
 
 enum {
-    BH_PREC_FP64 = 0,            /* plain FP64 forces; each weight m / (r^2 + eps2) from the
-                                    hardware reciprocal with one third-order refinement
-                                    (within about one ulp of the quotient) */
-    BH_PREC_FP32_KAHAN = 1,      /* FP32 cell-relative, Kahan-summed 64-term tiles */
+    BH_PREC_FP64 = 0,            /* FP64 forces; weights m / (r^2 + eps2) from hardware
+                                    reciprocals with one third-order refinement, one
+                                    for up to four terms (within a few ulp of the
+                                    quotient).  Passes of 4e9 far terms and more group
+                                    the far field (to about 1e-15 of it) */
+    BH_PREC_FP32_KAHAN = 1,      /* FP32 cell-relative, tile sums in FP64 or Kahan-summed.
+                                    Passes of 2e10 far terms and more group the far
+                                    field (to about 1e-10 of it) and are FP64 */
     BH_PREC_FP32_KAHAN_TERM = 2, /* FP32 cell-relative, Kahan per term */
     BH_PREC_FP32_PLAIN = 3,      /* FP32 cell-relative, uncompensated */
     BH_PREC_FP32_MFMA = 4,       /* FP32 cell-relative, far-field sums on the matrix cores,
@@ -68,7 +72,11 @@ typedef struct bh_law {
     double r2_cut;
 } bh_law;
 
-/* Launch shape of the force kernel. p: particles per lane (1, 2 or 4);
+/* Launch shape of the force kernels that take work items from a queue: the
+ * precisions 2 to 5, FP32 passes of several systems and 4e9 far terms or more that
+ * are not grouped, and every pass while the cost log is on.  (Grouped passes, and
+ * passes whose waves share chunks of particles, have shapes of their own; p and
+ * yspan still cut the items.)  p: particles per lane (1, 2 or 4);
  * yspan: max rows per work item (>= 1); waves_per_cu: persistent waves per
  * compute unit (>= 1); tail_split: the FP32 kernels run each of the last
  * tail_items queue entries as tail_split far-field slices (1 = off, <= 16;
@@ -120,7 +128,8 @@ int bh_calculate_box_cumm(void* ctx, void* stream);
 int bh_sort_particles(void* ctx, const bh_particles* src, const bh_particles* dst, void* stream);
 int bh_summarize(void* ctx, const bh_particles* p, void* stream);
 /* order: device int32 [n_items] queue order of the work items, or NULL for
- * the static (natural) order; it must come from this step's items. */
+ * the static (natural) order; it must come from this step's items.  A pass that
+ * takes no items from a queue (see bh_tuning) does not read it. */
 int bh_build_items(void* ctx, void* stream);
 int bh_evaluate_boxes(void* ctx, const bh_particles* p, const bh_law* law, int32_t precision,
                       const int32_t* order, void* stream);
@@ -131,7 +140,8 @@ int bh_force_pass(void* ctx, const bh_particles* p, const bh_law* law, int32_t p
                   const int32_t* order, void* stream);
 /* bh_force_pass in nparts launches: call it for part = 0 .. nparts-1 in
  * order (same arguments otherwise); part k runs the k-th contiguous range of
- * the work queue, the last part adds the slices and runs the recompute.  The
+ * the work queue or of the particles' chunks (a grouped pass forms the far field
+ * in part 0), the last part adds the slices and runs the recompute.  The
  * result is bit-identical to bh_force_pass (a particle's sums do not depend
  * on which launch runs its pieces).  For callers that need to return to the
  * host during a long pass (progress, deadlines).  No reference counterpart. */
@@ -148,7 +158,8 @@ int bh_tick_particles(void* ctx, const bh_particles* p, double dt, void* stream)
  * like eps32 * B, so particles with B > kappa * |a| (a in the law's units
  * divided by G / step) are evaluated again with the FP64 kernel's terms and
  * their FP32 result is replaced.  bh_read_stats()[6] is the number of
- * particles recomputed by the last pass.  kappa <= 0 turns it off (then the
+ * particles recomputed by the last pass (0 after a grouped pass: its sums are
+ * FP64, and bh_recompute after it has nothing to do).  kappa <= 0 turns it off (then the
  * FP32 pass writes no per-particle scratch).  deferred = 0: bh_force_pass,
  * bh_evaluate_boxes and the step calls run it; deferred = 1: bh_force_pass
  * stops after the FP32 kernels and the caller runs bh_recompute before
