@@ -911,12 +911,12 @@ int bh_build_items(void* ctx, void* stream)
     }
     unsigned g = (unsigned)c->ncols;   // one wave per grid column
     hipLaunchKernelGGL(k_items<false>, dim3(g), dim3(64), 0, st, (const SysDev*)c->sys, c->S,
-                       c->ncols, (const int32_t*)c->counts, (const int32_t*)c->offsets, pitem,
-                       c->tune.yspan, c->col_items, c->items, c->max_items, c->stats);
+                       c->ncols, (const int32_t*)c->offsets, pitem, c->tune.yspan,
+                       c->col_items, c->items, c->max_items, c->stats);
     run_scan(c, false, c->col_items, c->ncols, c->col_off, nullptr, ST_NITEMS, c->max_items, st);
     hipLaunchKernelGGL(k_items<true>, dim3(g), dim3(64), 0, st, (const SysDev*)c->sys, c->S,
-                       c->ncols, (const int32_t*)c->counts, (const int32_t*)c->offsets, pitem,
-                       c->tune.yspan, c->col_off, c->items, c->max_items, c->stats);
+                       c->ncols, (const int32_t*)c->offsets, pitem, c->tune.yspan,
+                       c->col_off, c->items, c->max_items, c->stats);
     LAUNCH_CHECK("items");
     return BH_OK;
 }

@@ -33,15 +33,29 @@
 // column offsets.
 //
 // Where no run of pitem particles reaches the row span, those are the column's
-// items, found a lane each (700k particles on 750^2 cells: 15 us a pass instead of
-// 50; 512 systems: 13 and 23 us instead of 100 and 120).  Else the column's counts and offsets are
-// read 64 rows at a time, and the greedy cut walks the non-empty rows with
-// wave-uniform values (every lane holds the same state; lane 0 writes).  A row's
-// values come by v_readlane: through shuffles the walk of a 1024-row column took
-// 160 us, of which the chip idles all but 1024 waves.
+// items, found a lane each.  Else the wave goes from item to item, the row of a
+// particle found by 64 lanes at a time.  The two passes, and with a walk of the
+// column's rows: 700k particles on 750^2 cells 13 us, 95; 4.2M in clusters on
+// 1024^2 39 us, 181; 512 systems 36 us, 220.
+
+// The row of a column that particle p lies in: the last with o[y] <= p, o[0 .. G].
+__device__ __forceinline__ int row_of(const int32_t* __restrict__ o, int G, int p)
+{
+    const int lane = threadIdx.x & 63;
+    int lo = 0, n = G;   // the row is in [lo, lo + n)
+    while (n > 1) {
+        const int step = (n + 63) >> 6;
+        const bool in = lane * step < n;
+        const unsigned long long b = __ballot(in && o[lo + (in ? lane * step : 0)] <= p);
+        const int k = __popcll(b) - 1;
+        n = min(step, n - k * step);
+        lo += k * step;
+    }
+    return lo;
+}
+
 template <bool WRITE>
 __device__ __forceinline__ int column_items(const SysDev* __restrict__ sys, int S, int64_t col,
-                                            const int32_t* __restrict__ counts,
                                             const int32_t* __restrict__ offsets, int pitem,
                                             int yspan, int64_t out, Item* __restrict__ items,
                                             int64_t max_items, int32_t* stats)
@@ -51,79 +65,48 @@ __device__ __forceinline__ int column_items(const SysDev* __restrict__ sys, int 
     const SysDev& d = sys[s];
     const int G = d.G;
     const int x = (int)(col - d.col_off);
-    const int64_t cb = d.c_off + (int64_t)x * G;
-    const int runs = (offsets[cb + G] - offsets[cb] + pitem - 1) / pitem;
+    const int32_t* o = offsets + d.c_off + (int64_t)x * G;
+    const int pb = uniform_int(o[G]);
+    int p = uniform_int(o[0]);
+    const int runs = (pb - p + pitem - 1) / pitem;
     bool wide = false;
     for (int i = lane; i < runs && G > yspan; i += BH_WAVE) {
-        const Item it = run_item(offsets + cb, G, s, x, i, pitem);
+        const Item it = run_item(o, G, s, x, i, pitem);
         wide = wide || it.y1 - it.y0 >= yspan;
     }
     if (!__any(wide)) {
         for (int i = lane; WRITE && i < runs; i += BH_WAVE) {
-            if (out + i < max_items) items[out + i] = run_item(offsets + cb, G, s, x, i, pitem);
+            if (out + i < max_items) items[out + i] = run_item(o, G, s, x, i, pitem);
             else atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
         }
         return runs;
     }
     int n_out = 0;
-    bool open = false;
-    int p0 = 0, np = 0, y0 = 0, y1 = 0;
-    auto emit = [&]() {
-        if (WRITE && lane == 0) {
-            int64_t k = out + n_out;
-            if (k < max_items) {
-                Item it;
-                it.p0 = p0;
-                it.np = np;
-                it.sys = s;
-                it.cx = x;
-                it.y0 = y0;
-                it.y1 = y1;
-                it.pad0 = 0;
-                it.pad1 = 0;
-                items[k] = it;
-            } else {
-                atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
+    while (p < pb) {   // the same on every lane; lane 0 writes
+        Item it;
+        it.p0 = p;
+        it.y0 = row_of(o, G, p);
+        const int end = it.y0 + yspan < G ? uniform_int(o[it.y0 + yspan]) : pb;
+        p = min(p + pitem, end);
+        if (WRITE) {
+            it.np = p - it.p0;
+            it.y1 = row_of(o, G, p - 1);
+            it.sys = s;
+            it.cx = x;
+            it.pad0 = 0;
+            it.pad1 = 0;
+            if (lane == 0) {
+                if (out + n_out < max_items) items[out + n_out] = it;
+                else atomicOr(&stats[ST_ERR], BH_ERR_ITEMS);
             }
         }
         ++n_out;
-        open = false;
-    };
-    for (int yb = 0; yb < G; yb += BH_WAVE) {
-        const int yl = yb + lane;
-        const int ncl = yl < G ? counts[cb + yl] : 0;
-        const int pcl = yl < G ? offsets[cb + yl] : 0;
-        unsigned long long nz = __ballot(ncl > 0);
-        while (nz) {
-            const int l = __ffsll((long long)nz) - 1;
-            nz &= nz - 1;
-            const int yy = yb + l;
-            int nc = __builtin_amdgcn_readlane(ncl, l);
-            int pc = __builtin_amdgcn_readlane(pcl, l);
-            if (open && yy - y0 >= yspan) emit();
-            while (nc > 0) {
-                if (!open) {
-                    open = true;
-                    p0 = pc;
-                    np = 0;
-                    y0 = yy;
-                }
-                int take = min(nc, pitem - np);
-                np += take;
-                pc += take;
-                nc -= take;
-                y1 = yy;
-                if (np == pitem) emit();
-            }
-        }
     }
-    if (open) emit();
     return n_out;
 }
 
 template <bool WRITE>
 __global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, int S, int64_t ncols,
-                                              const int32_t* __restrict__ counts,
                                               const int32_t* __restrict__ offsets, int pitem,
                                               int yspan, int32_t* __restrict__ col_items,
                                               Item* __restrict__ items, int64_t max_items,
@@ -131,15 +114,15 @@ __global__ __launch_bounds__(64) void k_items(const SysDev* __restrict__ sys, in
 {
     const int64_t col = blockIdx.x;
     if (col >= ncols) return;
-    const int n = column_items<WRITE>(sys, S, col, counts, offsets, pitem, yspan,
+    const int n = column_items<WRITE>(sys, S, col, offsets, pitem, yspan,
                                       WRITE ? col_items[col] : 0, items, max_items, stats);
     if (!WRITE && threadIdx.x == 0) col_items[col] = n;
 }
 
-template __global__ void k_items<false>(const SysDev*, int, int64_t, const int32_t*, const int32_t*,
-                                        int, int, int32_t*, Item*, int64_t, int32_t*);
-template __global__ void k_items<true>(const SysDev*, int, int64_t, const int32_t*, const int32_t*,
-                                       int, int, int32_t*, Item*, int64_t, int32_t*);
+template __global__ void k_items<false>(const SysDev*, int, int64_t, const int32_t*, int, int,
+                                        int32_t*, Item*, int64_t, int32_t*);
+template __global__ void k_items<true>(const SysDev*, int, int64_t, const int32_t*, int, int,
+                                       int32_t*, Item*, int64_t, int32_t*);
 
 // items_runs as a launch of its own: the count, scan, clamp and write of a
 // 16,384-particle step were six launches and 24 us.

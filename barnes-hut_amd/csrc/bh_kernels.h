@@ -463,9 +463,9 @@ __global__ void k_rc_combine(const int32_t* stats, const int32_t* rc_cnt, const 
                              double Gc, double* ax, double* ay);
 
 template <bool WRITE>
-__global__ void k_items(const SysDev* sys, int S, int64_t ncols, const int32_t* counts,
-                        const int32_t* offsets, int pitem, int yspan, int32_t* col_items,
-                        Item* items, int64_t max_items, int32_t* stats);
+__global__ void k_items(const SysDev* sys, int S, int64_t ncols, const int32_t* offsets, int pitem,
+                        int yspan, int32_t* col_items, Item* items, int64_t max_items,
+                        int32_t* stats);
 __global__ void k_items_runs(const SysDev* sys, int S, int ncols, const int32_t* offsets, int pitem,
                              int32_t* col_off, Item* items, int64_t max_items, int32_t* stats,
                              int write);
