@@ -414,12 +414,20 @@ __global__ __launch_bounds__(256) void k_scan_reduce(const int32_t* __restrict__
     int ev, ef, tv, tf;
     block_excl_scan2(v, f, ev, ef, tv, tf, sh);
     if (CNT) {
+        // at most one atomic a block, and only if it raises the maximum: one per
+        // wave, all on one word, made this kernel 28 us for 1M cells instead of 10
         mx = wave_max(mx);
-        if ((threadIdx.x & 63) == 0) atomicMax(&stats[ST_MAXCOUNT], mx);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mx;
+        __syncthreads();
     }
     if (threadIdx.x == 0) {
         bsum[blockIdx.x] = tv;
-        if (CNT) bne[blockIdx.x] = tf;
+        if (CNT) {
+            bne[blockIdx.x] = tf;
+            mx = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
+            if (mx > __atomic_load_n(&stats[ST_MAXCOUNT], __ATOMIC_RELAXED))
+                atomicMax(&stats[ST_MAXCOUNT], mx);
+        }
     }
 }
 
