@@ -187,7 +187,19 @@ __device__ __forceinline__ void cloud_sum(const CloudArgs& A, double* buf, int64
         if (A.mask_self && t0 < base + P * groups && t0 + CL_THREADS > base)
             cloud_tile<LAW, SOFT, P, 1, FAST>(sx, sy, sm, cnt, lane, L, t0, ti, xi, yi, ax, ay,
                                               A.eps2, A.r2cut);
-        else
+        else if (FAST) {
+            // a tile's sum first: fewer lanes per target make each lane's chain
+            // longer, and in one chain its rounding grew with it (70,000 rows: 9e-16
+            // of the sums, 4.5e-16 on twice the lanes, 1.8e-16 by tiles)
+            double tx[P] = {}, ty[P] = {};
+            cloud_tile<LAW, SOFT, P, 0, FAST>(sx, sy, sm, cnt, lane, L, t0, ti, xi, yi, tx, ty,
+                                              A.eps2, A.r2cut);
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                ax[p] += tx[p];
+                ay[p] += ty[p];
+            }
+        } else
             cloud_tile<LAW, SOFT, P, 0, FAST>(sx, sy, sm, cnt, lane, L, t0, ti, xi, yi, ax, ay,
                                               A.eps2, A.r2cut);
     }
@@ -254,7 +266,7 @@ __device__ __forceinline__ void cloud_block(const CloudArgs& A, int64_t blk)
 }
 
 template <int LAW, int SOFT, int P, int FAST>
-__global__ __launch_bounds__(CL_THREADS) void k_cloud(CloudArgs A)
+__global__ __launch_bounds__(CL_THREADS, 6) void k_cloud(CloudArgs A)
 {
     cloud_block<LAW, SOFT, P, FAST>(A, blockIdx.x);
 }

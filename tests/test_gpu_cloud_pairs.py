@@ -79,3 +79,26 @@ def test_two_clouds_both_sides_in_pairs():
     hiplib.cloud_gravity(w[:9000], second, eps2=1e-6, r2_cut=0.0)
     hiplib.cloud_gravity(w[4000:], first, eps2=1e-6, r2_cut=0.0)
     np.testing.assert_array_equal(whole.cpu().numpy(), w.cpu().numpy())
+
+
+@pytest.mark.parametrize("n", [6001, 30011, 70000])
+def test_rounding_does_not_grow_with_the_cloud(n):
+    """Sums by tiles of 256 rows: at most 16 + n / 256 roundings in a lane's
+    chain, of independent signs, so a few 1e-16 of the sums at any size."""
+    import torch
+    rng = np.random.default_rng(n)
+    rows = np.zeros((n, 10))
+    rows[:, :2], rows[:, 2] = rng.random((n, 2)), rng.uniform(1, 2, n)
+    dev = torch.as_tensor(rows, device="cuda")
+    hiplib.cloud_gravity(dev, None, eps2=0.0, r2_cut=1e-5)
+    got = dev.cpu().numpy()
+    x, y, m = (rows[:, k].astype(np.longdouble) for k in range(3))
+    num = den = 0.0
+    for i in rng.choice(n, 60, replace=False):
+        dx, dy = x - x[i], y - y[i]
+        r2 = dx * dx + dy * dy
+        w = np.where(r2 > 1e-5, m / np.where(r2 > 0, r2, 1), 0)
+        ex, ey = (dx * w).sum(), (dy * w).sum()
+        num += (got[i, 5] - ex) ** 2 + (got[i, 6] - ey) ** 2
+        den += ex * ex + ey * ey
+    assert float((num / den) ** 0.5) <= 4e-16
