@@ -219,13 +219,14 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 // (bh_fmm.hip) is used, per precision.
 //
 // fp64: a term-by-term pass (k_force64s) and a grouped one took, on uniform and
-// on clustered particles (tiles of 8 cells),
-//   131,072 on  90^2 (1.1e9 terms)  0.50, 0.61 ms    0.53, 0.98 ms
-//   600,000 on  60^2 (2.2e9)        1.36, 4.12       1.40, 4.09
-//   262,144 on 128^2 (4.3e9)        1.63, 1.85       0.58, 1.20
-//   600,000 on 110^2 (7.3e9)        2.90, 3.96       0.80, 2.35
-//   1M      on 140^2 (2.0e10)       7.36, 9.17       1.20, 3.44
-// so they meet below the line.  The allocation-free step has no scratch for the
+// on clustered particles,
+//   300,000 on  60^2 (1.1e9 terms)  0.57, 1.31 ms    0.51, 2.07 ms
+//   300,000 on  80^2 (1.9e9)        0.82, 1.33       0.46, 1.33
+//   600,000 on  60^2 (2.2e9)        1.27, 3.88       0.87, 3.72
+//   2M      on  34^2 (2.3e9)        13.6, 62.8       10.3, 48.5
+//   1M      on  60^2 (3.6e9)        2.41, 9.57       1.57, 8.24
+//   600,000 on 110^2 (7.3e9)        2.90, 3.96       0.65, 2.42
+// so they meet at the line.  The allocation-free step has no scratch for the
 // squares and gives the bits of bh_step, so single systems within its limits
 // stay term by term (at most 1.7e10 terms, 6 ms).
 // fp32: at 2.2e10 terms (600,001 particles, 193^2 cells) 4.5 and 1.1 ms.  The
@@ -234,7 +235,7 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 // items, which grouped passes do not have), and because the recompute, whose
 // flags callers read, belongs to the term-by-term pass.
 static constexpr double FP32_SHARED_TERMS = 4e9;
-static constexpr double FMM_MIN_TERMS_FP64 = 4e9;
+static constexpr double FMM_MIN_TERMS_FP64 = 2e9;
 static constexpr double FMM_MIN_TERMS_FP32 = 2e10;
 static constexpr double FMM_MAX_BYTES = 48.0 * (1 << 30);
 

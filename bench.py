@@ -87,7 +87,7 @@ LANE_OPS = 256 * 4 * 16 * 2.4e9
 ISSUE_CEILING64_TFLOPS = LANE_OPS / 11 * FLOP_PER_INTERACTION / 1e12
 # From these many far terms a pass groups its far field (library rule), in all
 # precisions in FP64 (see grouped_work)
-GROUPED_TERMS = {"fp64": 4e9, "fp32": 2e10}
+GROUPED_TERMS = {"fp64": 2e9, "fp32": 2e10}
 # FP64 recompute threshold of the FP32 paths (--recompute-kappa)
 RECOMPUTE_KAPPA = 1.5
 

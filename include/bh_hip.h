@@ -44,7 +44,7 @@ enum {
     BH_PREC_FP64 = 0,            /* FP64 forces; weights m / (r^2 + eps2) from hardware
                                     reciprocals with one third-order refinement, one
                                     for up to four terms (within a few ulp of the
-                                    quotient).  Passes of 4e9 far terms and more group
+                                    quotient).  Passes of 2e9 far terms and more group
                                     the far field (to about 1e-15 of it) */
     BH_PREC_FP32_KAHAN = 1,      /* FP32 cell-relative, tile sums in FP64 or Kahan-summed.
                                     Passes of 2e10 far terms and more group the far

@@ -102,6 +102,7 @@ def test_grouped_pass_against_oracle(kind, eps2, r2_cut):
 
 @pytest.mark.parametrize("n,G,precisions", [
     (70001, 600, "64"),          # 0.2 particles a cell: tiles of 24 cells
+    (600001, 60, "64"),          # 167: 5, near the least far terms that are grouped
     (150001, 500, "64 32"),      # 0.6: 22 and 14
     (400001, 301, "64 32"),      # 4.4: 13 and 8
     (1000003, 97, "64"),         # 106: 6
