@@ -878,7 +878,7 @@ int bh_summarize(void* ctx, const bh_particles* p, void* stream)
     // one wave per non-empty cell; the grid is sized for the worst case
     int64_t waves = std::min<int64_t>(c->C, (int64_t)c->num_cu * 64);
     hipLaunchKernelGGL(k_com, dim3(grid_for(waves * 64, 256)), dim3(256), 0, st,
-                       (const SysDev*)c->sys, c->S, (const int32_t*)c->ne_list,
+                       c->sys, c->S, (const int32_t*)c->ne_list,
                        (const int32_t*)c->stats, (const int32_t*)c->offsets,
                        (const double*)p->px, (const double*)p->py, (const double*)p->mass,
                        c->com_dense, c->l64, c->l32);
@@ -1194,7 +1194,7 @@ static int step_impl(void* ctx, const bh_particles* a, const bh_particles* b, co
         const int write = c->N <= ITEMS_ONE;
         const int64_t waves = std::min<int64_t>(c->C, (int64_t)c->num_cu * 64);
         hipLaunchKernelGGL(k_com_items, dim3(grid_for(waves * 64, 256) + 1), dim3(256), 0, st,
-                           (const SysDev*)c->sys, c->S, (const int32_t*)c->ne_list, c->stats,
+                           c->sys, c->S, (const int32_t*)c->ne_list, c->stats,
                            (const int32_t*)c->offsets, (const double*)b->px, (const double*)b->py,
                            (const double*)b->mass, c->com_dense, c->l64, c->l32, (int)c->ncols,
                            64 * c->tune.p, c->col_off, c->items, c->max_items, write);

@@ -32,7 +32,7 @@ enum {
 };
 
 // Per-system parameters. Host fills p_off, n, c_off, col_off, k_off, b_off, G, Gb;
-// the bounding-box kernels fill the FP64 box fields every step.
+// the bounding-box kernels fill the FP64 box fields and clear com_out every step.
 struct SysDev {
     int64_t p_off;
     int64_t n;
@@ -43,6 +43,8 @@ struct SysDev {
     int32_t G;
     int32_t Gb;
     double min_x, min_y, max_x, max_y, step;
+    int32_t com_out;   // != 0: a COM of this placement lies outside its cell (com_out)
+    int32_t pad;
 };
 
 #define RC_BLOCK 16   // cells per side of the blocks the recompute bound aggregates

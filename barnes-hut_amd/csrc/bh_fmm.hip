@@ -272,7 +272,7 @@ __global__ __launch_bounds__(FMM_THREADS) void k_fmm_p2m(FmmArgs A,
                     f.Y = fma((double)c.ky + 0.5, d.step, d.min_y) * sig;
                 }
                 A.list[e0 + r] = f;
-                // masses of both signs can put a COM outside its cell, where
+                // masses of both signs can put a COM outside its tile, where
                 // the interpolation does not hold: that system goes term by term
                 if (up && c.M != 0.0 && !(fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN))
                     A.sbad[tl.sys] = 1;
@@ -824,12 +824,12 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
 
     // mid entries: 3x3 tiles, or every tile where the grouped part does not
     // hold: a system of one tile, a cutoff that reaches past a tile, COMs
-    // outside their cells, particles moved since they were placed
+    // outside their tiles, particles that left theirs since they were placed
     const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
     const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
                      uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
-    // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
-    const bool plain = LAW == 0 || r2cut < 0.99;
+    const bool plain = placed_apart<LAW>(d, r2cut, act, (0.5 * (ux + 1.0) + ttx) * T - cx,
+                                         (0.5 * (uy + 1.0) + tty) * T - cy);
     const int nt = fs.n[0];
     const int mx0 = all ? 0 : max(ttx - 1, 0), mx1 = all ? nt - 1 : min(ttx + 1, nt - 1);
     const int my0 = all ? 0 : max(tty - 1, 0), my1 = all ? nt - 1 : min(tty + 1, nt - 1);

@@ -584,12 +584,16 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
     double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0;
     int cx = -100000, cy = -100000;
     if (act) {
-        x = A.x[gi] * sig;
-        y = A.y[gi] * sig;
+        x = A.x[gi];
+        y = A.y[gi];
         const int key = A.key_sorted[gi] - (int)coff;
         cx = key / G;
         cy = key - cx * G;
     }
+    const bool plain = placed_apart<LAW>(d, r2cut, act, (x - d.min_x) / d.step - cx,
+                                         (y - d.min_y) / d.step - cy);
+    x *= sig;
+    y *= sig;
     const int cxl = uniform_int(wave_min(act ? cx : 0x7fffffff));
     const int cxh = uniform_int(wave_max(act ? cx : -1));
     const int cyl = uniform_int(wave_min(act ? cy : 0x7fffffff));
@@ -649,8 +653,6 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
     const int mhi = uniform_int(A.neprefix[coff + (int64_t)min(cxh + 2, G) * G]);
     const int per = (((ne1 - ne0 + W - 1) / W) + 3) & ~3;
     const int f0 = min(ne1, ne0 + w * per), f1 = min(ne1, f0 + per);
-    // a COM outside the 3x3 cells is a cell side (>= 1) away: beyond most cutoffs
-    const bool plain = LAW == 0 || r2cut < 0.99;
     if (f0 < f1) {
         // the list is padded by a quad, so whole quads are in bounds
         fd8 p = *(cptr<fd8>)(as_const(A.l64) + f0), q = *(cptr<fd8>)(as_const(A.l64) + f0 + 2);

@@ -144,7 +144,7 @@ struct FmmArgs {
     int32_t *tcnt;             // per square: particles
     int32_t *tstart, *tne;     // per tile: its run of list
     int32_t* cnt;              // FMM_HEAVY .. FMM_QHEAVY, then per system sbad
-    int32_t* sbad;             // != 0: a COM lies outside its cell
+    int32_t* sbad;             // != 0: a COM lies outside its tile
     FmmChunk* chunks;
     FmmCom* list;
     FmmPart* pack;
@@ -259,6 +259,28 @@ __device__ __forceinline__ double step_scale(double step)
     int e2;
     (void)frexp(step, &e2);
     return ldexp(1.0, 1 - e2);
+}
+
+// Whether (fx, fy), in cell sides from a cell's corner, lies in the cell, up to
+// a thousandth of it (rounding of a COM's sums).
+__device__ __forceinline__ bool in_cell(double fx, double fy)
+{
+    return fabs(fx - 0.5) <= 0.501 && fabs(fy - 0.5) <= 0.501;
+}
+
+// Whether every COM outside a lane's 3x3 cells is beyond the cutoff r2cut (in
+// units of step_scale) for all lanes of the wave, so that its term needs no
+// test: the cutoff is below a cell side (at least 1; 0.996 squared with
+// in_cell's margins), the system's COMs lie in their cells and the lanes'
+// particles, (fx, fy) in cell sides from the corner of the cell that they were
+// placed in, are still there.
+template <int LAW>
+__device__ __forceinline__ bool placed_apart(const SysDev& d, double r2cut, bool act, double fx,
+                                             double fy)
+{
+    if (LAW == 0) return true;
+    if (!(r2cut < 0.99) || d.com_out != 0) return false;
+    return __ballot(act && !in_cell(fx, fy)) == 0ull;
 }
 
 // 1 / q as in wdiv64.
@@ -413,11 +435,11 @@ __global__ void k_gather(SortFields S, BhParticles D, int64_t N, const int32_t* 
                          const int32_t* stats, int32_t* perm_out);
 
 // summarize + tick
-__global__ void k_com(const SysDev* sys, int S, const int32_t* ne_list, const int32_t* stats,
+__global__ void k_com(SysDev* sys, int S, const int32_t* ne_list, const int32_t* stats,
                       const int32_t* offsets, const double* x, const double* y, const double* m,
                       double* com_dense, Com64* l64, Com32* l32);
 // k_com, and in its last block the items (k_items_runs) of at most ITEMS_COLS columns
-__global__ void k_com_items(const SysDev* sys, int S, const int32_t* ne_list, int32_t* stats,
+__global__ void k_com_items(SysDev* sys, int S, const int32_t* ne_list, int32_t* stats,
                             const int32_t* offsets, const double* x, const double* y,
                             const double* m, double* com_dense, Com64* l64, Com32* l32, int ncols,
                             int pitem, int32_t* col_off, Item* items, int64_t max_items, int write);

@@ -199,6 +199,7 @@ __device__ __forceinline__ bool store_box(SysDev& sys, const Box& d)
     sys.max_x = d.max_x;
     sys.max_y = d.max_y;
     sys.step = d.step;
+    sys.com_out = 0;
     return d.step > 0.0 && isfinite(d.step);
 }
 

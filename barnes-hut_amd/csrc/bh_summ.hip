@@ -8,7 +8,10 @@
 #include "bh_kernels.h"
 
 // Entry w of the lists and cell c's place in the dense array, from its sums.
-__device__ __forceinline__ void com_out(const SysDev& d, int64_t w, int c, double sx, double sy,
+// Masses of both signs, or rows moved since they were placed, can put a COM
+// outside its cell: the system is marked, since the force kernels take a COM
+// outside a particle's 3x3 cells to be a cell side away (see placed_apart).
+__device__ __forceinline__ void com_out(SysDev& d, int64_t w, int c, double sx, double sy,
                                         double sm, double* __restrict__ com_dense,
                                         Com64* __restrict__ l64, Com32* __restrict__ l32)
 {
@@ -30,9 +33,12 @@ __device__ __forceinline__ void com_out(const SysDev& d, int64_t w, int c, doubl
     e64.kx = kx;
     e64.ky = ky;
     l64[w] = e64;
+    const double fx = (X - d.min_x) / d.step - (double)kx;
+    const double fy = (Y - d.min_y) / d.step - (double)ky;
+    if (M != 0.0 && !in_cell(fx, fy)) d.com_out = 1;
     Com32 e32;
-    e32.fx = (float)((X - d.min_x) / d.step - (double)kx);
-    e32.fy = (float)((Y - d.min_y) / d.step - (double)ky);
+    e32.fx = (float)fx;
+    e32.fy = (float)fy;
     e32.rM = 1.0f / (float)M;
     e32.kxy = (kx << 16) | ky;
     l32[w] = e32;
@@ -50,7 +56,7 @@ __device__ __forceinline__ void com_out(const SysDev& d, int64_t w, int c, doubl
 // others.  262,144 particles in 16 clusters on 256^2 cells (up to 9,900 in a
 // cell): 144 -> 20 us; 4.2M on 1024^2 99 -> 89 us.
 __device__ __forceinline__ void com_cells(
-    const SysDev* __restrict__ sys, int S, const int32_t* __restrict__ ne_list,
+    SysDev* sys, int S, const int32_t* __restrict__ ne_list,
     const int32_t* __restrict__ stats, const int32_t* __restrict__ offsets,
     const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ m,
     double* __restrict__ com_dense, Com64* __restrict__ l64, Com32* __restrict__ l32, int nblocks,
@@ -130,7 +136,7 @@ __device__ __forceinline__ void com_cells(
     }
 }
 
-__global__ __launch_bounds__(256) void k_com(const SysDev* __restrict__ sys, int S,
+__global__ __launch_bounds__(256) void k_com(SysDev* sys, int S,
                                              const int32_t* __restrict__ ne_list,
                                              const int32_t* __restrict__ stats,
                                              const int32_t* __restrict__ offsets,
@@ -147,7 +153,7 @@ __global__ __launch_bounds__(256) void k_com(const SysDev* __restrict__ sys, int
 // The last block builds the work items meanwhile: a launch of its own for them is
 // 5 us of a 2,000-particle step, 11 us of one of 40 small systems.
 __global__ __launch_bounds__(256) void k_com_items(
-    const SysDev* __restrict__ sys, int S, const int32_t* __restrict__ ne_list, int32_t* stats,
+    SysDev* sys, int S, const int32_t* __restrict__ ne_list, int32_t* stats,
     const int32_t* __restrict__ offsets, const double* __restrict__ x,
     const double* __restrict__ y, const double* __restrict__ m, double* __restrict__ com_dense,
     Com64* __restrict__ l64, Com32* __restrict__ l32, int ncols, int pitem, int32_t* col_off,
