@@ -826,7 +826,8 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
     // hold: a system of one tile, a cutoff that reaches past a tile, COMs
     // outside their tiles, particles that left theirs since they were placed
     const bool in = !act || (fabs(ux) <= FMM_IN && fabs(uy) <= FMM_IN);
-    const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.999999 * h * h)) ||
+    // (0.9995: FMM_IN lets either end be 5e-5 of a tile nearer)
+    const bool all = fs.nlev == 0 || (LAW == 1 && !(r2cutp < 0.9995 * h * h)) ||
                      uniform_int(A.sbad[s]) != 0 || __ballot(!in) != 0ull;
     const bool plain = placed_apart<LAW>(d, r2cut, act, (0.5 * (ux + 1.0) + ttx) * T - cx,
                                          (0.5 * (uy + 1.0) + tty) * T - cy);

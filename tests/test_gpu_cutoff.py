@@ -42,3 +42,31 @@ def test_far_terms_within_the_cutoff_are_dropped(kind, n, G, r2_cut, precisions)
             assert norm <= (1e-11 if kind == "signed" else NORM[prec])
             assert (num / den).max() <= (1e-5 if kind == "signed" else EACH[prec])
     eng.close()
+
+
+def test_cutoff_just_below_a_tile_side():
+    """A grouped pass keeps every distant term where the cutoff ends before a
+    tile's side h, so it must end before the closest that a distant COM can
+    come: a particle 3e-5 h past its tile's edge still counts as inside."""
+    n, G, T = 300000, 90, 8          # 2.4e9 far terms, tiles of (130000 G^2 / n)^(1/4) cells
+    d = inputs.uniform(n, seed=73)
+    h = T / G
+    y = 4.5 / G
+    d["px"][:4] = [0.0, 1.0, h - 1e-8, 2 * h + 1e-8]   # the box, the particle, a heavy source
+    d["py"][:4] = [0.0, 1.0, y, y]
+    d["mass"][3] = 1e9
+    eng = _engine([n], [G], d)
+    i = int(np.nonzero(eng.fetch()["pid"] == d["pid"][2])[0][0])
+    off, keys = eng.offsets().astype(np.int64), eng.keys().astype(np.int64)
+    assert keys[i] == (T - 1) * G + 4
+    com = eng.com()
+    for moved in (0.0, 3e-5 * h):
+        eng.parts["px"][i] = h - 1e-8 + moved
+        law = (1e-6, 0.0, 0.99996 * h * h)
+        r = _pass(eng, law, "fp64")
+        rx, ry = orc.forces(G, off, keys, r["px"], r["py"], r["mass"], com, *law,
+                            targets=np.array([i]))
+        err = np.hypot(r["ax"][i] - rx, r["ay"][i] - ry)[0] / np.hypot(rx, ry)[0]
+        print(f"[cutoff] tile side, moved {moved:.1e}: {err:.2e}", flush=True)
+        assert err <= EACH["fp64"]
+    eng.close()
