@@ -945,6 +945,58 @@ int bh_force_pass(void* ctx, const bh_particles* p, const bh_law* law, int32_t p
     return bh_force_pass_part(ctx, p, law, precision, order, 0, 1, stream);
 }
 
+// Flags the particles of an FP32 pass's planes (rc_a32) by their bound and adds
+// the others' sums, or the flagged ones' FP64 terms, to the accelerations.
+static void recompute(Ctx* c, const bh_particles* p, const bh_law* law, hipStream_t st)
+{
+    const int64_t ntiles = c->nblocks * (RC_BLOCK / RC_TILE) * (RC_BLOCK / RC_TILE);
+    const unsigned nb = grid_for(c->nblocks, 4, (int64_t)c->num_cu * 4);
+    hipLaunchKernelGGL(k_rc_sums, dim3(nb + grid_for(ntiles, 256, (int64_t)c->num_cu * 8)),
+                       dim3(256), 0, st, (const SysDev*)c->sys, c->S, c->nblocks, ntiles, (int)nb,
+                       (const double*)c->com_dense, c->rc_blk, c->rc_tiles, c->rc_cnt, c->stats);
+    hipLaunchKernelGGL(k_rc_blockfar, dim3(grid_for(c->nblocks, 1, (int64_t)c->num_cu * 16)),
+                       dim3(64), 0, st, (const SysDev*)c->sys, c->S, c->nblocks,
+                       (const double*)c->rc_blk, c->rc_bfar);
+    // four waves an item where items of 64 P particles span 16 rows and more on
+    // average and do not fill the chip by themselves (k_rc_flag)
+    const bool wide = c->C * 64 * c->tune.p >= 16 * c->N && c->N <= (int64_t)c->num_cu * 4096;
+    hipLaunchKernelGGL(wide ? k_rc_flag<4> : k_rc_flag<1>,
+                       dim3(grid_for(c->max_items, 1, (int64_t)c->num_cu * 32)),
+                       dim3(wide ? 256 : 64), 0, st, (const Item*)c->items, (const SysDev*)c->sys,
+                       (const int32_t*)c->key_sorted, (const int32_t*)c->neprefix,
+                       (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
+                       (const double*)c->com_dense, (const double*)c->rc_tiles,
+                       (const double*)c->rc_blk, (const double*)c->rc_bfar,
+                       (const double*)c->rc_a32, (const double*)(c->rc_a32 + c->N),
+                       (const double*)(c->rc_a32 + 2 * c->N), law->G, c->rc_kappa * c->rc_kappa,
+                       (const int32_t*)c->stats, c->rc_cnt, c->rc_list, p->ax, p->ay);
+    hipLaunchKernelGGL(k_rc_groups, dim3(1), dim3(256), 0, st, (const int32_t*)c->rc_cnt, c->S,
+                       c->rc_gofs, c->stats);
+    const unsigned g = (unsigned)((int64_t)c->num_cu * 4);
+    if (law->r2_cut > 0.0)
+        hipLaunchKernelGGL(k_rc_fix64<1>, dim3(g), dim3(RC_THREADS), 0, st,
+                           (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
+                           (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
+                           (const SysDev*)c->sys, (const int32_t*)c->key_sorted,
+                           (const int32_t*)c->offsets, (const int32_t*)c->neprefix,
+                           (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
+                           (const double*)p->mass, law->G, law->eps2, law->r2_cut, c->rc_part,
+                           p->ax, p->ay);
+    else
+        hipLaunchKernelGGL(k_rc_fix64<0>, dim3(g), dim3(RC_THREADS), 0, st,
+                           (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
+                           (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
+                           (const SysDev*)c->sys, (const int32_t*)c->key_sorted,
+                           (const int32_t*)c->offsets, (const int32_t*)c->neprefix,
+                           (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
+                           (const double*)p->mass, law->G, law->eps2, law->r2_cut, c->rc_part,
+                           p->ax, p->ay);
+    hipLaunchKernelGGL(k_rc_combine, dim3(grid_for((int64_t)RC_PART_CAP * RC_GROUP, 256, 512)),
+                       dim3(256), 0, st, (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
+                       (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
+                       (const SysDev*)c->sys, (const double*)c->rc_part, law->G, p->ax, p->ay);
+}
+
 // Whether an FP32 pass goes by shared chunks (k_force32s) or by the queue of
 // work items (k_force32).  Chunks were faster on all of 28 single systems from
 // 2,000 to 4M particles but the densest (4M clustered particles on 30^2 cells,
@@ -977,21 +1029,29 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     ForceArgs fa;
     if ((precision == 0 || precision == 1) && (c->fmm_on >> precision & 1) && !c->cost_log_on) {
         // Grouped far field: its chunks replace the work items, so the queue
-        // order does not enter.  Near and mid terms are FP64 in both
-        // precisions: nothing is left for the recompute to mend.
+        // order does not enter.  An FP64 pass's sums are complete.  An FP32 pass's
+        // are FP64 too, but their far part is interpolated to ~1e-10 of it: the
+        // particles whose terms nearly cancel are recomputed here, term by term,
+        // and a call to bh_recompute finds nothing left.
         FmmArgs A = c->fa[precision];
         A.x = p->px;
         A.y = p->py;
         A.m = p->mass;
-        A.ax = p->ax;
-        A.ay = p->ay;
         const bool rc = precision == 1 && c->rc_kappa > 0.0;
+        A.ax = rc ? c->rc_a32 : p->ax;
+        A.ay = rc ? c->rc_a32 + c->N : p->ay;
+        A.s2n = rc ? c->rc_a32 + 2 * c->N : nullptr;
         if (part == 0) c->rc_ready = 0;
         bh_fmm_pass(A, c->fmm[precision], precision == 0, law->G, law->eps2, law->r2_cut, part, nparts,
                     c->num_cu, st);
         if (part == nparts - 1) {
-            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
-                               (int64_t)2, 0);
+            if (rc && law->G != 0.0) {
+                recompute(c, p, law, st);
+                hipLaunchKernelGGL(k_rc_grouped, dim3(1), dim3(64), 0, st, c->stats);
+            } else {
+                hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
+                                   (int64_t)4, 0);
+            }
             c->rc_ready = rc ? 2 : 0;
         }
         LAUNCH_CHECK("evaluate");
@@ -1070,7 +1130,7 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
     }
     if (!rc)   // the recomputed count describes the last pass
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP,
-                           (int64_t)2, 0);
+                           (int64_t)4, 0);
     LAUNCH_CHECK("evaluate");
     c->rc_ready = rc ? 1 : 0;
     if (rc && !c->rc_deferred) return bh_recompute(ctx, p, law, stream);
@@ -1098,59 +1158,13 @@ int bh_recompute(void* ctx, const bh_particles* p, const bh_law* law, void* stre
     if (!(law->eps2 >= 0.0) || !(law->r2_cut >= 0.0) || !std::isfinite(law->G))
         return fail(BH_EINVAL, "law needs finite G, eps2 >= 0, r2_cut >= 0");
     if (!c->rc_ready) return fail(BH_ESTATE, "no FP32 force pass prepared a recompute");
-    if (c->rc_ready == 2) return BH_OK;   // the pass formed its sums in FP64: nothing flagged
+    if (c->rc_ready == 2) return BH_OK;   // a grouped pass: done in the pass
     hipStream_t st = (hipStream_t)stream;
-    if (law->G == 0.0) {   // every term, and so the FP32 result, is zero
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP, (int64_t)2,
+    if (law->G == 0.0)   // every term, and so the FP32 result, is zero
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->stats + ST_NRECOMP, (int64_t)4,
                            0);
-        return BH_OK;
-    }
-    const int64_t ntiles = c->nblocks * (RC_BLOCK / RC_TILE) * (RC_BLOCK / RC_TILE);
-    const unsigned nb = grid_for(c->nblocks, 4, (int64_t)c->num_cu * 4);
-    hipLaunchKernelGGL(k_rc_sums, dim3(nb + grid_for(ntiles, 256, (int64_t)c->num_cu * 8)),
-                       dim3(256), 0, st, (const SysDev*)c->sys, c->S, c->nblocks, ntiles, (int)nb,
-                       (const double*)c->com_dense, c->rc_blk, c->rc_tiles, c->rc_cnt, c->stats);
-    hipLaunchKernelGGL(k_rc_blockfar, dim3(grid_for(c->nblocks, 1, (int64_t)c->num_cu * 16)),
-                       dim3(64), 0, st, (const SysDev*)c->sys, c->S, c->nblocks,
-                       (const double*)c->rc_blk, c->rc_bfar);
-    // four waves an item where items of 64 P particles span 16 rows and more on
-    // average and do not fill the chip by themselves (k_rc_flag)
-    const bool wide = c->C * 64 * c->tune.p >= 16 * c->N && c->N <= (int64_t)c->num_cu * 4096;
-    hipLaunchKernelGGL(wide ? k_rc_flag<4> : k_rc_flag<1>,
-                       dim3(grid_for(c->max_items, 1, (int64_t)c->num_cu * 32)),
-                       dim3(wide ? 256 : 64), 0, st, (const Item*)c->items, (const SysDev*)c->sys,
-                       (const int32_t*)c->key_sorted, (const int32_t*)c->neprefix,
-                       (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
-                       (const double*)c->com_dense, (const double*)c->rc_tiles,
-                       (const double*)c->rc_blk, (const double*)c->rc_bfar,
-                       (const double*)c->rc_a32, (const double*)(c->rc_a32 + c->N),
-                       (const double*)(c->rc_a32 + 2 * c->N), law->G, c->rc_kappa * c->rc_kappa,
-                       (const int32_t*)c->stats, c->rc_cnt, c->rc_list, p->ax, p->ay);
-    hipLaunchKernelGGL(k_rc_groups, dim3(1), dim3(256), 0, st, (const int32_t*)c->rc_cnt, c->S,
-                       c->rc_gofs, c->stats);
-    const unsigned g = (unsigned)((int64_t)c->num_cu * 4);
-    if (law->r2_cut > 0.0)
-        hipLaunchKernelGGL(k_rc_fix64<1>, dim3(g), dim3(RC_THREADS), 0, st,
-                           (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
-                           (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
-                           (const SysDev*)c->sys, (const int32_t*)c->key_sorted,
-                           (const int32_t*)c->offsets, (const int32_t*)c->neprefix,
-                           (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
-                           (const double*)p->mass, law->G, law->eps2, law->r2_cut, c->rc_part,
-                           p->ax, p->ay);
     else
-        hipLaunchKernelGGL(k_rc_fix64<0>, dim3(g), dim3(RC_THREADS), 0, st,
-                           (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
-                           (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
-                           (const SysDev*)c->sys, (const int32_t*)c->key_sorted,
-                           (const int32_t*)c->offsets, (const int32_t*)c->neprefix,
-                           (const Com64*)c->l64, (const double*)p->px, (const double*)p->py,
-                           (const double*)p->mass, law->G, law->eps2, law->r2_cut, c->rc_part,
-                           p->ax, p->ay);
-    hipLaunchKernelGGL(k_rc_combine, dim3(grid_for((int64_t)RC_PART_CAP * RC_GROUP, 256, 512)),
-                       dim3(256), 0, st, (const int32_t*)c->stats, (const int32_t*)c->rc_cnt,
-                       (const int32_t*)c->rc_gofs, c->S, (const int32_t*)c->rc_list,
-                       (const SysDev*)c->sys, (const double*)c->rc_part, law->G, p->ax, p->ay);
+        recompute(c, p, law, st);
     LAUNCH_CHECK("recompute");
     return BH_OK;
 }

@@ -28,6 +28,7 @@ enum {
     ST_NPASS = 5,      // merge passes the within-cell sort needed
     ST_NRECOMP = 6,    // particles flagged for the FP64 recompute (last FP32 pass)
     ST_RCGROUPS = 7,   // their groups (up to RC_GROUP particles of one system)
+    ST_NGROUPED = 8,   // the same two of a grouped pass, which recomputes by itself
     ST_COUNT = 16
 };
 

@@ -689,10 +689,10 @@ __global__ __launch_bounds__(256) void k_fmm_pack(FmmArgs A)
 // k_force64s, which loads ahead, the branch costs 5 to 8 % on clusters.)
 // (Loading a quad ahead, as k_force64s does, is 5 % slower here: the second set of
 // registers spills scalars that the outer loops hold.)
-template <int LAW>
+template <int LAW, bool SQ>
 __device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int g0, int g1, int gi,
                                           double x, double y, double eps2, double r2cut, int step,
-                                          double& sx, double& sy)
+                                          double& sx, double& sy, double& s2)
 {
     const cptr<FmmPart> E = as_const(pack);
     for (; j + 3 < b; j += step) {
@@ -701,28 +701,28 @@ __device__ __forceinline__ void near_cell(const FmmPart* pack, int j, int b, int
         const double wy[4] = {p[1] - y, p[5] - y, q[1] - y, q[5] - y};
         const double m[4] = {p[2], p[6], q[2], q[6]};
         if (j + 3 < g0 || j > g1)
-            quad_terms<LAW, false>(wx, wy, m, {true, true, true, true}, eps2, r2cut, sx, sy);
+            quad_terms<LAW, false, SQ>(wx, wy, m, {true, true, true, true}, eps2, r2cut, sx, sy, &s2);
         else
-            quad_terms<LAW, true>(wx, wy, m, {j != gi, j + 1 != gi, j + 2 != gi, j + 3 != gi},
-                                  eps2, r2cut, sx, sy);
+            quad_terms<LAW, true, SQ>(wx, wy, m, {j != gi, j + 1 != gi, j + 2 != gi, j + 3 != gi},
+                                  eps2, r2cut, sx, sy, &s2);
     }
     if (j + 1 < b) {
         const fd8 p = *(cptr<fd8>)(E + j);
-        pair_terms<LAW, true>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
-                              j + 1 != gi, eps2, r2cut, sx, sy);
+        pair_terms<LAW, true, SQ>(p[0] - x, p[1] - y, p[2], p[4] - x, p[5] - y, p[6], j != gi,
+                              j + 1 != gi, eps2, r2cut, sx, sy, &s2);
         j += 2;
     }
     if (j < b)   // the last of an odd count, with a copy of itself without mass
-        pair_terms<LAW, true>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0, j != gi,
-                              j != gi, eps2, r2cut, sx, sy);
+        pair_terms<LAW, true, SQ>(E[j].x - x, E[j].y - y, E[j].m, E[j].x - x, E[j].y - y, 0.0, j != gi,
+                              j != gi, eps2, r2cut, sx, sy, &s2);
 }
 
 // A lane's own near candidates in column xc (OWN: its own column, which holds
 // the particle itself), every W-th pair from the w-th on.  gi < 0: no particle.
-template <int LAW, bool OWN>
+template <int LAW, bool OWN, bool SQ>
 __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G, int xc, int cy,
                                            int gi, int w, int W, double x, double y, double eps2,
-                                           double r2cut, double& sx, double& sy)
+                                           double r2cut, double& sx, double& sy, double& s2)
 {
     if (gi < 0 || xc < 0 || xc >= G) return;
     const int64_t cl = coff + (int64_t)xc * G;
@@ -733,8 +733,8 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
         const bool two = j + 1 < b;
         const FmmPart* E1 = two ? E + 1 : E;
         const double m1 = two ? E1->m : 0.0;
-        pair_terms<LAW, OWN>(E->x - x, E->y - y, E->m, E1->x - x, E1->y - y, m1, j != gi,
-                             (two ? j + 1 : j) != gi, eps2, r2cut, sx, sy);
+        pair_terms<LAW, OWN, SQ>(E->x - x, E->y - y, E->m, E1->x - x, E1->y - y, m1, j != gi,
+                             (two ? j + 1 : j) != gi, eps2, r2cut, sx, sy, &s2);
     }
 }
 
@@ -748,10 +748,12 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
 // loads and a row test; otherwise each lane walks its own three ranges with
 // vector loads (a union would spend most of its terms on the test).  Terms go in
 // quads, or a lane's own in pairs, that share a reciprocal; only quads that hold
-// the lanes themselves are tested for the particle itself.
-template <int P, int LAW>
+// the lanes themselves are tested for the particle itself.  SQ: r2 is the sum of
+// the near terms' (m / r)^2, r in cell sides, for the FP64 recompute's bound.
+template <int P, int LAW, bool SQ>
 __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int W, double eps2p,
-                                            double r2cutp, int& gi, double& rx, double& ry)
+                                            double r2cutp, int& gi, double& rx, double& ry,
+                                            double& r2)
 {
     constexpr int Q = P * P;
     const int lane = threadIdx.x & 63;
@@ -779,7 +781,7 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
         r -= b - a;
     }
     const bool act = gi >= 0;
-    double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, fx = 0.0, fy = 0.0;
+    double x = 0.0, y = 0.0, sx = 0.0, sy = 0.0, s2 = 0.0, fx = 0.0, fy = 0.0;
     int cx = -100000, cy = -100000;
     if (act) {
         const FmmPart p = A.pack[gi];
@@ -813,13 +815,14 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
                 const int j = a + 4 * ((w - turn) & (W - 1));
                 turn += (b - a + 3) >> 2;
                 if (!(act && abs(row - cy) <= 1)) continue;
-                near_cell<LAW>(A.pack, j, b, g0, g1, gi, x, y, eps2, r2cut, 4 * W, sx, sy);
+                near_cell<LAW, SQ>(A.pack, j, b, g0, g1, gi, x, y, eps2, r2cut, 4 * W, sx, sy,
+                                   s2);
             }
         }
     } else {
-        near_range<LAW, false>(A, coff, G, cx - 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
-        near_range<LAW, true>(A, coff, G, cx, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
-        near_range<LAW, false>(A, coff, G, cx + 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy);
+        near_range<LAW, false, SQ>(A, coff, G, cx - 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy, s2);
+        near_range<LAW, true, SQ>(A, coff, G, cx, cy, gi, w, W, x, y, eps2, r2cut, sx, sy, s2);
+        near_range<LAW, false, SQ>(A, coff, G, cx + 1, cy, gi, w, W, x, y, eps2, r2cut, sx, sy, s2);
     }
 
     // mid entries: 3x3 tiles, or every tile where the grouped part does not
@@ -911,17 +914,27 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
     }
     rx = fma(sx, sig, fx);
     ry = fma(sy, sig, fy);
+    if (SQ) r2 = s2 * ((step * sig) * (step * sig));
+}
+
+// A particle's sums as the pass leaves them: added to its acceleration, or (SQ)
+// in the recompute's planes, which add them or the FP64 terms in their place.
+template <bool SQ>
+__device__ __forceinline__ void put_sum(double* a, int gi, double v)
+{
+    if (SQ) a[gi] = v;
+    else a[gi] += v;
 }
 
 // Chunks of dense tiles, each shared by the eight waves of a block: a particle
 // of a cluster's core may have 10^4 near candidates where the others have a
 // hundred, and on a wave of its own such a chunk would outlast the rest of the
 // pass.  1M particles, 400^2 cells, cores of 10^3 a cell: 10.7 -> 7.9 ms.
-template <int P, int LAW>
+template <int P, int LAW, bool SQ>
 __global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double Gc, double eps2,
                                                               double r2cut, int qpart, int nqparts)
 {
-    __shared__ double part[2][FMM_WAVES][BH_WAVE];
+    __shared__ double part[SQ ? 3 : 2][FMM_WAVES][BH_WAVE];
     __shared__ int unit;
     const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
     const int64_t n = A.cnt[FMM_HEAVY];
@@ -933,17 +946,18 @@ __global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double 
         const int ci = uniform_int(unit);
         if (ci >= q1) break;
         int gi;
-        double rx, ry;
-        chunk_terms<P, LAW>(A, ci, w, FMM_WAVES, eps2, r2cut, gi, rx, ry);
+        double rx, ry, r2;
+        chunk_terms<P, LAW, SQ>(A, ci, w, FMM_WAVES, eps2, r2cut, gi, rx, ry, r2);
         part[0][w][lane] = rx;
         part[1][w][lane] = ry;
+        if (SQ) part[SQ ? 2 : 0][w][lane] = r2;
         __syncthreads();
-        if (w < 2 && gi >= 0) {   // wave 0 adds x, wave 1 adds y
+        if (w < (SQ ? 3 : 2) && gi >= 0) {   // wave 0 adds x, wave 1 y, wave 2 the near squares
             double t = 0.0;
 #pragma unroll
             for (int v = 0; v < FMM_WAVES; ++v) t += part[w][v][lane];
-            double* a = w ? A.ay : A.ax;
-            a[gi] += Gc * t;
+            if (SQ && w == 2) A.s2n[gi] = t;
+            else put_sum<SQ>(w ? A.ay : A.ax, gi, Gc * t);
         }
     }
 }
@@ -956,7 +970,7 @@ __global__ __launch_bounds__(64 * FMM_WAVES) void k_fmm_dense(FmmArgs A, double 
 // ms on 512 systems (7.1 with tiles of 6); 2.16 and 9.9 ms with terms in pairs
 // and every entry of a tile that the 3x3 cells touch tested, 2.8 and 12.8 ms with
 // entries loaded one by one.
-template <int P, int LAW>
+template <int P, int LAW, bool SQ>
 __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double eps2, double r2cut,
                                                   int qpart, int nqparts)
 {
@@ -964,11 +978,12 @@ __global__ __launch_bounds__(64) void k_fmm_force(FmmArgs A, double Gc, double e
     const int q0 = (int)(n * qpart / nqparts), q1 = (int)(n * (qpart + 1) / nqparts);
     for (int u = q0 + blockIdx.x; u < q1; u += gridDim.x) {
         int gi;
-        double rx, ry;
-        chunk_terms<P, LAW>(A, (int)(A.max_chunks - 1 - u), 0, 1, eps2, r2cut, gi, rx, ry);
+        double rx, ry, r2;
+        chunk_terms<P, LAW, SQ>(A, (int)(A.max_chunks - 1 - u), 0, 1, eps2, r2cut, gi, rx, ry, r2);
         if (gi >= 0) {
-            A.ax[gi] += Gc * rx;
-            A.ay[gi] += Gc * ry;
+            put_sum<SQ>(A.ax, gi, Gc * rx);
+            put_sum<SQ>(A.ay, gi, Gc * ry);
+            if (SQ) A.s2n[gi] = r2;
         }
     }
 }
@@ -999,21 +1014,17 @@ static void fmm_prepare(const FmmArgs& A, const FmmPlan& pl, double eps2, int nu
                            dim3(FMM_THREADS), 0, st, A, tb.shift, tb.cheb, tb.fine, l);
 }
 
-template <int P>
+template <int P, int LAW, bool SQ>
 static void fmm_force(const FmmArgs& A, double Gc, double eps2, double r2cut, int part, int nparts,
                       int num_cu, hipStream_t st)
 {
     if (part > 0)   // the queue of this launch
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, A.cnt + FMM_QHEAVY, (int64_t)1, 0);
     const int64_t cap = A.max_chunks, most = (int64_t)num_cu * 256;
-    const dim3 gd(num_cu * 4), bd(64 * FMM_WAVES), g((unsigned)(cap < most ? cap : most)), b(64);
-    if (r2cut > 0.0) {
-        hipLaunchKernelGGL((k_fmm_dense<P, 1>), gd, bd, 0, st, A, Gc, eps2, r2cut, part, nparts);
-        hipLaunchKernelGGL((k_fmm_force<P, 1>), g, b, 0, st, A, Gc, eps2, r2cut, part, nparts);
-    } else {
-        hipLaunchKernelGGL((k_fmm_dense<P, 0>), gd, bd, 0, st, A, Gc, eps2, r2cut, part, nparts);
-        hipLaunchKernelGGL((k_fmm_force<P, 0>), g, b, 0, st, A, Gc, eps2, r2cut, part, nparts);
-    }
+    hipLaunchKernelGGL((k_fmm_dense<P, LAW, SQ>), dim3(num_cu * 4), dim3(64 * FMM_WAVES), 0, st, A,
+                       Gc, eps2, r2cut, part, nparts);
+    hipLaunchKernelGGL((k_fmm_force<P, LAW, SQ>), dim3((unsigned)(cap < most ? cap : most)),
+                       dim3(64), 0, st, A, Gc, eps2, r2cut, part, nparts);
 }
 
 void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, double eps2,
@@ -1023,6 +1034,9 @@ void bh_fmm_pass(const FmmArgs& A, const FmmPlan& pl, bool fp64, double Gc, doub
         if (fp64) fmm_prepare<FMM_P64>(A, pl, eps2, num_cu, st);
         else fmm_prepare<FMM_P32>(A, pl, eps2, num_cu, st);
     }
-    if (fp64) fmm_force<FMM_P64>(A, Gc, eps2, r2cut, part, nparts, num_cu, st);
-    else fmm_force<FMM_P32>(A, Gc, eps2, r2cut, part, nparts, num_cu, st);
+    const bool law = r2cut > 0.0, sq = A.s2n != nullptr;
+    const auto force = fp64 ? (law ? fmm_force<FMM_P64, 1, false> : fmm_force<FMM_P64, 0, false>)
+                     : sq   ? (law ? fmm_force<FMM_P32, 1, true> : fmm_force<FMM_P32, 0, true>)
+                            : (law ? fmm_force<FMM_P32, 1, false> : fmm_force<FMM_P32, 0, false>);
+    force(A, Gc, eps2, r2cut, part, nparts, num_cu, st);
 }

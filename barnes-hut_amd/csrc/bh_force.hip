@@ -572,7 +572,7 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
         }
         s = uniform_int(s);
     }
-    if (blockIdx.x == 0 && threadIdx.x < 2) A.stats[ST_NRECOMP + threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 4) A.stats[ST_NRECOMP + threadIdx.x] = 0;
     const SysDev& d = A.sys[s];
     const int G = d.G;
     const int64_t coff = d.c_off;

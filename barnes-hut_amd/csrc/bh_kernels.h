@@ -139,6 +139,7 @@ struct FmmArgs {
     const Com64* l64;
     const double *x, *y, *m;
     double *ax, *ay;
+    double* s2n;               // the near terms' (m / r)^2, if the recompute follows
     const FmmTile* tiles;      // every square, level by level
     const FmmGroup* groups;
     int32_t *tcnt;             // per square: particles
@@ -297,10 +298,12 @@ __device__ __forceinline__ double rcp64(double q)
 // cutoff, a wave none of whose lanes drops either term (all but the closest
 // pairs) takes the plain form after one test of the smaller distance: ~14 issue
 // slots a term instead of 19 with a select per q and weight.
-template <int LAW, bool MASK>
+// SQ: s2 gains the sum of m w, which is (m / r)^2, r softened.
+template <int LAW, bool MASK, bool SQ = false>
 __device__ __forceinline__ void pair_terms(double wx0, double wy0, double m0, double wx1,
                                            double wy1, double m1, bool k0, bool k1, double eps2,
-                                           double r2cut, double& sx, double& sy)
+                                           double r2cut, double& sx, double& sy,
+                                           double* s2 = nullptr)
 {
     double q0, q1;
     bool sel = MASK;   // wave-uniform
@@ -334,6 +337,7 @@ __device__ __forceinline__ void pair_terms(double wx0, double wy0, double m0, do
     sy = fma(wy0, w0, sy);
     sx = fma(wx1, w1, sx);
     sy = fma(wy1, w1, sy);
+    if (SQ) *s2 = fma(m1, w1, fma(m0, w0, *s2));
 }
 
 // Four terms from one reciprocal: pairs are brought to common denominators,
@@ -341,10 +345,11 @@ __device__ __forceinline__ void pair_terms(double wx0, double wy0, double m0, do
 // instructions and one reciprocal (of several issue slots) after the
 // separations, where two pairs take 34 and two: 10M particles over 120^2 cells,
 // 6.7e10 terms, 26.5 -> 24.3 ms.
-template <int LAW, bool MASK>
+template <int LAW, bool MASK, bool SQ = false>
 __device__ __forceinline__ void quad_terms(const double (&wx)[4], const double (&wy)[4],
                                            const double (&m)[4], const bool (&keep)[4],
-                                           double eps2, double r2cut, double& sx, double& sy)
+                                           double eps2, double r2cut, double& sx, double& sy,
+                                           double* s2 = nullptr)
 {
     double q[4], t[4];
     bool k[4] = {keep[0], keep[1], keep[2], keep[3]};
@@ -383,6 +388,10 @@ __device__ __forceinline__ void quad_terms(const double (&wx)[4], const double (
     sy = fma(ny0, u0, sy);
     sx = fma(nx1, u1, sx);
     sy = fma(ny1, u1, sy);
+    if (SQ) {
+        *s2 = fma(fma(m[1], t[1], m[0] * t[0]), u0, *s2);
+        *s2 = fma(fma(m[3], t[3], m[2] * t[2]), u1, *s2);
+    }
 }
 
 // grid-method potential
@@ -459,6 +468,7 @@ __global__ void k_force_combine(const Item* items, const int32_t* order, const i
                                 int64_t part_n, double* ax, double* ay);
 // FP64 recompute of the particles whose FP32 rounding-error estimate is
 // large against their acceleration
+__global__ void k_rc_grouped(int32_t* stats);
 __global__ void k_rc_sums(const SysDev* sys, int S, int64_t nblocks, int64_t ntiles, int nb,
                           const double* com_dense, double* blk, double* tl, int32_t* rc_cnt,
                           int32_t* stats);

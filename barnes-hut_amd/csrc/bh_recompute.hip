@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void k_rc_sums(const SysDev* __restrict__ sys,
 {
     if (blockIdx.x == 0) {
         for (int s = threadIdx.x; s < S; s += 256) rc_cnt[s] = 0;
-        if (threadIdx.x < 2) stats[ST_NRECOMP + threadIdx.x] = 0;
+        if (threadIdx.x < 4) stats[ST_NRECOMP + threadIdx.x] = 0;
     }
     if ((int)blockIdx.x < nb) rc_blocks(sys, S, nblocks, com_dense, blk, blockIdx.x, nb);
     else rc_tiles(sys, S, ntiles, com_dense, tl, blockIdx.x - nb, gridDim.x - nb);
@@ -435,6 +435,16 @@ __global__ __launch_bounds__(256) void k_rc_groups(const int32_t* __restrict__ r
         stats[ST_NRECOMP] = carry_n;
         stats[ST_RCGROUPS] = carry_g;
     }
+}
+
+// A grouped pass's counts to their own place, off the list of an FP32 pass whose
+// recompute the caller may run.
+__global__ void k_rc_grouped(int32_t* stats)
+{
+    const int k = threadIdx.x;
+    if (k >= 2) return;
+    stats[ST_NGROUPED + k] = stats[ST_NRECOMP + k];
+    stats[ST_NRECOMP + k] = 0;
 }
 
 template <int LAW>

@@ -47,8 +47,9 @@ enum {
                                     quotient).  Passes of 2e9 far terms and more group
                                     the far field (to about 1e-15 of it) */
     BH_PREC_FP32_KAHAN = 1,      /* FP32 cell-relative, tile sums in FP64 or Kahan-summed.
-                                    Passes of 2e10 far terms and more group the far
-                                    field (to about 1e-10 of it) and are FP64 */
+                                    Passes of 2e10 far terms and more are summed in
+                                    FP64 with the far field grouped (to about 1e-10
+                                    of it) */
     BH_PREC_FP32_KAHAN_TERM = 2, /* FP32 cell-relative, Kahan per term */
     BH_PREC_FP32_PLAIN = 3,      /* FP32 cell-relative, uncompensated */
     BH_PREC_FP32_MFMA = 4,       /* FP32 cell-relative, far-field sums on the matrix cores,
@@ -158,12 +159,14 @@ int bh_tick_particles(void* ctx, const bh_particles* p, double dt, void* stream)
  * like eps32 * B, so particles with B > kappa * |a| (a in the law's units
  * divided by G / step) are evaluated again with the FP64 kernel's terms and
  * their FP32 result is replaced.  bh_read_stats()[6] is the number of
- * particles recomputed by the last pass (0 after a grouped pass: its sums are
- * FP64, and bh_recompute after it has nothing to do).  kappa <= 0 turns it off (then the
+ * particles recomputed by the last pass.  kappa <= 0 turns it off (then the
  * FP32 pass writes no per-particle scratch).  deferred = 0: bh_force_pass,
  * bh_evaluate_boxes and the step calls run it; deferred = 1: bh_force_pass
  * stops after the FP32 kernels and the caller runs bh_recompute before
- * anything else touches the particles (the step calls still run it).
+ * anything else touches the particles (the step calls still run it).  A
+ * grouped FP32 pass takes the same particles term by term in the pass itself,
+ * deferred or not: their number is bh_read_stats()[8], [6] stays 0, and
+ * bh_recompute after it has nothing left to do.
  * Default: kappa 1.5, deferred 0. */
 int bh_set_recompute(void* ctx, double kappa, int32_t deferred);
 /* The recompute stage alone, for the last FP32 bh_force_pass on p (same law);
@@ -189,7 +192,8 @@ int bh_step_learned(void* ctx, const bh_particles* a, const bh_particles* b, con
 
 /* Synchronises the stream, copies the int32 stats block (16 entries:
  * [0] error bits, [1] max cell count, [2] work items, [4] non-empty cells,
- * [6] particles recomputed in FP64 by the last FP32 pass, [7] their groups)
+ * [6] particles recomputed in FP64 by the last FP32 pass, [7] their groups,
+ * [8] and [9] the same of a grouped FP32 pass)
  * to host memory out16, and returns BH_EDEVICE if an error bit is set. */
 int bh_read_stats(void* ctx, int32_t* out16, void* stream);
 /* Copies state `what` into dst (device or host memory), count elements. */
