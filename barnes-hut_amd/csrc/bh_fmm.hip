@@ -887,6 +887,34 @@ __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int
         }
     }
 
+    // terms one by one (see one_term), by all waves of the chunk (SQ: the
+    // recompute takes particles whose sums are not finite)
+    const bool bad = !SQ && !is_finite(sx, sy);
+    if (!SQ && (W > 1 ? (bool)__syncthreads_or(bad) : __any(bad))) {
+        sx = sy = 0.0;
+        for (int xc = max(cx - 1, 0); act && xc <= min(cx + 1, G - 1); ++xc) {
+            const int64_t cl = coff + (int64_t)xc * G;
+            const int b = A.offsets[cl + min(cy + 1, G - 1) + 1];
+#pragma unroll 1
+            for (int j = A.offsets[cl + max(cy - 1, 0)] + w; j < b; j += W) {
+                const FmmPart q = A.pack[j];
+                one_term<LAW>(q.x - x, q.y - y, q.m, j != gi, eps2, r2cut, sx, sy);
+            }
+        }
+        for (int mx = mx0; mx <= mx1; ++mx) {
+            for (int my = my0; my <= my1; ++my) {
+                const int mt = fs.off[0] + mx * nt + my;
+                const int e0 = A.tstart[mt], ne = A.tne[mt];
+#pragma unroll 1
+                for (int e = e0 + w; e < e0 + ne; e += W) {
+                    const FmmCom f = A.list[e];
+                    one_term<LAW>(f.X - x, f.Y - y, f.M, abs(f.kx - cx) > 1 || abs(f.ky - cy) > 1,
+                                  eps2, r2cut, sx, sy);
+                }
+            }
+        }
+    }
+
     // distant part: the tile's Chebyshev series
     if (!all && act) {
         double ty[P];

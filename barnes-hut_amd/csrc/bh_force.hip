@@ -691,6 +691,23 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
             q = qn;
         }
     }
+    if (__syncthreads_or(!is_finite(sx, sy))) {   // one by one (see one_term)
+        sx = sy = 0.0;
+        for (int xc = max(cx - 1, 0); act && xc <= min(cx + 1, G - 1); ++xc) {
+            const int64_t cl = coff + (int64_t)xc * G;
+            const int b = A.offsets[cl + min(cy + 1, G - 1) + 1];
+#pragma unroll 1
+            for (int j = A.offsets[cl + max(cy - 1, 0)] + w; j < b; j += W)
+                one_term<LAW>(fma(A.x[j], sig, -x), fma(A.y[j], sig, -y), A.m[j], j != gi, eps2,
+                              r2cut, sx, sy);
+        }
+#pragma unroll 1
+        for (int e = f0; e < f1; ++e) {
+            const Com64 f = A.l64[e];
+            one_term<LAW>(fma(f.X, sig, -x), fma(f.Y, sig, -y), f.M,
+                          abs(f.kx - cx) > 1 || abs(f.ky - cy) > 1, eps2, r2cut, sx, sy);
+        }
+    }
     part[0][w][lane] = sx;
     part[1][w][lane] = sy;
     __syncthreads();

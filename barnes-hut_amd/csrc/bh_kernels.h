@@ -394,6 +394,26 @@ __device__ __forceinline__ void quad_terms(const double (&wx)[4], const double (
     }
 }
 
+// One term, by a reciprocal of its own.  The products above leave a double's
+// range where softening is below ~1e-77 cell sides squared (and particles
+// coincide) or above 1e77, and then leave an infinite or NaN sum: the kernels
+// take such a wave's or block's terms again, one by one, which says what the sum
+// is where it is not finite by itself.
+template <int LAW>
+__device__ __forceinline__ void one_term(double wx, double wy, double m, bool keep, double eps2,
+                                         double r2cut, double& sx, double& sy)
+{
+    double w = near_w64<LAW, 1>(wx, wy, m, eps2, r2cut);
+    w = keep ? w : 0.0;
+    sx = fma(wx, w, sx);
+    sy = fma(wy, w, sy);
+}
+
+__device__ __forceinline__ bool is_finite(double sx, double sy)
+{
+    return fabs(sx) < __builtin_huge_val() && fabs(sy) < __builtin_huge_val();
+}
+
 // grid-method potential
 __global__ void k_sys_mass(const SysDev* sys, const int32_t* neprefix, const Com64* l64,
                            double* msys);
