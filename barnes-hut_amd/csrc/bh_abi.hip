@@ -109,6 +109,7 @@ struct bh_ctx_s {
     int fmm_on = 0;          // bit 0: fp64 passes, bit 1: fp32 passes
     FmmPlan fmm[2];          // per precision (0: fp64, 1: fp32)
     FmmArgs fa[2] = {};      // device buffers and sizes; the per-pass fields are set by each pass
+    int fmm_live = -1;       // precision whose far field the shared buffers hold
     hipStream_t cap_stream = nullptr;   // graph capture only; replays run on the caller's stream
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     GraphKey gkey[2];
@@ -329,17 +330,25 @@ static std::vector<double> fmm_table(int P)
     return v;
 }
 
-// Lays out the squares of every system for one precision and allocates the
-// grouped far field's buffers (c->sys_h and the sizes are set).
-static int fmm_configure(Ctx* c, int precision)
+// What the host fills in of a precision's squares.
+struct FmmHost {
+    std::vector<FmmSys> fs;
+    std::vector<FmmTile> tiles;
+    std::vector<FmmGroup> groups;
+    int64_t slots = 0;   // node-mass slots of a plane, all levels
+};
+
+// Lays out the squares of every system for one precision (c->sys_h and the sizes
+// are set).
+static void fmm_squares(Ctx* c, int precision, FmmHost& h)
 {
-    const int P = precision == 0 ? FMM_P64 : FMM_P32, F = fmm_far(P);
+    const int P = precision == 0 ? FMM_P64 : FMM_P32;
     const int S = c->S;
-    std::vector<FmmSys> fs(S);
+    h.fs.resize(S);
     int nlev = 0;
     for (int s = 0; s < S; ++s) {
         const int G = c->sys_h[s].G;
-        FmmSys& f = fs[s];
+        FmmSys& f = h.fs[s];
         std::memset(&f, 0, sizeof(f));
         f.T = fmm_tile(c->sys_h[s].n, G, P);
         f.n[0] = (int32_t)cdiv(G, f.T);
@@ -353,53 +362,58 @@ static int fmm_configure(Ctx* c, int precision)
     FmmPlan& plan = c->fmm[precision];
     FmmArgs& a = c->fa[precision];
     a = FmmArgs{};
-    std::vector<FmmTile> tiles;
-    std::vector<FmmGroup> groups;
-    int64_t slots = 0;
     // 64 targets share a wave's slice of the law; where that leaves fewer waves
     // than SIMDs, 16 (a wave then takes 0.3 instead of 0.8 ms at P = 20)
     int64_t squares = 0;
-    for (const FmmSys& f : fs)
+    for (const FmmSys& f : h.fs)
         for (int l = 0; l < f.nlev; ++l) squares += (int64_t)f.n[l] * f.n[l];
     const int gsize = squares < 64 * 48 ? 16 : 64;
     for (int l = 0; l < nlev; ++l) {
-        a.lev_off[l] = (int64_t)tiles.size();
+        a.lev_off[l] = (int64_t)h.tiles.size();
         for (int s = 0; s < S; ++s) {
-            FmmSys& f = fs[s];
+            FmmSys& f = h.fs[s];
             if (l >= std::max(f.nlev, 1)) continue;
-            f.off[l] = (int32_t)tiles.size();
+            f.off[l] = (int32_t)h.tiles.size();
             const int n = f.n[l];
             for (int x = 0; x < n; ++x)
-                for (int y = 0; y < n; ++y) tiles.push_back({s, (int16_t)x, (int16_t)y});
+                for (int y = 0; y < n; ++y) h.tiles.push_back({s, (int16_t)x, (int16_t)y});
             if (f.nlev == 0) continue;
-            f.moff[l] = slots;
-            slots += fmm_plane(n);
+            f.moff[l] = h.slots;
+            h.slots += fmm_plane(n);
             for (int p = 0; p < 4; ++p) {
                 const int ga = p >> 1, gb = p & 1;
                 const int cnt = ((n - ga + 1) / 2) * ((n - gb + 1) / 2);
                 for (int t0 = 0; t0 < cnt; t0 += gsize)
-                    groups.push_back({s, t0, std::min(gsize, cnt - t0), (int16_t)l, (int8_t)ga,
-                                      (int8_t)gb});
+                    h.groups.push_back({s, t0, std::min(gsize, cnt - t0), (int16_t)l, (int8_t)ga,
+                                        (int8_t)gb});
             }
         }
     }
-    for (int l = nlev; l <= FMM_LEVELS; ++l) a.lev_off[l] = (int64_t)tiles.size();
+    for (int l = nlev; l <= FMM_LEVELS; ++l) a.lev_off[l] = (int64_t)h.tiles.size();
     a.S = S;
     a.N = c->N;
     a.nleaf = a.lev_off[1];
-    a.ntiles = (int64_t)tiles.size();
+    a.ntiles = (int64_t)h.tiles.size();
     a.max_chunks = cdiv(c->N, 64) + a.nleaf;
     plan.nlev = nlev;
-    plan.ngroups = (int64_t)groups.size();
+    plan.ngroups = (int64_t)h.groups.size();
+}
+
+// The grouped far field's buffers for the precisions in `wanted` (fmm_wanted), in
+// one allocation (each costs ~50 us): first what the host fills in, then the node
+// masses, whose borders stay zero, then what every pass forms anew, which the
+// two precisions share.
+static int fmm_configure(Ctx* c, int wanted)
+{
     static const std::vector<double> tabs[2] = {fmm_table(FMM_P64), fmm_table(FMM_P32)};
-    const std::vector<double>& tab = tabs[precision];
-    // one allocation (each costs ~50 us): first what the host fills in, then the
-    // node masses, whose borders stay zero, then the rest
-    FmmSys* dfs = nullptr;
-    FmmTile* dt = nullptr;
-    FmmGroup* dg = nullptr;
-    double* dtab = nullptr;
-    size_t size = 0, host = 0, zero = 0;
+    FmmHost h[2];
+    FmmSys* dfs[2] = {};
+    FmmTile* dt[2] = {};
+    FmmGroup* dg[2] = {};
+    double* dtab[2] = {};
+    for (int i = 0; i < 2; ++i)
+        if (wanted >> i & 1) fmm_squares(c, i, h[i]);
+    size_t size = 0, host = 0, zero = 0, end = 0;
     unsigned char* base = nullptr;
     auto carve = [&](auto*& p, int64_t count) {
         p = base ? (std::remove_reference_t<decltype(p)>)(base + size) : nullptr;
@@ -407,54 +421,75 @@ static int fmm_configure(Ctx* c, int precision)
     };
     auto layout = [&] {
         size = 0;
-        carve(dtab, (int64_t)tab.size());
-        carve(dfs, S);
-        carve(dt, a.ntiles);
-        carve(dg, (int64_t)groups.size());
+        for (int i = 0; i < 2; ++i) {
+            if (!(wanted >> i & 1)) continue;
+            carve(dtab[i], (int64_t)tabs[i].size());
+            carve(dfs[i], c->S);
+            carve(dt[i], (int64_t)h[i].tiles.size());
+            carve(dg[i], (int64_t)h[i].groups.size());
+        }
         host = size;
-        carve(a.mult, slots * P * P);
-        carve(a.multf, slots * F * F);
-        zero = size;
-        carve(a.tcnt, a.ntiles);
-        carve(a.tstart, a.nleaf);
-        carve(a.tne, a.nleaf);
-        carve(a.cnt, FMM_NCNT + S);
-        carve(a.chunks, a.max_chunks);
-        carve(a.list, c->C + 4 * a.nleaf);
-        carve(a.pack, c->N);
-        carve(a.loc, a.ntiles * 2 * P * P);
-        carve(a.locf, a.ntiles * 2 * F * F);
+        for (int i = 0; i < 2; ++i) {
+            if (!(wanted >> i & 1)) continue;
+            const int P = i ? FMM_P32 : FMM_P64, F = fmm_far(P);
+            carve(c->fa[i].mult, h[i].slots * P * P);
+            carve(c->fa[i].multf, h[i].slots * F * F);
+        }
+        zero = end = size;
+        for (int i = 0; i < 2; ++i) {
+            if (!(wanted >> i & 1)) continue;
+            const int P = i ? FMM_P32 : FMM_P64, F = fmm_far(P);
+            FmmArgs& a = c->fa[i];
+            size = zero;
+            carve(a.pack, a.N);
+            carve(a.tcnt, a.ntiles);
+            carve(a.tstart, a.nleaf);
+            carve(a.tne, a.nleaf);
+            carve(a.cnt, FMM_NCNT + a.S);
+            carve(a.chunks, a.max_chunks);
+            carve(a.list, c->C + 4 * a.nleaf);
+            carve(a.loc, a.ntiles * 2 * P * P);
+            carve(a.locf, a.ntiles * 2 * F * F);
+            end = std::max(end, size);
+        }
     };
     layout();
-    int r = dalloc(c, &base, (int64_t)size);
+    int r = dalloc(c, &base, (int64_t)end);
     if (r) return r;
     layout();
     std::vector<unsigned char> up(host);
-    auto fill = [&](const void* dst, const void* src, size_t bytes) {
-        std::memcpy(up.data() + ((const unsigned char*)dst - base), src, bytes);
+    auto fill = [&](const void* dst, const auto& v) {
+        std::memcpy(up.data() + ((const unsigned char*)dst - base), v.data(),
+                    v.size() * sizeof(v[0]));
     };
-    fill(dtab, tab.data(), tab.size() * sizeof(double));
-    plan.tab.nodes = dtab;
-    plan.tab.cheb = dtab + P;
-    plan.tab.shift = plan.tab.cheb + P * P;
-    plan.tab.fnodes = plan.tab.shift + 2 * P * P;
-    plan.tab.fine = plan.tab.fnodes + F;
-    fill(dfs, fs.data(), sizeof(FmmSys) * S);
-    fill(dt, tiles.data(), sizeof(FmmTile) * tiles.size());
-    fill(dg, groups.data(), sizeof(FmmGroup) * groups.size());
+    for (int i = 0; i < 2; ++i) {
+        if (!(wanted >> i & 1)) continue;
+        const int P = i ? FMM_P32 : FMM_P64;
+        FmmTables& tab = c->fmm[i].tab;
+        tab.nodes = dtab[i];
+        tab.cheb = tab.nodes + P;
+        tab.shift = tab.cheb + P * P;
+        tab.fnodes = tab.shift + 2 * P * P;
+        tab.fine = tab.fnodes + fmm_far(P);
+        fill(dtab[i], tabs[i]);
+        fill(dfs[i], h[i].fs);
+        fill(dt[i], h[i].tiles);
+        fill(dg[i], h[i].groups);
+        FmmArgs& a = c->fa[i];
+        a.sbad = a.cnt + FMM_NCNT;
+        a.fsys = dfs[i];
+        a.tiles = dt[i];
+        a.groups = dg[i];
+        a.sys = c->sys;
+        a.sys_of = c->sys_of;
+        a.offsets = c->offsets;
+        a.neprefix = c->neprefix;
+        a.key_sorted = c->key_sorted;
+        a.l64 = c->l64;
+    }
     HIP_TRY(hipMemcpy(base, up.data(), host, hipMemcpyHostToDevice));
     HIP_TRY(hipMemset(base + host, 0, zero - host));
-    a.sbad = a.cnt + FMM_NCNT;
-    a.fsys = dfs;
-    a.tiles = dt;
-    a.groups = dg;
-    a.sys = c->sys;
-    a.sys_of = c->sys_of;
-    a.offsets = c->offsets;
-    a.neprefix = c->neprefix;
-    a.key_sorted = c->key_sorted;
-    a.l64 = c->l64;
-    c->fmm_on |= 1 << precision;
+    c->fmm_on = wanted;
     return BH_OK;
 }
 
@@ -524,6 +559,7 @@ static void unconfigure(Ctx* c)
     c->energy_buf = nullptr;
     c->rc_ready = 0;
     c->fmm_on = 0;
+    c->fmm_live = -1;
 }
 
 // Allocates and initialises the buffers for sizes already validated by
@@ -544,9 +580,8 @@ static int configure(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, i
     HIP_TRY(hipMemset(c->neprefix, 0, sizeof(int32_t) * (C + 1)));
     c->fmm_on = 0;
     const int wanted = fmm_wanted(c->sys_h);
-    for (int precision = 0; precision < 2; ++precision) {
-        const size_t held = c->allocs.size();
-        if (!(wanted >> precision & 1) || fmm_configure(c, precision) == BH_OK) continue;
+    const size_t held = c->allocs.size();
+    if (wanted && fmm_configure(c, wanted) != BH_OK) {
         while (c->allocs.size() > held) {   // no room: these passes stay term by term
             (void)hipFree(c->allocs.back());
             c->allocs.pop_back();
@@ -1041,6 +1076,10 @@ int bh_force_pass_part(void* ctx, const bh_particles* p, const bh_law* law, int3
         A.ax = rc ? c->rc_a32 : p->ax;
         A.ay = rc ? c->rc_a32 + c->N : p->ay;
         A.s2n = rc ? c->rc_a32 + 2 * c->N : nullptr;
+        if (part > 0 && c->fmm_live != precision)
+            return fail(BH_ESTATE, "the far field of this pass's part 0 is gone: a pass of the other "
+                                   "precision ran since");
+        c->fmm_live = precision;
         if (part == 0) c->rc_ready = 0;
         bh_fmm_pass(A, c->fmm[precision], precision == 0, law->G, law->eps2, law->r2_cut, part, nparts,
                     c->num_cu, st);

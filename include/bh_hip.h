@@ -142,7 +142,9 @@ int bh_force_pass(void* ctx, const bh_particles* p, const bh_law* law, int32_t p
 /* bh_force_pass in nparts launches: call it for part = 0 .. nparts-1 in
  * order (same arguments otherwise); part k runs the k-th contiguous range of
  * the work queue or of the particles' chunks (a grouped pass forms the far field
- * in part 0), the last part adds the slices and runs the recompute.  The
+ * in part 0, for this pass alone: a grouped pass of the other precision between
+ * two parts makes the next one BH_ESTATE), the last part adds the slices and runs
+ * the recompute.  The
  * result is bit-identical to bh_force_pass (a particle's sums do not depend
  * on which launch runs its pieces).  For callers that need to return to the
  * host during a long pass (progress, deadlines).  No reference counterpart. */

@@ -52,3 +52,27 @@ def test_kappa_holds_for_grouped_passes(kind, law):
     _pass(eng, law, "fp64")
     assert int(eng.ctx.stats()[8]) == 0
     eng.close()
+
+
+def test_parts_of_two_grouped_passes_are_not_mixed():
+    """FP64 and FP32 passes form their far fields in one scratch: a part whose
+    far field the other precision has replaced is refused, and nothing is added."""
+    from barneshut.kernels.hiplib import BhError
+    n, G, d = _input("clusters")
+    eng = _engine([n], [G], d)
+    eng.ctx.build_items()
+    law = (1e-6, 1e-10, 0.0)
+    want = {p: _pass(eng, law, p) for p in ("fp64", "fp32")}
+    for p, other in (("fp64", "fp32"), ("fp32", "fp64")):
+        eng.ctx.force_pass(eng.parts, *law, p, part=0, nparts=2)
+        eng.ctx.force_pass(eng.parts, *law, other)
+        for k in ("ax", "ay"):
+            eng.parts[k].zero_()
+        with pytest.raises(BhError):
+            eng.ctx.force_pass(eng.parts, *law, p, part=1, nparts=2)
+        assert not eng.parts["ax"].any()
+        for part in range(2):
+            eng.ctx.force_pass(eng.parts, *law, p, part=part, nparts=2)
+        np.testing.assert_array_equal(eng.fetch()["ax"], want[p]["ax"])
+        eng.parts["ax"].zero_()
+    eng.close()
