@@ -130,11 +130,12 @@ static void free_all(Ctx* c)
 }
 
 template <typename T>
-static int dalloc(Ctx* c, T** p, int64_t count)
+static int dalloc(Ctx* c, T** p, int64_t count, bool* no_room = nullptr)
 {
     size_t bytes = (size_t)std::max<int64_t>(count, 1) * sizeof(T);
     void* q = nullptr;
     hipError_t e = hipMalloc(&q, bytes);
+    if (no_room) *no_room = e == hipErrorOutOfMemory;
     if (e != hipSuccess)
         return fail(BH_EHIP, "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
     c->allocs.push_back(q);
@@ -402,7 +403,8 @@ static void fmm_squares(Ctx* c, int precision, FmmHost& h)
 // The grouped far field's buffers for the precisions in `wanted` (fmm_wanted), in
 // one allocation (each costs ~50 us): first what the host fills in, then the node
 // masses, whose borders stay zero, then what every pass forms anew, which the
-// two precisions share.
+// two precisions share.  Without room for them (and only then) the passes stay
+// term by term, which bh_query tells.
 static int fmm_configure(Ctx* c, int wanted)
 {
     static const std::vector<double> tabs[2] = {fmm_table(FMM_P64), fmm_table(FMM_P32)};
@@ -454,7 +456,12 @@ static int fmm_configure(Ctx* c, int wanted)
         }
     };
     layout();
-    int r = dalloc(c, &base, (int64_t)end);
+    bool no_room = false;
+    int r = dalloc(c, &base, (int64_t)end, &no_room);
+    if (no_room) {
+        (void)hipGetLastError();
+        return BH_OK;
+    }
     if (r) return r;
     layout();
     std::vector<unsigned char> up(host);
@@ -580,14 +587,7 @@ static int configure(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, i
     HIP_TRY(hipMemset(c->neprefix, 0, sizeof(int32_t) * (C + 1)));
     c->fmm_on = 0;
     const int wanted = fmm_wanted(c->sys_h);
-    const size_t held = c->allocs.size();
-    if (wanted && fmm_configure(c, wanted) != BH_OK) {
-        while (c->allocs.size() > held) {   // no room: these passes stay term by term
-            (void)hipFree(c->allocs.back());
-            c->allocs.pop_back();
-        }
-        (void)hipGetLastError();
-    }
+    if (wanted && (r = fmm_configure(c, wanted))) return r;
     HIP_TRY(hipDeviceSynchronize());
     return BH_OK;
 }
@@ -1417,6 +1417,14 @@ int bh_query(void* ctx, int32_t what, int64_t* out)
     case 3: *out = c->ncols; break;
     case 4: *out = c->max_items; break;
     case 5: *out = c->num_cu; break;
+    case 6:
+    case 7: *out = !(c->fmm_on >> (what - 6) & 1) ? 0 : what == 6 ? FMM_P64 : FMM_P32; break;
+    case 8:
+    case 9:
+        *out = c->fmm_on >> (what - 8) & 1
+                   ? fmm_tile(c->sys_h[0].n, c->sys_h[0].G, what == 8 ? FMM_P64 : FMM_P32)
+                   : 0;
+        break;
     default: return fail(BH_EINVAL, "unknown query " + std::to_string(what));
     }
     return BH_OK;

@@ -252,7 +252,9 @@ int bh_order_by_cost(void* ctx, const float* cost, int32_t* order, void* stream)
 int bh_learned_order(void* ctx, const float* params, int32_t* order, void* stream);
 
 /* Context sizes: what = 0 particles, 1 cells, 2 systems, 3 columns,
- * 4 work-item capacity, 5 compute units. */
+ * 4 work-item capacity, 5 compute units; the grouped far field of FP64 (6) and
+ * FP32 (7) passes: Chebyshev nodes per side of a square, 0 where passes go term by
+ * term; and the cells per side of the first system's tiles (8 and 9; 0 likewise). */
 int bh_query(void* ctx, int32_t what, int64_t* out);
 
 /* Cloud-to-cloud direct gravity: the reference's gravity plugin
