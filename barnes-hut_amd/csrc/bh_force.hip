@@ -468,8 +468,8 @@ __global__ __launch_bounds__(64) void k_force64(ForceArgs A)
 // order.  A pass has N / 64 W waves instead of N / 128 and each a W-th of the
 // chain, so small passes fill the chip; the terms come by scalar loads, so
 // they cost neither LDS reads nor a staging round per tile.  A chunk is 64
-// consecutive sorted particles of one system: a particle's terms and their
-// order depend on its system alone.
+// consecutive sorted particles of one system: in passes of this form a particle's
+// terms and their order depend on its system alone.
 //
 // Near candidates: if the chunk lies in one column and spans two rows at most
 // (dense cells), its waves walk the union of the lanes' cells, four candidates

@@ -117,7 +117,13 @@ int bh_destroy(void* ctx);
  * holds n[s] >= 1 particles at rows [sum_{t<s} n[t], ...) and a
  * grid_dim[s]^2 grid, 1 <= grid_dim[s] <= 32767 (the FP32 COM list packs a
  * cell's column and row in 16 bits each; such a grid already needs ~170 B of
- * per-cell state, ~180 GB). (Re)allocates the context's scratch. */
+ * per-cell state, ~180 GB). (Re)allocates the context's scratch.
+ * Systems do not act on each other, and a pass takes one form for all of them:
+ * far terms grouped or one by one, FP32 work shared by chunks or taken from a
+ * queue.  The form follows from the far terms of all systems together and, for
+ * grouping, from free memory (bh_query 6 and 7).  A system's accelerations are
+ * the same bit for bit in any company under one form, and to rounding (the
+ * forms' accuracy, see the precisions) under another. */
 int bh_set_systems(void* ctx, int32_t nsys, const int64_t* n, const int32_t* grid_dim);
 int bh_set_tuning(void* ctx, const bh_tuning* t);
 int bh_get_tuning(void* ctx, bh_tuning* t);
