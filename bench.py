@@ -30,15 +30,15 @@ per-cell COM, forces, tick.  Paths on the same input:
     refinement (within about one ulp of the quotient);
   * the same with the IEEE division per weight (`fp64_ieee`, secondary);
   * the FP32 precision, static order: at this size its pass is grouped and in
-    FP64, to a remainder of 1e-9 (term by term, below 2e10 far terms, it is FP32
+    FP64, to a remainder of 1e-10 (term by term, below 2e10 far terms, it is FP32
     cell-relative forces with FP64 tile sums);
   * the same with the learned work-queue order (the cost model in
     barnes-hut_amd/costmodels/clusters256.npz; --cost-model none disables), which
     is formed but orders nothing where the pass is grouped.
-Term-by-term FP32 paths include the FP64 recompute of the particles whose FP32
-terms nearly cancel (kappa 1.5, --recompute-kappa 0 disables), timed apart from
-the force kernel; a grouped pass has none.  `value` is the FP32 + learned-order path's whole-job
-throughput.
+FP32 paths include the FP64 recompute of the particles whose terms nearly cancel
+(kappa 1.5, --recompute-kappa 0 disables): of a term-by-term pass timed apart
+from the force kernel, of a grouped one within it.  `value` is the FP32 +
+learned-order path's whole-job throughput.
 
 Secondary blocks (not in `value`): the cost-model workload (256 clusters,
 sigma [0.001, 0.03], lognormal masses, 1024^2: FP64, FP32 static, FP32
@@ -85,9 +85,9 @@ FLOP_PER_INTERACTION = 11
 # arithmetic, 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz.
 LANE_OPS = 256 * 4 * 16 * 2.4e9
 ISSUE_CEILING64_TFLOPS = LANE_OPS / 11 * FLOP_PER_INTERACTION / 1e12
-# From these many far terms a pass groups its far field (library rule), in all
-# precisions in FP64 (see grouped_work)
-GROUPED_TERMS = {"fp64": 2e9, "fp32": 2e10}
+# Nodes per square side that a grouped pass uses between squares further apart,
+# by its nodes per side
+FAR_NODES = {20: 16, 12: 10}
 # FP64 recompute threshold of the FP32 paths (--recompute-kappa)
 RECOMPUTE_KAPPA = 1.5
 
@@ -149,18 +149,14 @@ def run_path(eng, d, precision, steps, warmup, order_fn=None, kappa=RECOMPUTE_KA
     return (t1 - t0) / steps, kms, rms, near, far
 
 
-def grouped_work(counts, precision):
-    """FP64 operations of a grouped pass over G x G cells with these counts: near
-    and mid terms one by one (11 each), and per square with particles the products
-    of the nodes' masses with the law between nodes (2 components, a multiply and an
-    add each; 12 offsets at P^2 x P^2 nodes, 15 at F^2 x F^2).  None where the pass
-    is not grouped."""
+def grouped_work(counts, P, T):
+    """FP64 operations of a grouped pass over G x G cells with these counts, tiles of
+    T cells a side and P nodes a side: near and mid terms one by one (11 each), and
+    per square with particles the products of the nodes' masses with the law between
+    nodes (2 components, a multiply and an add each; 12 offsets at P^2 x P^2 nodes,
+    15 at F^2 x F^2).  The FP64 recompute's terms are not among them."""
     G = counts.shape[0]
-    n, ne = int(counts.sum()), int((counts > 0).sum())
-    if precision not in GROUPED_TERMS or n * min(n, ne) < GROUPED_TERMS[precision]:
-        return None
-    P, F, c = (20, 16, 130000.0) if precision == "fp64" else (12, 10, 22000.0)
-    T = min(max(round((c * G * G / n) ** 0.25), 4), 24)   # cells per tile side
+    n, F = int(counts.sum()), FAR_NODES[P]
     nt = -(-G // T)
 
     def around(a):   # sums over 3 x 3
@@ -209,8 +205,11 @@ def measure(d, G, precision, tuning, steps, warmup, model=None, kappa=RECOMPUTE_
             return order_buf
     sec, kms, rms, near, far = run_path(eng, d, precision, steps, warmup, order_fn, kappa)
     st = eng.ctx.stats()
-    n_items, n_rc = int(st[2]), int(st[6])
-    grouped = grouped_work(eng.counts().reshape(G, G).astype(np.int64), precision)
+    n_items, n_rc = int(st[2]), int(st[6]) + int(st[8])
+    # the pass's form, as the library chose it: nodes and cells per tile side
+    q = {"fp64": 6, "fp32": 7}.get(precision)
+    P, T = (eng.ctx.query(q), eng.ctx.query(q + 2)) if q else (0, 0)
+    grouped = grouped_work(eng.counts().reshape(G, G).astype(np.int64), P, T) if P else None
     eng.close()
     inter = (near + far).astype(np.float64)
     flops = FLOP_PER_INTERACTION * inter if grouped is None else np.full(steps, grouped["flop"])
@@ -261,7 +260,8 @@ def force_errors(d, G, runs, kappa=RECOMPUTE_KAPPA):
                          p99=float(np.quantile(per, 0.99)), max=float(per.max()),
                          n_over_1e5=int((per > 1e-5).sum()))
         if kap > 0 and not prec.startswith("fp64"):
-            out[name]["recomputed"] = int(eng.ctx.stats()[6])
+            st = eng.ctx.stats()
+            out[name]["recomputed"] = int(st[6]) + int(st[8])
     eng.check()
     eng.close()
     return out
@@ -419,7 +419,8 @@ def batched_line(steps, model_path, seed=0):
                            tuning="auto", autotune_candidates=BATCHED_CANDIDATES)
         out["tuning"] = b.tune_result["tuning"]
         sec = b.run(steps, warmup=1)
-        out["recomputed_last_step"] = int(b.eng.ctx.stats()[6])
+        st = b.eng.ctx.stats()
+        out["recomputed_last_step"] = int(st[6]) + int(st[8])
         inter = b.eng.interactions()[-1].astype(np.float64)    # placement of the last step
         out[name] = {"ms_per_step": sec * 1e3, "value": float(sizes.sum()) / sec / 1e6,
                      "interactions_last_step": float(inter.sum()),

@@ -63,3 +63,20 @@ def test_a_system_and_its_copies(n, G, prec, same):
     print(f"[rule] {n} {G} {prec}: {norm:.2e}, max {(num / den).max():.2e}", flush=True)
     assert 0 < norm <= (NORM["fp64"] if prec == "fp64" else 1e-6)   # fp32 by terms: 4e-8
     assert (num / den).max() <= EACH[prec]
+
+
+@pytest.mark.parametrize("n,G,prec,tile", [
+    (262144, 256, "fp64", None), (262145, 256, "fp64", 13),
+    (600001, 193, "fp32", 6), (600001, 193, "fp64", 9)])   # (c G^2 / n)^(1/4): 6.08, 9.48
+def test_benchmark_counts_the_form_that_ran(n, G, prec, tile):
+    """The benchmark's accounting of a pass follows the library's form, on
+    clusters too, where few cells hold particles."""
+    import bench
+    d = inputs.gaussian_mixture(n, 8, (0.005, 0.03), seed=86)
+    r = bench.measure(d, G, prec, None, 1, 0)
+    if tile is None:
+        assert r["grouped"] is None
+        assert r["flop_per_launch"] == bench.FLOP_PER_INTERACTION * (r["near"][0] + r["far"][0])
+    else:
+        assert r["grouped"]["tile_side"] == tile
+        assert r["grouped"]["near_terms"] == r["near"][0]
