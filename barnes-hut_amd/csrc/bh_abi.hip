@@ -231,11 +231,14 @@ static void set_sizes(Ctx* c, int32_t nsys, int64_t N, int64_t C, int64_t cols, 
 // so they meet at the line.  The allocation-free step has no scratch for the
 // squares and gives the bits of bh_step, so single systems within its limits
 // stay term by term (at most 1.7e10 terms, 6 ms).
-// fp32: at 2.2e10 terms (600,001 particles, 193^2 cells) 4.5 and 1.1 ms.  The
-// line is above the crossing because short FP32 passes over many uneven
-// systems are where a learned queue order shortens the pass (it orders work
-// items, which grouped passes do not have), and because the recompute, whose
-// flags callers read, belongs to the term-by-term pass.
+// fp32: 600,001 particles on 182^2 cells (1.99e10 terms) take 4.18 (uniform) and
+// 4.14 ms (16 clusters) term by term, on 183^2 0.71 and 3.56 grouped, each with
+// the recompute.  The line is above the crossing because short FP32 passes over
+// many uneven systems are where a learned queue order shortens the pass (it orders
+// work items, which grouped passes do not have), and because callers that defer
+// the recompute or read its count (stats [6]) find both in the term-by-term pass
+// only.  Grouped FP32 passes with P = 20 instead of the recompute were 6.0 against
+// 5.6 ms (4.2M clustered on 1024^2), 25.5 against 15.7 (512 systems).
 static constexpr double FP32_SHARED_TERMS = 4e9;
 static constexpr double FMM_MIN_TERMS_FP64 = 2e9;
 static constexpr double FMM_MIN_TERMS_FP32 = 2e10;

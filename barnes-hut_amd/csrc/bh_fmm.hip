@@ -749,7 +749,8 @@ __device__ __forceinline__ void near_range(const FmmArgs& A, int64_t coff, int G
 // vector loads (a union would spend most of its terms on the test).  Terms go in
 // quads, or a lane's own in pairs, that share a reciprocal; only quads that hold
 // the lanes themselves are tested for the particle itself.  SQ: r2 is the sum of
-// the near terms' (m / r)^2, r in cell sides, for the FP64 recompute's bound.
+// the near terms' (m / r)^2, r in cell sides, for the FP64 recompute's bound: 2 to 3
+// % (4.2M FP32 particles over 1024^2 cells 2.14 -> 2.20 ms, 512 systems 7.14 -> 7.27).
 template <int P, int LAW, bool SQ>
 __device__ __forceinline__ void chunk_terms(const FmmArgs& A, int ci, int w, int W, double eps2p,
                                             double r2cutp, int& gi, double& rx, double& ry,

@@ -35,7 +35,7 @@
 // Where no run of pitem particles reaches the row span, those are the column's
 // items, found a lane each.  Else the wave goes from item to item, the row of a
 // particle found by 64 lanes at a time.  The two passes, and with a walk of the
-// column's rows: 700k particles on 750^2 cells 13 us, 95; 4.2M in clusters on
+// column's rows: 700k particles on 601^2 cells 13 us, 95; 4.2M in clusters on
 // 1024^2 39 us, 181; 512 systems 36 us, 220.
 
 // The row of a column that particle p lies in: the last with o[y] <= p, o[0 .. G].
