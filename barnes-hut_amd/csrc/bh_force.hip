@@ -483,6 +483,8 @@ __global__ __launch_bounds__(64) void k_force64(ForceArgs A)
 // candidates of a cell exceed an XCD's L2, a third.  W = 4 and 16 are within
 // 10 % of W = 8 from 65k particles on and slower below (W = 4: 29 against 24 us
 // at 16,384) or above (W = 16).
+// At most 80 registers, so that three blocks share a CU: with 81 under a cutoff,
+// 184,442 particles on 46^2 cells took 438 instead of 393 us.
 typedef double fd4a __attribute__((ext_vector_type(4), aligned(8)));
 
 struct Four {   // four candidates in scalar registers
@@ -558,9 +560,10 @@ __device__ __forceinline__ void near_cell(const ForceArgs& A, int j, int b, int 
 }
 
 template <int W, int LAW>
-__global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
+__global__ __launch_bounds__(64 * W, 6) void k_force64s(ForceArgs A, int S)
 {
     __shared__ double part[2][W][BH_WAVE];
+    __shared__ int bad[W];
     const int lane = threadIdx.x & 63, w = uniform_int(threadIdx.x >> 6);
     const int64_t ci = A.chunk0 + blockIdx.x;
     int s = 0;
@@ -691,7 +694,14 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
             q = qn;
         }
     }
-    if (__syncthreads_or(!is_finite(sx, sy))) {   // one by one (see one_term)
+    part[0][w][lane] = sx;
+    part[1][w][lane] = sy;
+    if (lane == 0) bad[w] = 0;
+    if (!is_finite(sx, sy)) bad[w] = 1;
+    __syncthreads();
+    // one by one, by all waves of the block (see one_term); told by a word a wave
+    // beside the sums, since a barrier of its own costs 1 % of a short block
+    if (__any(bad[lane & (W - 1)])) {
         sx = sy = 0.0;
         for (int xc = max(cx - 1, 0); act && xc <= min(cx + 1, G - 1); ++xc) {
             const int64_t cl = coff + (int64_t)xc * G;
@@ -707,10 +717,10 @@ __global__ __launch_bounds__(64 * W) void k_force64s(ForceArgs A, int S)
             one_term<LAW>(fma(f.X, sig, -x), fma(f.Y, sig, -y), f.M,
                           abs(f.kx - cx) > 1 || abs(f.ky - cy) > 1, eps2, r2cut, sx, sy);
         }
+        part[0][w][lane] = sx;
+        part[1][w][lane] = sy;
+        __syncthreads();
     }
-    part[0][w][lane] = sx;
-    part[1][w][lane] = sy;
-    __syncthreads();
     if (w < 2 && act) {   // wave 0 adds x, wave 1 adds y
         double t = 0.0;
 #pragma unroll
